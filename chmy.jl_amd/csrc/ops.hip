@@ -1,5 +1,5 @@
-// Per-point Launcher kernels: generic GridOperators, diffusion, update_old!,
-// thermal flux/update and the viscosity max-neighbourhood.  Each thread owns
+// Per-point Launcher kernels: diffusion, update_old!, thermal flux/update and
+// the viscosity max-neighbourhood.  Each thread owns
 // one logical index I of the box; blocks are one wave64 wide along x (the
 // contiguous dim) so loads and stores coalesce.  These are bandwidth-bound
 // streaming kernels; the fused Stokes iteration lives in stokes.hip.
@@ -29,211 +29,6 @@ __device__ __forceinline__ Ix3 sh(Ix3 I, int d, int64_t s) {
     if (d == 0) I.i += s; else if (d == 1) I.j += s; else I.k += s;
     return I;
 }
-// il/ir of an operator on a field at its own location (GridOperators.jl:23-36)
-template <class T>
-__device__ __forceinline__ T leftv(const DFL<T>& f, int D, Ix3 I) { return f.loc[D] == 0 ? g_at(f, sh(I, D, -1)) : g_at(f, I); }
-template <class T>
-__device__ __forceinline__ T rightv(const DFL<T>& f, int D, Ix3 I) { return f.loc[D] == 0 ? g_at(f, I) : g_at(f, sh(I, D, 1)); }
-template <class T>
-__device__ __forceinline__ T ddv(const DFL<T>& f, T isp, int D, Ix3 I) { return (rightv(f, D, I) - leftv(f, D, I)) * isp; }
-
-// lerp (interpolation.jl:14-94): knots over the differing dims, reduced with
-// fma(0.5, b-a, a) from the first differing dim (innermost) to the last.
-template <class T>
-__device__ T lerpv(const DFL<T>& f, const int32_t* to, Ix3 I) {
-    int dims[3], m = 0;
-    for (int d = 0; d < f.nd; ++d)
-        if (f.loc[d] != to[d]) dims[m++] = d;
-    T v[8];
-    for (int q = 0; q < (1 << m); ++q) {
-        Ix3 J = I;
-        for (int b = 0; b < m; ++b) {
-            int D = dims[b];
-            bool right = (q >> b) & 1;
-            // Center->Vertex knots (I-e, I); Vertex->Center knots (I, I+e)
-            int64_t s = f.loc[D] == 0 ? (right ? 0 : -1) : (right ? 1 : 0);
-            J = sh(J, D, s);
-        }
-        v[q] = g_at(f, J);
-    }
-    for (int b = 0; b < m; ++b) {
-        int half = 1 << (m - b - 1);
-        for (int q = 0; q < half; ++q) {
-            T a = v[2 * q], c = v[2 * q + 1];
-            v[q] = fma(T(0.5), c - a, a);
-        }
-    }
-    return v[0];
-}
-
-struct OpArgs {
-    int op, nd, D, nsrc;
-};
-
-template <class T>
-__global__ void __launch_bounds__(256) op_kernel(Box3 b, DFL<T> dst, DFL<T> s0, DFL<T> s1, DFL<T> s2, OpArgs a,
-                                                 T isp0, T isp1, T isp2) {
-    bool ok;
-    Ix3 I = box_index(b, ok);
-    if (!ok) return;
-    const DFL<T>* s[3] = {&s0, &s1, &s2};
-    const T isp[3] = {isp0, isp1, isp2};
-    T v = T(0);
-    switch (a.op) {
-        case CHMY_OP_PARTIAL: v = ddv(s0, isp[a.D], a.D, I); break;
-        case CHMY_OP_LERP: v = lerpv(s0, dst.loc, I); break;
-        case CHMY_OP_DIVG: {
-            v = ddv(*s[0], isp[0], 0, I);
-            for (int d = 1; d < a.nd; ++d) v = v + ddv(*s[d], isp[d], d, I);
-        } break;
-        case CHMY_OP_VMAG: {
-            const int32_t c[3] = {0, 0, 0};
-            T x = lerpv(*s[0], c, I);
-            T acc = x * x;
-            for (int d = 1; d < a.nd; ++d) { T y = lerpv(*s[d], c, I); acc = acc + y * y; }
-            v = sqrt(acc);
-        } break;
-        case CHMY_OP_LEFT: v = leftv(s0, a.D, I); break;
-        case CHMY_OP_RIGHT: v = rightv(s0, a.D, I); break;
-    }
-    g_at(dst, I) = v;
-}
-
-// ------------------------------------------------------------------ masked and second-order operators
-// Masked forms (masked_operators.jl:11-39): left/right multiply the knot
-// value by the mask at the field's own location at that knot,
-// left(f, ω)[I] = f[Il]·ω[Il]; with M = false the plain forms, bitwise those
-// of leftv/rightv/ddv.  ∂² and ∂k∂ (partial_derivatives.jl:7-21) take
-// differences of ∂ at the two knots of the flipped location; ∂k∂ weights
-// them with lerp(k) at those knots (the coefficient is never masked).
-//
-// On a FunctionAxis (NU, non-NULL table along the dim) the metrics are the
-// reference's: ∂ scales δ by iΔ(grid, loc(f), dim, I) (partial_derivatives.jl:5,
-// field_operators.jl:20-24: the source field's location, at the output
-// index), ∂² and ∂k∂ their difference by iΔ(loc(f), I) (:7-21), and the
-// Center -> Vertex lerp weight at vertex i is 0.5 Δc(i-1) iΔv(i)
-// (interpolation.jl:29); Vertex -> Center stays 0.5 (:28).
-__device__ __forceinline__ int64_t ix_of(Ix3 I, int D) { return D == 0 ? I.i : D == 1 ? I.j : I.k; }
-
-template <class T, bool NU>
-__device__ __forceinline__ T isp_at(const Axes3& ax, const T* isp, int D, int loc, Ix3 I) {
-    if (!NU || !ax.a[D].p) return isp[D];
-    return T(ax.a[D].at(loc == 0 ? CHMY_AX_IDC : CHMY_AX_IDV, ix_of(I, D)));
-}
-
-template <class T, bool M>
-__device__ __forceinline__ T knot(const DFL<T>& f, const DFL<T>& w, Ix3 J) {
-    const T v = g_at(f, J);
-    return M ? v * g_at(w, J) : v;
-}
-template <class T, bool M>
-__device__ __forceinline__ T leftk(const DFL<T>& f, const DFL<T>& w, int D, Ix3 I) {
-    return knot<T, M>(f, w, f.loc[D] == 0 ? sh(I, D, -1) : I);
-}
-template <class T, bool M>
-__device__ __forceinline__ T rightk(const DFL<T>& f, const DFL<T>& w, int D, Ix3 I) {
-    return knot<T, M>(f, w, f.loc[D] == 0 ? I : sh(I, D, 1));
-}
-template <class T, bool M, bool NU>
-__device__ __forceinline__ T ddk(const DFL<T>& f, const DFL<T>& w, const Axes3& ax, const T* isp, int D, Ix3 I) {
-    return (rightk<T, M>(f, w, D, I) - leftk<T, M>(f, w, D, I)) * isp_at<T, NU>(ax, isp, D, f.loc[D], I);
-}
-// knots of the flipped location around I: Center f -> (I, I+e), Vertex f -> (I-e, I)
-__device__ __forceinline__ void flip_knots(int loc, int D, Ix3 I, Ix3& Il, Ix3& Ir) {
-    Il = loc == 0 ? I : sh(I, D, -1);
-    Ir = loc == 0 ? sh(I, D, 1) : I;
-}
-// lerp and hlerp with the weights of the axis (HARM: the harmonic rule
-// inv(muladd(t, inv(b) - inv(a), inv(a))), interpolation.jl:15,101); knots
-// over the differing dims, first differing dim innermost
-template <class T, bool NU, bool HARM>
-__device__ T itpw(const DFL<T>& f, const int32_t* to, const Axes3& ax, Ix3 I) {
-    int dims[3], m = 0;
-    for (int d = 0; d < f.nd; ++d)
-        if (f.loc[d] != to[d]) dims[m++] = d;
-    T v[8];
-    for (int q = 0; q < (1 << m); ++q) {
-        Ix3 J = I;
-        for (int b = 0; b < m; ++b) {
-            int D = dims[b];
-            bool right = (q >> b) & 1;
-            int64_t s = f.loc[D] == 0 ? (right ? 0 : -1) : (right ? 1 : 0);
-            J = sh(J, D, s);
-        }
-        v[q] = g_at(f, J);
-    }
-    for (int b = 0; b < m; ++b) {
-        const int D = dims[b];
-        const T t = (NU && ax.a[D].p && f.loc[D] == 0) ? T(ax.a[D].at(CHMY_AX_WCV, ix_of(I, D))) : T(0.5);
-        int half = 1 << (m - b - 1);
-        for (int q = 0; q < half; ++q) {
-            T a = v[2 * q], c = v[2 * q + 1];
-            v[q] = HARM ? T(1) / fma(t, T(1) / c - T(1) / a, T(1) / a) : fma(t, c - a, a);
-        }
-    }
-    return v[0];
-}
-template <class T, bool M, bool NU>
-__device__ T d2k(const DFL<T>& f, const DFL<T>& w, const Axes3& ax, const T* isp, int D, Ix3 I) {
-    Ix3 Il, Ir;
-    flip_knots(f.loc[D], D, I, Il, Ir);
-    return (ddk<T, M, NU>(f, w, ax, isp, D, Ir) - ddk<T, M, NU>(f, w, ax, isp, D, Il)) *
-           isp_at<T, NU>(ax, isp, D, f.loc[D], I);
-}
-template <class T, bool M, bool NU>
-__device__ T dkdk(const DFL<T>& f, const DFL<T>& w, const DFL<T>& k, const Axes3& ax, const T* isp, int D, Ix3 I) {
-    Ix3 Il, Ir;
-    flip_knots(f.loc[D], D, I, Il, Ir);
-    int32_t floc[3] = {f.loc[0], f.loc[1], f.loc[2]};
-    floc[D] = 1 - floc[D];
-    return (itpw<T, NU, false>(k, floc, ax, Ir) * ddk<T, M, NU>(f, w, ax, isp, D, Ir) -
-            itpw<T, NU, false>(k, floc, ax, Il) * ddk<T, M, NU>(f, w, ax, isp, D, Il)) *
-           isp_at<T, NU>(ax, isp, D, f.loc[D], I);
-}
-
-template <class T, bool M, bool NU>
-__global__ void __launch_bounds__(256) op_ext_kernel(Box3 b, DFL<T> dst, DFL<T> s0, DFL<T> s1, DFL<T> s2, DFL<T> w0,
-                                                     DFL<T> w1, DFL<T> w2, DFL<T> k, OpArgs a, T isp0, T isp1,
-                                                     T isp2, Axes3 ax) {
-    bool ok;
-    Ix3 I = box_index(b, ok);
-    if (!ok) return;
-    const DFL<T>* s[3] = {&s0, &s1, &s2};
-    const DFL<T>* w[3] = {&w0, &w1, &w2};
-    const T isp[3] = {isp0, isp1, isp2};
-    T v = T(0);
-    switch (a.op) {
-        case CHMY_OP_PARTIAL: v = ddk<T, M, NU>(s0, w0, ax, isp, a.D, I); break;
-        case CHMY_OP_DELTA: v = rightk<T, M>(s0, w0, a.D, I) - leftk<T, M>(s0, w0, a.D, I); break;
-        case CHMY_OP_LEFT: v = leftk<T, M>(s0, w0, a.D, I); break;
-        case CHMY_OP_RIGHT: v = rightk<T, M>(s0, w0, a.D, I); break;
-        case CHMY_OP_DIVG: {
-            v = ddk<T, M, NU>(*s[0], *w[0], ax, isp, 0, I);
-            for (int d = 1; d < a.nd; ++d) v = v + ddk<T, M, NU>(*s[d], *w[d], ax, isp, d, I);
-        } break;
-        case CHMY_OP_D2: v = d2k<T, M, NU>(s0, w0, ax, isp, a.D, I); break;
-        case CHMY_OP_DKD: v = dkdk<T, M, NU>(s0, w0, k, ax, isp, a.D, I); break;
-        case CHMY_OP_LAPL: {
-            v = d2k<T, M, NU>(s0, w0, ax, isp, 0, I);
-            for (int d = 1; d < a.nd; ++d) v = v + d2k<T, M, NU>(s0, w0, ax, isp, d, I);
-        } break;
-        case CHMY_OP_DIVG_GRAD: {
-            v = dkdk<T, M, NU>(s0, w0, k, ax, isp, 0, I);
-            for (int d = 1; d < a.nd; ++d) v = v + dkdk<T, M, NU>(s0, w0, k, ax, isp, d, I);
-        } break;
-        case CHMY_OP_LERP: v = itpw<T, NU, false>(s0, dst.loc, ax, I); break;
-        case CHMY_OP_HLERP: v = itpw<T, NU, true>(s0, dst.loc, ax, I); break;
-        case CHMY_OP_VMAG: {
-            const int32_t c[3] = {0, 0, 0};
-            T x = itpw<T, NU, false>(*s[0], c, ax, I);
-            T acc = x * x;
-            for (int d = 1; d < a.nd; ++d) { T y = itpw<T, NU, false>(*s[d], c, ax, I); acc = acc + y * y; }
-            v = sqrt(acc);
-        } break;
-    }
-    g_at(dst, I) = v;
-}
-
 // ------------------------------------------------------------------ diffusion
 template <class T>
 __global__ void __launch_bounds__(256) diffusion_flux_kernel(Box3 b, DFL<T> C, DFL<T> q0, DFL<T> q1, DFL<T> q2,
@@ -537,11 +332,6 @@ __global__ void __launch_bounds__(256) maxloc_kernel(Box3 b, DFL<T> dst, DFL<T> 
 }
 
 // ------------------------------------------------------------------ host side
-template <class T>
-DFL<T> lv_or(const chmy_field_t* f, const DFL<T>& fallback) {
-    return f ? lview<T>(*f) : fallback;
-}
-
 static dim3 blk2() { return dim3(kBX, kBY, 1); }
 
 template <class T>
@@ -606,120 +396,6 @@ static int thermal_launch(const chmy_grid_t* g, const chmy_box_t& bx, const chmy
 using namespace chmy;
 
 extern "C" {
-
-int chmy_op(int op, const chmy_grid_t* g, const chmy_box_t* box, const chmy_field_t* dst, int nsrc,
-            const chmy_field_t* src, int dim, void* stream) {
-    CHMY_TRY(check_grid_any(g));
-    if (nonuniform(g)) return chmy_op_masked(op, g, box, dst, nsrc, src, nullptr, nullptr, dim, stream);
-    chmy_box_t bx;
-    CHMY_TRY(check_box(g, box, &bx));
-    CHMY_TRY(check_field(g, dst, "dst", nullptr, -1));
-    const int dt = dst->dtype;
-    const bool vec = op == CHMY_OP_DIVG || op == CHMY_OP_VMAG;
-    if (vec && nsrc != g->nd) return set_error(CHMY_E_ARG, "divg/vmag need nd source fields");
-    if (!vec && nsrc != 1) return set_error(CHMY_E_ARG, "operator needs one source field");
-    if (!src) return set_error(CHMY_E_ARG, "src is NULL");
-    if (op != CHMY_OP_PARTIAL && op != CHMY_OP_LERP && op != CHMY_OP_DIVG && op != CHMY_OP_VMAG &&
-        op != CHMY_OP_LEFT && op != CHMY_OP_RIGHT)
-        return set_error(CHMY_E_ARG, "unknown operator %d", op);
-    if ((op == CHMY_OP_PARTIAL || op == CHMY_OP_LEFT || op == CHMY_OP_RIGHT) && (dim < 0 || dim >= g->nd))
-        return set_error(CHMY_E_ARG, "dim %d out of range", dim);
-    for (int q = 0; q < nsrc; ++q) {
-        const int* want = nullptr;
-        int loc[3];
-        if (op == CHMY_OP_DIVG || op == CHMY_OP_VMAG) {
-            for (int d = 0; d < 3; ++d) loc[d] = d == q ? 1 : 0;
-            want = loc;
-        }
-        CHMY_TRY(check_field(g, &src[q], "src", want, dt));
-    }
-    Box3 b = box3(bx, g->nd);
-    if (no_work(b)) return 0;
-    OpArgs a{op, g->nd, dim, nsrc};
-    hipStream_t s = (hipStream_t)stream;
-    dim3 grd = grid_for(b, blk2());
-    if (dt == CHMY_F64) {
-        DFL<double> d = lview<double>(*dst), s0 = lview<double>(src[0]);
-        DFL<double> s1 = nsrc > 1 ? lview<double>(src[1]) : s0, s2 = nsrc > 2 ? lview<double>(src[2]) : s0;
-        hipLaunchKernelGGL(op_kernel<double>, grd, blk2(), 0, s, b, d, s0, s1, s2, a, g->inv_spacing[0],
-                           g->inv_spacing[1], g->inv_spacing[2]);
-    } else {
-        DFL<float> d = lview<float>(*dst), s0 = lview<float>(src[0]);
-        DFL<float> s1 = nsrc > 1 ? lview<float>(src[1]) : s0, s2 = nsrc > 2 ? lview<float>(src[2]) : s0;
-        hipLaunchKernelGGL(op_kernel<float>, grd, blk2(), 0, s, b, d, s0, s1, s2, a, (float)g->inv_spacing[0],
-                           (float)g->inv_spacing[1], (float)g->inv_spacing[2]);
-    }
-    CHMY_HIP(hipGetLastError());
-    return 0;
-}
-
-int chmy_op_masked(int op, const chmy_grid_t* g, const chmy_box_t* box, const chmy_field_t* dst, int nsrc,
-                   const chmy_field_t* src, const chmy_field_t* masks, const chmy_field_t* k, int dim, void* stream) {
-    CHMY_TRY(check_grid_any(g));
-    chmy_box_t bx;
-    CHMY_TRY(check_box(g, box, &bx));
-    CHMY_TRY(check_field(g, dst, "dst", nullptr, -1));
-    const int dt = dst->dtype;
-    const bool vec = op == CHMY_OP_DIVG || op == CHMY_OP_VMAG;
-    const bool per_dim = op == CHMY_OP_PARTIAL || op == CHMY_OP_DELTA || op == CHMY_OP_LEFT || op == CHMY_OP_RIGHT ||
-                         op == CHMY_OP_D2 || op == CHMY_OP_DKD;
-    const bool known = per_dim || vec || op == CHMY_OP_LERP || op == CHMY_OP_HLERP || op == CHMY_OP_LAPL ||
-                       op == CHMY_OP_DIVG_GRAD;
-    if (!known) return set_error(CHMY_E_ARG, "unknown operator %d", op);
-    const bool maskable = op != CHMY_OP_LERP && op != CHMY_OP_HLERP && op != CHMY_OP_VMAG;
-    const bool needs_k = op == CHMY_OP_DKD || op == CHMY_OP_DIVG_GRAD;
-    if (vec && nsrc != g->nd) return set_error(CHMY_E_ARG, "divg/vmag need nd source fields");
-    if (!vec && nsrc != 1) return set_error(CHMY_E_ARG, "operator needs one source field");
-    if (!src) return set_error(CHMY_E_ARG, "src is NULL");
-    if (per_dim && (dim < 0 || dim >= g->nd)) return set_error(CHMY_E_ARG, "dim %d out of range", dim);
-    if (masks && !maskable) return set_error(CHMY_E_ARG, "operator %d has no masked form", op);
-    if (needs_k != (k != nullptr)) return set_error(CHMY_E_ARG, needs_k ? "k is NULL" : "k is given to an operator without a coefficient");
-    for (int q = 0; q < nsrc; ++q) {
-        const int* want = nullptr;
-        int loc[3];
-        if (vec) {
-            for (int d = 0; d < 3; ++d) loc[d] = d == q ? 1 : 0;
-            want = loc;
-        }
-        CHMY_TRY(check_field(g, &src[q], "src", want, dt));
-        // the mask component read with src[q] is the one at src[q]'s location
-        if (masks) CHMY_TRY(check_field(g, &masks[q], "mask", src[q].loc, dt));
-    }
-    if (k) CHMY_TRY(check_field(g, k, "k", nullptr, dt));
-    Box3 b = box3(bx, g->nd);
-    if (no_work(b)) return 0;
-    OpArgs a{op, g->nd, dim, nsrc};
-    hipStream_t s = (hipStream_t)stream;
-    dim3 grd = grid_for(b, blk2());
-    auto run = [&](auto tag) {
-        using T = decltype(tag);
-        DFL<T> d = lview<T>(*dst), s0 = lview<T>(src[0]);
-        DFL<T> s1 = nsrc > 1 ? lview<T>(src[1]) : s0, s2 = nsrc > 2 ? lview<T>(src[2]) : s0;
-        DFL<T> w0 = masks ? lview<T>(masks[0]) : s0;
-        DFL<T> w1 = masks && nsrc > 1 ? lview<T>(masks[1]) : w0, w2 = masks && nsrc > 2 ? lview<T>(masks[2]) : w0;
-        DFL<T> kk = k ? lview<T>(*k) : s0;
-        const T i0 = (T)g->inv_spacing[0], i1 = (T)g->inv_spacing[1], i2 = (T)g->inv_spacing[2];
-        const Axes3 ax = axes_of(g);
-        if (nonuniform(g)) {
-            if (masks)
-                hipLaunchKernelGGL((op_ext_kernel<T, true, true>), grd, blk2(), 0, s, b, d, s0, s1, s2, w0, w1, w2, kk, a,
-                                   i0, i1, i2, ax);
-            else
-                hipLaunchKernelGGL((op_ext_kernel<T, false, true>), grd, blk2(), 0, s, b, d, s0, s1, s2, w0, w1, w2, kk, a,
-                                   i0, i1, i2, ax);
-        } else if (masks) {
-            hipLaunchKernelGGL((op_ext_kernel<T, true, false>), grd, blk2(), 0, s, b, d, s0, s1, s2, w0, w1, w2, kk, a,
-                               i0, i1, i2, ax);
-        } else {
-            hipLaunchKernelGGL((op_ext_kernel<T, false, false>), grd, blk2(), 0, s, b, d, s0, s1, s2, w0, w1, w2, kk, a,
-                               i0, i1, i2, ax);
-        }
-    };
-    if (dt == CHMY_F64) run(double{});
-    else run(float{});
-    CHMY_HIP(hipGetLastError());
-    return 0;
-}
 
 int chmy_diffusion_flux(const chmy_grid_t* g, const chmy_box_t* box, const chmy_field_t* q, const chmy_field_t* C,
                         double chi, void* stream) {

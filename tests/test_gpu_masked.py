@@ -178,3 +178,32 @@ def test_masked_argument_errors(arch):
     w32 = chmy.FieldMask(arch, g, dtype=torch.float32)
     with pytest.raises(chmy.ChmyError, match="dtype"):
         L(arch, g, (chmy.kernels.partial, (d_, s, w32, 0, g)))
+
+
+@pytest.mark.parametrize("dims", [(63, 2, 3), (64, 130, 165), (126, 131, 127), (62, 255, 62), (2047, 66, 0)])
+def test_operators_over_tiles_and_plane_chunks(arch, dims):
+    """Boxes that end inside, at and past the 64 x 4 tile and the chunks of
+    1, 2 and 4 planes, bitwise against the oracle: a first difference, an
+    interpolation, and the masked second differences (Center and Vertex
+    coefficient)."""
+    nd = 3 if dims[2] else 2
+    g = chmy.UniformGrid(origin=(-0.5,) * nd, extent=(1.0, 1.1, 1.2)[:nd], dims=dims[:nd])
+    og = ogrid(g)
+    rng = np.random.default_rng(81)
+    L, K, T, c, v = chmy.Launcher(arch, g), chmy.kernels, np.float64, (Cc(),) * nd, (Vv(),) * nd
+    s, hs = pair(arch, g, og, c, T, rng=rng)
+    w, hw = mask_pair(arch, g, og, T, rng, "fraction")
+    d_, hd = pair(arch, g, og, flipped(c, nd - 1), T, fill=0)
+    L(arch, g, (K.partial, (d_, s, nd - 1, g)))
+    O.op("partial", og, hd, hs, dim=nd - 1)
+    assert_same(d_, hd, "∂")
+    d_, hd = pair(arch, g, og, v, T, fill=0)
+    L(arch, g, (K.lerp, (d_, s, g)))
+    O.op("lerp", og, hd, hs)
+    assert_same(d_, hd, "lerp")
+    for kloc in (c, v):
+        k, hk = pair(arch, g, og, kloc, T, rng=rng, lo=0.5, hi=2.0)
+        d_, hd = pair(arch, g, og, c, T, fill=0)
+        L(arch, g, (K.divg_grad, (d_, s, k, w, g)))
+        O.op_masked("divg_grad", og, hd, hs, hw[codes(c)], k=hk)
+        assert_same(d_, hd, f"masked divg_grad, k at {codes(kloc)}")
