@@ -1,4 +1,5 @@
 // Runtime part of the C ABI: errors, device selection, memory, descriptor checks.
+#include <atomic>
 #include <cmath>
 #include <cstdarg>
 #include <cstring>
@@ -116,6 +117,18 @@ int check_tensor(const chmy_grid_t* g, const chmy_field_t* tau, const char* name
         CHMY_TRY(check_field(g, &tau[c], nm, loc, dtype, allow_bf16));
     }
     return 0;
+}
+
+int cu_count() {
+    static std::atomic<int> ncu[64];
+    int dev = 0;
+    if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) dev = 0;
+    int n = ncu[dev].load(std::memory_order_relaxed);
+    if (n == 0) {
+        if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n <= 0) n = 256;
+        ncu[dev].store(n, std::memory_order_relaxed);
+    }
+    return n;
 }
 
 }  // namespace chmy

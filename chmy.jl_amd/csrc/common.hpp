@@ -171,6 +171,9 @@ inline dim3 grid_for(const Box3& b, dim3 blk) {
                 (unsigned)((b.len[2] + blk.z - 1) / blk.z));
 }
 
+// Compute units of the current device, read once per device (api.hip).
+int cu_count();
+
 // Block id -> tile, so that the blocks an XCD receives (ids congruent mod 8,
 // dispatched round-robin over the 8 XCDs) form one contiguous run of tiles and
 // share halo rows in that XCD's L2.

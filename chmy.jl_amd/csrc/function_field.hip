@@ -10,6 +10,28 @@
 // kernel argument, so every wave runs the same operation at the same time
 // (the switch is uniform) and the only per-lane state is the register file.
 //
+// Before the launch the host lowers the program (plan_program):
+//  - constants become operands instead of operations;
+//  - a wave owns 64 x points of one row and marches a chunk of the last dim;
+//    operations that do not depend on the last dim (the x and y parts of a
+//    distance, say) run once per chunk, the others at every plane;
+//  - registers are assigned to slots by their last use.  8 or 16 slots are a
+//    vector in VGPRs addressed by a uniform index, so no register lives in
+//    memory (with one f64 per SSA register the file was 1 KB a lane of
+//    scratch, and that traffic was the time);
+//  - each operation runs on 4 (8 slots) or 2 (16 slots) planes at once, which
+//    shares its decoding and gives independent work to overlap.
+// Programs that need more slots keep the file in LDS; those, and the ones that
+// call sin, cos, tanh or pow, whose code is large, run one plane at a time.
+//  - sums, products, negations and squares become FMA with constant operands
+//    that give the same bits, so most operations take the first branch.
+// Bound by instruction issue: per operation and 4 planes about 65 vector and 83
+// scalar instructions (counters), most of them operand moves and decoding.
+// Measured, one launch, us, before -> now (register file in scratch, one
+// point a lane): 160x144x127 FP64, 42 operations with two exp 295 -> 64, 27
+// operations with one exp 188 -> 46, 11 operations with two loads 96 -> 32;
+// 255^3: 1503 -> 212, 980 -> 154, 689 -> 148.
+//
 // Continuous functions read the coordinates at the destination's location,
 // coord(grid, loc, I...) with the fma forms of uniform_axis.jl:18-19;
 // discrete ones read logical indices and other fields at constant index
@@ -19,6 +41,7 @@
 // so programs made of + - * / sqrt, comparisons and ifelse give the bits of
 // the same expressions evaluated on the host; exp, log, sin, cos, tanh and
 // pow are the device math library's and may differ from the host's by an ulp.
+#include <algorithm>
 #include <cmath>
 
 #include "common.hpp"
@@ -36,21 +59,23 @@ struct PSrc {
     int32_t esize;
 };
 
-struct PProg {
-    int32_t n, nd;
-    double o[3], h[3], ih[3];
-    Axes3 ax;            // FunctionAxis tables (p == nullptr: uniform dim)
-    chmy_pop_t op[kPMaxOps];
-    double k[kPMaxConst];
-    PSrc src[kPMaxSrc];
+// A lowered operation: operands are slots (>= 0) or constants (-1 - index),
+// or the fields of the leaf operations as in chmy_pop_t.
+struct PIns {
+    int16_t op, dst;
+    int32_t a, b, c;
 };
 
-__device__ __forceinline__ double load_src(const PSrc& s, int64_t i, int64_t j, int64_t k) {
-    const int64_t o = i * s.st[0] + j * s.st[1] + k * s.st[2];
-    if (s.dtype == CHMY_F64) return reinterpret_cast<const double*>(s.p)[o];
-    if (s.dtype == CHMY_F32) return (double)reinterpret_cast<const float*>(s.p)[o];
-    return (double)bf16_to_f32(reinterpret_cast<const uint16_t*>(s.p)[o]);
-}
+struct PProg {
+    int32_t npro, n;     // operations [0, npro) once per chunk, [npro, n) per plane
+    int32_t out;         // the stored value's operand
+    int32_t m;           // the marched dim (nd - 1; 2 in 1D, of length 1)
+    double o[3], h[3], ih[3];
+    Axes3 ax;            // FunctionAxis tables (p == nullptr: uniform dim)
+    PIns op[kPMaxOps + 1];   // (one past the end is read ahead)
+    double k[kPMaxConst + 3];   // the program's, then 1, -1 and -0.0
+    PSrc src[kPMaxSrc];
+};
 
 __host__ __device__ __forceinline__ int off8(int32_t packed, int d) { return (int)(int8_t)((packed >> (8 * d)) & 0xff); }
 
@@ -64,82 +89,169 @@ __device__ __forceinline__ double jl_max(double x, double y) {
     return (y > x || (!signbit(y) && signbit(x))) ? y : x;
 }
 
-template <class T>
-__global__ void __launch_bounds__(256) program_kernel(const PProg P, DF<T> dst, Box3 b) {
-    const int64_t i = b.lo[0] + (int64_t)blockIdx.x * 64 + threadIdx.x;
-    const int64_t j = b.lo[1] + (int64_t)blockIdx.y * 4 + threadIdx.y;
-    const int64_t k = b.lo[2] + blockIdx.z;
-    if (i >= b.lo[0] + b.len[0] || j >= b.lo[1] + b.len[1]) return;
-    const int64_t I[3] = {i, j, k};
-    double r[kPMaxOps];
-    for (int q = 0; q < P.n; ++q) {
-        const chmy_pop_t o = P.op[q];
-        double v = 0.0;
-        switch (o.op) {
-            case CHMY_P_CONST: v = P.k[o.a]; break;
-            case CHMY_P_INDEX: v = (double)(I[o.a] + o.b); break;
-            case CHMY_P_COORD: {
-                if (P.ax.a[o.a].p) {
-                    v = P.ax.a[o.a].at(o.b == CHMY_VERTEX ? CHMY_AX_VERTEX : CHMY_AX_CENTER, I[o.a] + o.c);
-                    break;
-                }
-                const double i1 = (double)(I[o.a] + o.c - 1);
+// The register file of one plane: a VGPR vector of S slots, or (S = 0) the
+// block's LDS, one f64 a lane and slot.
+typedef double slots8 __attribute__((ext_vector_type(8)));
+typedef double slots16 __attribute__((ext_vector_type(16)));
+extern __shared__ double slot_lds[];
+template <int S>
+struct Slots {
+    __device__ __forceinline__ double get(int s) const { return slot_lds[64 * s + threadIdx.x]; }
+    __device__ __forceinline__ void set(int s, double x) { slot_lds[64 * s + threadIdx.x] = x; }
+};
+template <>
+struct Slots<8> {
+    slots8 v;
+    __device__ __forceinline__ double get(int s) const { return v[s]; }
+    __device__ __forceinline__ void set(int s, double x) { v[s] = x; }
+};
+template <>
+struct Slots<16> {
+    slots16 v;
+    __device__ __forceinline__ double get(int s) const { return v[s]; }
+    __device__ __forceinline__ void set(int s, double x) { v[s] = x; }
+};
+
+// x^n as repeated products, left to right (Julia's literal powers x^2 = x*x,
+// x^3 = x*x*x; x^-1 = inv(x), x^-2 = inv(x)^2)
+__device__ __forceinline__ double powi(double r, int e) {
+    const double x = e < 0 ? 1.0 / r : r;
+    const int n = e < 0 ? -e : e;
+    double v = n == 0 ? 1.0 : x;
+    for (int q = 1; q < n; ++q) v = v * x;
+    return v;
+}
+
+template <int S, int N, bool HEAVY>
+__device__ __forceinline__ void program_run(const PProg& P, int q0, int q1, Slots<S>* r, const int64_t* I,
+                                            const int64_t* Im) {
+    PIns next = P.op[q0];
+    for (int q = q0; q < q1; ++q) {
+        const PIns o = next;
+        next = P.op[q + 1];   // in flight while this one runs
+        double v[N], x[N], y[N], z[N];
+        auto get = [&](int s, double* t) {
+            if (s >= 0) {
+#pragma unroll
+                for (int u = 0; u < N; ++u) t[u] = r[u].get(s);
+            } else {
+                const double k = P.k[-1 - s];
+#pragma unroll
+                for (int u = 0; u < N; ++u) t[u] = k;
+            }
+        };
+        // index of plane u along dim d
+        auto at = [&](int d, int u) -> int64_t { return d == P.m ? Im[u] : (d == 0 ? I[0] : d == 1 ? I[1] : I[2]); };
+#define CHMY_P_EACH(expr)                      \
+    do {                                       \
+        _Pragma("unroll") for (int u = 0; u < N; ++u) v[u] = (expr); \
+    } while (0)
+        // the operations that fill most programs first, each one branch away
+        if (o.op == CHMY_P_FMA) {
+            get(o.a, x);
+            get(o.b, y);
+            get(o.c, z);
+            CHMY_P_EACH(fma(x[u], y[u], z[u]));
+        } else if (o.op == CHMY_P_LOAD) {
+            const PSrc& s = P.src[o.a];
+            const int64_t off = off8(o.b, 0) * s.st[0] + off8(o.b, 1) * s.st[1] + off8(o.b, 2) * s.st[2];
+            int64_t w[N];
+#pragma unroll
+            for (int u = 0; u < N; ++u) w[u] = off + at(0, u) * s.st[0] + at(1, u) * s.st[1] + at(2, u) * s.st[2];
+            if (s.dtype == CHMY_F64) CHMY_P_EACH(reinterpret_cast<const double*>(s.p)[w[u]]);
+            else if (s.dtype == CHMY_F32) CHMY_P_EACH((double)reinterpret_cast<const float*>(s.p)[w[u]]);
+            else CHMY_P_EACH((double)bf16_to_f32(reinterpret_cast<const uint16_t*>(s.p)[w[u]]));
+        } else if (o.op == CHMY_P_SELECT) {
+            get(o.a, x);
+            get(o.b, y);
+            get(o.c, z);
+            CHMY_P_EACH(x[u] != 0.0 ? y[u] : z[u]);
+        } else if (o.op == CHMY_P_LT) {
+            get(o.a, x);
+            get(o.b, y);
+            CHMY_P_EACH(x[u] < y[u] ? 1.0 : 0.0);
+        } else if (o.op == CHMY_P_COORD) {
+            const AxisT ax = P.ax.a[o.a];
+            if (ax.p) {
+                CHMY_P_EACH(ax.at(o.b == CHMY_VERTEX ? CHMY_AX_VERTEX : CHMY_AX_CENTER, at(o.a, u) + o.c));
+            } else {
                 const double h = P.h[o.a], og = P.o[o.a];
-                v = o.b == CHMY_VERTEX ? fma(i1, h, og) : fma(i1, h, fma(0.5, h, og));
-                break;
+                const double o1 = o.b == CHMY_VERTEX ? og : fma(0.5, h, og);
+                CHMY_P_EACH(fma((double)(at(o.a, u) + o.c - 1), h, o1));
             }
-            case CHMY_P_SPACING:
-                v = P.ax.a[o.a].p ? P.ax.a[o.a].at(o.b == CHMY_VERTEX ? CHMY_AX_DV : CHMY_AX_DC, I[o.a] + o.c)
-                                  : P.h[o.a];
-                break;
-            case CHMY_P_INV_SPACING:
-                v = P.ax.a[o.a].p ? P.ax.a[o.a].at(o.b == CHMY_VERTEX ? CHMY_AX_IDV : CHMY_AX_IDC, I[o.a] + o.c)
-                                  : P.ih[o.a];
-                break;
-            case CHMY_P_LOAD:
-                v = load_src(P.src[o.a], i + off8(o.b, 0), j + off8(o.b, 1), k + off8(o.b, 2));
-                break;
-            case CHMY_P_NEG: v = -r[o.a]; break;
-            case CHMY_P_ABS: v = fabs(r[o.a]); break;
-            case CHMY_P_SQRT: v = sqrt(r[o.a]); break;
-            case CHMY_P_EXP: v = exp(r[o.a]); break;
-            case CHMY_P_LOG: v = log(r[o.a]); break;
-            case CHMY_P_SIN: v = sin(r[o.a]); break;
-            case CHMY_P_COS: v = cos(r[o.a]); break;
-            case CHMY_P_TANH: v = tanh(r[o.a]); break;
-            case CHMY_P_FLOOR: v = floor(r[o.a]); break;
-            case CHMY_P_NOT: v = r[o.a] == 0.0 ? 1.0 : 0.0; break;
-            case CHMY_P_ADD: v = r[o.a] + r[o.b]; break;
-            case CHMY_P_SUB: v = r[o.a] - r[o.b]; break;
-            case CHMY_P_MUL: v = r[o.a] * r[o.b]; break;
-            case CHMY_P_DIV: v = r[o.a] / r[o.b]; break;
-            case CHMY_P_POW: v = pow(r[o.a], r[o.b]); break;
-            case CHMY_P_MIN: v = jl_min(r[o.a], r[o.b]); break;
-            case CHMY_P_MAX: v = jl_max(r[o.a], r[o.b]); break;
-            case CHMY_P_LT: v = r[o.a] < r[o.b] ? 1.0 : 0.0; break;
-            case CHMY_P_LE: v = r[o.a] <= r[o.b] ? 1.0 : 0.0; break;
-            case CHMY_P_GT: v = r[o.a] > r[o.b] ? 1.0 : 0.0; break;
-            case CHMY_P_GE: v = r[o.a] >= r[o.b] ? 1.0 : 0.0; break;
-            case CHMY_P_EQ: v = r[o.a] == r[o.b] ? 1.0 : 0.0; break;
-            case CHMY_P_NE: v = r[o.a] != r[o.b] ? 1.0 : 0.0; break;
-            case CHMY_P_AND: v = (r[o.a] != 0.0 && r[o.b] != 0.0) ? 1.0 : 0.0; break;
-            case CHMY_P_OR: v = (r[o.a] != 0.0 || r[o.b] != 0.0) ? 1.0 : 0.0; break;
-            case CHMY_P_POWI: {
-                // x^n as repeated products, left to right (Julia's literal
-                // powers x^2 = x*x, x^3 = x*x*x; x^-1 = inv(x), x^-2 = inv(x)^2)
-                const double x = o.b < 0 ? 1.0 / r[o.a] : r[o.a];
-                const int n = o.b < 0 ? -o.b : o.b;
-                v = n == 0 ? 1.0 : x;
-                for (int e = 1; e < n; ++e) v = v * x;
-                break;
+        } else if (o.op == CHMY_P_EXP) {
+            get(o.a, x);
+            CHMY_P_EACH(exp(x[u]));
+        } else if (o.op < CHMY_P_NEG) {
+            const AxisT ax = P.ax.a[o.a];
+            if (o.op == CHMY_P_INDEX) CHMY_P_EACH((double)(at(o.a, u) + o.b));
+            else if (o.op == CHMY_P_SPACING)
+                CHMY_P_EACH(ax.p ? ax.at(o.b == CHMY_VERTEX ? CHMY_AX_DV : CHMY_AX_DC, at(o.a, u) + o.c) : P.h[o.a]);
+            else
+                CHMY_P_EACH(ax.p ? ax.at(o.b == CHMY_VERTEX ? CHMY_AX_IDV : CHMY_AX_IDC, at(o.a, u) + o.c)
+                                 : P.ih[o.a]);
+        } else {
+            get(o.a, x);
+            if (o.op >= CHMY_P_ADD && o.op != CHMY_P_POWI) get(o.b, y);
+            switch (o.op) {
+                case CHMY_P_ABS: CHMY_P_EACH(fabs(x[u])); break;
+                case CHMY_P_SQRT: CHMY_P_EACH(sqrt(x[u])); break;
+                case CHMY_P_LOG: CHMY_P_EACH(log(x[u])); break;
+                case CHMY_P_FLOOR: CHMY_P_EACH(floor(x[u])); break;
+                case CHMY_P_NOT: CHMY_P_EACH(x[u] == 0.0 ? 1.0 : 0.0); break;
+                case CHMY_P_DIV: CHMY_P_EACH(x[u] / y[u]); break;
+                case CHMY_P_MIN: CHMY_P_EACH(jl_min(x[u], y[u])); break;
+                case CHMY_P_MAX: CHMY_P_EACH(jl_max(x[u], y[u])); break;
+                case CHMY_P_LE: CHMY_P_EACH(x[u] <= y[u] ? 1.0 : 0.0); break;
+                case CHMY_P_EQ: CHMY_P_EACH(x[u] == y[u] ? 1.0 : 0.0); break;
+                case CHMY_P_NE: CHMY_P_EACH(x[u] != y[u] ? 1.0 : 0.0); break;
+                case CHMY_P_AND: CHMY_P_EACH((x[u] != 0.0 && y[u] != 0.0) ? 1.0 : 0.0); break;
+                case CHMY_P_OR: CHMY_P_EACH((x[u] != 0.0 || y[u] != 0.0) ? 1.0 : 0.0); break;
+                case CHMY_P_POWI: CHMY_P_EACH(powi(x[u], o.b)); break;
+                default:
+                    if constexpr (HEAVY) {
+                        if (o.op == CHMY_P_SIN) CHMY_P_EACH(sin(x[u]));
+                        else if (o.op == CHMY_P_COS) CHMY_P_EACH(cos(x[u]));
+                        else if (o.op == CHMY_P_TANH) CHMY_P_EACH(tanh(x[u]));
+                        else CHMY_P_EACH(pow(x[u], y[u]));
+                    }
+                    break;
             }
-            case CHMY_P_SELECT: v = r[o.a] != 0.0 ? r[o.b] : r[o.c]; break;
-            case CHMY_P_FMA: v = fma(r[o.a], r[o.b], r[o.c]); break;
-            default: break;
         }
-        r[q] = v;
+#undef CHMY_P_EACH
+#pragma unroll
+        for (int u = 0; u < N; ++u) r[u].set(o.dst, v[u]);
     }
-    put(dst(i, j, k), r[P.n - 1]);
+}
+
+// One wave: 64 x points of a row, a chunk of planes of the marched dim, N
+// planes at a time.  Lanes and planes past the box evaluate clamped indices
+// and store nothing.
+template <class T, int S, int N, bool HEAVY>
+__global__ void __launch_bounds__(64) program_kernel(const PProg P, DF<T> dst, Box3 b, int nbx, int nby, int chunk) {
+    const int t = blockIdx.x;
+    const int bx = t % nbx, by = (t / nbx) % nby, bc = t / (nbx * nby);
+    const int m = P.m;
+    const int64_t i = b.lo[0] + (int64_t)bx * 64 + threadIdx.x, hi0 = b.lo[0] + b.len[0];
+    const int64_t j = b.lo[1] + by;   // nby == 1 in 2D and 1D, where j is marched or the only one
+    const int64_t m0 = b.lo[m] + (int64_t)bc * chunk;
+    const int64_t hm = b.lo[m] + b.len[m], m1 = m0 + chunk < hm ? m0 + chunk : hm;
+    const int64_t I[3] = {i < hi0 ? i : hi0 - 1, j, b.lo[2]};
+    Slots<S> r[N];
+    int64_t Im[N];
+#pragma unroll
+    for (int u = 0; u < N; ++u) Im[u] = m0;
+    program_run<S, N, HEAVY>(P, 0, P.npro, r, I, Im);
+    for (int64_t p = m0; p < m1; p += N) {
+#pragma unroll
+        for (int u = 0; u < N; ++u) Im[u] = p + u < m1 ? p + u : m1 - 1;
+        program_run<S, N, HEAVY>(P, P.npro, P.n, r, I, Im);
+#pragma unroll
+        for (int u = 0; u < N; ++u) {
+            const double v = P.out >= 0 ? r[u].get(P.out) : P.k[-1 - P.out];
+            if (i < hi0 && p + u < m1) put(m == 2 ? dst(i, j, p + u) : dst(i, p + u, 0), v);
+        }
+    }
 }
 
 static bool unary(int op) { return op >= CHMY_P_NEG && op <= CHMY_P_NOT; }
@@ -197,6 +309,138 @@ static int check_program(const chmy_grid_t* g, const chmy_pop_t* prog, int nprog
     return 0;
 }
 
+static int nargs_of(int op) {
+    if (op == CHMY_P_SELECT || op == CHMY_P_FMA) return 3;
+    return binary(op) ? 2 : unary(op) || op == CHMY_P_POWI ? 1 : 0;
+}
+
+// Lowers a checked program into P (operations, split point, output operand);
+// returns the number of slots it needs, and whether it calls sin, cos, tanh
+// or pow.  Slots are reused after a register's last use; a value that the
+// per-plane part reads from the per-chunk part keeps its slot to the end.
+static int plan_program(const chmy_pop_t* prog, int n, PProg* P, bool* heavy) {
+    bool plane[kPMaxOps], live[kPMaxOps] = {};
+    int last[kPMaxOps];          // position of the last use in the lowered order
+    int order[kPMaxOps], no = 0;
+    *heavy = false;
+    auto arg = [](const chmy_pop_t& o, int k) { return k == 0 ? o.a : k == 1 ? o.b : o.c; };
+    live[n - 1] = true;
+    for (int q = n - 1; q >= 0; --q)
+        for (int k = 0; live[q] && k < nargs_of(prog[q].op); ++k) live[arg(prog[q], k)] = true;
+    for (int q = 0; q < n; ++q) {
+        const chmy_pop_t& o = prog[q];
+        if (o.op == CHMY_P_LOAD) plane[q] = true;
+        else if (o.op >= CHMY_P_INDEX && o.op <= CHMY_P_INV_SPACING) plane[q] = o.a == P->m;
+        else plane[q] = false;
+        for (int k = 0; k < nargs_of(o.op); ++k) plane[q] = plane[q] || plane[arg(o, k)];
+    }
+    for (int part = 0; part < 2; ++part) {
+        if (part == 1) P->npro = no;
+        for (int q = 0; q < n; ++q)
+            if (live[q] && prog[q].op != CHMY_P_CONST && plane[q] == (part == 1)) order[no++] = q;
+    }
+    P->n = no;
+    for (int q = 0; q < n; ++q) last[q] = -1;
+    for (int p = 0; p < no; ++p) {
+        const chmy_pop_t& o = prog[order[p]];
+        for (int k = 0; k < nargs_of(o.op); ++k) {
+            const int r = arg(o, k);
+            last[r] = !plane[r] && p >= P->npro ? no : std::max(last[r], p);
+        }
+    }
+    last[n - 1] = no;
+    int slot[kPMaxOps], used = 0;
+    bool busy[kPMaxOps] = {};
+    auto operand = [&](int r) { return prog[r].op == CHMY_P_CONST ? -1 - prog[r].a : slot[r]; };
+    for (int p = 0; p < no; ++p) {
+        const int q = order[p];
+        const chmy_pop_t& o = prog[q];
+        const int na = nargs_of(o.op);
+        PIns& w = P->op[p];
+        w.op = (int16_t)o.op;
+        w.a = na > 0 ? operand(o.a) : o.a;
+        w.b = na > 1 ? operand(o.b) : o.b;
+        w.c = na > 2 ? operand(o.c) : o.c;
+        for (int k = 0; k < na; ++k) {
+            const int r = arg(o, k);
+            if (prog[r].op != CHMY_P_CONST && last[r] == p) busy[slot[r]] = false;
+        }
+        int s = 0;
+        while (busy[s]) ++s;
+        busy[s] = true;
+        slot[q] = s;
+        used = std::max(used, s + 1);
+        w.dst = (int16_t)s;
+        *heavy = *heavy || o.op == CHMY_P_SIN || o.op == CHMY_P_COS || o.op == CHMY_P_TANH || o.op == CHMY_P_POW;
+    }
+    P->out = operand(n - 1);
+    // the sums, products and negations as the FMA that gives the same bits:
+    // a + b = fma(a, 1, b), a - b = fma(b, -1, a), a b = fma(a, b, -0.0),
+    // -a = fma(a, -1, -0.0); a > b and a >= b as b < a and b <= a
+    const int one = -1 - kPMaxConst, minus = one - 1, nzero = one - 2;
+    for (int p = 0; p < no; ++p) {
+        PIns& w = P->op[p];
+        const int32_t a = w.a, b = w.b;
+        auto as_fma = [&w](int32_t x, int32_t y, int32_t z) {
+            w.op = CHMY_P_FMA;
+            w.a = x;
+            w.b = y;
+            w.c = z;
+        };
+        switch (w.op) {
+            case CHMY_P_ADD: as_fma(a, one, b); break;
+            case CHMY_P_SUB: as_fma(b, minus, a); break;
+            case CHMY_P_MUL: as_fma(a, b, nzero); break;
+            case CHMY_P_NEG: as_fma(a, minus, nzero); break;
+            case CHMY_P_POWI:
+                if (b == 2) as_fma(a, a, nzero);
+                break;
+            case CHMY_P_GT:
+            case CHMY_P_GE:
+                w.op = w.op == CHMY_P_GT ? CHMY_P_LT : CHMY_P_LE;
+                w.a = b;
+                w.b = a;
+                break;
+            default: break;
+        }
+    }
+    P->k[kPMaxConst] = 1.0;
+    P->k[kPMaxConst + 1] = -1.0;
+    P->k[kPMaxConst + 2] = -0.0;
+    return used;
+}
+
+template <class T>
+static int program_launch(const PProg& P, const chmy_field_t* dst, const Box3& b, int slots, bool heavy,
+                          hipStream_t st) {
+    const int64_t nbx = (b.len[0] + 63) / 64, nby = P.m == 2 ? b.len[1] : 1, nm = b.len[P.m];
+    // planes per wave: fill whole rounds of the waves the chip holds (12 a CU
+    // at these kernels' registers); a wave also spends about two planes' time
+    // on the per-chunk operations.  160x144x127: 20 planes, one round
+    const int64_t room = 12 * (int64_t)cu_count();
+    int64_t chunk = 4, best = INT64_MAX;
+    for (int64_t c = 4; c <= 64; c += 4) {
+        const int64_t waves = nbx * nby * ((nm + c - 1) / c), cost = (waves + room - 1) / room * (c + 2);
+        if (cost < best) {
+            best = cost;
+            chunk = c;
+        }
+    }
+    const int64_t nb = nbx * nby * ((nm + chunk - 1) / chunk);
+    if (nb > INT32_MAX) return set_error(CHMY_E_SIZE, "point program: box too large");
+    const dim3 grd((unsigned)nb), blk(64);
+    const DF<T> d = view<T>(*dst);
+    const int ix = (int)nbx, iy = (int)nby, ic = (int)chunk;
+    if (slots > 16)
+        hipLaunchKernelGGL((program_kernel<T, 0, 1, true>), grd, blk, (size_t)slots * 64 * sizeof(double), st, P, d, b, ix,
+                           iy, ic);
+    else if (heavy) hipLaunchKernelGGL((program_kernel<T, 16, 1, true>), grd, blk, 0, st, P, d, b, ix, iy, ic);
+    else if (slots > 8) hipLaunchKernelGGL((program_kernel<T, 16, 2, false>), grd, blk, 0, st, P, d, b, ix, iy, ic);
+    else hipLaunchKernelGGL((program_kernel<T, 8, 4, false>), grd, blk, 0, st, P, d, b, ix, iy, ic);
+    CHMY_HIP(hipGetLastError());
+    return 0;
+}
+
 }  // namespace chmy
 
 using namespace chmy;
@@ -226,15 +470,15 @@ int chmy_set_program(const chmy_grid_t* g, const chmy_field_t* dst, const chmy_b
     if (b.len[0] == 0 || b.len[1] == 0 || b.len[2] == 0) return 0;
     PProg P;
     std::memset(&P, 0, sizeof P);
-    P.n = nprog;
-    P.nd = g->nd;
+    P.m = g->nd == 1 ? 2 : g->nd - 1;
     for (int d = 0; d < 3; ++d) {
         P.o[d] = d < g->nd ? g->origin[d] : 0.0;
         P.h[d] = d < g->nd ? g->spacing[d] : 0.0;
         P.ih[d] = d < g->nd ? g->inv_spacing[d] : 0.0;
     }
     P.ax = axes_of(g);
-    std::memcpy(P.op, prog, sizeof(chmy_pop_t) * nprog);
+    bool heavy;
+    const int slots = plan_program(prog, nprog, &P, &heavy);
     if (nconst) std::memcpy(P.k, consts, sizeof(double) * nconst);
     for (int s = 0; s < nsrc; ++s) {
         const chmy_field_t& f = srcs[s];
@@ -251,16 +495,9 @@ int chmy_set_program(const chmy_grid_t* g, const chmy_field_t* dst, const chmy_b
         P.src[s].esize = es;
     }
     hipStream_t st = (hipStream_t)stream;
-    const dim3 blk(64, 4, 1);
-    const dim3 grd((unsigned)((b.len[0] + 63) / 64), (unsigned)((b.len[1] + 3) / 4), (unsigned)b.len[2]);
-    if (dst->dtype == CHMY_F64)
-        hipLaunchKernelGGL(program_kernel<double>, grd, blk, 0, st, P, view<double>(*dst), b);
-    else if (dst->dtype == CHMY_F32)
-        hipLaunchKernelGGL(program_kernel<float>, grd, blk, 0, st, P, view<float>(*dst), b);
-    else
-        hipLaunchKernelGGL(program_kernel<bf16s>, grd, blk, 0, st, P, view<bf16s>(*dst), b);
-    CHMY_HIP(hipGetLastError());
-    return 0;
+    if (dst->dtype == CHMY_F64) return program_launch<double>(P, dst, b, slots, heavy, st);
+    if (dst->dtype == CHMY_F32) return program_launch<float>(P, dst, b, slots, heavy, st);
+    return program_launch<bf16s>(P, dst, b, slots, heavy, st);
 }
 
 }  // extern "C"

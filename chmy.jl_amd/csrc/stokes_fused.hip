@@ -1556,19 +1556,12 @@ constexpr int kTW3 = std::is_same<T, double>::value ? CHMY_FUSED_TW64 : CHMY_FUS
 // lengths 16 / 22 / 24 / 26 / 37 / 43 / 52: 0.784 / 0.739 / 0.775 / 0.734 /
 // 0.694 / 0.760 / 0.705, the order this cost gives).
 static int32_t tb3_chunk(int64_t tiles, int64_t planes) {
-    static int ncu[64] = {0};
-    int dev = 0;
-    if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) dev = 0;
-    if (ncu[dev] == 0) {
-        int n = 0;
-        if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n <= 0) n = 256;
-        ncu[dev] = n;
-    }
+    const int ncu = cu_count();
     int64_t best = -1, bestk = planes;
     for (int64_t c = 1; c <= planes; ++c) {
         const int64_t k = (planes + c - 1) / c;
         if (k < kTB3Z) break;
-        const int64_t cost = ((tiles * c + ncu[dev] - 1) / ncu[dev]) * (k + 3);
+        const int64_t cost = ((tiles * c + ncu - 1) / ncu) * (k + 3);
         if (best < 0 || cost < best) {
             best = cost;
             bestk = k;

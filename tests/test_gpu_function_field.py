@@ -256,3 +256,30 @@ def test_program_errors(arch):
     prog = trace(lambda g_, l, ix, iy, H: H[ix + 3, iy], g, Cc(), discrete=True, parameters=(H,))
     with pytest.raises(_lib.ChmyError, match="storage"):
         prog.run(g, f)
+
+
+@pytest.mark.parametrize("dims", [(1,), (130,), (64, 1), (63, 13), (65, 3, 1), (70, 5, 21), (129, 2, 66)])
+@pytest.mark.parametrize("wide,sine", [(3, False), (6, False), (12, False), (20, False), (3, True), (12, True), (20, True)])
+def test_program_register_files_and_plane_chunks(arch, dims, wide, sine):
+    """Programs that keep 3 to 20 values live at once (registers in 8 or 16
+    slots, or in LDS), with parts that depend on the last dim and parts that do
+    not, over boxes that end inside and past the chunks of planes; `sine` adds
+    0·sin, which selects the one-plane variants and leaves the bits alone.
+    Only + - × and comparisons, so bitwise against the host."""
+    nd = len(dims)
+    g = chmy.UniformGrid(arch, origin=(-0.4,) * nd, extent=(1.0, 1.3, 0.9)[:nd], dims=dims)
+    f = chmy.Field(arch, g, Cc())
+
+    def func(*xs):
+        first, last = xs[0], xs[-1]
+        square = (xs[nd // 2] - 0.05) ** 2
+        v = [first * (0.3 + k) + (last if k % 2 else square) for k in range(wide)]
+        s = v[0] * v[-1]
+        for k in range(1, wide):
+            s = s - v[k] * v[wide - 1 - k]
+        s = chmy.ifelse(s > first, s, -s + last)
+        return 0.0 * np.sin(last) + s if sine else s
+
+    chmy.set_(f, func, g)
+    want = host_values(ogrid(g), f, func, ())
+    assert np.array_equal(f.interior().cpu().numpy(), want)
