@@ -141,7 +141,9 @@ __device__ __forceinline__ void program_run(const PProg& P, int q0, int q1, Slot
             }
         };
         // index of plane u along dim d
-        auto at = [&](int d, int u) -> int64_t { return d == P.m ? Im[u] : (d == 0 ? I[0] : d == 1 ? I[1] : I[2]); };
+        auto at = [&](int d, int u) -> int64_t {
+            return d == P.m ? Im[u] : (d == 0 ? I[0] : d == 1 ? I[1] : I[2]);
+        };
 #define CHMY_P_EACH(expr)                      \
     do {                                       \
         _Pragma("unroll") for (int u = 0; u < N; ++u) v[u] = (expr); \

@@ -505,7 +505,8 @@ int chmy_op_masked(int op, const chmy_grid_t* g, const chmy_box_t* box, const ch
     if (!src) return set_error(CHMY_E_ARG, "src is NULL");
     if (per_dim && (dim < 0 || dim >= g->nd)) return set_error(CHMY_E_ARG, "dim %d out of range", dim);
     if (masks && !maskable) return set_error(CHMY_E_ARG, "operator %d has no masked form", op);
-    if (needs_k != (k != nullptr)) return set_error(CHMY_E_ARG, needs_k ? "k is NULL" : "k is given to an operator without a coefficient");
+    if (needs_k != (k != nullptr))
+        return set_error(CHMY_E_ARG, needs_k ? "k is NULL" : "k is given to an operator without a coefficient");
     for (int q = 0; q < nsrc; ++q) {
         const int* want = nullptr;
         int loc[3];

@@ -159,6 +159,144 @@ __global__ void __launch_bounds__(256) diffusion_step_bc_kernel(Box3 box, Box3 r
     g_at(Co, P) = w;
 }
 
+// Up to KS steps of the loop in one launch (build extension), C and its face
+// ghosts only: a block loads its TX x TY (x TZ) cells with a ring of KS and
+// advances them on chip, the valid region shrinking by one ring a step; the
+// ring is computed again by the neighbouring blocks.  A thread holds PT
+// consecutive points of the last dim in registers and finds its neighbours
+// along the other dims in LDS (two buffers, one barrier a step).  A cell's
+// value is the expression of diffusion_value on the same operands; the
+// neighbour beyond a boundary is the batch's own fma step of the cell (the
+// stored ghost in the first step), so every stored value has the bits of as
+// many launches of the step.  q is not stored and the corner ghosts (which no
+// cell reads) are left alone: the caller runs the last two steps one by one,
+// and they write both buffers' ghosts, corners included, and q.
+//
+// Why: a step of 256^2 cells is one 5 us launch for 0.5 MB of data, most of it
+// the wait for the launch before it.  Measured, us per step of a 100-step call,
+// one launch each -> now: 2D FP64 64^2 4.7 -> 0.95, 256^2 5.1 -> 0.96, 500x480
+// 5.5 -> 1.5, 1024^2 11.4 -> 3.5 (FP32 10.0 -> 2.8); 3D 20^3 5.6 -> 3.5, 64^3
+// 12.6 -> 3.7, 160^3 58.6 -> 25.7 (FP32 45 -> 15).  Bound by the chain of LDS
+// reads and barriers (0.1 us a step) and the launches on small grids, by
+// vector issue and LDS on large ones.
+template <class T>
+struct DiffTile {
+    DF<T> C, Co;
+    int32_t n[3], nb[3];
+    int32_t steps;   // 1..KS
+    T nchi, dt, isp[3];
+    SideRules r;
+};
+
+template <class T>
+__device__ __forceinline__ T ghost_of(const SideRules& r, int d, int side, T w) {
+    const T val = T(r.val[d][side]);
+    if (r.kind[d][side] == CHMY_DIRICHLET) return fma(T(2), val - w, w);
+    return fma(T(r.h[d]), side == 0 ? -val : val, w);
+}
+
+template <class T, int ND, int TX, int TY, int TZ, int KS, int PT>
+struct DiffShape {
+    static constexpr int RX = TX + 2 * KS, RY = TY + 2 * KS, RZ = ND == 3 ? TZ + 2 * KS : 1;
+    static constexpr int M = ND - 1, RM = ND == 3 ? RZ : RY, SM = ND == 3 ? RX * RY : RX;   // the last dim
+    static constexpr int COLS = ND == 3 ? RX * RY : RX, NT = COLS * (RM / PT);
+    static_assert(RM % PT == 0 && NT <= 1024, "strips tile the last dim");
+};
+
+template <class T, int ND, int TX, int TY, int TZ, int KS, int PT, int NT = DiffShape<T, ND, TX, TY, TZ, KS, PT>::NT>
+__global__ void __launch_bounds__(NT) diffusion_tile_kernel(const DiffTile<T> p) {
+    using Sh = DiffShape<T, ND, TX, TY, TZ, KS, PT>;
+    constexpr int RX = Sh::RX, RY = Sh::RY, M = Sh::M, SM = Sh::SM;
+    __shared__ T buf[2][Sh::COLS * Sh::RM];
+    const int t = xcd_remap(blockIdx.x, gridDim.x);
+    const int bx = t % p.nb[0], by = (t / p.nb[0]) % p.nb[1], bz = ND == 3 ? t / (p.nb[0] * p.nb[1]) : 0;
+    const int col = threadIdx.x % Sh::COLS, strip = threadIdx.x / Sh::COLS;
+    const int a[3] = {col % RX, ND == 3 ? col / RX : strip * PT, strip * PT};
+    const int org[3] = {1 + bx * TX - KS, 1 + by * TY - KS, ND == 3 ? 1 + bz * TZ - KS : 0};
+    const int len[3] = {RX, RY, Sh::RZ};
+    int ring0 = KS;
+    bool cell0 = true, stored0 = true, edge = false, g0[2][2] = {};
+#pragma unroll
+    for (int d = 0; d < ND; ++d) {
+        edge = edge || org[d] < 1 || org[d] + len[d] > p.n[d] + 1;   // the region holds a boundary (block-uniform)
+        if (d == M) continue;
+        const int c = org[d] + a[d];
+        stored0 = stored0 && c >= 0 && c <= p.n[d] + 1;
+        cell0 = cell0 && c >= 1 && c <= p.n[d];
+        ring0 = min(ring0, min(a[d], len[d] - 1 - a[d]));
+        g0[d][0] = c == 1;
+        g0[d][1] = c == p.n[d];
+    }
+    const int l0 = ND == 3 ? col + a[2] * SM : col + a[1] * SM;
+    const int64_t base = (int64_t)(org[0] + a[0]) + (int64_t)(org[1] + a[1]) * p.C.sy +
+                         (ND == 3 ? (int64_t)(org[2] + a[2]) * p.C.sz : 0);
+    const int64_t sm = ND == 3 ? p.C.sz : p.C.sy;
+    T c[PT];
+    int ring[PT];   // steps the point is advanced: 0 where it is no cell of the region
+#pragma unroll
+    for (int q = 0; q < PT; ++q) {
+        const int m = a[M] + q, i = org[M] + m;
+        const bool in = i >= 1 && i <= p.n[M];
+        ring[q] = cell0 && in ? min(ring0, min(m, Sh::RM - 1 - m)) - (KS - p.steps) : 0;
+        c[q] = T(0);
+        if (stored0 && i >= 0 && i <= p.n[M] + 1) c[q] = p.C.p[base + q * sm];
+        buf[0][l0 + q * SM] = c[q];
+    }
+    __syncthreads();
+    auto advance = [&](auto edge_) {
+        constexpr bool EDGE = decltype(edge_)::value;
+#pragma unroll 1
+        for (int s = 1; s <= p.steps; ++s) {
+            const T* in = buf[(s - 1) & 1];
+            T* out = buf[s & 1];
+            const bool by_rule = EDGE && s > 1;
+            const T below = strip > 0 ? in[l0 - SM] : T(0), above = strip + 1 < Sh::RM / PT ? in[l0 + PT * SM] : T(0);
+            T old = below;
+#pragma unroll
+            for (int q = 0; q < PT; ++q) {
+                const T cq = c[q];
+                const T next = q + 1 < PT ? c[q + 1] : above;
+                if (ring[q] >= s) {
+                    const int l = l0 + q * SM, i = org[M] + a[M] + q;
+                    T dv = T(0);
+#pragma unroll
+                    for (int d = 0; d < ND; ++d) {
+                        T lo = d == M ? old : in[l - (d == 0 ? 1 : RX)], hi = d == M ? next : in[l + (d == 0 ? 1 : RX)];
+                        if (by_rule) {
+                            if (d == M ? i == 1 : g0[d & 1][0]) lo = ghost_of(p.r, d, 0, cq);
+                            if (d == M ? i == p.n[M] : g0[d & 1][1]) hi = ghost_of(p.r, d, 1, cq);
+                        }
+                        const T ql = p.nchi * ((cq - lo) * p.isp[d]);
+                        const T qr = p.nchi * ((hi - cq) * p.isp[d]);
+                        const T x = (qr - ql) * p.isp[d];
+                        dv = d == 0 ? x : dv + x;
+                    }
+                    c[q] = cq - p.dt * dv;
+                    out[l] = c[q];
+                }
+                old = cq;
+            }
+            __syncthreads();
+        }
+    };
+    if (edge) advance(std::true_type{});
+    else advance(std::false_type{});
+#pragma unroll
+    for (int q = 0; q < PT; ++q) {
+        if (ring[q] < p.steps) continue;   // the tile's own cells
+        const int64_t o = base + q * sm;
+        p.Co.p[o] = c[q];
+        if (!edge) continue;
+        const int i = org[M] + a[M] + q;
+#pragma unroll
+        for (int d = 0; d < ND; ++d) {
+            const int64_t st = d == 0 ? 1 : d == 1 ? p.C.sy : p.C.sz;
+            if (d == M ? i == 1 : g0[d & 1][0]) p.Co.p[o - st] = ghost_of(p.r, d, 0, c[q]);
+            if (d == M ? i == p.n[M] : g0[d & 1][1]) p.Co.p[o + st] = ghost_of(p.r, d, 1, c[q]);
+        }
+    }
+}
+
 // ------------------------------------------------------------------ update_old!
 template <class T>
 struct Copy7 {
@@ -355,6 +493,77 @@ static int diffusion_launch(const chmy_grid_t* g, const chmy_box_t* box, const c
     return 0;
 }
 
+template <class T, int ND, int TX, int TY, int TZ, int KS, int PT>
+static int diffusion_tile_launch(const DiffTile<T>& base, int steps, const DF<T>* C, int p, hipStream_t s) {
+    DiffTile<T> a = base;
+    a.steps = steps;
+    a.C = C[p];
+    a.Co = C[1 - p];
+    const int tile[3] = {TX, TY, TZ};
+    int64_t nb = 1;
+    for (int d = 0; d < 3; ++d) {
+        const int64_t q = d < ND ? ((int64_t)a.n[d] + tile[d] - 1) / tile[d] : 1;
+        a.nb[d] = (int32_t)q;
+        nb *= q;
+    }
+    hipLaunchKernelGGL((diffusion_tile_kernel<T, ND, TX, TY, TZ, KS, PT>), dim3((unsigned)nb),
+                       dim3(DiffShape<T, ND, TX, TY, TZ, KS, PT>::NT), 0, s, a);
+    CHMY_HIP(hipGetLastError());
+    return 0;
+}
+
+// Tiles.  Small grids, whose time is latency, take one point a thread (2D) or
+// 3 (3D) and as many waves as a block holds; grids that fill the chip several
+// times over take larger tiles, which compute less ring, with more points a
+// thread.  The lines lie where the two cross (f64 us per step, small / large
+// tile: 2D 240 k cells 1.75 / 1.50, 65 k 0.95 / 1.5; 3D 262 k cells 3.7 / 6.1,
+// 4.1 M 35.9 / 25.7).
+constexpr int kDiffK2 = 8, kDiffK3 = 2;
+template <class T>
+static int diffusion_tile_any(int nd, int k, int64_t cells, const DiffTile<T>& a, const DF<T>* C, int p,
+                              hipStream_t s) {
+    if (nd == 2)
+        return cells < (1 << 17) ? diffusion_tile_launch<T, 2, 16, 16, 1, kDiffK2, 1>(a, k, C, p, s)
+                                 : diffusion_tile_launch<T, 2, 32, 32, 1, kDiffK2, 3>(a, k, C, p, s);
+    return cells < 3 * (1 << 18) ? diffusion_tile_launch<T, 3, 16, 8, 8, kDiffK3, 3>(a, k, C, p, s)
+                                 : diffusion_tile_launch<T, 3, 28, 12, 12, kDiffK3, 8>(a, k, C, p, s);
+}
+
+// All but the last two steps in passes of up to 8 (2D) or 2 (3D) steps, as many
+// passes as leave the buffers where single steps would (a pass flips the
+// parity once); *done steps were taken.
+template <class T>
+static int diffusion_passes(const chmy_grid_t* g, const chmy_field_t* C0, const chmy_field_t* C1, const SideRules& r,
+                            double chi, double dt, int niter, int* p, int* done, hipStream_t s) {
+    const int steps = niter - 2, nd = g->nd;
+    int64_t cells = 1;
+    for (int d = 0; d < nd; ++d) cells *= g->n[d];
+    if (nd < 2 || steps < 2) return 0;
+    DiffTile<T> a;
+    std::memset(&a, 0, sizeof a);
+    for (int d = 0; d < 3; ++d) {
+        if (d < nd && g->n[d] > (int64_t(1) << 30)) return 0;
+        a.n[d] = d < nd ? (int32_t)g->n[d] : 1;
+        a.isp[d] = T(g->inv_spacing[d]);
+    }
+    a.nchi = -T(chi);
+    a.dt = T(dt);
+    a.r = r;
+    const DF<T> C[2] = {view<T>(*C0), view<T>(*C1)};
+    if (C[0].sy != C[1].sy || C[0].sz != C[1].sz) return 0;   // the kernel takes one stride set
+    const int K = nd == 2 ? kDiffK2 : kDiffK3;
+    int m = (steps + K - 1) / K;
+    if ((m ^ steps) & 1) ++m;   // passes and steps of the same parity
+    if (m > steps) return 0;
+    for (int q = 0; q < m; ++q) {
+        const int k = steps / m + (q < steps % m ? 1 : 0);
+        CHMY_TRY(diffusion_tile_any<T>(nd, k, cells, a, C, *p, s));
+        *p = 1 - *p;
+        *done += k;
+    }
+    return 0;
+}
+
 template <class T>
 static int copy_launch(const chmy_grid_t* g, const chmy_box_t& bx, const chmy_field_t* Tf, const chmy_field_t* tau,
                        const chmy_field_t* To, const chmy_field_t* tauo, hipStream_t s) {
@@ -490,8 +699,10 @@ int chmy_diffusion_iterate(const chmy_grid_t* g, const chmy_field_t* C0, const c
             DFL<T> c[2] = {lview<T>(*C0), lview<T>(*C1)};
             DFL<T> q0 = lview<T>(q[0]);
             DFL<T> q1 = g->nd > 1 ? lview<T>(q[1]) : q0, q2 = g->nd > 2 ? lview<T>(q[2]) : q0;
+            int it = 0;
+            CHMY_TRY(diffusion_passes<T>(g, C0, C1, rules, chi, dt, niter, &p, &it, (hipStream_t)stream));
             const dim3 grd = grid_for(reg, blk2());
-            for (int it = 0; it < niter; ++it) {
+            for (; it < niter; ++it) {
                 hipLaunchKernelGGL(diffusion_step_bc_kernel<T>, grd, blk2(), 0, (hipStream_t)stream, b, reg, c[p],
                                    c[1 - p], q0, q1, q2, g->nd, -T(chi), T(dt), T(g->inv_spacing[0]),
                                    T(g->inv_spacing[1]), T(g->inv_spacing[2]), rules);

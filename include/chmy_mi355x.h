@@ -202,8 +202,9 @@ int chmy_diffusion_step(const chmy_grid_t* grid, const chmy_box_t* box, const ch
  * *parity_inout into 1-p, then the C batch (bc_counts[2*dim+side-1] <= 1
  * entries, the conditions in bcs, as chmy_bc_batchset) on 1-p.  When every
  * (dim, side) has one rule with a scalar (or no) value, the batch runs inside
- * the step's launch (one launch per step, same bits).  On return
- * *parity_inout names the buffer holding C (build extension). */
+ * the step's launch, and in 2D and 3D all but the last two steps run several
+ * to a launch (same bits in both buffers and q).  On return *parity_inout
+ * names the buffer holding C (build extension). */
 int chmy_diffusion_iterate(const chmy_grid_t* grid, const chmy_field_t* C0, const chmy_field_t* C1,
                            const chmy_field_t* q, const int32_t* bc_counts, const chmy_bc_t* bcs, double chi,
                            double dt, int niter, int* parity_inout, void* stream);

@@ -669,3 +669,43 @@ def test_maxabs_items(arch, dtype, dims):
         assert ss == chmy.kernels.sumsq(f)
     f.interior()[spots[-1]] = float("nan")
     assert np.isnan(chmy.kernels.maxabs(f))
+
+
+@pytest.mark.parametrize("T", TYPES)
+@pytest.mark.parametrize("dims,steps,halo1", [
+    ((1, 1), 7, 1), ((2, 3), 12, 1), ((15, 17), 11, 1), ((16, 33), 21, 1), ((70, 33), 40, 1), ((70, 33), 9, 2),
+    ((1, 130), 30, 1), ((391, 350), 13, 1), ((2, 1, 3), 7, 1), ((16, 8, 9), 8, 1), ((33, 17, 7), 11, 1),
+    ((93, 92, 97), 9, 1)])
+def test_diffusion_iterate_passes_equal_single_steps(arch, T, dims, steps, halo1):
+    """Several steps per launch (tiles of every shape and grids that end
+    inside, at and past them; up to 8 steps, with remainders; both parities)
+    against one call per step: both buffers' whole storage and q, bitwise, on
+    random storage with Dirichlet and Neumann values.  Buffers of different
+    padding (halo1) keep single steps."""
+    import ctypes as C
+    from chmy import _lib
+    from chmy.kernels import _arr
+    nd = len(dims)
+    g = chmy.UniformGrid(arch, origin=(-1.0,) * nd, extent=(2.0, 1.7, 1.4)[:nd], dims=dims)
+    rng = np.random.default_rng(31)
+    rules = [(_lib.DIRICHLET, 0.7), (_lib.NEUMANN, -1.3), (_lib.NEUMANN, 0.0), (_lib.DIRICHLET, -0.4),
+             (_lib.NEUMANN, 0.25), (_lib.DIRICHLET, 1.1)][:2 * nd]
+    counts = (C.c_int32 * 6)(*([1] * (2 * nd) + [0] * (6 - 2 * nd)))
+    bcs = (_lib.ChmyBC * (2 * nd))(*[_lib.ChmyBC(k, _lib.VALUE_SCALAR, v, None) for k, v in rules])
+    dt = 0.1 * min(chmy.spacing(g)) ** 2
+    sets = []
+    for _ in range(2):
+        Cs = [chmy.Field(arch, g, Cc(), NP2TORCH[T]), chmy.Field(arch, g, Cc(), NP2TORCH[T], halo=halo1)]
+        sets.append((Cs, [chmy.Field(arch, g, vloc(D, nd), NP2TORCH[T]) for D in range(nd)]))
+    for a, b in zip(sets[0][0] + sets[0][1], sets[1][0] + sets[1][1]):
+        a.data.copy_(torch.from_numpy(rng.uniform(-1.0, 1.0, tuple(a.data.shape))))
+        b.data.copy_(a.data)
+    par = [C.c_int(1), C.c_int(1)]
+    for (Cs, q), p, calls in ((sets[0], par[0], [steps]), (sets[1], par[1], [1] * steps)):
+        for n in calls:
+            _lib.call("chmy_diffusion_iterate", C.byref(g.desc()), C.byref(Cs[0].desc()), C.byref(Cs[1].desc()),
+                      _arr(q), counts, bcs, 0.9, dt, n, C.byref(p), chmy.current_stream())
+    chmy.synchronize()
+    assert par[0].value == par[1].value
+    for a, b in zip(sets[0][0] + sets[0][1], sets[1][0] + sets[1][1]):
+        assert torch.equal(a.data, b.data)
