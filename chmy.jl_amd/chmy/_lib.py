@@ -118,6 +118,7 @@ SIGNATURES = {
     "chmy_op_masked": [C.c_int, PG, PB, PF, C.c_int, PF, PF, PF, C.c_int, VP],
     "chmy_set_program": [PG, PF, PB, P(ChmyPop), C.c_int, P(C.c_double), C.c_int, PF, C.c_int, VP],
     "chmy_maxabs_dev": [PF, PB, P(C.c_double), VP],
+    "chmy_maxabs_many": [C.c_int, PF, P(C.c_double), VP],
     "chmy_maxabs": [PF, PB, P(C.c_double), VP],
     "chmy_sumsq": [PF, PB, P(C.c_double), VP],
 }

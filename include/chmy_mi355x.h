@@ -489,7 +489,10 @@ int chmy_set_program(const chmy_grid_t* grid, const chmy_field_t* dst, const chm
  * exact (order-independent); result in f64 written to *out_dev (device).
  * NaN in the box yields NaN. */
 int chmy_maxabs_dev(const chmy_field_t* f, const chmy_box_t* box, double* out_dev, void* stream);
-/* Same, synchronizing and returning the scalar on the host. */
+/* The same over the interiors of n fields (any of the three dtypes each) in
+ * one launch per 16 fields: out_dev[q] for f[q] (build extension). */
+int chmy_maxabs_many(int n, const chmy_field_t* f, double* out_dev, void* stream);
+/* chmy_maxabs_dev, synchronizing and returning the scalar on the host. */
 int chmy_maxabs(const chmy_field_t* f, const chmy_box_t* box, double* out_host, void* stream);
 /* Σ f² over a box in f64, deterministic order (run-to-run identical); host result. */
 int chmy_sumsq(const chmy_field_t* f, const chmy_box_t* box, double* out_host, void* stream);

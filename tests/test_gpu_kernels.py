@@ -709,3 +709,32 @@ def test_diffusion_iterate_passes_equal_single_steps(arch, T, dims, steps, halo1
     assert par[0].value == par[1].value
     for a, b in zip(sets[0][0] + sets[0][1], sets[1][0] + sets[1][1]):
         assert torch.equal(a.data, b.data)
+
+
+@pytest.mark.parametrize("dims", [(1020, 3), (1021, 3), (4093, 2), (9000,), (3, 2000), (1, 1, 1), (2, 3, 700), (127, 31, 5)])
+def test_maxabs_many_runs(arch, dims):
+    """One reduction over fields of the three dtypes: rows shorter and longer
+    than a run, bands with a remainder, runs that start inside a 16 B granule
+    (Vertex rows, halo 2); the maximum planted at the first, the last and some
+    inner elements, infinity and NaN; larger values in the padding are ignored."""
+    nd = len(dims)
+    g = chmy.UniformGrid(arch, origin=(0.0,) * nd, extent=(1.0,) * nd, dims=dims)
+    rng = np.random.default_rng(7)
+    locs = [(Cc(),) * nd, (Vv(),) * nd]
+    fields = [chmy.Field(arch, g, loc, dt, halo=h) for dt in (torch.float64, torch.float32, torch.bfloat16)
+              for loc in locs for h in (1, 2)]
+    for trial in range(6):
+        want = []
+        for k, f in enumerate(fields):
+            inner = rng.uniform(-1.0, 1.0, f.dims)
+            spot = [(0,) * nd, tuple(m - 1 for m in f.dims)][trial] if trial < 2 else tuple(
+                int(rng.integers(0, m)) for m in f.dims)
+            inner[spot] = float("nan") if trial == 5 and k % 2 else (-np.inf if trial == 4 else 3.0 + k * 0.25)
+            f.data.fill_(500.0)
+            f.interior().copy_(torch.from_numpy(inner))
+            want.append(np.max(np.abs(inner)))
+        got = chmy.kernels.maxabs_many(fields)
+        if trial < 4:   # other magnitudes stay below 1: the planted one is exact in every dtype
+            assert got == want
+        else:
+            assert np.array_equal(got, want, equal_nan=True)
