@@ -111,6 +111,7 @@ SIGNATURES = {
     "chmy_sia_step": [PG, PF, PF, PF, PF, D, C.c_int, D, D, D, D, VP],
     "chmy_sia_step_adjoint": [PG, PF, PF, PF, PF, PF, PF, D, C.c_int, D, D, D, D, PF, VP],
     "chmy_sia_run": [PG, PF, C.c_int, PF, PF, D, C.c_int, D, D, D, P(C.c_double), VP],
+    "chmy_sia_run_adaptive": [PG, PF, C.c_int, PF, PF, D, C.c_int, D, D, D, D, D, PF, P(C.c_double), VP],
     "chmy_sia_reverse": [PG, PF, C.c_int, C.c_int, C.c_int, PF, PF, PF, PF, PF, PF, D, C.c_int, D, D, D,
                          P(C.c_double), P(C.c_int), VP],
     "chmy_sia_reverse_noalloc": [PG, PF, C.c_int, C.c_int, C.c_int, PF, PF, PF, PF, D, C.c_int, D, D, D,

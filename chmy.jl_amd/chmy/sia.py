@@ -111,6 +111,19 @@ class SIA:
         _lib.call("chmy_sia_run", C.byref(self.grid.desc()), _arr(states), len(states), *self._args(), d,
                   current_stream())
 
+    def run_adaptive(self, states):
+        """states[q] -> states[q+1] with the Δt of dt_rule(states[q]), the rule
+        evaluated on the device (no wait between steps); returns the Δt's.
+        self.D holds the last state's D, as dt_rule leaves it."""
+        n = len(states) - 1
+        if n < 1:
+            return []
+        work = torch.empty(2 * n, dtype=torch.float64, device=states[0].data.device)
+        _lib.call("chmy_sia_run_adaptive", C.byref(self.grid.desc()), _arr(states), n + 1, *self._args(),
+                  min(spacing(self.grid)) ** 2, self.dt_max, C.byref(self.D.desc()),
+                  C.cast(C.c_void_p(work.data_ptr()), C.POINTER(C.c_double)), current_stream())
+        return work[:n].tolist()
+
     def _field(self):
         return Field(self.arch, self.grid, Center(), torch.float64)
 
@@ -135,10 +148,7 @@ class SIA:
         if states[0] is not self.H:
             states[0].data.copy_(self.H.data)
         if dts is None:
-            out = []
-            for k in range(nsteps):
-                out.append(self.dt_rule(states[k]))
-                self.run(states[k:k + 2], out[-1:])
+            out = self.run_adaptive(states)
         else:
             out = [float(x) for x in dts[:nsteps]]
             self.run(states, out)

@@ -311,8 +311,24 @@ struct SiaStep {   // one forward step H -> Ho (+ the H Neumann batch when bc !=
     DF<T> Dout;
 };
 
-template <class T>
-__device__ __forceinline__ void sia_step_block(const SiaStep<T>& p, int64_t nx, int64_t ny, T* lds) {
+// The time step from max(D) on the device (sia.jl:76-78): Δt =
+// min(h2 / max(D) / 4.1, dt_max), with max(D) as the bits of its magnitude in
+// *dmax.  Every block forms the same Δt; the first stores it.
+struct SiaRule {
+    const unsigned long long* dmax;
+    double h2, dt_max;
+    double* dt_out;
+};
+__device__ __forceinline__ double sia_rule_dt(const SiaRule& r) {
+    const double m = __longlong_as_double((long long)*r.dmax);
+    const double d = m > 0.0 ? r.h2 / m / 4.1 : __longlong_as_double(0x7ff0000000000000ll);
+    return r.dt_max < d ? r.dt_max : d;
+}
+
+// READ_D: D(H) is in Dout already (stored with its maximum for the time-step
+// rule), the same bits as evaluated here.
+template <class T, bool READ_D = false>
+__device__ __forceinline__ void sia_step_block(const SiaStep<T>& p, int64_t nx, int64_t ny, T* lds, T dt) {
     constexpr int W = kSX + 2, Hh = kSY + 2;
     using LS = SiaLds<T, 2>;
     T(*Ds)[W] = reinterpret_cast<T(*)[W]>(lds + LS::W * LS::HH);
@@ -326,9 +342,9 @@ __device__ __forceinline__ void sia_step_block(const SiaStep<T>& p, int64_t nx, 
         const int a = q % W, b = q / W;
         const int64_t i = i0 - 1 + a, j = j0 - 1 + b;
         const bool in = i >= 1 && i <= nx && j >= 1 && j <= ny;
-        const T d = in ? L.D(i, j) : T(0);
+        const T d = in ? (READ_D ? p.Dout(i, j, 0) : L.D(i, j)) : T(0);
         Ds[b][a] = d;
-        if (p.wd && in && a >= 1 && a <= kSX && b >= 1 && b <= kSY) p.Dout(i, j, 0) = d;
+        if (!READ_D && p.wd && in && a >= 1 && a <= kSX && b >= 1 && b <= kSY) p.Dout(i, j, 0) = d;
     }
     __syncthreads();
     for (int q = tid; q < kSX * kSY; q += kST) {
@@ -346,7 +362,7 @@ __device__ __forceinline__ void sia_step_block(const SiaStep<T>& p, int64_t nx, 
             return -fma(T(0.5), Dr - Dl, Dl) * L.gy(i, f);
         };
         const T dv = (qx(i + 1, a + 1) - qx(i, a)) * s.ix + (qy(j + 1, b + 1) - qy(j, b)) * s.iy;
-        const T h = jmax0(s.H(i, j, 0) + p.dt * (-dv + L.M(i, j)));
+        const T h = jmax0(s.H(i, j, 0) + dt * (-dv + L.M(i, j)));
         const DF<T>& Ho = p.Ho;
         Ho(i, j, 0) = h;
         if (p.bc) {
@@ -525,7 +541,43 @@ template <class T, int NP>
 __global__ void __launch_bounds__(kST) sia_step_tile(SiaStep<T> f, int64_t nx, int64_t ny) {
     __shared__ T lds[(kSX + 4) * (kSY + 4) + (kSX + 2) * (kSY + 2)];
     if constexpr (NP > 0) f.s.n = NP;
-    sia_step_block(f, nx, ny, lds);
+    sia_step_block(f, nx, ny, lds, f.dt);
+}
+
+// The step whose Δt follows from the stored D and its maximum.
+template <class T>
+__global__ void __launch_bounds__(kST) sia_step_rule_tile(SiaStep<T> f, SiaRule r, int64_t nx, int64_t ny) {
+    __shared__ T lds[(kSX + 4) * (kSY + 4) + (kSX + 2) * (kSY + 2)];
+    const double dt = sia_rule_dt(r);
+    if (blockIdx.x == 0 && blockIdx.y == 0 && threadIdx.x == 0) *r.dt_out = dt;
+    sia_step_block<T, true>(f, nx, ny, lds, dt);
+}
+
+// D at cells 1..n and the maximum of its magnitude (bits; NaN above infinity)
+template <class T, int NP>
+__global__ void __launch_bounds__(256) sia_d_max_kernel(SiaF<T> s, DF<T> D, int64_t nx, int64_t ny,
+                                                        unsigned long long* dmax) {
+    __shared__ unsigned long long part[4];
+    if constexpr (NP > 0) s.n = NP;
+    int64_t i, j;
+    bool ok;
+    cell_index<T>(i, j, nx, ny, ok);
+    unsigned long long m = 0;
+    if (ok) {
+        const T d = s.D(i, j);
+        D(i, j, 0) = d;
+        m = (unsigned long long)__double_as_longlong((double)d) & 0x7fffffffffffffffull;
+    }
+    for (int o = 32; o > 0; o >>= 1) {
+        const unsigned long long q = __shfl_xor(m, o, 64);
+        m = q > m ? q : m;
+    }
+    if (threadIdx.x == 0) part[threadIdx.y] = m;
+    __syncthreads();
+    if (threadIdx.x == 0 && threadIdx.y == 0) {
+        for (int q = 1; q < 4; ++q) m = part[q] > m ? part[q] : m;
+        if (m > __hip_atomic_load(dmax, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) atomicMax(dmax, m);
+    }
 }
 
 // blockIdx.z == 0: adjoint tile; blockIdx.z == 1: forward tile of an independent step
@@ -537,7 +589,7 @@ __global__ void __launch_bounds__(kST) sia_adj_tile(SiaAdj<T> a, SiaStep<T> f, i
         f.s.n = NP;
     }
     if (blockIdx.z == 0) sia_adj_block(a, nx, ny, lds);
-    else sia_step_block(f, nx, ny, lds);
+    else sia_step_block(f, nx, ny, lds, f.dt);
 }
 
 // n = 3 (Glen's law as sia.jl uses it) takes the unrolled kernels
@@ -878,6 +930,46 @@ int chmy_sia_run(const chmy_grid_t* g, const chmy_field_t* states, int nstates, 
     for (int q = 0; q + 1 < nstates; ++q) {
         SiaStep<double> f = sia_stepper(g, &states[q], &states[q + 1], B, A, p, dts[q]);
         launch_step_tile(sia_tiles(g->n[0], g->n[1], 1), st, f, g->n[0], g->n[1]);
+    }
+    CHMY_HIP(hipGetLastError());
+    return 0;
+}
+
+// Per step: D and its maximum, then the step, which reads both; no host wait
+// until the caller reads the Δt.  The host-side rule took three launches, a
+// copy and a wait per step (57 us a step at 250x230; now 11).
+int chmy_sia_run_adaptive(const chmy_grid_t* g, const chmy_field_t* states, int nstates, const chmy_field_t* B,
+                          const chmy_field_t* A, double As, int npow, double mb_a, double mb_b, double mb_c, double h2,
+                          double dt_max, const chmy_field_t* D, double* work_dev, void* stream) {
+    if (nstates < 1) return set_error(CHMY_E_ARG, "nstates=%d < 1", nstates);
+    CHMY_TRY(check_grid(g));
+    CHMY_TRY(sia_check_states(g, states, nstates, "states"));
+    CHMY_TRY(sia_check(g, &states[0], B, A, npow));
+    CHMY_TRY(check_center(g, D, "D", CHMY_F64));
+    if (nstates > 1 && !work_dev) return set_error(CHMY_E_ARG, "work_dev is NULL");
+    for (int q = 0; q + 1 < nstates; ++q)
+        if (states[q].data == states[q + 1].data)
+            return set_error(CHMY_E_ARG, "states[%d] and states[%d] share storage", q, q + 1);
+    for (int q = 0; q < nstates; ++q)
+        if (states[q].data == D->data) return set_error(CHMY_E_ARG, "D shares storage with states[%d]", q);
+    if (nstates == 1) return 0;
+    const SiaPar p{As, npow, mb_a, mb_b, mb_c, 0.0};
+    hipStream_t st = (hipStream_t)stream;
+    const int64_t nx = g->n[0], ny = g->n[1];
+    const int n = nstates - 1;
+    unsigned long long* dmax = reinterpret_cast<unsigned long long*>(work_dev + n);
+    hipLaunchKernelGGL(sia_fill_zero, dim3((unsigned)std::min((n + 255) / 256, 64)), dim3(256), 0, st, work_dev + n,
+                       (int64_t)n);
+    const dim3 grd((unsigned)((nx + 63) / 64), (unsigned)((ny + 3) / 4), 1);
+    for (int q = 0; q < n; ++q) {
+        SiaStep<double> f = sia_stepper(g, &states[q], &states[q + 1], B, A, p, 0.0);
+        f.Dout = view<double>(*D);
+        if (npow == 3)
+            hipLaunchKernelGGL((sia_d_max_kernel<double, 3>), grd, sia_blk(), 0, st, f.s, f.Dout, nx, ny, dmax + q);
+        else
+            hipLaunchKernelGGL((sia_d_max_kernel<double, 0>), grd, sia_blk(), 0, st, f.s, f.Dout, nx, ny, dmax + q);
+        const SiaRule r{dmax + q, h2, dt_max, work_dev + q};
+        hipLaunchKernelGGL(sia_step_rule_tile<double>, sia_tiles(nx, ny, 1), dim3(kST), 0, st, f, r, nx, ny);
     }
     CHMY_HIP(hipGetLastError());
     return 0;

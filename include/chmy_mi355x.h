@@ -407,6 +407,16 @@ int chmy_sia_step_adjoint(const chmy_grid_t* grid, const chmy_field_t* H, const 
 int chmy_sia_run(const chmy_grid_t* grid, const chmy_field_t* states, int nstates, const chmy_field_t* B,
                  const chmy_field_t* A, double As, int npow, double mb_a, double mb_b, double mb_c,
                  const double* dts, void* stream);
+/* chmy_sia_run with the reference's time-step rule evaluated on the device
+ * before each step (sia.jl:76-78): D (a Center field) = D(states[q]) as
+ * chmy_sia_diffusivity stores it, Δt = min(h2 / max|D| / 4.1, dt_max) (h2:
+ * the squared smallest spacing; dt_max where max|D| is 0), then the step.
+ * work_dev: 2 (nstates-1) doubles on the device; its first nstates-1 receive
+ * the Δt sequence.  Equal to chmy_sia_diffusivity + chmy_maxabs + chmy_sia_run
+ * per step bitwise, without their host waits (build extension). */
+int chmy_sia_run_adaptive(const chmy_grid_t* grid, const chmy_field_t* states, int nstates, const chmy_field_t* B,
+                          const chmy_field_t* A, double As, int npow, double mb_a, double mb_b, double mb_c,
+                          double h2, double dt_max, const chmy_field_t* D, double* work_dev, void* stream);
 /* Reverse sweep of a checkpointed run (build extension): ckpt[s] holds the
  * state before step s*stride (nckpt = ceil(nsteps/stride)); each segment is
  * recomputed once into seg (2*(stride-1) Center fields, two alternating

@@ -347,3 +347,31 @@ def test_sia_gradient_matches_cpu_reference(arch):
         fd = (J_cpu(logA0 + h * v) - J_cpu(logA0 - h * v)) / (2 * h)
         ad = float(np.sum(gn * v[2:-2, 2:-2].T))
         assert abs(fd - ad) <= 1e-6 * abs(fd), (fd, ad)
+
+
+@pytest.mark.parametrize("dims", [(1, 1), (31, 9), (64, 8), (65, 17), (130, 70)])
+@pytest.mark.parametrize("npow,with_A,dt_max", [(3, True, 1.0), (3, False, math.inf), (2, True, 0.3)])
+def test_adaptive_run_equals_rule_and_step(arch, dims, npow, with_A, dt_max):
+    """The time-step rule on the device against dt_rule and run step by step:
+    the Δt sequence, every state and D, bitwise, from ice and from none (where
+    max(D) is 0 and Δt the largest allowed)."""
+    g = chmy.UniformGrid(arch, origin=(0.0, 0.0), extent=(40e3, 30e3), dims=dims)
+    rng = np.random.default_rng(5)
+    pad = (dims[1] + 4, dims[0] + 4)
+    S = SIA(arch, g, 800.0 * rng.random(pad), np.log(1e-4) + 0.3 * rng.random(pad) if with_A else None, As=0.2,
+            npow=npow, mb=(0.01, 500.0, 2.0), dt_max=dt_max)
+    for H0 in (300.0 * rng.random(pad), np.zeros(pad)):
+        if dt_max == math.inf and not H0.any():
+            continue
+        S.reset(H0)
+        want_states, want_dts = [S.H] + [S._field() for _ in range(5)], []
+        for k in range(5):
+            want_dts.append(S.dt_rule(want_states[k]))
+            S.run(want_states[k:k + 2], want_dts[-1:])
+        want_D = S.D.data.clone()
+        S.D.data.zero_()
+        states = [S.H] + [S._field() for _ in range(5)]
+        assert S.run_adaptive(states) == want_dts
+        assert torch.equal(S.D.data, want_D)
+        for a, b in zip(states, want_states):
+            assert torch.equal(a.data, b.data)
