@@ -34,26 +34,9 @@
 // kernels (stokes.hip), so the results are bitwise those of update_stress! +
 // update_velocity!; the default fast form (Arith<T, false>) is algebraically
 // equal and agrees to a few ulp per iteration.
-#include <type_traits>
-
-#include "common.hpp"
+#include "stokes_pt.hpp"
 
 namespace chmy {
-
-constexpr int kFX = 64;
-enum { LC = 0, LVX = 1, LVY = 2, LVZ = 3, LXY = 4, LXZ = 5, LYZ = 6, NLOC = 7 };
-
-// Scalars shared by both arithmetic forms.
-template <class T>
-struct Kc {
-    T Gs, dts, Gdt, dPr, dr, nu, eta_s, eve_s;   // reference inputs
-    T iGdt, omdr, third, a_s, b_s, cv_s;         // fast-form constants (host computed)
-};
-
-struct LocStride {
-    uint32_t sy, sz;     // element strides
-    uint32_t o0;         // element offset of logical (0, 0, 0)
-};
 
 template <class T>
 struct Fused3 {
@@ -70,99 +53,6 @@ struct Fused3 {
     T ix, iy, iz;
     Kc<T> k;
 };
-
-#ifndef CHMY_FUSED_NT_STORE
-#define CHMY_FUSED_NT_STORE 0
-#endif
-
-template <class T>
-__device__ __forceinline__ T ldo(const T* p, uint32_t boff) {
-    return *reinterpret_cast<const T*>(reinterpret_cast<const char*>(p) + boff);
-}
-// Loads of the sweep's read-only forcing (tau_old, f_V, f_P): in the sweep
-// precision, or (BF, FP32 sweeps only) from bf16 storage at half the byte
-// offset of the FP32 layout.
-template <class T, bool BF>
-__device__ __forceinline__ T ldf(const T* p, uint32_t boff) {
-    if constexpr (BF) {
-        static_assert(sizeof(T) == 4, "bf16 forcing goes with FP32 sweeps");
-        return T(bf16_to_f32(*reinterpret_cast<const uint16_t*>(reinterpret_cast<const char*>(p) + (boff >> 1))));
-    } else {
-        return *reinterpret_cast<const T*>(reinterpret_cast<const char*>(p) + boff);
-    }
-}
-
-template <class T>
-__device__ __forceinline__ void sto(T* p, uint32_t boff, T v) {
-#if CHMY_FUSED_NT_STORE
-    // streaming store: the advanced state is not re-read in this launch
-    __builtin_nontemporal_store(v, reinterpret_cast<T*>(reinterpret_cast<char*>(p) + boff));
-#else
-    *reinterpret_cast<T*>(reinterpret_cast<char*>(p) + boff) = v;
-#endif
-}
-
-// EXACT: the reference's expressions (stokes_3d_inc_ve_T.jl:23-57), bitwise.
-// FAST: the same update with eta_ve*(1/(G dt) + 1/eta) = 1 used to cancel
-// tau/eta: tau_new = tau(1 - dtau_r) + eta_ve dtau_r (tau_old/(G dt) + 2 eps'),
-// eta_ve = eta/(1 + eta/(G dt)), Pr_new = Pr - divV eta_ve dtau_Pr and
-// V_new = V + r nudtau (1/eta_V + 1/(G dt)): 7 divisions per point instead
-// of 31, results within a few ulp per iteration of the exact form.
-template <class T, bool EXACT>
-struct Arith;
-
-template <class T>
-struct Arith<T, true> {
-    struct Loc { T eta, eve; };
-    __device__ static Loc field(T eta, const Kc<T>& k) { return Loc{eta, visc_ve(eta, k.Gs, k.dts)}; }
-    __device__ static Loc scalar(const Kc<T>& k) { return Loc{k.eta_s, k.eve_s}; }
-    __device__ static T diag(T t, T to, T e, T dV, Loc L, const Kc<T>& k) {
-        T r = ((-(t - to)) / k.Gdt - t / L.eta) + T(2) * (e - dV / T(3));
-        return t + (r * L.eve) * k.dr;
-    }
-    __device__ static T off(T t, T to, T e, Loc L, const Kc<T>& k) {
-        T r = ((-(t - to)) / k.Gdt - t / L.eta) + T(2) * e;
-        return t + (r * L.eve) * k.dr;
-    }
-    __device__ static T pr(T P, T dv, Loc L, const Kc<T>& k) { return P - (dv * L.eve) * k.dPr; }
-    __device__ static T vcoef_field(T em, const Kc<T>& k) { return visc_ve(em, k.Gs, k.dts); }
-    __device__ static T vcoef_scalar(const Kc<T>& k) { return k.eve_s; }
-    __device__ static T vel(T v, T r, T c, const Kc<T>& k) { return v + (r * k.nu) / c; }
-};
-
-// Divisions of the fast form: IEEE in FP64; in FP32 (the defect-correction
-// sweeps) a times the hardware reciprocal of b (v_rcp_f32, 1 ulp), for its 7
-// divisions per point
-__device__ __forceinline__ double fast_div(double a, double b) { return a / b; }
-__device__ __forceinline__ float fast_div(float a, float b) { return a * __builtin_amdgcn_rcpf(b); }
-
-template <class T>
-struct Arith<T, false> {
-    struct Loc { T a, b; };   // a = eta_ve dtau_r, b = eta_ve dtau_Pr
-    __device__ static Loc field(T eta, const Kc<T>& k) {
-        const T eve = fast_div(eta, fma(eta, k.iGdt, T(1)));
-        return Loc{eve * k.dr, eve * k.dPr};
-    }
-    __device__ static Loc scalar(const Kc<T>& k) { return Loc{k.a_s, k.b_s}; }
-    __device__ static T diag(T t, T to, T e, T dV, Loc L, const Kc<T>& k) {
-        return fma(t, k.omdr, L.a * fma(to, k.iGdt, T(2) * fma(-dV, k.third, e)));
-    }
-    __device__ static T off(T t, T to, T e, Loc L, const Kc<T>& k) {
-        return fma(t, k.omdr, L.a * fma(to, k.iGdt, T(2) * e));
-    }
-    __device__ static T pr(T P, T dv, Loc L, const Kc<T>& k) { return fma(-dv, L.b, P); }
-    __device__ static T vcoef_field(T em, const Kc<T>& k) { return k.nu * (fast_div(T(1), em) + k.iGdt); }
-    __device__ static T vcoef_scalar(const Kc<T>& k) { return k.cv_s; }
-    __device__ static T vel(T v, T r, T c, const Kc<T>& k) { return fma(r, c, v); }
-};
-
-template <class T>
-__device__ __forceinline__ T lerp4(T a0, T a1, T b0, T b1) {
-    // knots (lo,lo),(hi,lo),(lo,hi),(hi,hi); first dim innermost (interpolation.jl:37-56)
-    T A = fma(T(0.5), a1 - a0, a0);
-    T B = fma(T(0.5), b1 - b0, b0);
-    return fma(T(0.5), B - A, A);
-}
 
 // Tuning knobs fixed at build time: rows per block (FP64 / FP32 sweeps) and
 // the minimum waves per SIMD the register allocation must allow (0 = no bound).
@@ -425,24 +315,6 @@ __global__ void __launch_bounds__(TW * BY, CHMY_FUSED_WPE) fused3d_kernel(Fused3
 // staggered location (C, Vx, Vy, xy), advanced by one row per step; lanes
 // right of the storage address the last stored column (their values reach no
 // output), so every load is unconditional.
-enum { L2C = 0, L2X = 1, L2Y = 2, L2XY = 3, NLOC2 = 4 };
-
-template <class T>
-struct Fused2 {
-    const T *Vx, *Vy, *Pr, *txx, *tyy, *txy;
-    T *oVx, *oVy, *oPr, *otxx, *otyy, *otxy;
-    const T *Oxx, *Oyy, *Oxy;
-    const T *eta, *eml, *rg;
-    const T *fVx, *fVy, *fP;
-    T *dV, *rVx, *rVy;
-    LocStride L[NLOC2];
-    int32_t n[2];
-    int32_t ntx, nchunks, ychunk;
-    int32_t has_rg, write_res, has_f;
-    T ix, iy;
-    Kc<T> k;
-};
-
 template <class T>
 __device__ __forceinline__ T shup(T v) { return __shfl_up(v, 1, kFX); }     // value of lane l-1
 template <class T>
@@ -456,21 +328,6 @@ constexpr int kW2 = CHMY_FUSED_W2;   // waves (x-tiles) per block
 #define CHMY_FUSED_YCHUNK2 8
 #endif
 constexpr int kYChunk2 = CHMY_FUSED_YCHUNK2;   // rows per wave (the march is unrolled over them)
-
-// Raw load of a forcing value (kept as bf16 bits until use, so the load can
-// stay in flight across a row of the march) and its conversion.
-template <class T, bool BF>
-using Fraw = typename std::conditional<BF, uint16_t, T>::type;
-template <class T, bool BF>
-__device__ __forceinline__ Fraw<T, BF> ldr(const T* p, uint32_t boff) {
-    if constexpr (BF) return *reinterpret_cast<const uint16_t*>(reinterpret_cast<const char*>(p) + (boff >> 1));
-    else return *reinterpret_cast<const T*>(reinterpret_cast<const char*>(p) + boff);
-}
-template <class T, bool BF>
-__device__ __forceinline__ T cvf(Fraw<T, BF> v) {
-    if constexpr (BF) return T(bf16_to_f32(v));
-    else return v;
-}
 
 // What one row j of the y-march reads: Center values at row j, the y-face,
 // vertex and η values at row j+1, and Vx at row j+1 (Vx at row j is carried).
@@ -633,14 +490,6 @@ __global__ void __launch_bounds__(kFX * kW2) fused2d_kernel(Fused2<T> a) {
 }
 
 // ------------------------------------------------------------------ 2D, two PT iterations per pass
-// The V batch a 2D free-slip solve applies after every iteration
-// (stokes_2d_inc_ve_T.jl's bc of update_velocity!): Vx Dirichlet on its x
-// nodes 1 / n+1 and Neumann in y, Vy Neumann in x and Dirichlet on its y
-// nodes 1 / n+1, scalar values [side 1, side 2]; h the spacings.
-struct FreeSlip2 {
-    double ax[2], qy[2], by[2], qx[2];
-    double hx, hy;
-};
 
 #ifndef CHMY_FUSED_TB
 #define CHMY_FUSED_TB 1   // 0: chmy_stokes_iterate runs single iterations only
@@ -942,20 +791,6 @@ template <class T>
 constexpr int kTB3Y = std::is_same<T, double>::value ? CHMY_FUSED_TB3_BY64 : CHMY_FUSED_TB3_BY32;
 constexpr int kTB3Z = CHMY_FUSED_TB3_ZCHUNK;
 static_assert(kTB3Z >= 2, "B's first plane of a chunk above the bottom one must be >= 1");
-
-// x neighbours inside a row's wave by DPP whole-wave shifts: xm1 gives lane l
-// the value of lane l-1, xp1 that of lane l+1 (lanes 0 / 63 receive 0, and
-// reach no output).
-__device__ __forceinline__ int dpp_shr1(int v) { return __builtin_amdgcn_update_dpp(0, v, 0x138, 0xf, 0xf, false); }
-__device__ __forceinline__ int dpp_shl1(int v) { return __builtin_amdgcn_update_dpp(0, v, 0x130, 0xf, 0xf, false); }
-__device__ __forceinline__ double xm1(double v) {
-    return __hiloint2double(dpp_shr1(__double2hiint(v)), dpp_shr1(__double2loint(v)));
-}
-__device__ __forceinline__ double xp1(double v) {
-    return __hiloint2double(dpp_shl1(__double2hiint(v)), dpp_shl1(__double2loint(v)));
-}
-__device__ __forceinline__ float xm1(float v) { return __int_as_float(dpp_shr1(__float_as_int(v))); }
-__device__ __forceinline__ float xp1(float v) { return __int_as_float(dpp_shl1(__float_as_int(v))); }
 
 // Two PT iterations in one pass over a 64 x BY tile marching z.  Thread
 // (tx, ty) owns column (i, j) = (i0 - 2 + tx, j0 - 2 + ty); the row index is
@@ -1769,6 +1604,11 @@ static int fused_launch(const chmy_grid_t* g, const chmy_field_t* V, const chmy_
         a.iy = T(g->inv_spacing[1]);
         a.k = make_consts<T>(eta_s, eve_s, G, dt, dPr, dr, nu);
         const int64_t nbx = g->n[0] + 2, nby = g->n[1] + 2;
+        if (tb && tb->iters > 2) {   // several iterations, the free-slip batch between them
+            multi2d_launch<T>(a, *tb, fv, exact, bf, rg != nullptr, s);
+            CHMY_HIP(hipGetLastError());
+            return 0;
+        }
         if (tb) {   // two iterations, the free-slip batch between them
             a.ntx = (int32_t)((nbx + kFX - 5) / (kFX - 4));
             a.ychunk = exact ? kTBC<T, true> : kTBC<T, false>;
@@ -1979,6 +1819,7 @@ static bool free_slip_2d(const chmy_grid_t* g, const int32_t* counts, const int3
     }
     fs->hx = g->spacing[0];
     fs->hy = g->spacing[1];
+    fs->iters = 2;
     return true;
 }
 
@@ -2061,10 +1902,10 @@ int chmy_stokes_iterate(const chmy_grid_t* g, const chmy_field_t* V0, const chmy
         for (int q = 0; q < total; ++q) fset[p][q] = Vs[p][bc_comp[q]];
     const chmy_field_t* T[2] = {tau0, tau1};
     const chmy_field_t* P[2] = {Pr0, Pr1};
-    // free-slip batches run iterations in pairs (one pass, the batch in-kernel
-    // between them); the pair writes the other set, as one iteration does, so
-    // the parity flips once per pair.  CHMY_ITER_SINGLE keeps single
-    // iterations (CHMY_ITER_PAIRS, once the 3D opt-in, is accepted and ignored)
+    // free-slip batches run iterations in passes (the batch in-kernel between
+    // them), two in 3D and up to `most` in 2D; a pass writes the other set, as
+    // one iteration does, so the parity flips once per pass.  CHMY_ITER_SINGLE
+    // keeps single iterations (CHMY_ITER_PAIRS, once the 3D opt-in, is accepted and ignored)
     const bool single = ((flags | flags_last) & CHMY_ITER_SINGLE) != 0;
     flags &= ~(CHMY_ITER_PAIRS | CHMY_ITER_SINGLE);
     flags_last &= ~(CHMY_ITER_PAIRS | CHMY_ITER_SINGLE);
@@ -2073,11 +1914,22 @@ int chmy_stokes_iterate(const chmy_grid_t* g, const chmy_field_t* V0, const chmy
     const bool tb2 = CHMY_FUSED_TB && !single && nd == 2 && free_slip_2d(g, bc_counts, bc_comp, bcs, &fs);
     const bool tb3 = !single && !(rhog && f_V) && nd == 3 && free_slip_3d(g, bc_counts, bc_comp, bcs, &fs3);
     const bool tb = tb2 || tb3;
+    const int most = tb2 ? multi2d_most(g) : 1;
     int p = *parity_inout;
     for (int it = 0; it < niter;) {
         const int fl = it == niter - 1 ? flags_last : flags;
         const int fl2 = it + 1 == niter - 1 ? flags_last : flags;
-        if (tb && it + 1 < niter && fl == fl2 && !(fl & CHMY_ITER_RESIDUAL)) {
+        // 2D: as many iterations of the same flags as a pass takes, three or more
+        int m = 1;
+        while (m < most && it + m < niter && (it + m == niter - 1 ? flags_last : flags) == fl) ++m;
+        if (tb2 && m > 2 && !(fl & CHMY_ITER_RESIDUAL)) {
+            fs.iters = m;
+            CHMY_TRY(stokes_iter_impl(g, Vs[p], T[p], P[p], Vs[1 - p], T[1 - p], P[1 - p], tau_old, eta, eta_ml, rhog,
+                                      f_V, f_P, divV, r_V, fl, eta_s, eta_ve_s, G, dt, dtau_Pr, dtau_r, nudtau,
+                                      stream, &fs, nullptr));
+            fs.iters = 2;
+            it += m;
+        } else if (tb && it + 1 < niter && fl == fl2 && !(fl & CHMY_ITER_RESIDUAL)) {
             CHMY_TRY(stokes_iter_impl(g, Vs[p], T[p], P[p], Vs[1 - p], T[1 - p], P[1 - p], tau_old, eta, eta_ml, rhog,
                                       f_V, f_P, divV, r_V, fl, eta_s, eta_ve_s, G, dt, dtau_Pr, dtau_r, nudtau,
                                       stream, tb2 ? &fs : nullptr, tb3 ? &fs3 : nullptr));

@@ -284,11 +284,11 @@ int chmy_stokes_iter(const chmy_grid_t* grid, const chmy_field_t* V, const chmy_
  * *parity_inout names the set holding the new state.
  * Build extension: with a free-slip V batch (each component Dirichlet on its
  * own dim, Neumann on the others, scalar values) and no residual fields,
- * iterations run in pairs, one pass each with the batch applied in-kernel
- * between the two (as chmy_stokes_iter2; in 3D not with rho g and forcing
- * together); CHMY_ITER_SINGLE (in `flags`) keeps single iterations, and
- * CHMY_ITER_PAIRS is accepted and ignored.  A pair writes set 1-p like one
- * iteration, so the parity flips once per pair; results are bitwise those of
+ * iterations run in passes with the batch applied in-kernel between them, two
+ * in 3D (as chmy_stokes_iter2; not with rho g and forcing together) and up to
+ * eight in 2D; CHMY_ITER_SINGLE (in `flags`) keeps single iterations, and
+ * CHMY_ITER_PAIRS is accepted and ignored.  A pass writes set 1-p like one
+ * iteration, so the parity flips once per pass; results are bitwise those of
  * single iterations. */
 int chmy_stokes_iterate(const chmy_grid_t* grid, const chmy_field_t* V0, const chmy_field_t* tau0,
                         const chmy_field_t* Pr0, const chmy_field_t* V1, const chmy_field_t* tau1,

@@ -358,3 +358,19 @@ def test_iter2_rejects_other_batches(arch):
                   C.byref(sets[0].Pr.desc()), _arr(list(sets[1].V)), _arr(list(sets[1].tau)),
                   C.byref(sets[1].Pr.desc()), _arr(list(told)), None, None, None, None, None, counts, comp, conds,
                   0, 0.8, 0.5, 1.0, 0.37, p["dtau_Pr"], p["dtau_r"], p["nudtau"], chmy.current_stream())
+
+
+@pytest.mark.parametrize("T,forcing", [(np.float64, None), (np.float64, "same"), (np.float32, "bf16")])
+@pytest.mark.parametrize("exact,visc,rhog", [(False, "field", True), (True, "field", False), (False, "scalar", False)])
+@pytest.mark.parametrize("dims,niter", [
+    ((49, 3), 10), ((48, 2), 7), ((2, 130), 9), ((101, 66), 15),             # one row a thread
+    ((260, 140), 13), ((155, 399), 10), ((207, 258), 6),                     # two rows
+    ((641, 500), 17), ((478, 638), 11)])                                     # three rows
+def test_several_iterations_per_pass_2d(arch, T, forcing, exact, visc, rhog, dims, niter):
+    """2D passes of up to 7, 6 and 8 iterations (the three tile shapes, grids
+    that end inside, at and past their tiles, whole passes and remainders of 1
+    and 2) against single iterations, bitwise over the storage."""
+    g = chmy.UniformGrid(arch, origin=(-0.5, -0.5), extent=(1.0, 1.3), dims=dims)
+    a = _run(arch, g, T, exact, visc, forcing, GENERAL, niter, True, 23, rhog=rhog)
+    b = _run(arch, g, T, exact, visc, forcing, GENERAL, niter, False, 23, rhog=rhog)
+    _compare(a, b, f"dims {dims} niter {niter}")
