@@ -295,6 +295,83 @@ __global__ void __launch_bounds__(256) bc_set_kernel(BCSetLaunch L) {
     static_cast<T*>(F.p)[pofs] = v;
 }
 
+// The same for sets of numbers on uniform axes (what the solvers apply after
+// every iteration), where the launch itself is the time: a tenth of the kernel
+// argument, 32-bit indices, and the chain as one pass down the dims.  The dims
+// above D that also write the point move it to their inner node; from the
+// value stored there, each of them and then D applies its rule, a Dirichlet on
+// a vertex dropping what came before.  Measured, us per set, bc_set_kernel ->
+// this: V of 127x95 4.7 -> 3.8, T of 64^2 5.8 -> 3.1, V of 159x143x127 12.2 ->
+// 5-6, T 8.0 -> 4.5, V of 255^3 24.6 -> 16-20 (a 128 B line per point on the x
+// faces).
+struct BCNum {
+    void* p;               // logical (0,0,0)
+    int64_t sy, sz;
+    double val[3][2];
+    int32_t m[3];
+    // -1 none, 0 Dirichlet on a vertex, 1 Dirichlet, 2 Neumann.  Words, indexed
+    // by constants only: with bytes indexed by the block's dim the compiler
+    // split m's address into two parts that were not word-aligned, whose low
+    // bits a scalar load drops.
+    int32_t kind[3][2];
+};
+struct BCNumLaunch {
+    int32_t tn[3];         // n_d + 3
+    double h[3];
+    BCNum f[kSetFields];
+};
+
+// blockIdx.y = (dim, side), blockIdx.z = field; x threads over the dim's plane
+template <class T, int ND>
+__global__ void __launch_bounds__(256) bc_num_kernel(const BCNumLaunch L) {
+    const BCNum& F = L.f[blockIdx.z];
+    const int D = blockIdx.y >> 1, sd = blockIdx.y & 1;
+    int kd = -1, node = 0;   // this rule's kind and the node it writes
+#pragma unroll
+    for (int k = 0; k < ND; ++k) {
+        if (k != D) continue;
+        kd = sd == 0 ? F.kind[k][0] : F.kind[k][1];
+        node = sd == 0 ? (kd == 0 ? 1 : 0) : (kd == 0 ? F.m[k] : F.m[k] + 1);
+    }
+    if (kd < 0) return;
+    const uint32_t t = blockIdx.x * 256u + threadIdx.x;
+    uint32_t w0 = 1, w1 = 1;   // the dim's plane
+    if (ND > 1) w0 = (uint32_t)(D == 0 ? L.tn[1] : L.tn[0]);
+    if (ND == 3) w1 = (uint32_t)(D == 2 ? L.tn[1] : L.tn[2]);
+    if (t >= w0 * w1) return;
+    const int v = ND == 3 ? (int)(t / w0) : 0, u = (int)(t - (uint32_t)v * w0);
+    const int c[3] = {D == 0 ? node : u, D == 1 ? node : D == 0 ? u : v, D == 2 ? node : v};
+    int o[3] = {c[0], c[1], c[2]};
+    int side[3];           // the side of dim k's rule that writes the point, or -1
+    bool fixed = false;    // a Dirichlet on a vertex among them: nothing stored is read
+#pragma unroll
+    for (int k = 0; k < ND; ++k) {
+        const int k0 = F.kind[k][0], k1 = F.kind[k][1];
+        int q = -1;
+        if (k1 >= 0 && c[k] == (k1 == 0 ? F.m[k] : F.m[k] + 1)) q = 1;
+        if (k0 >= 0 && c[k] == (k0 == 0 ? 1 : 0)) q = 0;
+        if (k == D) q = sd;
+        if (k < D && q >= 0) return;   // a lower dim writes this point last
+        side[k] = k < D ? -1 : q;
+        if (side[k] >= 0) {
+            o[k] = side[k] == 0 ? 1 : F.m[k];
+            fixed = fixed || (side[k] == 0 ? k0 : k1) == 0;
+        }
+    }
+    T* p = static_cast<T*>(F.p);
+    T x = fixed ? T(0) : p[o[0] + o[1] * F.sy + o[2] * F.sz];
+#pragma unroll
+    for (int k = ND - 1; k >= 0; --k) {
+        if (side[k] < 0) continue;
+        const T val = T(side[k] == 0 ? F.val[k][0] : F.val[k][1]);
+        const int kind = side[k] == 0 ? F.kind[k][0] : F.kind[k][1];
+        if (kind == 0) x = val;
+        else if (kind == 1) x = fma(T(2), val - x, x);
+        else x = fma(T(L.h[k]), side[k] == 0 ? -val : val, x);
+    }
+    p[c[0] + c[1] * F.sy + c[2] * F.sz] = x;
+}
+
 static bool same_field(const chmy_field_t& a, const chmy_field_t& b) {
     if (a.nd != b.nd || a.dtype != b.dtype) return false;
     for (int d = 0; d < 3; ++d)
@@ -360,6 +437,53 @@ static int pack_set(const chmy_grid_t* g, const int32_t* counts, const chmy_fiel
     return L->nf > 0 ? 1 : 0;
 }
 
+// Sets of numbers on uniform axes whose planes count in 32 bits take
+// bc_num_kernel; returns 1 when launched, 0 when not.
+static int launch_num(const BCSetLaunch& L, int dtype, hipStream_t s) {
+    BCNumLaunch q;
+    std::memset(&q, 0, sizeof q);
+    int64_t tot = 1;
+    for (int d = 0; d < 3; ++d) {
+        if (L.ax.a[d].p || L.tn[d] > INT32_MAX / 2) return 0;
+        q.tn[d] = (int32_t)L.tn[d];
+        q.h[d] = L.h[d];
+    }
+    for (int d = 0; d < L.nd; ++d) {
+        int64_t p = 1;
+        for (int e = 0; e < L.nd; ++e)
+            if (e != d) p *= L.tn[e];
+        tot = std::max(tot, p);
+    }
+    if (tot > INT32_MAX) return 0;
+    for (int i = 0; i < L.nf; ++i) {
+        const BCSetField& a = L.f[i];
+        BCNum& b = q.f[i];
+        b.p = a.p;
+        b.sy = a.st[1];
+        b.sz = a.st[2];
+        for (int d = 0; d < 3; ++d) {
+            b.m[d] = (int32_t)a.m[d];
+            for (int e = 0; e < 2; ++e) {
+                const BCRule& r = a.r[d][e];
+                if (r.kind >= 0 && r.vkind == CHMY_VALUE_FIELD) return 0;
+                b.kind[d][e] = r.kind < 0 ? -1 : r.kind == CHMY_NEUMANN ? 2 : a.vertex[d] ? 0 : 1;
+                b.val[d][e] = r.kind >= 0 && r.vkind == CHMY_VALUE_SCALAR ? r.value : 0.0;
+            }
+        }
+    }
+    const dim3 blk(256), grd((unsigned)((tot + 255) / 256), (unsigned)(2 * L.nd), (unsigned)L.nf);
+    auto go = [&](auto zero) {
+        using T = decltype(zero);
+        if (L.nd == 1) hipLaunchKernelGGL((bc_num_kernel<T, 1>), grd, blk, 0, s, q);
+        else if (L.nd == 2) hipLaunchKernelGGL((bc_num_kernel<T, 2>), grd, blk, 0, s, q);
+        else hipLaunchKernelGGL((bc_num_kernel<T, 3>), grd, blk, 0, s, q);
+    };
+    if (dtype == CHMY_F64) go(0.0);
+    else go(0.0f);
+    CHMY_HIP(hipGetLastError());
+    return 1;
+}
+
 static int launch_set(const BCSetLaunch& L, int dtype, hipStream_t s) {
     int64_t tot = 1;
     for (int d = 0; d < L.nd; ++d) {
@@ -409,7 +533,11 @@ int chmy_bc_batchset(const chmy_grid_t* g, const int32_t* counts, const chmy_fie
         int dtype;
         const int ok = pack_set(g, counts, fields, bcs, &L, &dtype);
         if (ok < 0) return ok;
-        if (ok) return launch_set(L, dtype, (hipStream_t)stream);
+        if (ok) {
+            const int num = launch_num(L, dtype, (hipStream_t)stream);
+            if (num) return num == 1 ? 0 : num;
+            return launch_set(L, dtype, (hipStream_t)stream);
+        }
     }
     for (int D = g->nd - 1; D >= 0; --D) {
         int Ks[2] = {counts[2 * D], counts[2 * D + 1]};

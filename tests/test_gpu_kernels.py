@@ -738,3 +738,32 @@ def test_maxabs_many_runs(arch, dims):
             assert got == want
         else:
             assert np.array_equal(got, want, equal_nan=True)
+
+
+@pytest.mark.parametrize("dims", [(2,), (300,), (2, 2), (253, 2), (3, 254), (2, 2, 2), (14, 15, 3), (2, 127, 126)])
+def test_bc_sets_of_numbers_at_plane_edges(arch, dims):
+    """The one-launch batch of numbers against the per-side launches, bitwise
+    over the storage: planes that end inside, at and past a block, the
+    smallest grids, 8 fields of every location with rules missing on some
+    sides, so that corners meet every pair of rules."""
+    nd = len(dims)
+    g = chmy.UniformGrid(arch, origin=(0.0,) * nd, extent=(1.0, 1.3, 0.8)[:nd], dims=dims)
+    rng = np.random.default_rng(9)
+    D, N = chmy.Dirichlet, chmy.Neumann
+    pool = [D(), N(), D(1.25), N(-0.75), None, D(-0.5), N(0.3)]
+    pairs = []
+    for q in range(8):
+        loc = tuple(Vv() if (q >> d) & 1 else Cc() for d in range(nd))
+        spec = {k: (pool[int(rng.integers(0, 7))], pool[int(rng.integers(0, 7))]) for k in "xyz"[:nd]}
+        a = chmy.Field(arch, g, loc)
+        a.data.copy_(torch.from_numpy(rng.uniform(-1.0, 1.0, tuple(a.data.shape))))
+        b = chmy.Field(arch, g, loc)
+        b.data.copy_(a.data)
+        pairs.append((a, b, spec))
+    chmy.batch(g, *[(a, spec) for a, _, spec in pairs]).apply()
+    per_side = chmy.batch(g, *[(b, spec) for _, b, spec in pairs])
+    for d in reversed(range(nd)):
+        for s in (1, 2):
+            per_side.apply_side(d, s)
+    for q, (a, b, spec) in enumerate(pairs):
+        assert torch.equal(a.data, b.data), f"field {q} {spec}"
