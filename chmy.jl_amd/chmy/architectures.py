@@ -70,8 +70,10 @@ def heuristic_groupsize(backend, nd):
 
 
 def current_stream():
-    """hipStream_t of torch's current stream, as a void* for the C ABI."""
-    return torch.cuda.current_stream().cuda_stream
+    """hipStream_t of torch's current stream, as a void* for the C ABI.  Read
+    as the raw handle: every entry point takes one, and building torch's Stream
+    object for it costs 2.9 us a call against 0.2."""
+    return torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice())
 
 
 def synchronize(backend=None):

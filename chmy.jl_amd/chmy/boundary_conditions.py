@@ -175,6 +175,10 @@ class BatchSet:
         self.grid = grid
         self.per_dim = per_dim
         self._c = None
+        # the distinct fields and conditions named
+        pairs = [(f, c) for sides in per_dim for b in sides for f, c in zip(b.fields, b.conditions)]
+        self._fields = tuple({id(f): f for f, _ in pairs}.values())
+        self._conds = tuple({id(c): c for _, c in pairs}.values())
 
     def __getitem__(self, d):
         return self.per_dim[d]
@@ -182,15 +186,8 @@ class BatchSet:
     def _key(self):
         """Storage pointers the cached descriptors were built from (fields swap
         storage under double buffering)."""
-        key = []
-        for d in range(self.grid.nd):
-            for s in range(2):
-                b = self.per_dim[d][s]
-                for f, cond in zip(b.fields, b.conditions):
-                    key.append(f.data.data_ptr())
-                    if isinstance(cond.value, Field):
-                        key.append(cond.value.data.data_ptr())
-        return tuple(key)
+        return tuple([f.data.data_ptr() for f in self._fields] +
+                     [c.value.data.data_ptr() for c in self._conds if isinstance(c.value, Field)])
 
     def _descriptors(self):
         key = self._key()

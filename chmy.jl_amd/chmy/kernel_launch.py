@@ -31,6 +31,7 @@ class Launcher:
         self.grid = grid
         self.nd = grid.nd
         self.worksize = tuple(n + 2 for n in grid.dims)
+        self.origin = (0,) * grid.nd   # Offset(-1) of the 1-based worksize
         self.outer_width = None if outer_width is None else tuple(outer_width)
         self.sync = sync
         if self.outer_width is not None:
@@ -57,17 +58,16 @@ class Launcher:
 
     def __call__(self, arch, grid, kernel_and_args, bc=None):
         kernel, args = kernel_and_args
-        base = -1  # Offset(-1)
         if self.outer_width is None:
-            kernel.launch(grid, tuple(base + 1 for _ in range(self.nd)), self.worksize, *args)
+            kernel.launch(grid, self.origin, self.worksize, *args)
             if bc is not None:
                 bc.apply()
         else:
-            lo = tuple(base + 1 + o for o in self.inner_offset())
+            lo = tuple(self.inner_offset())
             kernel.launch(grid, lo, self.inner_worksize(), *args)
             for D in reversed(range(self.nd)):
                 for S in (1, 2):
-                    lo = tuple(base + 1 + o for o in self.outer_offset(D, S))
+                    lo = self.outer_offset(D, S)
                     ws = self.outer_worksize(D)
                     if all(w > 0 for w in ws):
                         kernel.launch(grid, lo, ws, *args)
