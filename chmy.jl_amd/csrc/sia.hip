@@ -25,7 +25,7 @@
 
 #include <vector>
 
-#include "common.hpp"
+#include "stokes_pt.hpp"
 
 namespace chmy {
 
@@ -248,74 +248,81 @@ __global__ void __launch_bounds__(256) sia_adj5(SiaF<T> s, SiaW<T> w, DF<T> lo, 
     lo(i, j, 0) = l;
 }
 
-// ---------------------------------------------------------------- tiled one-pass forms
-// The forward step and the adjoint step as one launch each: a block owns a
-// kSX x kSY tile of cells and stages the lazily evaluated fields it needs in
-// LDS (D on the tile + 1 ring for the step; D on +3, mu on +2 and abar on +1
-// for the adjoint), so D is evaluated once per cell instead of once per use.
-// The arithmetic of every value is the one of the per-point kernels above,
-// so the results are bitwise equal to them.  With blockIdx.z = 1 a launch of
-// the adjoint also advances an independent forward step (the recompute of
-// the previous checkpoint segment), which fills the GPU at small grids.
-#ifndef CHMY_SIA_TX
-#define CHMY_SIA_TX 32
-#endif
-#ifndef CHMY_SIA_TY
-#define CHMY_SIA_TY 8
-#endif
-#ifndef CHMY_SIA_THREADS
-#define CHMY_SIA_THREADS 256
-#endif
-constexpr int kSX = CHMY_SIA_TX, kSY = CHMY_SIA_TY, kST = CHMY_SIA_THREADS;
-
-// S = B + H staged in LDS on the tile + R ring (zero outside cells 0..n+1,
-// which no evaluation reads); the formulas are those of SiaF.
-template <class T, int R>
-struct SiaLds {
-    static constexpr int W = kSX + 2 * R, HH = kSY + 2 * R;
-    const T* Ss;
-    int64_t i0, j0;
-    const SiaF<T>* f;
-    __device__ static void load(const SiaF<T>& s, T* Ss, int64_t i0, int64_t j0, int64_t nx, int64_t ny) {
-        for (int q = threadIdx.x; q < W * HH; q += kST) {
-            const int a = q % W, b = q / W;
-            const int64_t i = i0 - R + a, j = j0 - R + b;
-            Ss[q] = (i >= 0 && i <= nx + 1 && j >= 0 && j <= ny + 1) ? s.S(i, j) : T(0);
-        }
+// ---------------------------------------------------------------- one-pass forms
+// The forward steps and the adjoint step as one launch each.  A block is a
+// region of 64 columns (one lane each) by NW x R rows: wave w holds rows
+// w R .. w R + R - 1 of its column in registers.  x neighbours come by DPP
+// lane shifts, y neighbours from the thread's own rows, and only a wave's
+// first and last rows pass through LDS.  Every value of a cell is formed once
+// per region and its row index is wave-uniform, so the row conditions and
+// addresses are scalar.  The ring a stage cannot form right (2 cells per
+// forward step, 1 more for the next state's D, 3 to 4 for the adjoint) is
+// work that other blocks own.  The arithmetic of every value is the one of the
+// per-point kernels above, so the results are bitwise equal to them.
+template <int NW, int R>
+struct SiaCol {
+    static constexpr int NR = NW * R;
+    using Edge = double[2][NW][64];   // first and last row of every wave
+    int lane, w, i, jb;               // column, first row
+    uint32_t ic;                      // column clamped into the stored 0..nx+1
+    int rx, ry;                       // columns and rows around the owned ones
+    int nx, ny;
+    __device__ __forceinline__ SiaCol(int bx, int by, int rx_, int ry_, int64_t nx_, int64_t ny_) : rx(rx_), ry(ry_) {
+        lane = threadIdx.x;
+        w = __builtin_amdgcn_readfirstlane(threadIdx.y);
+        nx = (int)nx_;
+        ny = (int)ny_;
+        i = 1 + bx * (64 - 2 * rx) - rx + lane;
+        jb = 1 + by * (NR - 2 * ry) - ry + w * R;
+        ic = (uint32_t)min(max(i, 0), nx + 1);
     }
-    __device__ T S(int64_t i, int64_t j) const { return Ss[(j - j0 + R) * W + (i - i0 + R)]; }
-    __device__ T gx(int64_t i, int64_t j) const { return (S(i, j) - S(i - 1, j)) * f->ix; }
-    __device__ T gy(int64_t i, int64_t j) const { return (S(i, j) - S(i, j - 1)) * f->iy; }
-    __device__ T ax(int64_t i, int64_t j) const { T l = gx(i, j), r = gx(i + 1, j); return fma(T(0.5), r - l, l); }
-    __device__ T ay(int64_t i, int64_t j) const { T l = gy(i, j), r = gy(i, j + 1); return fma(T(0.5), r - l, l); }
-    __device__ T D(int64_t i, int64_t j) const {
-        const T h = f->H(i, j, 0);
-        const T a = f->hasA ? f->A(i, j, 0) : T(1);
-        const T u = ax(i, j), w = ay(i, j);
-        const T vm = sqrt(u * u + w * w);
-        return (a * ipow_(h, f->n + 2) + f->As * ipow_(h, f->n)) * ipow_(vm, f->n - 1);
+    __device__ __forceinline__ int j(int r) const { return jb + r; }
+    __device__ __forceinline__ int jc(int r) const { return min(max(jb + r, 0), ny + 1); }
+    __device__ __forceinline__ bool inside(int r) const { return i >= 1 && i <= nx && j(r) >= 1 && j(r) <= ny; }
+    __device__ __forceinline__ bool own(int r) const {
+        const int y = w * R + r;
+        return lane >= rx && lane < 64 - rx && y >= ry && y < NR - ry && inside(r);
     }
-    __device__ T M(int64_t i, int64_t j) const {
-        const T m = f->mba * (S(i, j) - f->mbb);
-        return m < f->mbc ? m : f->mbc;
+    __device__ __forceinline__ double ld(const DF<double>& f, int r) const {
+        return (f.p + (int64_t)jc(r) * f.sy)[ic];
+    }
+    __device__ __forceinline__ double& at(const DF<double>& f, int r) const {   // owned cells only
+        return (f.p + (int64_t)j(r) * f.sy)[ic];
+    }
+    __device__ __forceinline__ void put(Edge& e, const double* v) const {
+        e[0][w][lane] = v[0];
+        e[1][w][lane] = v[R - 1];
+    }
+    // the rows below the first and above the last (a row of the block's rim
+    // gets its own value: it reaches ring cells only)
+    __device__ __forceinline__ void get(const Edge& e, const double* v, double& lo, double& hi) const {
+        lo = w > 0 ? e[1][w - 1][lane] : v[0];
+        hi = w + 1 < NW ? e[0][w + 1][lane] : v[R - 1];
     }
 };
 
 template <class T>
-struct SiaStep {   // one forward step H -> Ho (+ the H Neumann batch when bc != 0)
+struct SiaStep {   // forward steps H -> Ho, H's Neumann batch included
     SiaF<T> s;
     DF<T> Ho;
-    T dt;
-    int bc;
-    int wd;        // also store D(H) of the tile's cells into Dout (for a later adjoint step at H)
+    int wd;        // also store D(H) of the cells into Dout (for a later adjoint step at H)
     DF<T> Dout;
+};
+
+// Steps a launch may take: their time steps travel in its argument.
+constexpr int kSiaSteps = 8;
+struct SiaDts {
+    double dt[kSiaSteps];
+    int n;
 };
 
 // The time step from max(D) on the device (sia.jl:76-78): Δt =
 // min(h2 / max(D) / 4.1, dt_max), with max(D) as the bits of its magnitude in
-// *dmax.  Every block forms the same Δt; the first stores it.
+// *dmax.  Every block forms the same Δt; the first stores it.  next (or
+// NULL) receives the new state's max(D) the same way.
 struct SiaRule {
     const unsigned long long* dmax;
+    unsigned long long* next;
     double h2, dt_max;
     double* dt_out;
 };
@@ -324,64 +331,161 @@ __device__ __forceinline__ double sia_rule_dt(const SiaRule& r) {
     const double d = m > 0.0 ? r.h2 / m / 4.1 : __longlong_as_double(0x7ff0000000000000ll);
     return r.dt_max < d ? r.dt_max : d;
 }
+__device__ __forceinline__ unsigned long long sia_mag(double d) {
+    return (unsigned long long)__double_as_longlong(d) & 0x7fffffffffffffffull;
+}
 
-// READ_D: D(H) is in Dout already (stored with its maximum for the time-step
-// rule), the same bits as evaluated here.
-template <class T, bool READ_D = false>
-__device__ __forceinline__ void sia_step_block(const SiaStep<T>& p, int64_t nx, int64_t ny, T* lds, T dt) {
-    constexpr int W = kSX + 2, Hh = kSY + 2;
-    using LS = SiaLds<T, 2>;
-    T(*Ds)[W] = reinterpret_cast<T(*)[W]>(lds + LS::W * LS::HH);
-    const SiaF<T>& s = p.s;
-    const int tid = threadIdx.x;
-    const int64_t i0 = 1 + (int64_t)blockIdx.x * kSX, j0 = 1 + (int64_t)blockIdx.y * kSY;
-    LS::load(s, lds, i0, j0, nx, ny);
-    const LS L{lds, i0, j0, &s};
-    __syncthreads();
-    for (int q = tid; q < W * Hh; q += kST) {
-        const int a = q % W, b = q / W;
-        const int64_t i = i0 - 1 + a, j = j0 - 1 + b;
-        const bool in = i >= 1 && i <= nx && j >= 1 && j <= ny;
-        const T d = in ? (READ_D ? p.Dout(i, j, 0) : L.D(i, j)) : T(0);
-        Ds[b][a] = d;
-        if (!READ_D && p.wd && in && a >= 1 && a <= kSX && b >= 1 && b <= kSY) p.Dout(i, j, 0) = d;
+// One column's rows of H with B and A, and the surface gradients and D of the
+// current H.  H's rows -1 and R (and the ghost cells) are kept with it.
+template <int NW, int R>
+struct SiaRows {
+    using Col = SiaCol<NW, R>;
+    double h[R + 2], b[R + 2], a[R];   // [r + 1]: row r
+    double gx[R], gy[R + 1], u[R], v[R];
+    __device__ __forceinline__ void load(const SiaF<double>& s, const Col& c) {
+#pragma unroll
+        for (int r = -1; r <= R; ++r) {
+            h[r + 1] = c.ld(s.H, r);
+            b[r + 1] = c.ld(s.B, r);
+        }
+#pragma unroll
+        for (int r = 0; r < R; ++r) a[r] = s.hasA ? c.ld(s.A, r) : 1.0;
     }
-    __syncthreads();
-    for (int q = tid; q < kSX * kSY; q += kST) {
-        const int a = q % kSX + 1, b = q / kSX + 1;   // LDS position of the cell
-        const int64_t i = i0 + a - 1, j = j0 + b - 1;
-        if (i > nx || j > ny) continue;
-        auto qx = [&](int64_t f, int la) -> T {   // x-vertex f, right cell at LDS column la
-            if (f <= 1 || f >= nx + 1) return T(0);
-            const T Dl = Ds[b][la - 1], Dr = Ds[b][la];
-            return -fma(T(0.5), Dr - Dl, Dl) * L.gx(f, j);
-        };
-        auto qy = [&](int64_t f, int lb) -> T {
-            if (f <= 1 || f >= ny + 1) return T(0);
-            const T Dl = Ds[lb - 1][a], Dr = Ds[lb][a];
-            return -fma(T(0.5), Dr - Dl, Dl) * L.gy(i, f);
-        };
-        const T dv = (qx(i + 1, a + 1) - qx(i, a)) * s.ix + (qy(j + 1, b + 1) - qy(j, b)) * s.iy;
-        const T h = jmax0(s.H(i, j, 0) + dt * (-dv + L.M(i, j)));
-        const DF<T>& Ho = p.Ho;
-        Ho(i, j, 0) = h;
-        if (p.bc) {
-            // Neumann(0) batch, dims y then x (batch.jl:20-29): ghosts copy the
-            // adjacent cell (fma(Δ, -0, f) == f), corners the diagonal cell
-            if (i == 1) Ho(0, j, 0) = h;
-            if (i == nx) Ho(nx + 1, j, 0) = h;
-            if (j == 1) {
-                Ho(i, 0, 0) = h;
-                if (i == 1) Ho(0, 0, 0) = h;
-                if (i == nx) Ho(nx + 1, 0, 0) = h;
-            }
-            if (j == ny) {
-                Ho(i, ny + 1, 0) = h;
-                if (i == 1) Ho(0, ny + 1, 0) = h;
-                if (i == nx) Ho(nx + 1, ny + 1, 0) = h;
+    __device__ __forceinline__ double S(int r) const { return b[r + 1] + h[r + 1]; }
+    // after a step: the neighbouring waves' rows, then the Neumann(0) ghosts
+    // (a ghost copies the adjacent cell: fma(Δ, -0, f) == f; corners are not read)
+    __device__ __forceinline__ void refresh(const Col& c, typename Col::Edge& e) {
+        c.put(e, h + 1);
+        __syncthreads();
+        c.get(e, h + 1, h[0], h[R + 1]);
+#pragma unroll
+        for (int r = -1; r < R; ++r)
+            if (c.j(r) == 0) h[r + 1] = h[r + 2];
+#pragma unroll
+        for (int r = R; r >= 0; --r)
+            if (c.j(r) == c.ny + 1) h[r + 1] = h[r];
+        const int i0 = c.i - c.lane;
+        if (i0 <= 0 || i0 + 63 > c.nx) {   // block-uniform
+#pragma unroll
+            for (int r = -1; r <= R; ++r) {
+                const double up = xp1(h[r + 1]), dn = xm1(h[r + 1]);
+                h[r + 1] = c.i == 0 ? up : c.i == c.nx + 1 ? dn : h[r + 1];
             }
         }
     }
+    __device__ __forceinline__ void gradients(const SiaF<double>& s) {
+#pragma unroll
+        for (int r = 0; r <= R; ++r) gy[r] = (S(r) - S(r - 1)) * s.iy;
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+            gx[r] = (S(r) - xm1(S(r))) * s.ix;
+            const double gr = xp1(gx[r]);
+            u[r] = fma(0.5, gr - gx[r], gx[r]);
+            v[r] = fma(0.5, gy[r + 1] - gy[r], gy[r]);
+        }
+    }
+    __device__ __forceinline__ double D(const SiaF<double>& s, int r) const {
+        const double vm = sqrt(u[r] * u[r] + v[r] * v[r]);
+        return (a[r] * ipow_(h[r + 1], s.n + 2) + s.As * ipow_(h[r + 1], s.n)) * ipow_(vm, s.n - 1);
+    }
+    // H - Δt(divg q - M) of row r before max(., 0), from D's lerps on the faces
+    __device__ __forceinline__ void update(const SiaF<double>& s, const Col& c, const double* fx, const double* fy,
+                                           double dt, double* x) const {
+        double qy[R + 1];
+#pragma unroll
+        for (int r = 0; r <= R; ++r) qy[r] = c.j(r) <= 1 || c.j(r) >= c.ny + 1 ? 0.0 : -fy[r] * gy[r];
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+            const double q = c.i <= 1 || c.i >= c.nx + 1 ? 0.0 : -fx[r] * gx[r];
+            const double dv = (xp1(q) - q) * s.ix + (qy[r + 1] - qy[r]) * s.iy;
+            const double m = s.mba * (S(r) - s.mbb);
+            x[r] = h[r + 1] + dt * (-dv + (m < s.mbc ? m : s.mbc));
+        }
+    }
+};
+
+// D's lerps on a column's x faces (left of each row's cell) and y faces
+template <int NW, int R>
+__device__ __forceinline__ void sia_face_d(const double* D, double lo, double hi, double* fx, double* fy) {
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+        const double l = xm1(D[r]);
+        fx[r] = fma(0.5, D[r] - l, l);
+    }
+#pragma unroll
+    for (int r = 0; r <= R; ++r) {
+        const double l = r > 0 ? D[r - 1] : lo, g = r < R ? D[r] : hi;
+        fy[r] = fma(0.5, g - l, l);
+    }
+}
+
+// n forward steps on the region (a ring of 2 n); the owned cells' final H and
+// its ghosts are stored.  With MAXD (a ring of 2 n + 1) the magnitude bits of
+// the new state's largest owned D come back.
+template <int NW, int R, bool MAXD>
+__device__ __forceinline__ unsigned long long sia_step_cols(const SiaStep<double>& p, const SiaCol<NW, R>& c,
+                                                            const double* dts, int n, double (*ldsH)[NW][64],
+                                                            double (*ldsD)[NW][64]) {
+    using Col = SiaCol<NW, R>;
+    const SiaF<double>& s = p.s;
+    typename Col::Edge& eH = *reinterpret_cast<typename Col::Edge*>(ldsH);
+    typename Col::Edge& eD = *reinterpret_cast<typename Col::Edge*>(ldsD);
+    SiaRows<NW, R> k;
+    k.load(s, c);
+#pragma unroll 1
+    for (int q = 0; q < n; ++q) {
+        if (q > 0) k.refresh(c, eH);
+        k.gradients(s);
+        double D[R];
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+            D[r] = c.inside(r) ? k.D(s, r) : 0.0;
+            if (p.wd && c.own(r)) c.at(p.Dout, r) = D[r];
+        }
+        c.put(eD, D);
+        __syncthreads();
+        double lo, hi, fx[R], fy[R + 1], x[R];
+        c.get(eD, D, lo, hi);
+        sia_face_d<NW, R>(D, lo, hi, fx, fy);
+        k.update(s, c, fx, fy, dts[q], x);
+#pragma unroll
+        for (int r = 0; r < R; ++r) k.h[r + 1] = c.inside(r) ? jmax0(x[r]) : k.h[r + 1];
+    }
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+        if (!c.own(r)) continue;
+        const double h = k.h[r + 1];
+        double* row = &c.at(p.Ho, r);
+        row[0] = h;
+        // Neumann(0) batch, dims y then x (batch.jl:20-29): ghosts copy the
+        // adjacent cell, corners the diagonal cell
+        const bool x0 = c.i == 1, x1 = c.i == c.nx;
+        if (x0) row[-1] = h;
+        if (x1) row[1] = h;
+        if (c.j(r) == 1) {
+            double* g = row - p.Ho.sy;
+            g[0] = h;
+            if (x0) g[-1] = h;
+            if (x1) g[1] = h;
+        }
+        if (c.j(r) == c.ny) {
+            double* g = row + p.Ho.sy;
+            g[0] = h;
+            if (x0) g[-1] = h;
+            if (x1) g[1] = h;
+        }
+    }
+    unsigned long long m = 0;
+    if constexpr (MAXD) {
+        k.refresh(c, eH);
+        k.gradients(s);
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+            const unsigned long long d = c.own(r) ? sia_mag(k.D(s, r)) : 0ull;
+            m = d > m ? d : m;
+        }
+    }
+    return m;
 }
 
 template <class T>
@@ -393,164 +497,161 @@ struct SiaAdj {    // one adjoint step at state s.H: lam -> lo, gA += dJ/dlog A
     DF<T> Din;
 };
 
-template <class T>
-__device__ __forceinline__ void sia_adj_block(const SiaAdj<T>& p, int64_t nx, int64_t ny, T* lds) {
-    constexpr int W3 = kSX + 6, H3 = kSY + 6, W2 = kSX + 4, H2 = kSY + 4, W1 = kSX + 2, H1 = kSY + 2;
-    using LS = SiaLds<T, 4>;
-    T* base = lds + LS::W * LS::HH;
-    T(*Ds)[W3] = reinterpret_cast<T(*)[W3]>(base);
-    T(*Ms)[W2] = reinterpret_cast<T(*)[W2]>(base + W3 * H3);
-    T(*Ax)[W1] = reinterpret_cast<T(*)[W1]>(base + W3 * H3 + W2 * H2);
-    T(*Ay)[W1] = reinterpret_cast<T(*)[W1]>(base + W3 * H3 + W2 * H2 + W1 * H1);
-    T(*HDs)[kSX] = reinterpret_cast<T(*)[kSX]>(base + W3 * H3 + W2 * H2 + 2 * W1 * H1);
-    const SiaF<T>& s = p.s;
-    const T dt = p.dt;
-    const int tid = threadIdx.x;
-    const int64_t i0 = 1 + (int64_t)blockIdx.x * kSX, j0 = 1 + (int64_t)blockIdx.y * kSY;
-    LS::load(s, lds, i0, j0, nx, ny);
-    const LS L{lds, i0, j0, &s};
-    __syncthreads();
-    auto inside = [nx, ny](int64_t i, int64_t j) { return i >= 1 && i <= nx && j >= 1 && j <= ny; };
-    // D on the tile + 3 ring; cell (i, j) at Ds[j - j0 + 3][i - i0 + 3]; the same
-    // bits whether evaluated here or stored by the forward step at this state
-    for (int q = tid; q < W3 * H3; q += kST) {
-        const int a = q % W3, b = q / W3;
-        const int64_t i = i0 - 3 + a, j = j0 - 3 + b;
-        Ds[b][a] = inside(i, j) ? (p.rd ? p.Din(i, j, 0) : L.D(i, j)) : T(0);
-    }
-    __syncthreads();
-    // pass A1: mu on the tile + 2 ring; cell at Ms[j - j0 + 2][i - i0 + 2]
-    for (int q = tid; q < W2 * H2; q += kST) {
-        const int a = q % W2, b = q / W2;
-        const int64_t i = i0 - 2 + a, j = j0 - 2 + b;
-        T mu = T(0);
-        if (inside(i, j)) {
-            const int da = a + 1, db = b + 1;   // the cell in Ds
-            auto qx = [&](int64_t f, int la) -> T {
-                if (f <= 1 || f >= nx + 1) return T(0);
-                const T Dl = Ds[db][la - 1], Dr = Ds[db][la];
-                return -fma(T(0.5), Dr - Dl, Dl) * L.gx(f, j);
-            };
-            auto qy = [&](int64_t f, int lb) -> T {
-                if (f <= 1 || f >= ny + 1) return T(0);
-                const T Dl = Ds[lb - 1][da], Dr = Ds[lb][da];
-                return -fma(T(0.5), Dr - Dl, Dl) * L.gy(i, f);
-            };
-            const T dv = (qx(i + 1, da + 1) - qx(i, da)) * s.ix + (qy(j + 1, db + 1) - qy(j, db)) * s.iy;
-            const T x = s.H(i, j, 0) + dt * (-dv + L.M(i, j));
-            mu = x > T(0) ? p.lam(i, j, 0) : T(0);
+// lam' reaches D of the cells 3 away, and an evaluated D the surface of the
+// cell beside that one: the rows -1 and R a wave holds cover it in y, one
+// more lane in x.
+constexpr int kAdjRing = 3;
+__host__ __device__ constexpr int sia_adj_ring(int rd) { return rd ? kAdjRing : kAdjRing + 1; }
+
+template <int NW, int R>
+__device__ __forceinline__ void sia_adj_cols(const SiaAdj<double>& p, const SiaCol<NW, R>& c, double (*lds0)[NW][64],
+                                             double (*lds1)[NW][64]) {
+    using Col = SiaCol<NW, R>;
+    const SiaF<double>& s = p.s;
+    typename Col::Edge& e0 = *reinterpret_cast<typename Col::Edge*>(lds0);
+    typename Col::Edge& e1 = *reinterpret_cast<typename Col::Edge*>(lds1);
+    const double dt = p.dt;
+    const int nx = c.nx, ny = c.ny;
+    SiaRows<NW, R> k;
+    k.load(s, c);
+    double lam[R], D[R], Dlo, Dhi, fx[R], fy[R + 1];
+#pragma unroll
+    for (int r = 0; r < R; ++r) lam[r] = c.ld(p.lam, r);
+    double gA[R];
+#pragma unroll
+    for (int r = 0; r < R; ++r) gA[r] = s.hasA ? c.ld(p.gA, r) : 0.0;
+    if (p.rd) {   // D of the wave's rows and the two beside them, stored by the forward step at this state
+        const double lo = c.ld(p.Din, -1), hi = c.ld(p.Din, R);
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+            const double d = c.ld(p.Din, r);
+            D[r] = c.inside(r) ? d : 0.0;
         }
-        Ms[b][a] = mu;
+        Dlo = c.inside(-1) ? lo : 0.0;
+        Dhi = c.inside(R) ? hi : 0.0;
+        k.gradients(s);
+    } else {
+        k.gradients(s);
+#pragma unroll
+        for (int r = 0; r < R; ++r) D[r] = c.inside(r) ? k.D(s, r) : 0.0;
+        c.put(e1, D);
+        __syncthreads();
+        c.get(e1, D, Dlo, Dhi);
     }
-    __syncthreads();
-    // passes A2+A3: Dbar and abar on the tile + 1 ring; HD and grad on the tile
-    for (int q = tid; q < W1 * H1; q += kST) {
-        const int a = q % W1, b = q / W1;
-        const int64_t i = i0 - 1 + a, j = j0 - 1 + b;
-        T abx = T(0), aby = T(0);
-        if (inside(i, j)) {
-            const int ma = a + 1, mb = b + 1;   // the cell in Ms
-            auto Dvx = [&](int64_t f, int la) -> T {   // x-vertex f, right cell at Ms column la
-                if (f < 2 || f > nx) return T(0);
-                const T qb = dt * s.ix * (Ms[mb][la] - Ms[mb][la - 1]);
-                return -L.gx(f, j) * qb;
-            };
-            auto Dvy = [&](int64_t f, int lb) -> T {
-                if (f < 2 || f > ny) return T(0);
-                const T qb = dt * s.iy * (Ms[lb][ma] - Ms[lb - 1][ma]);
-                return -L.gy(i, f) * qb;
-            };
-            const T Db = T(0.5) * (Dvx(i, ma) + Dvx(i + 1, ma + 1)) + T(0.5) * (Dvy(j, mb) + Dvy(j + 1, mb + 1));
-            const int n = s.n;
-            const T h = s.H(i, j, 0);
-            const T av = s.hasA ? s.A(i, j, 0) : T(1);
-            const T u = L.ax(i, j), v = L.ay(i, j);
-            const T vm = sqrt(u * u + v * v);
-            const T P = ipow_(vm, n - 1);
-            const T Cc = av * ipow_(h, n + 2) + s.As * ipow_(h, n);
-            const bool tile = a >= 1 && a <= kSX && b >= 1 && b <= kSY;
-            if (tile) {
-                if (s.hasA) p.gA(i, j, 0) = p.gA(i, j, 0) + av * (Db * ipow_(h, n + 2) * P);
-                HDs[b - 1][a - 1] = Db * (T(n + 2) * av * ipow_(h, n + 1) + T(n) * s.As * ipow_(h, n - 1)) * P;
-            }
-            T coef = T(0);
-            if (n >= 3) coef = T(n - 1) * ipow_(vm, n - 3);
-            else if (n == 2 && vm > T(0)) coef = T(1) / vm;
-            const T Pb = Db * Cc;
-            abx = Pb * coef * u;
-            aby = Pb * coef * v;
-        }
-        Ax[b][a] = abx;
-        Ay[b][a] = aby;
+    sia_face_d<NW, R>(D, Dlo, Dhi, fx, fy);
+    // A1: mu
+    double mu[R], mlo, mhi;
+    {
+        double x[R];
+        k.update(s, c, fx, fy, dt, x);
+#pragma unroll
+        for (int r = 0; r < R; ++r) mu[r] = c.inside(r) && x[r] > 0.0 ? lam[r] : 0.0;
     }
+    c.put(e0, mu);
     __syncthreads();
-    // passes A4+A5: gbar on the 4 faces of each tile cell, then lam'
-    for (int q = tid; q < kSX * kSY; q += kST) {
-        const int t = q % kSX, u = q / kSX;
-        const int64_t i = i0 + t, j = j0 + u;
-        if (i > nx || j > ny) continue;
-        const int a1 = t + 1, b1 = u + 1;   // cell in Ax/Ay
-        const int a2 = t + 2, b2 = u + 2;   // cell in Ms
-        const int a3 = t + 3, b3 = u + 3;   // cell in Ds
-        auto gbx = [&](int64_t f, int o) -> T {   // x-vertex f = i + o, o in {0, 1}
-            T g = T(0);
-            if (f >= 2 && f <= nx) {
-                const T qb = dt * s.ix * (Ms[b2][a2 + o] - Ms[b2][a2 + o - 1]);
-                const T Dl = Ds[b3][a3 + o - 1], Dr = Ds[b3][a3 + o];
-                g = -fma(T(0.5), Dr - Dl, Dl) * qb;
-            }
-            if (f - 1 >= 1) g = g + T(0.5) * Ax[b1][a1 + o - 1];
-            if (f <= nx) g = g + T(0.5) * Ax[b1][a1 + o];
-            return g;
-        };
-        auto gby = [&](int64_t f, int o) -> T {
-            T g = T(0);
-            if (f >= 2 && f <= ny) {
-                const T qb = dt * s.iy * (Ms[b2 + o][a2] - Ms[b2 + o - 1][a2]);
-                const T Dl = Ds[b3 + o - 1][a3], Dr = Ds[b3 + o][a3];
-                g = -fma(T(0.5), Dr - Dl, Dl) * qb;
-            }
-            if (f - 1 >= 1) g = g + T(0.5) * Ay[b1 + o - 1][a1];
-            if (f <= ny) g = g + T(0.5) * Ay[b1 + o][a1];
-            return g;
-        };
-        const T gx0 = gbx(i, 0), gx1 = gbx(i + 1, 1), gy0 = gby(j, 0), gy1 = gby(j + 1, 1);
-        T r = T(0);
-        r = r + s.ix * gx0;
-        r = r - s.ix * gx1;
-        r = r + s.iy * gy0;
-        r = r - s.iy * gy1;
-        const T mu = Ms[b2][a2];
-        T l = mu + HDs[u][t] + r;
-        const T m = s.mba * (L.S(i, j) - s.mbb);
-        if (m < s.mbc) l = l + dt * mu * s.mba;
-        if (i == 1) l = l + (-s.ix * gx0);
-        if (i == nx) l = l + s.ix * gx1;
-        if (j == 1) l = l + (-s.iy * gy0);
-        if (j == ny) l = l + s.iy * gy1;
-        p.lo(i, j, 0) = l;
+    c.get(e0, mu, mlo, mhi);
+    // A2 + A3: qbar on the faces, Dbar, abar; HD and the log A gradient
+    const bool fxin = c.i >= 2 && c.i <= nx;
+    double qbx[R], qby[R + 1], Dvy[R + 1], abx[R], aby[R], HD[R];
+#pragma unroll
+    for (int r = 0; r <= R; ++r) {
+        qby[r] = dt * s.iy * ((r < R ? mu[r] : mhi) - (r > 0 ? mu[r - 1] : mlo));
+        Dvy[r] = c.j(r) < 2 || c.j(r) > ny ? 0.0 : -k.gy[r] * qby[r];
+    }
+    const int n = s.n;
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+        qbx[r] = dt * s.ix * (mu[r] - xm1(mu[r]));
+        const double Dvx = fxin ? -k.gx[r] * qbx[r] : 0.0;
+        const double Db = 0.5 * (Dvx + xp1(Dvx)) + 0.5 * (Dvy[r] + Dvy[r + 1]);
+        const double h = k.h[r + 1], av = k.a[r], u = k.u[r], v = k.v[r];
+        const double vm = sqrt(u * u + v * v);
+        const double P = ipow_(vm, n - 1);
+        const double Cc = av * ipow_(h, n + 2) + s.As * ipow_(h, n);
+        if (s.hasA && c.own(r)) c.at(p.gA, r) = gA[r] + av * (Db * ipow_(h, n + 2) * P);
+        HD[r] = Db * (double(n + 2) * av * ipow_(h, n + 1) + double(n) * s.As * ipow_(h, n - 1)) * P;
+        double coef = 0.0;
+        if (n >= 3) coef = double(n - 1) * ipow_(vm, n - 3);
+        else if (n == 2 && vm > 0.0) coef = 1.0 / vm;
+        const double Pb = Db * Cc;
+        const bool in = c.inside(r);
+        abx[r] = in ? Pb * coef * u : 0.0;
+        aby[r] = in ? Pb * coef * v : 0.0;
+    }
+    double alo, ahi;
+    c.put(e1, aby);
+    __syncthreads();
+    c.get(e1, aby, alo, ahi);
+    // A4 + A5: gbar on the faces, then lam'
+    double gby[R + 1];
+#pragma unroll
+    for (int r = 0; r <= R; ++r) {
+        const int f = c.j(r);
+        double g = f >= 2 && f <= ny ? -fy[r] * qby[r] : 0.0;
+        if (f - 1 >= 1) g = g + 0.5 * (r > 0 ? aby[r - 1] : alo);
+        if (f <= ny) g = g + 0.5 * (r < R ? aby[r] : ahi);
+        gby[r] = g;
+    }
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+        double gx0 = fxin ? -fx[r] * qbx[r] : 0.0;
+        const double al = xm1(abx[r]);
+        gx0 = c.i - 1 >= 1 ? gx0 + 0.5 * al : gx0;
+        gx0 = c.i <= nx ? gx0 + 0.5 * abx[r] : gx0;
+        const double gx1 = xp1(gx0), gy0 = gby[r], gy1 = gby[r + 1];
+        if (!c.own(r)) continue;
+        double t = 0.0;
+        t = t + s.ix * gx0;
+        t = t - s.ix * gx1;
+        t = t + s.iy * gy0;
+        t = t - s.iy * gy1;
+        double l = mu[r] + HD[r] + t;
+        const double m = s.mba * (k.S(r) - s.mbb);
+        if (m < s.mbc) l = l + dt * mu[r] * s.mba;
+        if (c.i == 1) l = l + (-s.ix * gx0);
+        if (c.i == nx) l = l + s.ix * gx1;
+        if (c.j(r) == 1) l = l + (-s.iy * gy0);
+        if (c.j(r) == ny) l = l + s.iy * gy1;
+        c.at(p.lo, r) = l;
     }
 }
-
-constexpr int kAdjLds = (kSX + 8) * (kSY + 8) + (kSX + 6) * (kSY + 6) + (kSX + 4) * (kSY + 4) + 2 * (kSX + 2) * (kSY + 2) + kSX * kSY;
 
 // NP > 0: the Glen exponent as a compile-time constant (it must equal the
 // run-time one), so that every power's product loop unrolls; the products
 // and their order are the same as with NP = 0.
-template <class T, int NP>
-__global__ void __launch_bounds__(kST) sia_step_tile(SiaStep<T> f, int64_t nx, int64_t ny) {
-    __shared__ T lds[(kSX + 4) * (kSY + 4) + (kSX + 2) * (kSY + 2)];
+template <int NP, int NW, int R>
+__global__ void __launch_bounds__(NW * 64) sia_steps_kernel(SiaStep<double> f, SiaDts d, int ntx, int64_t nx,
+                                                            int64_t ny) {
+    __shared__ double lds[2][2][NW][64];
     if constexpr (NP > 0) f.s.n = NP;
-    sia_step_block(f, nx, ny, lds, f.dt);
+    const SiaCol<NW, R> c(blockIdx.x % ntx, blockIdx.x / ntx, 2 * d.n, 2 * d.n, nx, ny);
+    sia_step_cols<NW, R, false>(f, c, d.dt, d.n, lds[0], lds[1]);
 }
 
-// The step whose Δt follows from the stored D and its maximum.
-template <class T>
-__global__ void __launch_bounds__(kST) sia_step_rule_tile(SiaStep<T> f, SiaRule r, int64_t nx, int64_t ny) {
-    __shared__ T lds[(kSX + 4) * (kSY + 4) + (kSX + 2) * (kSY + 2)];
-    const double dt = sia_rule_dt(r);
-    if (blockIdx.x == 0 && blockIdx.y == 0 && threadIdx.x == 0) *r.dt_out = dt;
-    sia_step_block<T, true>(f, nx, ny, lds, dt);
+// The step whose Δt follows from its state's max(D), and the next state's.
+template <int NP, int NW, int R, bool MAXD>
+__global__ void __launch_bounds__(NW * 64) sia_rule_kernel(SiaStep<double> f, SiaRule rule, int ntx, int64_t nx,
+                                                           int64_t ny) {
+    __shared__ double lds[2][2][NW][64];
+    __shared__ unsigned long long part[NW];
+    if constexpr (NP > 0) f.s.n = NP;
+    const double dt = sia_rule_dt(rule);
+    if (blockIdx.x == 0 && threadIdx.x == 0 && threadIdx.y == 0) *rule.dt_out = dt;
+    constexpr int ring = MAXD ? 3 : 2;
+    const SiaCol<NW, R> c(blockIdx.x % ntx, blockIdx.x / ntx, ring, ring, nx, ny);
+    unsigned long long m = sia_step_cols<NW, R, MAXD>(f, c, &dt, 1, lds[0], lds[1]);
+    if constexpr (MAXD) {
+        for (int o = 32; o > 0; o >>= 1) {
+            const unsigned long long q = __shfl_xor(m, o, 64);
+            m = q > m ? q : m;
+        }
+        if (threadIdx.x == 0) part[threadIdx.y] = m;
+        __syncthreads();
+        if (threadIdx.x == 0 && threadIdx.y == 0) {
+            for (int q = 1; q < NW; ++q) m = part[q] > m ? part[q] : m;
+            if (m > __hip_atomic_load(rule.next, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) atomicMax(rule.next, m);
+        }
+    }
 }
 
 // D at cells 1..n and the maximum of its magnitude (bits; NaN above infinity)
@@ -566,7 +667,7 @@ __global__ void __launch_bounds__(256) sia_d_max_kernel(SiaF<T> s, DF<T> D, int6
     if (ok) {
         const T d = s.D(i, j);
         D(i, j, 0) = d;
-        m = (unsigned long long)__double_as_longlong((double)d) & 0x7fffffffffffffffull;
+        m = sia_mag((double)d);
     }
     for (int o = 32; o > 0; o >>= 1) {
         const unsigned long long q = __shfl_xor(m, o, 64);
@@ -580,28 +681,90 @@ __global__ void __launch_bounds__(256) sia_d_max_kernel(SiaF<T> s, DF<T> D, int6
     }
 }
 
-// blockIdx.z == 0: adjoint tile; blockIdx.z == 1: forward tile of an independent step
-template <class T, int NP>
-__global__ void __launch_bounds__(kST) sia_adj_tile(SiaAdj<T> a, SiaStep<T> f, int64_t nx, int64_t ny) {
-    __shared__ T lds[kAdjLds];
+// Blocks 0 .. na - 1: adjoint regions; the rest: an independent forward step
+// (the recompute of the previous checkpoint segment rides along).
+template <int NP, int NW, int RA, int RF>
+__global__ void __launch_bounds__(NW * 64) sia_adj_kernel(SiaAdj<double> a, SiaStep<double> f, double fdt, int na,
+                                                          int ntxa, int ntxf, int64_t nx, int64_t ny) {
+    __shared__ double lds[2][2][NW][64];
     if constexpr (NP > 0) {
         a.s.n = NP;
         f.s.n = NP;
     }
-    if (blockIdx.z == 0) sia_adj_block(a, nx, ny, lds);
-    else sia_step_block(f, nx, ny, lds, f.dt);
+    const int bid = blockIdx.x;
+    if (bid < na) {
+        const SiaCol<NW, RA> c(bid % ntxa, bid / ntxa, sia_adj_ring(a.rd), kAdjRing, nx, ny);
+        sia_adj_cols<NW, RA>(a, c, lds[0], lds[1]);
+    } else {
+        const SiaCol<NW, RF> c((bid - na) % ntxf, (bid - na) / ntxf, 2, 2, nx, ny);
+        sia_step_cols<NW, RF, false>(f, c, &fdt, 1, lds[0], lds[1]);
+    }
+}
+
+// Shapes, each the best measured of 4..16 waves by 1..6 rows.  A launch's floor
+// is its serial chain (about 4.5 us a forward step, 5.4 us an adjoint step for
+// one region alone), so forward steps go several to a launch (300 steps of
+// 512^2: 5.1 us each singly, 4.3 in twos, 3.8 in threes, 3.9 in fives on
+// regions of 64 x 64, where the ring's work eats the rest).  Regions of 32 rows while they
+// all fit the CUs at once, else 48 (250x177: 1.14 ms for the gradient of 100
+// steps with 32 rows, 1.20 with 48; 512^2: 4.86 and 4.68 for 300).  The
+// adjoint's regions are 16 rows with 24 for the steps riding along: 3 blocks a
+// CU hold them all at 512^2 (with 16 and 16 rows a second round starts: 5.04).
+constexpr int kSiaMax = 3;                        // forward steps per launch
+constexpr int kNWF = 16, kRF1 = 2, kRF2 = 3;      // forward: waves, rows per wave
+constexpr int kNWA = 8, kRA = 2, kRR = 3;         // adjoint, and the steps riding along
+constexpr int kNWD = 16, kRD = 1;                 // the adaptive step
+static_assert(kSiaMax <= kSiaSteps && kNWF * kRF1 > 4 * kSiaMax && 64 > 4 * kSiaMax && kNWA * kRA > 2 * kAdjRing &&
+                  kNWA * kRR > 4 && kNWD * kRD > 6,
+              "a region owns at least one row and column");
+
+static int sia_regions(int64_t nx, int64_t ny, int rx, int ry, int rows, int* ntx) {
+    const int64_t w = 64 - 2 * rx, h = rows - 2 * ry;
+    *ntx = (int)((nx + w - 1) / w);
+    return (int)(*ntx * ((ny + h - 1) / h));
 }
 
 // n = 3 (Glen's law as sia.jl uses it) takes the unrolled kernels
-static void launch_step_tile(dim3 grd, hipStream_t st, const SiaStep<double>& f, int64_t nx, int64_t ny) {
-    if (f.s.n == 3) hipLaunchKernelGGL((sia_step_tile<double, 3>), grd, dim3(kST), 0, st, f, nx, ny);
-    else hipLaunchKernelGGL((sia_step_tile<double, 0>), grd, dim3(kST), 0, st, f, nx, ny);
+template <int R>
+static void launch_steps_r(hipStream_t st, const SiaStep<double>& f, const SiaDts& d, int64_t nx, int64_t ny) {
+    int ntx;
+    const int nb = sia_regions(nx, ny, 2 * d.n, 2 * d.n, kNWF * R, &ntx);
+    const dim3 blk(64, kNWF);
+    if (f.s.n == 3) hipLaunchKernelGGL((sia_steps_kernel<3, kNWF, R>), dim3(nb), blk, 0, st, f, d, ntx, nx, ny);
+    else hipLaunchKernelGGL((sia_steps_kernel<0, kNWF, R>), dim3(nb), blk, 0, st, f, d, ntx, nx, ny);
 }
 
-static void launch_adj_tile(dim3 grd, hipStream_t st, const SiaAdj<double>& a, const SiaStep<double>& f, int64_t nx,
-                            int64_t ny) {
-    if (a.s.n == 3) hipLaunchKernelGGL((sia_adj_tile<double, 3>), grd, dim3(kST), 0, st, a, f, nx, ny);
-    else hipLaunchKernelGGL((sia_adj_tile<double, 0>), grd, dim3(kST), 0, st, a, f, nx, ny);
+static void launch_steps(hipStream_t st, const SiaStep<double>& f, const double* dts, int n, int64_t nx, int64_t ny) {
+    SiaDts d{};
+    d.n = n;
+    for (int q = 0; q < n; ++q) d.dt[q] = dts[q];
+    int ntx;
+    if (sia_regions(nx, ny, 2 * n, 2 * n, kNWF * kRF1, &ntx) <= cu_count()) launch_steps_r<kRF1>(st, f, d, nx, ny);
+    else launch_steps_r<kRF2>(st, f, d, nx, ny);
+}
+
+template <bool MAXD>
+static void launch_rule(hipStream_t st, const SiaStep<double>& f, const SiaRule& r, int64_t nx, int64_t ny) {
+    constexpr int NW = kNWD, R = kRD;
+    int ntx;
+    const int nb = sia_regions(nx, ny, MAXD ? 3 : 2, MAXD ? 3 : 2, NW * R, &ntx);
+    const dim3 blk(64, NW);
+    if (f.s.n == 3) hipLaunchKernelGGL((sia_rule_kernel<3, NW, R, MAXD>), dim3(nb), blk, 0, st, f, r, ntx, nx, ny);
+    else hipLaunchKernelGGL((sia_rule_kernel<0, NW, R, MAXD>), dim3(nb), blk, 0, st, f, r, ntx, nx, ny);
+}
+
+static void launch_adj(hipStream_t st, const SiaAdj<double>& a, const SiaStep<double>* f, double fdt, int64_t nx,
+                       int64_t ny) {
+    constexpr int NW = kNWA, RA = kRA, RF = kRR;
+    int ntxa, ntxf = 1;
+    const int na = sia_regions(nx, ny, sia_adj_ring(a.rd), kAdjRing, NW * RA, &ntxa);
+    const int nf = f ? sia_regions(nx, ny, 2, 2, NW * RF, &ntxf) : 0;
+    const SiaStep<double> g = f ? *f : SiaStep<double>{};
+    const dim3 blk(64, NW);
+    if (a.s.n == 3)
+        hipLaunchKernelGGL((sia_adj_kernel<3, NW, RA, RF>), dim3(na + nf), blk, 0, st, a, g, fdt, na, ntxa, ntxf, nx, ny);
+    else
+        hipLaunchKernelGGL((sia_adj_kernel<0, NW, RA, RF>), dim3(na + nf), blk, 0, st, a, g, fdt, na, ntxa, ntxf, nx, ny);
 }
 
 template <class T>
@@ -634,17 +797,11 @@ static int sia_check(const chmy_grid_t* g, const chmy_field_t* H, const chmy_fie
     return 0;
 }
 
-static dim3 sia_tiles(int64_t nx, int64_t ny, int z) {
-    return dim3((unsigned)((nx + kSX - 1) / kSX), (unsigned)((ny + kSY - 1) / kSY), (unsigned)z);
-}
-
 static SiaStep<double> sia_stepper(const chmy_grid_t* g, const chmy_field_t* H, const chmy_field_t* Ho,
-                                   const chmy_field_t* B, const chmy_field_t* A, const SiaPar& p, double dt) {
+                                   const chmy_field_t* B, const chmy_field_t* A, const SiaPar& p) {
     SiaStep<double> f;
     f.s = make_sia<double>(g, H, B, A, p);
     f.Ho = view<double>(*Ho);
-    f.dt = dt;
-    f.bc = 1;
     f.wd = 0;
     f.Dout = f.Ho;
     return f;
@@ -662,6 +819,30 @@ static SiaAdj<double> sia_adjointer(const chmy_grid_t* g, const chmy_field_t* H,
     a.rd = 0;
     a.Din = a.lo;
     return a;
+}
+
+// Steps the launch that starts at state q takes: states between its first and
+// its last are not stored, so each must have a later state in the same
+// storage (looked for over the next 8), and the output must not touch the
+// input (a block reads cells that its neighbours own).
+static int sia_run_length(const chmy_field_t* st, int nstates, int q) {
+    const auto same = [](const chmy_field_t& a, const chmy_field_t& b) {
+        return a.data == b.data && a.halo[0] == b.halo[0] && a.halo[1] == b.halo[1];
+    };
+    const auto apart = [](const chmy_field_t& a, const chmy_field_t& b) {
+        const char *pa = static_cast<const char*>(a.data), *pb = static_cast<const char*>(b.data);
+        return pa + pad_of(a, 0) * pad_of(a, 1) * 8 <= pb || pb + pad_of(b, 0) * pad_of(b, 1) * 8 <= pa;
+    };
+    const auto replaced = [&](int m) {
+        for (int t = m + 1; t < nstates && t <= m + 8; ++t)
+            if (same(st[t], st[m])) return true;
+        return false;
+    };
+    int most = 1;
+    while (most < kSiaMax && q + most + 1 < nstates && replaced(q + most)) ++most;
+    for (int n = most; n > 1; --n)
+        if (apart(st[q], st[q + n])) return n;
+    return 1;
 }
 
 static int sia_check_states(const chmy_grid_t* g, const chmy_field_t* st, int n, const char* what) {
@@ -709,12 +890,12 @@ static int sia_reverse_sweep(const chmy_grid_t* g, const chmy_field_t* ckpt, int
     // recompute the last segment on its own
     for (int q = 1; q < len(nseg - 1); ++q) {
         const chmy_field_t s0 = state(nseg - 1, q - 1), s1 = state(nseg - 1, q);
-        SiaStep<double> f = sia_stepper(g, &s0, &s1, B, A, p, dts[(nseg - 1) * stride + q - 1]);
+        SiaStep<double> f = sia_stepper(g, &s0, &s1, B, A, p);
         if (dbuf) {
             f.wd = 1;
             f.Dout = dfield(nseg - 1, q - 1);
         }
-        launch_step_tile(sia_tiles(nx, ny, 1), st, f, nx, ny);
+        launch_steps(st, f, &dts[(nseg - 1) * stride + q - 1], 1, nx, ny);
     }
     int slot = 0;   // lam_in of the next adjoint step: 0 = lam_a, 1 = lam_b
     for (int sg = nseg - 1; sg >= 0; --sg) {
@@ -726,14 +907,15 @@ static int sia_reverse_sweep(const chmy_grid_t* g, const chmy_field_t* ckpt, int
             SiaStep<double> f{};
             if (fw) {
                 const chmy_field_t s0 = state(sg - 1, r), s1 = state(sg - 1, r + 1);
-                f = sia_stepper(g, &s0, &s1, B, A, p, dts[(sg - 1) * stride + r]);
+                f = sia_stepper(g, &s0, &s1, B, A, p);
                 if (dbuf) {
                     f.wd = 1;
                     f.Dout = dfield(sg - 1, r);
                 }
             }
+            const double* fdt = fw ? &dts[(sg - 1) * stride + r] : nullptr;
             if (r >= L) {
-                launch_step_tile(sia_tiles(nx, ny, 1), st, f, nx, ny);
+                launch_steps(st, f, fdt, 1, nx, ny);
                 continue;
             }
             const int q = L - 1 - r;
@@ -746,7 +928,7 @@ static int sia_reverse_sweep(const chmy_grid_t* g, const chmy_field_t* ckpt, int
                 a.rd = 1;
                 a.Din = dfield(sg, q);
             }
-            launch_adj_tile(sia_tiles(nx, ny, fw ? 2 : 1), st, a, f, nx, ny);
+            launch_adj(st, a, fw ? &f : nullptr, fw ? *fdt : 0.0, nx, ny);
             slot ^= 1;
         }
     }
@@ -888,7 +1070,7 @@ int chmy_sia_step_adjoint(const chmy_grid_t* g, const chmy_field_t* H, const chm
     SiaPar p{As, npow, mb_a, mb_b, mb_c, dt};
     if (!work) {   // one tiled pass
         SiaAdj<double> a = sia_adjointer(g, H, lam_in, lam_out, A ? grad_logA : nullptr, B, A, p, dt);
-        launch_adj_tile(sia_tiles(g->n[0], g->n[1], 1), (hipStream_t)stream, a, SiaStep<double>{}, g->n[0], g->n[1]);
+        launch_adj((hipStream_t)stream, a, nullptr, 0.0, g->n[0], g->n[1]);
         CHMY_HIP(hipGetLastError());
         return 0;
     }
@@ -927,16 +1109,18 @@ int chmy_sia_run(const chmy_grid_t* g, const chmy_field_t* states, int nstates, 
             return set_error(CHMY_E_ARG, "states[%d] and states[%d] share storage", q, q + 1);
     const SiaPar p{As, npow, mb_a, mb_b, mb_c, 0.0};
     hipStream_t st = (hipStream_t)stream;
-    for (int q = 0; q + 1 < nstates; ++q) {
-        SiaStep<double> f = sia_stepper(g, &states[q], &states[q + 1], B, A, p, dts[q]);
-        launch_step_tile(sia_tiles(g->n[0], g->n[1], 1), st, f, g->n[0], g->n[1]);
+    for (int q = 0; q + 1 < nstates;) {
+        const int n = sia_run_length(states, nstates, q);
+        const SiaStep<double> f = sia_stepper(g, &states[q], &states[q + n], B, A, p);
+        launch_steps(st, f, dts + q, n, g->n[0], g->n[1]);
+        q += n;
     }
     CHMY_HIP(hipGetLastError());
     return 0;
 }
 
-// Per step: D and its maximum, then the step, which reads both; no host wait
-// until the caller reads the Δt.  The host-side rule took three launches, a
+// One launch per step: the step with the Δt of its state's max(D), then the new
+// state's max(D); no host wait until the caller reads the Δt.  The host-side rule took three launches, a
 // copy and a wait per step (57 us a step at 250x230; now 11).
 int chmy_sia_run_adaptive(const chmy_grid_t* g, const chmy_field_t* states, int nstates, const chmy_field_t* B,
                           const chmy_field_t* A, double As, int npow, double mb_a, double mb_b, double mb_c, double h2,
@@ -962,14 +1146,19 @@ int chmy_sia_run_adaptive(const chmy_grid_t* g, const chmy_field_t* states, int 
                        (int64_t)n);
     const dim3 grd((unsigned)((nx + 63) / 64), (unsigned)((ny + 3) / 4), 1);
     for (int q = 0; q < n; ++q) {
-        SiaStep<double> f = sia_stepper(g, &states[q], &states[q + 1], B, A, p, 0.0);
+        SiaStep<double> f = sia_stepper(g, &states[q], &states[q + 1], B, A, p);
         f.Dout = view<double>(*D);
-        if (npow == 3)
-            hipLaunchKernelGGL((sia_d_max_kernel<double, 3>), grd, sia_blk(), 0, st, f.s, f.Dout, nx, ny, dmax + q);
-        else
-            hipLaunchKernelGGL((sia_d_max_kernel<double, 0>), grd, sia_blk(), 0, st, f.s, f.Dout, nx, ny, dmax + q);
-        const SiaRule r{dmax + q, h2, dt_max, work_dev + q};
-        hipLaunchKernelGGL(sia_step_rule_tile<double>, sia_tiles(nx, ny, 1), dim3(kST), 0, st, f, r, nx, ny);
+        if (q == 0) {   // the first state's D and maximum
+            if (npow == 3)
+                hipLaunchKernelGGL((sia_d_max_kernel<double, 3>), grd, sia_blk(), 0, st, f.s, f.Dout, nx, ny, dmax);
+            else
+                hipLaunchKernelGGL((sia_d_max_kernel<double, 0>), grd, sia_blk(), 0, st, f.s, f.Dout, nx, ny, dmax);
+        }
+        const bool last = q + 1 == n;
+        f.wd = last;   // D keeps the last evaluated state's, as the rule leaves it
+        const SiaRule r{dmax + q, last ? nullptr : dmax + q + 1, h2, dt_max, work_dev + q};
+        if (last) launch_rule<false>(st, f, r, nx, ny);
+        else launch_rule<true>(st, f, r, nx, ny);
     }
     CHMY_HIP(hipGetLastError());
     return 0;

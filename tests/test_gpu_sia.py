@@ -375,3 +375,67 @@ def test_adaptive_run_equals_rule_and_step(arch, dims, npow, with_A, dt_max):
         assert torch.equal(S.D.data, want_D)
         for a, b in zip(states, want_states):
             assert torch.equal(a.data, b.data)
+
+
+@pytest.mark.parametrize("npow", [3, 2])
+@pytest.mark.parametrize("n", [(2, 3), (52, 20), (53, 37), (57, 11), (116, 45), (125, 61), (700, 402)])
+def test_multi_step_regions_equal_single_steps(arch, n, npow):
+    """Several steps to a launch, the adaptive step's next max(D) and the
+    adjoint's regions at their edges (owned columns 52, 56, 58, 60, rows 10,
+    20, 36 and one more; 32- and 48-row regions): bitwise the per-point step
+    with its Neumann batch, the rule on the stored D, and the five gather
+    passes."""
+    g, og, H, hH, B, hB, A, hA = _setup(arch, n=n, seed=19)
+    S = SIA(arch, g, hB.arr, logA=np.log(hA.arr), As=0.5, npow=npow, mb=(0.5, 0.3, 0.25))
+    dt = 1e-2 * min(e / m for e, m in zip(g.extent, n)) ** 2
+    dts = [dt * (1 + 0.1 * k) for k in range(8)]
+    want = [hH.arr.copy()]
+    S.reset(hH.arr)
+    for d in dts:
+        S.step(d)
+        S.H.swap(S.H2)
+        want.append(dev(S.H).copy())
+    S.reset(hH.arr)
+    S.forward(8, dts)
+    assert np.array_equal(dev(S.H), want[8]) and np.array_equal(dev(S.H2), want[7])
+    # every state kept, and buffers reused out of turn (0 1 0 2 1 2 0 1 3)
+    for order in (range(9), (0, 1, 0, 2, 1, 2, 0, 1, 3)):
+        f = [S._field() for _ in range(max(order) + 1)]
+        f[order[0]].data.copy_(torch.from_numpy(hH.arr))
+        S.run([f[q] for q in order], dts)
+        for q, x in enumerate(f):
+            k = max(p for p in range(9) if order[p] == q)
+            assert np.array_equal(dev(x), want[k]), (order, k)
+    # the adaptive rule over three steps
+    S.reset(hH.arr)
+    got = S.forward(3)
+    T = SIA(arch, g, hB.arr, logA=np.log(hA.arr), As=0.5, npow=npow, mb=(0.5, 0.3, 0.25))
+    T.reset(hH.arr)
+    for k in range(3):
+        d = T.dt_rule()
+        assert got[k] == d
+        T.step(d)
+        T.H.swap(T.H2)
+    assert np.array_equal(dev(S.H), dev(T.H)) and np.array_equal(dev(S.D), dev(T.D))
+    # the adjoint step against the five passes, and the reverse sweep (stored D, riding steps)
+    rng = np.random.default_rng(2)
+    lam0 = torch.from_numpy(rng.standard_normal((n[1], n[0])).T.copy()).to(S.lam.data.device)
+    out = []
+    for passes in (1, 5):
+        S.reset(want[3])
+        for a in (S.grad, S.lam, S.lam2):
+            a.data.zero_()
+        S.lam.interior().copy_(lam0)
+        S._adjoint_step(S.H, dt, passes=passes)
+        out.append((S.lam.interior().cpu().numpy().copy(), S.grad.interior().cpu().numpy().copy()))
+    assert np.array_equal(out[0][0], out[1][0]) and np.array_equal(out[0][1], out[1][1])
+    obs = torch.from_numpy(want[8][2:-2, 2:-2].T.copy()).to(S.lam.data.device) * 0.97
+    _, grad = S.gradient(hH.arr, obs, 8, dts, ncheck=2)
+    lam = S.lam.interior().clone()
+    for a in (S.grad, S.lam, S.lam2):
+        a.data.zero_()
+    S.lam.interior().copy_(torch.from_numpy(want[8][2:-2, 2:-2].T.copy()).to(S.lam.data.device) - obs)
+    for k in reversed(range(8)):
+        S.reset(want[k])
+        S._adjoint_step(S.H, dts[k], passes=5)
+    assert torch.equal(S.lam.interior(), lam) and torch.equal(S.grad.interior(), grad)
