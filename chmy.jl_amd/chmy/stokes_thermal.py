@@ -18,15 +18,18 @@ bitwise those of the reference's kernel sequence.
 """
 from __future__ import annotations
 
+import ctypes as C
 import math
 
 import torch
 
+from . import _lib
+from .architectures import current_stream
 from .boundary_conditions import Neumann, batch
 from .fields import Field, VectorField
 from .grids import Center, spacing
 from .kernel_launch import Launcher
-from .kernels import maxabs, thermal_step, update_old
+from .kernels import _arr, maxabs, thermal_step, update_old
 from .stokes import PTStokes
 
 
@@ -109,8 +112,11 @@ class StokesThermal:
                 # iterations q and q+1 in one pass; each thermal update reads
                 # the V of its own iteration (Stokes does not read T)
                 S.pass2_first(self._V1)
-                self._thermal(self._V1, dt)
-                self._thermal(S.V, dt)
+                if g.nd == 3 and q + 1 < niter:   # the call's last step stores qT
+                    self._thermal2(self._V1, S.V, dt)
+                else:
+                    self._thermal(self._V1, dt)
+                    self._thermal(S.V, dt)
                 q += 2
                 continue
             S.iteration(write_res=check)
@@ -131,6 +137,16 @@ class StokesThermal:
         src, dst = self._tp, 1 - self._tp
         self.launch(self.arch, g, (thermal_step, (self._Tbuf[src], self._Tbuf[dst], self.T_old, self.qT,
                                                   V, self.lam, dt, g)), bc=self._Tbcs[dst])
+        self._tp = dst
+
+    def _thermal2(self, V1, V2, dt):
+        """_thermal with V1, then with V2, in one launch (the T batch between
+        them in the kernel, qT not stored), and the T batch on the result."""
+        dst = 1 - self._tp
+        _lib.call("chmy_thermal_step2", C.byref(self.grid.desc()), C.byref(self.T.desc()),
+                  C.byref(self._Tbuf[dst].desc()), C.byref(self.T_old.desc()), _arr(V1), _arr(V2), self.lam, float(dt),
+                  current_stream())
+        self._Tbcs[dst].apply()
         self._tp = dst
 
     def run(self, nt=2, niter=None, ncheck=None, eps=1e-6):

@@ -5,7 +5,7 @@
 // streaming kernels; the fused Stokes iteration lives in stokes.hip.
 #include <cstring>
 
-#include "common.hpp"
+#include "stokes_pt.hpp"
 
 namespace chmy {
 
@@ -443,6 +443,113 @@ __global__ void __launch_bounds__(64 * kThY) thermal_step3_kernel(Box3 b, DF<T> 
     }
 }
 
+// Two thermal steps in one launch (3D), with T's Neumann(0) batch between
+// them: T -> T1 (V of the first step) -> T_out at cells 1..n (V of the
+// second).  T1 is never stored, nor any qT, so the two steps read T, T_old
+// and both V once and write T_out once: 9 arrays where two
+// thermal_step3_kernel launches move 18.  A block is 64 lanes x BY rows
+// marching z: at plane s the first step forms T1(s) from T's planes in
+// registers, and the second forms T_out(s - 1) from T1(s - 2 .. s) and T1's
+// neighbouring rows in LDS (two planes by parity, one barrier a plane); x
+// neighbours come by lane shifts.  T1 is exact on lanes 1..62 and all rows,
+// T_out on lanes 2..61 and rows 1..BY-2.  A plane's loads are issued one
+// plane ahead, since a block of one wave per row has few loads in flight.
+// Same expressions as thermal_step3_kernel, so bitwise the two launches with
+// chmy_bc_batchset between them.
+// 175x159x143 FP64: 2 x 81 us -> 92 us (286 MB at least: 3.1 TB/s; 8, 10 and
+// 12 rows a block and 2 to 4 blocks a CU were within 1%, so it runs at what
+// the 12 strided streams give, not at its occupancy).
+constexpr int kTh2Y = 16;
+
+template <class T>
+struct Thermal2 {
+    DF<T> Tf, Tout, To, V1[3], V2[3];
+    T nlam, dt, is[3];
+    int n[3], nbx, nby, kchunk;
+};
+
+template <class T>
+__global__ void __launch_bounds__(64 * kTh2Y) thermal_step2_kernel(Thermal2<T> a) {
+    __shared__ T s1[2][kTh2Y][64];
+    const int lane = threadIdx.x, ty = __builtin_amdgcn_readfirstlane(threadIdx.y);
+    const int lt = xcd_remap(blockIdx.x, gridDim.x);
+    const int bx = lt % a.nbx, by = (lt / a.nbx) % a.nby, bz = lt / (a.nbx * a.nby);
+    const int n0 = a.n[0], n1 = a.n[1], n2 = a.n[2];
+    const int i = bx * 60 - 1 + lane, j = by * (kTh2Y - 2) + ty;   // lane 2 and row 1 of the first tile: cell 1
+    const int kb = 1 + bz * a.kchunk, ke = min(kb + a.kchunk, n2 + 1);
+    const uint32_t ic = (uint32_t)min(max(i, 0), n0 + 1);
+    const int jc = min(max(j, 0), n1 + 1);
+    const bool own = lane >= 2 && lane <= 61 && i <= n0 && ty >= 1 && ty <= kTh2Y - 2 && j <= n1;
+    const T nlam = a.nlam, dt = a.dt, ix = a.is[0], iy = a.is[1], iz = a.is[2];
+    auto row = [](const DF<T>& f, int j, int k) -> T* { return f.p + ((int64_t)j * f.sy + (int64_t)k * f.sz); };
+    const int s0 = max(kb - 1, 1);
+    // plane s of T, its rows beside, V1 at the plane (z: the face above), T_old
+    T tc = row(a.Tf, jc, s0)[ic];
+    T qz = th_flux(tc, row(a.Tf, jc, s0 - 1)[ic], row(a.V1[2], jc, s0)[ic], nlam, iz);
+    T tp, tym, typ, vx, vy, vy1, vz1, to;
+    T wx, wy, wy1, wz1;   // V2 at the plane (z: the face above)
+    T toc = T(0), wxc = T(0), wyc = T(0), wy1c = T(0), wz1c = T(0);   // of plane s - 1
+    auto fetch = [&](int s) {
+        tp = row(a.Tf, jc, s + 1)[ic];
+        tym = row(a.Tf, jc - 1, s)[ic];
+        typ = row(a.Tf, jc + 1, s)[ic];
+        vx = row(a.V1[0], jc, s)[ic];
+        vy = row(a.V1[1], jc, s)[ic];
+        vy1 = row(a.V1[1], jc + 1, s)[ic];
+        vz1 = row(a.V1[2], jc, s + 1)[ic];
+        to = row(a.To, jc, s)[ic];
+        wx = row(a.V2[0], jc, s)[ic];
+        wy = row(a.V2[1], jc, s)[ic];
+        wy1 = row(a.V2[1], jc + 1, s)[ic];
+        wz1 = row(a.V2[2], jc, s + 1)[ic];
+    };
+    fetch(s0);
+    T t1m = T(0), t1c = T(0), q2z = T(0);
+    for (int s = s0; s <= ke; ++s) {
+        T t1;
+        if (s <= n2) {   // the first step at plane s
+            const T qx = th_flux(tc, xm1(tc), vx, nlam, ix);
+            const T qxr = xp1(qx);
+            const T qy = th_flux(tc, tym, vy, nlam, iy), qyr = th_flux(typ, tc, vy1, nlam, iy);
+            const T qzr = th_flux(tp, tc, vz1, nlam, iz);
+            const T dv = ((qxr - qx) * ix + (qyr - qy) * iy) + (qzr - qz) * iz;
+            t1 = to - dt * dv;
+            tc = tp;
+            qz = qzr;
+            // x ghosts: the adjacent cell (fma(h, -0, f) and fma(h, 0, f) of the batch)
+            const T up = xp1(t1), dn = xm1(t1) + T(0);
+            t1 = i <= 0 ? up : i == n0 + 1 ? dn : t1;
+        } else {
+            t1 = t1c + T(0);   // z's upper ghost
+        }
+        const T to_s = to, wx_s = wx, wy_s = wy, wy1_s = wy1, wz1_s = wz1;
+        if (s + 1 <= min(ke, n2)) fetch(s + 1);
+        s1[s & 1][ty][lane] = t1;
+        const int r = s - 1;
+        if (r >= kb) {   // the second step at plane s - 1
+            const int b = r & 1;
+            const T lo = s1[b][ty > 0 ? ty - 1 : ty][lane], hi = s1[b][ty < kTh2Y - 1 ? ty + 1 : ty][lane];
+            const T tm = j == 1 ? t1c : lo, tq = j == n1 ? t1c + T(0) : hi;
+            if (r == kb) q2z = th_flux(t1c, r == 1 ? t1c : t1m, row(a.V2[2], jc, r)[ic], nlam, iz);
+            const T qx = th_flux(t1c, xm1(t1c), wxc, nlam, ix);
+            const T qxr = xp1(qx);
+            const T qy = th_flux(t1c, tm, wyc, nlam, iy), qyr = th_flux(tq, t1c, wy1c, nlam, iy);
+            const T qzr = th_flux(t1, t1c, wz1c, nlam, iz);
+            const T dv = ((qxr - qx) * ix + (qyr - qy) * iy) + (qzr - q2z) * iz;
+            if (own) row(a.Tout, j, r)[ic] = toc - dt * dv;
+            q2z = qzr;
+        }
+        t1m = t1c;
+        t1c = t1;
+        toc = to_s;
+        wxc = wx_s;
+        wyc = wy_s;
+        wy1c = wy1_s;
+        wz1c = wz1_s;
+        __syncthreads();
+    }
+}
+
 template <class T>
 __global__ void __launch_bounds__(256) thermal_update_kernel(Box3 b, DFL<T> Tf, DFL<T> To, DFL<T> q0, DFL<T> q1,
                                                              DFL<T> q2, int nd, T dt, T i0, T i1, T i2) {
@@ -812,6 +919,55 @@ int chmy_thermal_step(const chmy_grid_t* g, const chmy_box_t* box, const chmy_fi
         hipLaunchKernelGGL(thermal_step_kernel<T>, grd, blk2(), 0, (hipStream_t)stream, b, t, to, o, v0, v1, v2, q0,
                            q1, q2, g->nd, -T(lam), T(dt), T(g->inv_spacing[0]), T(g->inv_spacing[1]),
                            T(g->inv_spacing[2]));
+        CHMY_HIP(hipGetLastError());
+        return 0;
+    };
+    return Tf->dtype == CHMY_F64 ? launch(0.0) : launch(0.0f);
+}
+
+int chmy_thermal_step2(const chmy_grid_t* g, const chmy_field_t* Tf, const chmy_field_t* T_out, const chmy_field_t* To,
+                       const chmy_field_t* V1, const chmy_field_t* V2, double lam, double dt, void* stream) {
+    CHMY_TRY(check_grid(g));
+    if (g->nd != 3) return set_error(CHMY_E_ARG, "chmy_thermal_step2 is 3D");
+    CHMY_TRY(check_center(g, Tf, "T", -1));
+    CHMY_TRY(check_center(g, T_out, "T_out", Tf->dtype));
+    CHMY_TRY(check_center(g, To, "T_old", Tf->dtype));
+    CHMY_TRY(check_vector(g, V1, "V1", Tf->dtype));
+    CHMY_TRY(check_vector(g, V2, "V2", Tf->dtype));
+    if (T_out->data == Tf->data || T_out->data == To->data)
+        return set_error(CHMY_E_ARG, "T_out must be distinct from T and T_old");
+    auto launch = [&](auto zero) -> int {
+        using T = decltype(zero);
+        Thermal2<T> a;
+        a.Tf = view<T>(*Tf);
+        a.Tout = view<T>(*T_out);
+        a.To = view<T>(*To);
+        for (int d = 0; d < 3; ++d) {
+            a.V1[d] = view<T>(V1[d]);
+            a.V2[d] = view<T>(V2[d]);
+            a.is[d] = T(g->inv_spacing[d]);
+            a.n[d] = (int)g->n[d];
+        }
+        a.nlam = -T(lam);
+        a.dt = T(dt);
+        a.nbx = (a.n[0] + 59) / 60;
+        a.nby = (a.n[1] + kTh2Y - 3) / (kTh2Y - 2);
+        // chunks of z that fill whole rounds of the CUs (one block a CU, 2
+        // planes a chunk recomputed), as the two-iteration Stokes pass picks its own
+        const int64_t tiles = (int64_t)a.nbx * a.nby, slots = cu_count();
+        int64_t best = INT64_MAX;
+        a.kchunk = a.n[2];
+        for (int nch = 1; nch <= a.n[2] && nch <= 64; ++nch) {
+            const int k = (a.n[2] + nch - 1) / nch;
+            const int64_t cost = (tiles * ((a.n[2] + k - 1) / k) + slots - 1) / slots * (k + 2);
+            if (cost < best) {
+                best = cost;
+                a.kchunk = k;
+            }
+        }
+        const int64_t nb = tiles * ((a.n[2] + a.kchunk - 1) / a.kchunk);
+        if (nb > INT32_MAX) return set_error(CHMY_E_SIZE, "thermal step: box too large");
+        hipLaunchKernelGGL(thermal_step2_kernel<T>, dim3((unsigned)nb), dim3(64, kTh2Y, 1), 0, (hipStream_t)stream, a);
         CHMY_HIP(hipGetLastError());
         return 0;
     };

@@ -250,6 +250,15 @@ int chmy_thermal_step(const chmy_grid_t* grid, const chmy_box_t* box, const chmy
                       const chmy_field_t* T_out, const chmy_field_t* T_old, const chmy_field_t* qT,
                       const chmy_field_t* V, double lambda_rhoCp, double dt, void* stream);
 
+/* Two thermal steps in one launch, 3D (build extension): chmy_thermal_step
+ * with V1, T's Neumann(0) batch on every side, chmy_thermal_step with V2.
+ * T holds its batch's ghosts; T_out (another buffer than T and T_old) receives
+ * the cells 1..n, bitwise those of the three launches; the caller applies the
+ * batch to it.  No qT is stored. */
+int chmy_thermal_step2(const chmy_grid_t* grid, const chmy_field_t* T, const chmy_field_t* T_out,
+                       const chmy_field_t* T_old, const chmy_field_t* V1, const chmy_field_t* V2, double lambda_rhoCp,
+                       double dt, void* stream);
+
 /* One fused PT iteration = update_stress! then update_velocity! over the
  * Launcher box (examples/stokes_3d_inc_ve_T.jl:164-165), double-buffered:
  * reads (V, tau, Pr) and writes (V_out, tau_out, Pr_out), so no block reads a

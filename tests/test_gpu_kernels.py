@@ -6,12 +6,15 @@ bitwise equality in f64 and f32: both sides evaluate the same IEEE
 expressions with no contraction and fma only at the reference's muladd
 sites.
 """
+import ctypes as C
+
 import numpy as np
 import pytest
 import torch
 
 import chmy
-from chmy import Center as Cc, Vertex as Vv
+from chmy import Center as Cc, Vertex as Vv, _lib
+from chmy.kernels import _arr
 import oracle as O
 from _helpers import NP2TORCH, assert_same, dev, ogrid, pair, vloc
 
@@ -480,6 +483,40 @@ def test_thermal_step_3d_march_equals_two_kernels(arch, T, dims):
         assert not np.any(dev(Tn)[sl] == 0)
         for a, b in zip(q, q2):
             assert np.array_equal(dev(a).view(bits), dev(b).view(bits)), f"qT box {lo} {ws}"
+
+
+@pytest.mark.parametrize("T", TYPES)
+@pytest.mark.parametrize("dims", [(60, 14, 5), (61, 15, 70), (130, 29, 45), (2, 1, 2), (3, 40, 1), (64, 16, 30)])
+def test_thermal_two_steps_in_one_launch(arch, T, dims):
+    """chmy_thermal_step2 at exactly full and one-over tiles (60 columns, 14
+    rows), one and several z chunks and the smallest grids: bitwise the two
+    steps with T's Neumann batch between them, on the cells and, after the
+    batch, on the ghosts."""
+    g = chmy.UniformGrid(origin=(-0.5, -0.5, -0.5), extent=(1.0, 0.9, 1.2), dims=dims)
+    og = ogrid(g)
+    rng = np.random.default_rng(sum(dims))
+    Ta, Tb, To, Tc = (pair(arch, g, og, (Cc(),) * 3, T, rng=rng)[0] for _ in range(4))
+    V1, V2, q = ([pair(arch, g, og, vloc(D, 3), T, rng=rng, lo=-1.0)[0] for D in range(3)] for _ in range(3))
+    lam, dt = 0.7, 0.21 * min(chmy.spacing(g)) ** 2
+    bcs = {id(f): chmy.batch(g, (f, chmy.Neumann())) for f in (Ta, Tb, Tc)}
+    bcs[id(Ta)].apply()
+    n = g.dims
+    lo, ws = (0, 0, 0), tuple(m + 2 for m in n)
+    _lib.call("chmy_thermal_step2", C.byref(g.desc()), C.byref(Ta.desc()), C.byref(Tc.desc()), C.byref(To.desc()),
+              _arr(V1), _arr(V2), lam, dt, chmy.current_stream())
+    bcs[id(Tc)].apply()
+    chmy.kernels.thermal_step.launch(g, lo, ws, Ta, Tb, To, q, V1, lam, dt, g)
+    bcs[id(Tb)].apply()
+    chmy.kernels.thermal_step.launch(g, lo, ws, Tb, Ta, To, q, V2, lam, dt, g)
+    bcs[id(Ta)].apply()
+    chmy.synchronize()
+    bits = np.int64 if T == np.float64 else np.int32
+    assert np.array_equal(dev(Tc)[2:-2, 2:-2, 2:-2].view(bits), dev(Ta)[2:-2, 2:-2, 2:-2].view(bits))
+    box = tuple(slice(1, 3 + m) for m in reversed(n))
+    assert np.array_equal(dev(Tc)[box].view(bits), dev(Ta)[box].view(bits))
+    with pytest.raises(chmy.ChmyError):
+        _lib.call("chmy_thermal_step2", C.byref(g.desc()), C.byref(Ta.desc()), C.byref(Ta.desc()),
+                  C.byref(To.desc()), _arr(V1), _arr(V2), lam, dt, chmy.current_stream())
 
 
 def test_empty_box_is_a_no_op(arch):
