@@ -29,7 +29,7 @@ from .boundary_conditions import Neumann, batch
 from .fields import Field, VectorField
 from .grids import Center, spacing
 from .kernel_launch import Launcher
-from .kernels import _arr, maxabs, thermal_step, update_old
+from .kernels import _arr, maxabs_many, thermal_step, update_old
 from .stokes import PTStokes
 
 
@@ -73,7 +73,7 @@ class StokesThermal:
         g = self.grid
         d = spacing(g)
         dt_diff = min(d) ** 2 / self.lam / g.nd / 2.1
-        vmax = [maxabs(self.S.V[D]) for D in range(g.nd)]
+        vmax = maxabs_many([self.S.V[D] for D in range(g.nd)])
         dt_adv = 0.1 * min(d[D] / vmax[D] if vmax[D] > 0 else math.inf for D in range(g.nd)) / g.nd / 2.1
         return min(dt_diff, dt_adv)
 
