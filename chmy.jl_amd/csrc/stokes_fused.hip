@@ -1820,6 +1820,7 @@ static bool free_slip_2d(const chmy_grid_t* g, const int32_t* counts, const int3
     fs->hx = g->spacing[0];
     fs->hy = g->spacing[1];
     fs->iters = 2;
+    fs->pre = 0;
     return true;
 }
 
@@ -1919,16 +1920,23 @@ int chmy_stokes_iterate(const chmy_grid_t* g, const chmy_field_t* V0, const chmy
     for (int it = 0; it < niter;) {
         const int fl = it == niter - 1 ? flags_last : flags;
         const int fl2 = it + 1 == niter - 1 ? flags_last : flags;
-        // 2D: as many iterations of the same flags as a pass takes, three or more
-        int m = 1;
-        while (m < most && it + m < niter && (it + m == niter - 1 ? flags_last : flags) == fl) ++m;
-        if (tb2 && m > 2 && !(fl & CHMY_ITER_RESIDUAL)) {
+        // 2D: a run of iterations of the same flags in passes of up to `most`, three
+        // or more each, evenly long (a remainder of one or two would take a launch
+        // that moves the state for itself)
+        const int run = flags == flags_last ? niter - it : it < niter - 1 ? niter - 1 - it : 1;
+        if (tb2 && run > 2 && !(fl & CHMY_ITER_RESIDUAL)) {
+            const int passes = (run + most - 1) / most, m = (run + passes - 1) / passes;
             fs.iters = m;
             CHMY_TRY(stokes_iter_impl(g, Vs[p], T[p], P[p], Vs[1 - p], T[1 - p], P[1 - p], tau_old, eta, eta_ml, rhog,
                                       f_V, f_P, divV, r_V, fl, eta_s, eta_ve_s, G, dt, dtau_Pr, dtau_r, nudtau,
                                       stream, &fs, nullptr));
-            fs.iters = 2;
             it += m;
+            fs.pre = m < run;   // the rest of the run is passes: the next applies the batch
+            if (fs.pre) {
+                p = 1 - p;
+                continue;
+            }
+            fs.iters = 2;
         } else if (tb && it + 1 < niter && fl == fl2 && !(fl & CHMY_ITER_RESIDUAL)) {
             CHMY_TRY(stokes_iter_impl(g, Vs[p], T[p], P[p], Vs[1 - p], T[1 - p], P[1 - p], tau_old, eta, eta_ml, rhog,
                                       f_V, f_P, divV, r_V, fl, eta_s, eta_ve_s, G, dt, dtau_Pr, dtau_r, nudtau,

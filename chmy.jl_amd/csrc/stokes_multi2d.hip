@@ -44,7 +44,9 @@ int multi2d_most(const chmy_grid_t* g) {
 // exact, and the tile's own are KM from each end.  Loads are clamped into the
 // stored range; clamped values reach no output.  The expressions are row2's,
 // so the results are bitwise those of single iterations with the batch
-// between them; the batch after the last one is the caller's.
+// between them; the batch after the last one is the caller's, or the next
+// pass's, which applies it to the V it reads (fs.pre; 4.5 us a launch and its
+// gap, a quarter of a pass at 127x95).
 // Bound by FP64 issue and by the one block a CU that 16 waves of 125 VGPRs
 // leave room for: loads and arithmetic of a block do not overlap.
 template <class T, bool FVISC, bool EXACT, bool HF, bool BF, bool RG, int KM, int W, int PT>
@@ -131,7 +133,7 @@ __global__ void __launch_bounds__(kFX * W) fused2d_multi_kernel(Fused2<T> a, Fre
     for (int it = 0; it < iters; ++it) {
         __syncthreads();
         T vxp = sV[1][wm][lane], vyn = sV[2][wp][lane];   // Vx at row j0 - 1, Vy at row j0 + PT
-        if (it > 0 && edge) {
+        if ((it > 0 || fs.pre) && edge) {
             const T first = vx[0];
             T rm = vxp;
 #pragma unroll

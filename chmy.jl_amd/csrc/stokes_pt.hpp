@@ -172,6 +172,7 @@ struct FreeSlip2 {
     double ax[2], qy[2], by[2], qx[2];
     double hx, hy;
     int32_t iters;   // iterations of the pass
+    int32_t pre;     // the batch is still to be applied to the V the pass reads
 };
 
 // The most iterations of a 2D pass over this grid (stokes_multi2d.hip).
