@@ -11,21 +11,28 @@ struct Shape2 {
 using Small2 = Shape2<7, 16, 1>;
 using Mid2 = Shape2<6, 16, 2>;
 using Large2 = Shape2<8, 16, 3>;
+using Dense2 = Shape2<5, 8, 3>;
 
-// Grids of at most a tile a CU take the flattest tile: their time is the
-// chain of iterations, and one row a thread makes it shortest.  Beyond that
-// the ring's share counts: 40% of the region's points are a tile's own in
-// Mid2, 50% in Large2, which pays once its tiles fill the chip several times.
-// FP64 us per iteration, Small2 / Mid2 / Large2 (two per pass before: 11.5 at
-// 127x95, 74 at 2047^2): 127x95 2.5 / 3.5 / 4; 500x400 - / 4.0 / 5.9; 1000x900
-// 11 (Mid2) / 10.1; 2047^2 45.7 / 38.5.  FP32 sweeps 2047^2 36 -> 24.
+// The first shape whose tiles all find a CU of their own is taken: the time is
+// then one block's chain of iterations, and the flatter the tile, the shorter
+// that chain.  Beyond, Dense2: two blocks of 8 waves a CU, so one computes
+// while the other loads and stores (16 waves of 125 VGPRs fill a CU alone),
+// at the same share of own points as Large2 (49% and 50%) but a pass of 5
+// iterations.  FP64 us for 33 iterations, Mid2 / Large2 / Dense2: 600x512 272 /
+// 231 / 246 (221 tiles of Large2), 800x640 340 / 313 / 297 (357 tiles),
+// 1400x1200 693 / 633 / 592; 41 at 2047^2 1734 (Large2) / 1584; other waves,
+// rows and lengths for the last one: <4, 8, 3> 1775, <6, 8, 3> 1668, <5, 16, 3>
+// 1982, <6, 12, 4> 1840, <5, 6, 4> 2512.  400x380: Mid2 and Dense2 alike.
 static int64_t tiles2(int64_t nbx, int64_t nby, int tx, int ty) { return ((nbx + tx - 1) / tx) * ((nby + ty - 1) / ty); }
+template <class Sh>
+static bool one_round(int64_t nbx, int64_t nby) {
+    return tiles2(nbx, nby, Sh::TX, Sh::TY) <= cu_count();
+}
 static int shape2(int64_t nbx, int64_t nby) {
-    if (tiles2(nbx, nby, Small2::TX, Small2::TY) <= cu_count()) return 0;
-    return nbx * nby < 300000 ? 1 : 2;
+    return one_round<Small2>(nbx, nby) ? 0 : one_round<Mid2>(nbx, nby) ? 1 : one_round<Large2>(nbx, nby) ? 2 : 3;
 }
 int multi2d_most(const chmy_grid_t* g) {
-    const int k[3] = {Small2::KM, Mid2::KM, Large2::KM};
+    const int k[4] = {Small2::KM, Mid2::KM, Large2::KM, Dense2::KM};
     return k[shape2(g->n[0] + 2, g->n[1] + 2)];
 }
 
@@ -47,10 +54,10 @@ int multi2d_most(const chmy_grid_t* g) {
 // between them; the batch after the last one is the caller's, or the next
 // pass's, which applies it to the V it reads (fs.pre; 4.5 us a launch and its
 // gap, a quarter of a pass at 127x95).
-// Bound by FP64 issue and by the one block a CU that 16 waves of 125 VGPRs
-// leave room for: loads and arithmetic of a block do not overlap.
+// Bound by FP64 issue: 16 waves of up to 128 VGPRs fill a CU (4 a SIMD, what
+// the launch bounds ask for), as one block or as two.
 template <class T, bool FVISC, bool EXACT, bool HF, bool BF, bool RG, int KM, int W, int PT>
-__global__ void __launch_bounds__(kFX * W) fused2d_multi_kernel(Fused2<T> a, FreeSlip2 fs, int iters) {
+__global__ void __launch_bounds__(kFX * W, 4) fused2d_multi_kernel(Fused2<T> a, FreeSlip2 fs, int iters) {
     using AR = Arith<T, EXACT>;
     using Loc = typename AR::Loc;
     constexpr int R = W * PT;
@@ -238,7 +245,8 @@ void multi2d_launch(Fused2<T> a, const FreeSlip2& fs, bool fv, bool exact, bool 
     switch (shape2(nbx, nby)) {
         case 0: go(Small2{}); break;
         case 1: go(Mid2{}); break;
-        default: go(Large2{}); break;
+        case 2: go(Large2{}); break;
+        default: go(Dense2{}); break;
     }
 }
 

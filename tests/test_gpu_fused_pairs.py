@@ -374,3 +374,14 @@ def test_several_iterations_per_pass_2d(arch, T, forcing, exact, visc, rhog, dim
     a = _run(arch, g, T, exact, visc, forcing, GENERAL, niter, True, 23, rhog=rhog)
     b = _run(arch, g, T, exact, visc, forcing, GENERAL, niter, False, 23, rhog=rhog)
     _compare(a, b, f"dims {dims} niter {niter}")
+
+
+@pytest.mark.parametrize("T,forcing", [(np.float64, None), (np.float32, "bf16")])
+@pytest.mark.parametrize("dims,niter", [((860, 559), 11), ((538, 1010), 8), ((1027, 640), 6)])
+def test_many_tiles_per_cu_2d(arch, T, forcing, dims, niter):
+    """Grids of several tiles a CU (8 waves, 54 x 14 points a tile; tiles that
+    end at, past and inside the box) against single iterations, bitwise."""
+    g = chmy.UniformGrid(arch, origin=(-0.5, -0.5), extent=(1.0, 1.3), dims=dims)
+    a = _run(arch, g, T, False, "field", forcing, GENERAL, niter, True, 29)
+    b = _run(arch, g, T, False, "field", forcing, GENERAL, niter, False, 29)
+    _compare(a, b, f"dims {dims} niter {niter}")
