@@ -171,6 +171,20 @@ inline dim3 grid_for(const Box3& b, dim3 blk) {
                 (unsigned)((b.len[2] + blk.z - 1) / blk.z));
 }
 
+// The q-th point of a plane of rows of len0 points, counted along the rows:
+// column a, row c (c >= len1 past the plane).  The 32-bit division unless the
+// plane has 2^32 points (uniform).
+__device__ __forceinline__ void plane_index(int64_t q, int64_t len0, int64_t len1, int64_t& a, int64_t& c) {
+    if (len0 * len1 + 0x10000 < 0x100000000ll) {
+        const uint32_t r = (uint32_t)q, n = (uint32_t)len0, k = r / n;
+        c = k;
+        a = r - k * n;
+    } else {
+        c = q / len0;
+        a = q - c * len0;
+    }
+}
+
 // Compute units of the current device, read once per device (api.hip).
 int cu_count();
 

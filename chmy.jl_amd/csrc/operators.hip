@@ -11,21 +11,22 @@
 // on the operator, the knots and the kernel's own arguments lived in scratch
 // memory, 224-368 B a lane, and that traffic was the time).
 //
-// One kernel walks the box for all of them: a block is 64 (x, one wave) x 4
-// (y) points and marches up to 4 planes in z, so that an operator's z
-// neighbour is still in L1 or L2; blocks are remapped so that each XCD gets a
-// contiguous run of tiles and the rows that y neighbours share stay in its
-// L2.  Bound by HBM (∂, divg, lerp, vmag), by loads served from L2 (lapl,
-// divg_grad: 7 and 21 loads a point) and by division (hlerp: 9 at an edge).
-// Measured, FP64, one launch, us, with the run-time switch -> now (one read
-// and one write of a field take 19 us at 191x175x167, 56 at 255^3):
-//   191x175x167  ∂ 295 -> 16, lerp to centres 430 -> 23, divg 430 -> 30,
-//                vmag 435 -> 33, lapl 440 -> 33, hlerp 227 -> 51,
-//                masked ∂ 540 -> 23, divg 804 -> 80, divg_grad 960 -> 85
-//   255^3        ∂ 57 (4.7 TB/s), divg 128 (4.2), lapl 100, divg_grad 302
-// Tiles of 8 and 16 rows and chunks of 1, 2, 8 and 16 planes were slower or
-// equal: 16 rows ∂ 32, 1 plane ∂ 29, 8 rows x 4 planes ∂ 19, 16 planes at
-// 255^3 ∂ 61.5.
+// One kernel walks the box for all of them: a block is 256 consecutive points
+// of a plane, counted along x and on into the next row, and marches up to 4
+// planes in z, so that an operator's z neighbour is still in L1 or L2; blocks
+// are remapped so that each XCD gets a contiguous run and the rows that y
+// neighbours share stay in its L2.  With one wave per 64 columns instead, a
+// row of 193 points took 4 waves, the last with one lane (1.33 times the
+// instructions).  The result is stored past the caches (non-temporal): no
+// point of it is read again.  Bound by HBM (∂, divg, lerp, vmag), by loads
+// served from L2 (lapl, divg_grad: 7 and 21 loads a point) and by division
+// (hlerp: 9 at an edge).
+// Measured, FP64 191x175x167, fields not in the caches, us a launch, 64 x 4
+// blocks -> flat -> and non-temporal (the bytes at 4.94 TB/s): ∂ 24 -> 20 -> 20
+// (18), lerp 33 -> 27 -> 27 (18), divg 48 -> 42 -> 39 (36), vmag 36 -> 31 ->
+// 29 (36), lapl 34 -> 29 -> 28 (18), hlerp 53 -> 37 -> 36 (18); masked ∂ 39 ->
+// 32 -> 31 (27), divg 91 -> 83 -> 68 (63), divg_grad 107 -> 85 -> 85 (63).
+// Chunks of 2 and 8 planes: divg_grad 84 and 93, ∂ 22 and 22.
 #include "common.hpp"
 
 namespace chmy {
@@ -282,18 +283,19 @@ struct OpVmag {
 };
 
 // ------------------------------------------------------------------ kernel
-constexpr int kOpX = 64, kOpY = 4, kOpZ = 4;
+constexpr int kOpB = 256, kOpZ = 4;
 
 template <class T, class Op>
-__global__ void __launch_bounds__(kOpX * kOpY) op_kernel(Box3 b, DF<T> dst, Op op, int nbx, int nby, int kchunk) {
+__global__ void __launch_bounds__(kOpB) op_kernel(Box3 b, DF<T> dst, Op op, int nbx, int kchunk) {
     const int t = xcd_remap(blockIdx.x, gridDim.x);
-    const int bx = t % nbx, by = (t / nbx) % nby, bz = t / (nbx * nby);
-    const int64_t a = (int64_t)bx * kOpX + threadIdx.x, c = (int64_t)by * kOpY + threadIdx.y;
-    if (a >= b.len[0] || c >= b.len[1]) return;
+    const int bx = t % nbx, bz = t / nbx;
+    int64_t a, c;
+    plane_index((int64_t)bx * kOpB + threadIdx.x, b.len[0], b.len[1], a, c);
+    if (c >= b.len[1]) return;
     const int64_t e0 = (int64_t)bz * kchunk, e1 = e0 + kchunk < b.len[2] ? e0 + kchunk : b.len[2];
     for (int64_t e = e0; e < e1; ++e) {
         const Pt p{{b.lo[0] + a, b.lo[1] + c, b.lo[2] + e}};
-        dst(p.i[0], p.i[1], p.i[2]) = op(p);
+        __builtin_nontemporal_store(op(p), &dst(p.i[0], p.i[1], p.i[2]));
     }
 }
 
@@ -377,13 +379,13 @@ struct OpCall {
 // smaller boxes, where blocks in flight count for more than reuse.
 template <class T, class Op>
 static int op_launch(const OpCall& c, const Op& op) {
-    const int64_t nbx = (c.b.len[0] + kOpX - 1) / kOpX, nby = (c.b.len[1] + kOpY - 1) / kOpY;
+    const int64_t nbx = (c.b.len[0] * c.b.len[1] + kOpB - 1) / kOpB;
     int kz = kOpZ;
-    while (kz > 1 && nbx * nby * ((c.b.len[2] + kz - 1) / kz) < 4096) kz /= 2;
-    const int64_t nb = nbx * nby * ((c.b.len[2] + kz - 1) / kz);
+    while (kz > 1 && nbx * ((c.b.len[2] + kz - 1) / kz) < 4096) kz /= 2;
+    const int64_t nb = nbx * ((c.b.len[2] + kz - 1) / kz);
     if (nb > INT32_MAX) return set_error(CHMY_E_SIZE, "operator: box too large");
-    hipLaunchKernelGGL((op_kernel<T, Op>), dim3((unsigned)nb), dim3(kOpX, kOpY, 1), 0, c.s, c.b, view<T>(*c.dst), op,
-                       (int)nbx, (int)nby, kz);
+    hipLaunchKernelGGL((op_kernel<T, Op>), dim3((unsigned)nb), dim3(kOpB, 1, 1), 0, c.s, c.b, view<T>(*c.dst), op, (int)nbx,
+                       kz);
     CHMY_HIP(hipGetLastError());
     return 0;
 }

@@ -81,6 +81,33 @@ def test_divg_vmag(arch, T, nd):
     assert_same(out, hout, "vmag")
 
 
+@pytest.mark.parametrize("T", TYPES)
+@pytest.mark.parametrize("dims", [(1, 1, 1), (62, 3, 5), (191, 4, 9), (254, 1, 3), (255, 2, 17), (3, 300, 2), (700, 5)])
+def test_operator_rows_across_blocks(arch, T, dims):
+    """Planes whose rows end inside, at and one past a block of 256 points,
+    several z chunks, and boxes inside the grid, against the oracle; points
+    outside the box keep their bits."""
+    nd = len(dims)
+    g = chmy.UniformGrid(arch, origin=(-1.0,) * nd, extent=(2.0,) * nd, dims=dims)
+    og = ogrid(g)
+    rng = np.random.default_rng(sum(dims))
+    V = [pair(arch, g, og, vloc(D, nd), T, rng=rng) for D in range(nd)]
+    out, hout = pair(arch, g, og, Cc(), T, rng=rng)
+    before = dev(out).copy()
+    chmy.kernels.divg.launch(g, (0,) * nd, tuple(n + 2 for n in dims), out, [v for v, _ in V], g)
+    O.op("divg", og, hout, [h for _, h in V])
+    chmy.synchronize()
+    assert_same(out, hout, "divg")
+    whole = dev(out).copy()
+    out.data.copy_(torch.from_numpy(before))
+    lo, ws = (1,) * nd, tuple(max(1, n - 1) for n in dims)
+    chmy.kernels.divg.launch(g, lo, ws, out, [v for v, _ in V], g)
+    chmy.synchronize()
+    sl = tuple(slice(1 + l, 1 + l + w) for l, w in zip(lo[::-1], ws[::-1]))
+    before[sl] = whole[sl]
+    assert np.array_equal(dev(out), before)
+
+
 def test_reference_operator_identities(arch):
     """test/test_grid_operators.jl:14-42,114-132 through the GPU Launcher:
     divg(V) == ∂xVx + ∂yVy + ∂zVz exactly; vmag of a constant 2-vector ≈ 3.4641."""
