@@ -165,12 +165,6 @@ inline Box3 box3(const chmy_box_t& b, int nd) {
 // KernelAbstractions launch over an empty worksize does no work).
 inline bool no_work(const Box3& b) { return b.len[0] <= 0 || b.len[1] <= 0 || b.len[2] <= 0; }
 
-// Block of 256 threads as 64 (x, one wave) x 4 (y); grid covers the box.
-inline dim3 grid_for(const Box3& b, dim3 blk) {
-    return dim3((unsigned)((b.len[0] + blk.x - 1) / blk.x), (unsigned)((b.len[1] + blk.y - 1) / blk.y),
-                (unsigned)((b.len[2] + blk.z - 1) / blk.z));
-}
-
 // The q-th point of a plane of rows of len0 points, counted along the rows:
 // column a, row c (c >= len1 past the plane).  The 32-bit division unless the
 // plane has 2^32 points (uniform).
@@ -183,6 +177,27 @@ __device__ __forceinline__ void plane_index(int64_t q, int64_t len0, int64_t len
         c = q / len0;
         a = q - c * len0;
     }
+}
+
+// Per-point kernels: blocks of 256 consecutive points of a plane (counted along
+// x and on into the next row, so no lane idles at a row's end), plane after
+// plane, each XCD a contiguous run of them: the planes and rows that a
+// neighbour's point shares are found in that XCD's L2.
+constexpr int kFlat = 256;
+inline dim3 flat_grid(const Box3& b) {
+    return dim3((unsigned)((b.len[0] * b.len[1] + kFlat - 1) / kFlat * b.len[2]), 1, 1);
+}
+__device__ __forceinline__ bool flat_point(const Box3& b, int64_t& i, int64_t& j, int64_t& k) {
+    const uint32_t per = (uint32_t)((b.len[0] * b.len[1] + kFlat - 1) / kFlat), nb = gridDim.x;
+    // xcd_remap on unsigned ids
+    const uint32_t run = nb / 8, id = blockIdx.x < 8 * run ? (blockIdx.x % 8) * run + blockIdx.x / 8 : blockIdx.x;
+    const uint32_t e = id / per;
+    int64_t a, c;
+    plane_index((int64_t)(id - e * per) * kFlat + threadIdx.x, b.len[0], b.len[1], a, c);
+    i = b.lo[0] + a;
+    j = b.lo[1] + c;
+    k = b.lo[2] + e;
+    return c < b.len[1];
 }
 
 // Compute units of the current device, read once per device (api.hip).

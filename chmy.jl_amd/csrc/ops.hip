@@ -1,26 +1,24 @@
 // Per-point Launcher kernels: diffusion, update_old!, thermal flux/update and
-// the viscosity max-neighbourhood.  Each thread owns
-// one logical index I of the box; blocks are one wave64 wide along x (the
-// contiguous dim) so loads and stores coalesce.  These are bandwidth-bound
-// streaming kernels; the fused Stokes iteration lives in stokes.hip.
+// the viscosity max-neighbourhood.  Each thread owns one logical index I of the
+// box, 256 consecutive points of a plane a block (flat_point).  These are
+// bandwidth-bound streaming kernels; the fused Stokes iteration lives in
+// stokes_fused.hip.  159x143x127 FP64, us, 64 x 4 blocks -> flat ones: thermal
+// flux 37.5 -> 31, update 34 -> 28.6, update_old! (loads before stores) 69 -> 60;
+// a diffusion step through the Launcher at 160x150x140 111 -> 94.
 #include <cstring>
 
 #include "stokes_pt.hpp"
 
 namespace chmy {
 
-constexpr int kBX = 64, kBY = 4;
-
 struct Ix3 {
     int64_t i, j, k;
 };
 
 __device__ __forceinline__ Ix3 box_index(const Box3& b, bool& ok) {
-    int64_t a = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
-    int64_t c = blockIdx.y * (int64_t)blockDim.y + threadIdx.y;
-    int64_t e = blockIdx.z * (int64_t)blockDim.z + threadIdx.z;
-    ok = a < b.len[0] && c < b.len[1] && e < b.len[2];
-    return Ix3{b.lo[0] + a, b.lo[1] + c, b.lo[2] + e};
+    Ix3 I;
+    ok = flat_point(b, I.i, I.j, I.k);
+    return I;
 }
 
 template <class T>
@@ -309,7 +307,13 @@ __global__ void __launch_bounds__(256) copy_kernel(Box3 b, Copy7<T> c) {
     bool ok;
     Ix3 I = box_index(b, ok);
     if (!ok) return;
-    for (int q = 0; q < c.n; ++q) g_at(c.dst[q], I) = g_at(c.src[q], I);
+    T v[7];
+#pragma unroll
+    for (int q = 0; q < 7; ++q)
+        if (q < c.n) v[q] = g_at(c.src[q], I);
+#pragma unroll
+    for (int q = 0; q < 7; ++q)
+        if (q < c.n) g_at(c.dst[q], I) = v[q];
 }
 
 // ------------------------------------------------------------------ thermal
@@ -577,7 +581,7 @@ __global__ void __launch_bounds__(256) maxloc_kernel(Box3 b, DFL<T> dst, DFL<T> 
 }
 
 // ------------------------------------------------------------------ host side
-static dim3 blk2() { return dim3(kBX, kBY, 1); }
+static dim3 blk2() { return dim3(kFlat, 1, 1); }
 
 template <class T>
 static int diffusion_launch(const chmy_grid_t* g, const chmy_box_t* box, const chmy_field_t* q,
@@ -589,7 +593,7 @@ static int diffusion_launch(const chmy_grid_t* g, const chmy_box_t* box, const c
     DFL<T> c = lview<T>(*Cf);
     DFL<T> q0 = lview<T>(q[0]);
     DFL<T> q1 = g->nd > 1 ? lview<T>(q[1]) : q0, q2 = g->nd > 2 ? lview<T>(q[2]) : q0;
-    dim3 grd = grid_for(b, blk2());
+    dim3 grd = flat_grid(b);
     if (flux)
         hipLaunchKernelGGL(diffusion_flux_kernel<T>, grd, blk2(), 0, s, b, c, q0, q1, q2, g->nd, -T(scalar),
                            T(g->inv_spacing[0]), T(g->inv_spacing[1]), T(g->inv_spacing[2]));
@@ -681,7 +685,7 @@ static int copy_launch(const chmy_grid_t* g, const chmy_box_t& bx, const chmy_fi
     for (int q = 0; q < nt; ++q) { c.src[c.n] = lview<T>(tau[q]); c.dst[c.n] = lview<T>(tauo[q]); ++c.n; }
     Box3 b = box3(bx, g->nd);
     if (no_work(b)) return 0;
-    hipLaunchKernelGGL(copy_kernel<T>, grid_for(b, blk2()), blk2(), 0, s, b, c);
+    hipLaunchKernelGGL(copy_kernel<T>, flat_grid(b), blk2(), 0, s, b, c);
     CHMY_HIP(hipGetLastError());
     return 0;
 }
@@ -694,7 +698,7 @@ static int thermal_launch(const chmy_grid_t* g, const chmy_box_t& bx, const chmy
     DFL<T> t = lview<T>(*Tf), o = lview<T>(other[0]);
     DFL<T> q0 = lview<T>(q[0]);
     DFL<T> q1 = g->nd > 1 ? lview<T>(q[1]) : q0, q2 = g->nd > 2 ? lview<T>(q[2]) : q0;
-    dim3 grd = grid_for(b, blk2());
+    dim3 grd = flat_grid(b);
     if (flux) {
         DFL<T> v1 = g->nd > 1 ? lview<T>(other[1]) : o, v2 = g->nd > 2 ? lview<T>(other[2]) : o;
         hipLaunchKernelGGL(thermal_flux_kernel<T>, grd, blk2(), 0, s, b, t, o, v1, v2, q0, q1, q2, g->nd, -T(scalar),
@@ -747,7 +751,7 @@ int chmy_diffusion_step(const chmy_grid_t* g, const chmy_box_t* box, const chmy_
         DFL<T> c = lview<T>(*C), co = lview<T>(*C_out);
         DFL<T> q0 = lview<T>(q[0]);
         DFL<T> q1 = g->nd > 1 ? lview<T>(q[1]) : q0, q2 = g->nd > 2 ? lview<T>(q[2]) : q0;
-        dim3 grd = grid_for(b, blk2());
+        dim3 grd = flat_grid(b);
         hipLaunchKernelGGL(diffusion_step_kernel<T>, grd, blk2(), 0, (hipStream_t)stream, b, c, co, q0, q1, q2,
                            g->nd, -T(chi), T(dt), T(g->inv_spacing[0]), T(g->inv_spacing[1]),
                            T(g->inv_spacing[2]));
@@ -808,7 +812,7 @@ int chmy_diffusion_iterate(const chmy_grid_t* g, const chmy_field_t* C0, const c
             DFL<T> q1 = g->nd > 1 ? lview<T>(q[1]) : q0, q2 = g->nd > 2 ? lview<T>(q[2]) : q0;
             int it = 0;
             CHMY_TRY(diffusion_passes<T>(g, C0, C1, rules, chi, dt, niter, &p, &it, (hipStream_t)stream));
-            const dim3 grd = grid_for(reg, blk2());
+            const dim3 grd = flat_grid(reg);
             for (; it < niter; ++it) {
                 hipLaunchKernelGGL(diffusion_step_bc_kernel<T>, grd, blk2(), 0, (hipStream_t)stream, b, reg, c[p],
                                    c[1 - p], q0, q1, q2, g->nd, -T(chi), T(dt), T(g->inv_spacing[0]),
@@ -915,7 +919,7 @@ int chmy_thermal_step(const chmy_grid_t* g, const chmy_box_t* box, const chmy_fi
             CHMY_HIP(hipGetLastError());
             return 0;
         }
-        dim3 grd = grid_for(b, blk2());
+        dim3 grd = flat_grid(b);
         hipLaunchKernelGGL(thermal_step_kernel<T>, grd, blk2(), 0, (hipStream_t)stream, b, t, to, o, v0, v1, v2, q0,
                            q1, q2, g->nd, -T(lam), T(dt), T(g->inv_spacing[0]), T(g->inv_spacing[1]),
                            T(g->inv_spacing[2]));
@@ -985,10 +989,10 @@ int chmy_maxloc(const chmy_grid_t* g, const chmy_box_t* box, const chmy_field_t*
     if (no_work(b)) return 0;
     hipStream_t s = (hipStream_t)stream;
     if (src->dtype == CHMY_F64)
-        hipLaunchKernelGGL(maxloc_kernel<double>, grid_for(b, blk2()), blk2(), 0, s, b, lview<double>(*dst),
+        hipLaunchKernelGGL(maxloc_kernel<double>, flat_grid(b), blk2(), 0, s, b, lview<double>(*dst),
                            lview<double>(*src), g->nd);
     else
-        hipLaunchKernelGGL(maxloc_kernel<float>, grid_for(b, blk2()), blk2(), 0, s, b, lview<float>(*dst),
+        hipLaunchKernelGGL(maxloc_kernel<float>, flat_grid(b), blk2(), 0, s, b, lview<float>(*dst),
                            lview<float>(*src), g->nd);
     CHMY_HIP(hipGetLastError());
     return 0;

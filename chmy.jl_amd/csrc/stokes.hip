@@ -3,11 +3,14 @@
 // examples/stokes_2d_inc_ve_T.jl:20-43) as per-point Launcher kernels.
 // Expressions keep the reference's association order; the library is built
 // with -ffp-contract=off so f64 results equal the CPU semantics bit for bit.
+// Both are bound by HBM (24 and 17 arrays a launch in 3D).  159x143x127 FP64,
+// 64 x 4 blocks with loads between stores -> flat blocks, each XCD a contiguous
+// run, every load before the first store, and divV and r_V (never read again
+// by the iteration) past the caches: stress 124 -> 109 us (5.1 TB/s), velocity
+// 100 -> 84 us (4.7 TB/s).
 #include "common.hpp"
 
 namespace chmy {
-
-constexpr int kSX = 64, kSY = 4;
 
 template <class T>
 struct StressArgs {
@@ -49,23 +52,30 @@ __device__ __forceinline__ T tau_new_off(T t, T to, T e, T eta, T eve, T Gdt, T 
 
 template <class T, int ND, bool FVISC>
 __global__ void __launch_bounds__(256) stress_kernel(Box3 b, StressArgs<T> a) {
-    const int64_t i = b.lo[0] + blockIdx.x * (int64_t)kSX + threadIdx.x;
-    const int64_t j = b.lo[1] + blockIdx.y * (int64_t)kSY + threadIdx.y;
-    const int64_t k = b.lo[2] + blockIdx.z;
-    if (i >= b.lo[0] + b.len[0] || j >= b.lo[1] + b.len[1]) return;
+    int64_t i, j, k;
+    if (!flat_point(b, i, j, k)) return;
     // every field shares the padded geometry along y/z except the staggered dim,
     // so offsets are computed per field
     auto O = [&](const DF<T>& f) { return i + j * f.sy + k * f.sz; };
     const DF<T>& Vx = a.V[0];
     const DF<T>& Vy = a.V[1];
     const int64_t ox = O(Vx), oy = O(Vy);
+    // every load before the first store (a store may alias, so none would be
+    // moved past one): a point's 26 loads in 3D are in flight together
+    constexpr int NT = ND == 2 ? 3 : 6;
+    const int64_t oc = O(a.Pr);
+    const T Pr0 = a.Pr.at(oc);
+    T t[NT], to[NT];
+#pragma unroll
+    for (int c = 0; c < NT; ++c) {
+        t[c] = a.tau[c].at(O(a.tau[c]));
+        to[c] = a.tauo[c].at(O(a.tauo[c]));
+    }
     if constexpr (ND == 2) {
         T exx = (Vx.at(ox + 1) - Vx.at(ox)) * a.ix;
         T eyy = (Vy.at(oy + Vy.sy) - Vy.at(oy)) * a.iy;
         T exy = T(0.5) * ((Vx.at(ox) - Vx.at(ox - Vx.sy)) * a.iy + (Vy.at(oy) - Vy.at(oy - 1)) * a.ix);
         T dv = exx + eyy;
-        const int64_t oc = O(a.Pr);
-        a.dV.at(O(a.dV)) = dv;
         T eta_c = a.eta_s, eve_c = a.eve_s, eta_e = a.eta_s, eve_e = a.eve_s;
         if constexpr (FVISC) {
             eta_c = a.eta.at(O(a.eta));
@@ -73,11 +83,11 @@ __global__ void __launch_bounds__(256) stress_kernel(Box3 b, StressArgs<T> a) {
             eta_e = lerp_cc_vv(a.eta, O(a.eta), 1, a.eta.sy);
             eve_e = visc_ve(eta_e, a.Gs, a.dts);
         }
-        a.Pr.at(oc) = a.Pr.at(oc) - (dv * eve_c) * a.dPr;
-        const int64_t o0 = O(a.tau[0]), o1 = O(a.tau[1]), o2 = O(a.tau[2]);
-        a.tau[0].at(o0) = tau_new_diag(a.tau[0].at(o0), a.tauo[0].at(O(a.tauo[0])), exx, dv, eta_c, eve_c, a.Gdt, a.dr);
-        a.tau[1].at(o1) = tau_new_diag(a.tau[1].at(o1), a.tauo[1].at(O(a.tauo[1])), eyy, dv, eta_c, eve_c, a.Gdt, a.dr);
-        a.tau[2].at(o2) = tau_new_off(a.tau[2].at(o2), a.tauo[2].at(O(a.tauo[2])), exy, eta_e, eve_e, a.Gdt, a.dr);
+        __builtin_nontemporal_store(dv, &a.dV.at(O(a.dV)));
+        a.Pr.at(oc) = Pr0 - (dv * eve_c) * a.dPr;
+        a.tau[0].at(O(a.tau[0])) = tau_new_diag(t[0], to[0], exx, dv, eta_c, eve_c, a.Gdt, a.dr);
+        a.tau[1].at(O(a.tau[1])) = tau_new_diag(t[1], to[1], eyy, dv, eta_c, eve_c, a.Gdt, a.dr);
+        a.tau[2].at(O(a.tau[2])) = tau_new_off(t[2], to[2], exy, eta_e, eve_e, a.Gdt, a.dr);
     } else {
         const DF<T>& Vz = a.V[2];
         const int64_t oz = O(Vz);
@@ -88,8 +98,6 @@ __global__ void __launch_bounds__(256) stress_kernel(Box3 b, StressArgs<T> a) {
         T exz = T(0.5) * ((Vx.at(ox) - Vx.at(ox - Vx.sz)) * a.iz + (Vz.at(oz) - Vz.at(oz - 1)) * a.ix);
         T eyz = T(0.5) * ((Vy.at(oy) - Vy.at(oy - Vy.sz)) * a.iz + (Vz.at(oz) - Vz.at(oz - Vz.sy)) * a.iy);
         T dv = (exx + eyy) + ezz;
-        const int64_t oc = O(a.Pr);
-        a.dV.at(O(a.dV)) = dv;
         T eta_c = a.eta_s, eve_c = a.eve_s;
         T exy_eta = a.eta_s, exz_eta = a.eta_s, eyz_eta = a.eta_s;
         T exy_eve = a.eve_s, exz_eve = a.eve_s, eyz_eve = a.eve_s;
@@ -104,20 +112,15 @@ __global__ void __launch_bounds__(256) stress_kernel(Box3 b, StressArgs<T> a) {
             exz_eve = visc_ve(exz_eta, a.Gs, a.dts);
             eyz_eve = visc_ve(eyz_eta, a.Gs, a.dts);
         }
-        a.Pr.at(oc) = a.Pr.at(oc) - (dv * eve_c) * a.dPr;
         const T e[6] = {exx, eyy, ezz, exy, exz, eyz};
         const T et[6] = {eta_c, eta_c, eta_c, exy_eta, exz_eta, eyz_eta};
         const T ev[6] = {eve_c, eve_c, eve_c, exy_eve, exz_eve, eyz_eve};
+        __builtin_nontemporal_store(dv, &a.dV.at(O(a.dV)));
+        a.Pr.at(oc) = Pr0 - (dv * eve_c) * a.dPr;
 #pragma unroll
-        for (int c = 0; c < 3; ++c) {
-            const int64_t o = O(a.tau[c]);
-            a.tau[c].at(o) = tau_new_diag(a.tau[c].at(o), a.tauo[c].at(O(a.tauo[c])), e[c], dv, et[c], ev[c], a.Gdt, a.dr);
-        }
-#pragma unroll
-        for (int c = 3; c < 6; ++c) {
-            const int64_t o = O(a.tau[c]);
-            a.tau[c].at(o) = tau_new_off(a.tau[c].at(o), a.tauo[c].at(O(a.tauo[c])), e[c], et[c], ev[c], a.Gdt, a.dr);
-        }
+        for (int c = 0; c < 6; ++c)
+            a.tau[c].at(O(a.tau[c])) = c < 3 ? tau_new_diag(t[c], to[c], e[c], dv, et[c], ev[c], a.Gdt, a.dr)
+                                             : tau_new_off(t[c], to[c], e[c], et[c], ev[c], a.Gdt, a.dr);
     }
 }
 
@@ -129,10 +132,8 @@ __device__ __forceinline__ T vel_eve(const VelArgs<T>& a, int64_t o, int64_t s) 
 
 template <class T, int ND, bool FVISC>
 __global__ void __launch_bounds__(256) velocity_kernel(Box3 b, VelArgs<T> a) {
-    const int64_t i = b.lo[0] + blockIdx.x * (int64_t)kSX + threadIdx.x;
-    const int64_t j = b.lo[1] + blockIdx.y * (int64_t)kSY + threadIdx.y;
-    const int64_t k = b.lo[2] + blockIdx.z;
-    if (i >= b.lo[0] + b.len[0] || j >= b.lo[1] + b.len[1]) return;
+    int64_t i, j, k;
+    if (!flat_point(b, i, j, k)) return;
     auto O = [&](const DF<T>& f) { return i + j * f.sy + k * f.sz; };
     const int64_t op = O(a.Pr);
     const T P = a.Pr.at(op);
@@ -146,10 +147,12 @@ __global__ void __launch_bounds__(256) velocity_kernel(Box3 b, VelArgs<T> a) {
                (txy.at(o2 + 1) - txy.at(o2)) * a.ix;
         if (a.has_rg) ry = ry - a.rg.at(O(a.rg));
         const int64_t vx = O(a.V[0]), vy = O(a.V[1]);
-        a.rV[0].at(O(a.rV[0])) = rx;
-        a.rV[1].at(O(a.rV[1])) = ry;
-        a.V[0].at(vx) = a.V[0].at(vx) + (rx * a.nu) / vel_eve<T, FVISC>(a, oe, 1);
-        a.V[1].at(vy) = a.V[1].at(vy) + (ry * a.nu) / vel_eve<T, FVISC>(a, oe, a.eml.sy);
+        const T vxn = a.V[0].at(vx) + (rx * a.nu) / vel_eve<T, FVISC>(a, oe, 1);
+        const T vyn = a.V[1].at(vy) + (ry * a.nu) / vel_eve<T, FVISC>(a, oe, a.eml.sy);
+        __builtin_nontemporal_store(rx, &a.rV[0].at(O(a.rV[0])));
+        __builtin_nontemporal_store(ry, &a.rV[1].at(O(a.rV[1])));
+        a.V[0].at(vx) = vxn;
+        a.V[1].at(vy) = vyn;
     } else {
         const DF<T>&txx = a.tau[0], &tyy = a.tau[1], &tzz = a.tau[2];
         const DF<T>&txy = a.tau[3], &txz = a.tau[4], &tyz = a.tau[5];
@@ -165,12 +168,15 @@ __global__ void __launch_bounds__(256) velocity_kernel(Box3 b, VelArgs<T> a) {
                (tyz.at(o5 + tyz.sy) - tyz.at(o5)) * a.iy;
         if (a.has_rg) rz = rz - a.rg.at(O(a.rg));
         const int64_t vx = O(a.V[0]), vy = O(a.V[1]), vz = O(a.V[2]);
-        a.rV[0].at(O(a.rV[0])) = rx;
-        a.rV[1].at(O(a.rV[1])) = ry;
-        a.rV[2].at(O(a.rV[2])) = rz;
-        a.V[0].at(vx) = a.V[0].at(vx) + (rx * a.nu) / vel_eve<T, FVISC>(a, oe, 1);
-        a.V[1].at(vy) = a.V[1].at(vy) + (ry * a.nu) / vel_eve<T, FVISC>(a, oe, a.eml.sy);
-        a.V[2].at(vz) = a.V[2].at(vz) + (rz * a.nu) / vel_eve<T, FVISC>(a, oe, a.eml.sz);
+        const T vxn = a.V[0].at(vx) + (rx * a.nu) / vel_eve<T, FVISC>(a, oe, 1);
+        const T vyn = a.V[1].at(vy) + (ry * a.nu) / vel_eve<T, FVISC>(a, oe, a.eml.sy);
+        const T vzn = a.V[2].at(vz) + (rz * a.nu) / vel_eve<T, FVISC>(a, oe, a.eml.sz);
+        __builtin_nontemporal_store(rx, &a.rV[0].at(O(a.rV[0])));
+        __builtin_nontemporal_store(ry, &a.rV[1].at(O(a.rV[1])));
+        __builtin_nontemporal_store(rz, &a.rV[2].at(O(a.rV[2])));
+        a.V[0].at(vx) = vxn;
+        a.V[1].at(vy) = vyn;
+        a.V[2].at(vz) = vzn;
     }
 }
 
@@ -199,8 +205,7 @@ static int stress_launch(const chmy_grid_t* g, const chmy_box_t& bx, const chmy_
     a.dr = T(dr);
     Box3 b = box3(bx, nd);
     if (no_work(b)) return 0;
-    dim3 blk(kSX, kSY, 1), grd((unsigned)((b.len[0] + kSX - 1) / kSX), (unsigned)((b.len[1] + kSY - 1) / kSY),
-                               (unsigned)b.len[2]);
+    const dim3 blk(kFlat, 1, 1), grd = flat_grid(b);
     if (nd == 2) {
         if (eta) hipLaunchKernelGGL((stress_kernel<T, 2, true>), grd, blk, 0, s, b, a);
         else hipLaunchKernelGGL((stress_kernel<T, 2, false>), grd, blk, 0, s, b, a);
@@ -234,8 +239,7 @@ static int velocity_launch(const chmy_grid_t* g, const chmy_box_t& bx, const chm
     a.nu = T(nu);
     Box3 b = box3(bx, nd);
     if (no_work(b)) return 0;
-    dim3 blk(kSX, kSY, 1), grd((unsigned)((b.len[0] + kSX - 1) / kSX), (unsigned)((b.len[1] + kSY - 1) / kSY),
-                               (unsigned)b.len[2]);
+    const dim3 blk(kFlat, 1, 1), grd = flat_grid(b);
     if (nd == 2) {
         if (eml) hipLaunchKernelGGL((velocity_kernel<T, 2, true>), grd, blk, 0, s, b, a);
         else hipLaunchKernelGGL((velocity_kernel<T, 2, false>), grd, blk, 0, s, b, a);

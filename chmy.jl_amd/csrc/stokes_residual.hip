@@ -11,11 +11,17 @@
 // Because the PT iteration is stationary in (V, tau, Pr), folding d into x and
 // restarting d at 0 continues the same iteration; the f64 residual sets the
 // attainable accuracy.
+// 207x191x175, bf16 forcing, us: residual 478 -> 374 with flat blocks, every
+// load before the first store and eta's form a template parameter (its
+// run-time test cut the loads into groups waited for one by one); 1.08 GB, 219
+// at the copy rate; the rest is about 60 loads a point at 4 waves a SIMD (106
+// VGPRs; held to 5 or 6 waves it takes 392 and 557).  Accumulate 316 -> 294
+// (1.38 GB, 4.7 TB/s).
+#include <type_traits>
+
 #include "common.hpp"
 
 namespace chmy {
-
-constexpr int kRX = 64, kRY = 4;
 
 template <class T, class TO>
 struct ResArgs {
@@ -23,7 +29,7 @@ struct ResArgs {
     DF<TO> toc[6], fV[3], fP;
     DF<T> dV, rV[3];
     T ix, iy, iz, eta_s, eve_s_unused, Gs, dts, Gdt;
-    int has_eta, has_rg, has_norm, has_fe;
+    int has_rg, has_norm, has_fe;
 };
 
 template <class T>
@@ -44,12 +50,10 @@ __device__ __forceinline__ T r_tau_off(T t, T to, T e, T eta, T Gdt) {
     return ((-(t - to)) / Gdt - t / eta) + T(2) * e;
 }
 
-template <class T, class TO, int ND>
+template <class T, class TO, int ND, bool HETA>
 __global__ void __launch_bounds__(256) residual_kernel(Box3 b, ResArgs<T, TO> a) {
-    const int64_t i = b.lo[0] + blockIdx.x * (int64_t)kRX + threadIdx.x;
-    const int64_t j = b.lo[1] + blockIdx.y * (int64_t)kRY + threadIdx.y;
-    const int64_t k = b.lo[2] + blockIdx.z;
-    if (i >= b.lo[0] + b.len[0] || j >= b.lo[1] + b.len[1]) return;
+    int64_t i, j, k;
+    if (!flat_point(b, i, j, k)) return;
     auto O = [i, j, k](const auto& f) { return i + j * f.sy + k * f.sz; };
     const DF<T>& Vx = a.V[0];
     const DF<T>& Vy = a.V[1];
@@ -71,23 +75,22 @@ __global__ void __launch_bounds__(256) residual_kernel(Box3 b, ResArgs<T, TO> a)
         e[5] = T(0.5) * ((Vy.at(oy) - Vy.at(oy - Vy.sz)) * a.iz + (Vz.at(oz) - Vz.at(oz - Vz.sy)) * a.iy);
         dv = (e[0] + e[1]) + e[2];
     }
-    const int nt = ND == 2 ? 3 : 6;
+    constexpr int NT = ND == 2 ? 3 : 6;
     const int64_t oe = O(a.eta);
-    for (int c = 0; c < nt; ++c) {
+    T rt[NT];   // stored below, after the last load
+#pragma unroll
+    for (int c = 0; c < NT; ++c) {
         T eta = a.eta_s;
         const bool diag = c < ND;
-        if (a.has_eta) {
+        if constexpr (HETA) {
             if (diag) eta = a.eta.at(oe);
-            else if (ND == 2) eta = lerp_e(a.eta, oe, 1, a.eta.sy);
-            else if (c == 3) eta = lerp_e(a.eta, oe, 1, a.eta.sy);
+            else if (ND == 2 || c == 3) eta = lerp_e(a.eta, oe, 1, a.eta.sy);
             else if (c == 4) eta = lerp_e(a.eta, oe, 1, a.eta.sz);
             else eta = lerp_e(a.eta, oe, a.eta.sy, a.eta.sz);
         }
         const T t = a.tau[c].at(O(a.tau[c])), to = a.told[c].at(O(a.told[c]));
-        const T r = diag ? r_tau_diag(t, to, e[c], dv, eta, a.Gdt) : r_tau_off(t, to, e[c], eta, a.Gdt);
-        put(a.toc[c].at(O(a.toc[c])), a.Gdt * r);
+        rt[c] = diag ? r_tau_diag(t, to, e[c], dv, eta, a.Gdt) : r_tau_off(t, to, e[c], eta, a.Gdt);
     }
-    put(a.fP.at(O(a.fP)), -dv);
     // R_V (update_velocity!'s r_V, stokes_3d_inc_ve_T.jl:51-53 / 2D stokes_2d_inc_ve_T.jl:39-40)
     const T P = a.Pr.at(oc);
     T r[3];
@@ -113,6 +116,10 @@ __global__ void __launch_bounds__(256) residual_kernel(Box3 b, ResArgs<T, TO> a)
     }
     if (a.has_fe)
         for (int d = 0; d < ND; ++d) r[d] = r[d] + a.fe[d].at(O(a.fe[d]));
+#pragma unroll
+    for (int c = 0; c < NT; ++c) put(a.toc[c].at(O(a.toc[c])), a.Gdt * rt[c]);
+    put(a.fP.at(O(a.fP)), -dv);
+#pragma unroll
     for (int d = 0; d < ND; ++d) {
         put(a.fV[d].at(O(a.fV[d])), r[d]);
         if (a.has_norm) a.rV[d].at(O(a.rV[d])) = r[d];
@@ -120,24 +127,22 @@ __global__ void __launch_bounds__(256) residual_kernel(Box3 b, ResArgs<T, TO> a)
     if (a.has_norm) a.dV.at(O(a.dV)) = dv;
 }
 
-template <class T, class TO>
+template <class T, class TO, int N>
 struct AccArgs {
-    DF<T> x[10];
-    DF<TO> d[10];
-    int n;
+    DF<T> x[N];
+    DF<TO> d[N];
 };
 
-template <class T, class TO>
-__global__ void __launch_bounds__(256) accumulate_kernel(Box3 b, AccArgs<T, TO> a) {
-    const int64_t i = b.lo[0] + blockIdx.x * (int64_t)kRX + threadIdx.x;
-    const int64_t j = b.lo[1] + blockIdx.y * (int64_t)kRY + threadIdx.y;
-    const int64_t k = b.lo[2] + blockIdx.z;
-    if (i >= b.lo[0] + b.len[0] || j >= b.lo[1] + b.len[1]) return;
-    for (int q = 0; q < a.n; ++q) {
-        const int64_t ox = i + j * a.x[q].sy + k * a.x[q].sz;
-        const int64_t od = i + j * a.d[q].sy + k * a.d[q].sz;
-        a.x[q].at(ox) = a.x[q].at(ox) + T(a.d[q].at(od));
-    }
+template <class T, class TO, int N>
+__global__ void __launch_bounds__(256) accumulate_kernel(Box3 b, AccArgs<T, TO, N> a) {
+    int64_t i, j, k;
+    if (!flat_point(b, i, j, k)) return;
+    T v[N];   // every load before the first store
+#pragma unroll
+    for (int q = 0; q < N; ++q)
+        v[q] = a.x[q].at(i + j * a.x[q].sy + k * a.x[q].sz) + T(a.d[q].at(i + j * a.d[q].sy + k * a.d[q].sz));
+#pragma unroll
+    for (int q = 0; q < N; ++q) a.x[q].at(i + j * a.x[q].sy + k * a.x[q].sz) = v[q];
 }
 
 template <class T, class TO>
@@ -166,7 +171,6 @@ static int residual_launch(const chmy_grid_t* g, const chmy_box_t& bx, const chm
     a.rg = rg ? view<T>(*rg) : a.Pr;
     a.fP = view<TO>(*fP);
     a.dV = dV ? view<T>(*dV) : a.Pr;
-    a.has_eta = eta != nullptr;
     a.has_rg = rg != nullptr;
     a.has_norm = dV != nullptr;
     a.ix = T(g->inv_spacing[0]);
@@ -178,10 +182,11 @@ static int residual_launch(const chmy_grid_t* g, const chmy_box_t& bx, const chm
     a.Gdt = T(G) * T(dt);
     Box3 b = box3(bx, nd);
     if (no_work(b)) return 0;
-    dim3 blk(kRX, kRY, 1), grd((unsigned)((b.len[0] + kRX - 1) / kRX), (unsigned)((b.len[1] + kRY - 1) / kRY),
-                               (unsigned)b.len[2]);
-    if (nd == 2) hipLaunchKernelGGL((residual_kernel<T, TO, 2>), grd, blk, 0, s, b, a);
-    else hipLaunchKernelGGL((residual_kernel<T, TO, 3>), grd, blk, 0, s, b, a);
+    const dim3 blk(kFlat, 1, 1), grd = flat_grid(b);
+    if (nd == 2 && eta) hipLaunchKernelGGL((residual_kernel<T, TO, 2, true>), grd, blk, 0, s, b, a);
+    else if (nd == 2) hipLaunchKernelGGL((residual_kernel<T, TO, 2, false>), grd, blk, 0, s, b, a);
+    else if (eta) hipLaunchKernelGGL((residual_kernel<T, TO, 3, true>), grd, blk, 0, s, b, a);
+    else hipLaunchKernelGGL((residual_kernel<T, TO, 3, false>), grd, blk, 0, s, b, a);
     CHMY_HIP(hipGetLastError());
     return 0;
 }
@@ -190,20 +195,19 @@ template <class T, class TO>
 static int accumulate_launch(const chmy_grid_t* g, const chmy_box_t& bx, const chmy_field_t* V,
                              const chmy_field_t* tau, const chmy_field_t* Pr, const chmy_field_t* Vc,
                              const chmy_field_t* tauc, const chmy_field_t* Prc, hipStream_t s) {
-    AccArgs<T, TO> a;
-    std::memset(&a, 0, sizeof a);
-    const int nd = g->nd, nt = nd == 2 ? 3 : 6;
-    a.n = 0;
-    for (int d = 0; d < nd; ++d) { a.x[a.n] = view<T>(V[d]); a.d[a.n] = view<TO>(Vc[d]); ++a.n; }
-    for (int c = 0; c < nt; ++c) { a.x[a.n] = view<T>(tau[c]); a.d[a.n] = view<TO>(tauc[c]); ++a.n; }
-    a.x[a.n] = view<T>(*Pr);
-    a.d[a.n] = view<TO>(*Prc);
-    ++a.n;
-    Box3 b = box3(bx, nd);
+    const Box3 b = box3(bx, g->nd);
     if (no_work(b)) return 0;
-    dim3 blk(kRX, kRY, 1), grd((unsigned)((b.len[0] + kRX - 1) / kRX), (unsigned)((b.len[1] + kRY - 1) / kRY),
-                               (unsigned)b.len[2]);
-    hipLaunchKernelGGL((accumulate_kernel<T, TO>), grd, blk, 0, s, b, a);
+    auto go = [&](auto nd) {
+        constexpr int ND = decltype(nd)::value, NT = ND == 2 ? 3 : 6;
+        AccArgs<T, TO, ND + NT + 1> a;
+        for (int d = 0; d < ND; ++d) { a.x[d] = view<T>(V[d]); a.d[d] = view<TO>(Vc[d]); }
+        for (int c = 0; c < NT; ++c) { a.x[ND + c] = view<T>(tau[c]); a.d[ND + c] = view<TO>(tauc[c]); }
+        a.x[ND + NT] = view<T>(*Pr);
+        a.d[ND + NT] = view<TO>(*Prc);
+        hipLaunchKernelGGL((accumulate_kernel<T, TO, ND + NT + 1>), flat_grid(b), dim3(kFlat, 1, 1), 0, s, b, a);
+    };
+    if (g->nd == 2) go(std::integral_constant<int, 2>{});
+    else go(std::integral_constant<int, 3>{});
     CHMY_HIP(hipGetLastError());
     return 0;
 }

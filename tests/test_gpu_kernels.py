@@ -831,3 +831,15 @@ def test_bc_sets_of_numbers_at_plane_edges(arch, dims):
             per_side.apply_side(d, s)
     for q, (a, b, spec) in enumerate(pairs):
         assert torch.equal(a.data, b.data), f"field {q} {spec}"
+
+
+@pytest.mark.parametrize("dims", [(62, 3, 5), (254, 1, 3), (255, 2, 9), (1, 300, 2), (510, 7), (1, 1), (700, 3)])
+def test_point_kernels_rows_across_blocks(arch, monkeypatch, dims):
+    """The per-point kernels where a plane's rows end inside, at and one past a
+    block of 256 points, and on the smallest planes."""
+    nd = len(dims)
+    monkeypatch.setitem(globals(), "grids", lambda _: chmy.UniformGrid(arch, origin=(-1.0,) * nd, extent=(2.0,) * nd,
+                                                                       dims=dims))
+    for visc in ("scalar", "field"):
+        test_stress_velocity(arch, np.float64, nd, visc)
+    test_update_old_and_thermal(arch, np.float64, nd)
