@@ -226,19 +226,28 @@ __device__ __forceinline__ void program_run(const PProg& P, int q0, int q1, Slot
     }
 }
 
-// One wave: 64 x points of a row, a chunk of planes of the marched dim, N
-// planes at a time.  Lanes and planes past the box evaluate clamped indices
-// and store nothing.
+// One wave: 64 consecutive points of a plane (of a row where y is marched), a
+// chunk of planes of the marched dim, N planes at a time.  Lanes and planes
+// past the box evaluate its first or last indices and store nothing.  With 64
+// columns of one row a wave instead, 160 points took three waves: us at
+// 160x144x127 FP64 66 -> 53 (42 operations), 46 -> 42 (27), 36 -> 29 (11 with
+// loads); all three and their host side at 140x187x170 FP32 238 -> 187,
+// 191x187x189 FP64 271 -> 256 (160x144x127 waits for the host: 161 both).
 template <class T, int S, int N, bool HEAVY>
-__global__ void __launch_bounds__(64) program_kernel(const PProg P, DF<T> dst, Box3 b, int nbx, int nby, int chunk) {
+__global__ void __launch_bounds__(64) program_kernel(const PProg P, DF<T> dst, Box3 b, int nbx, int chunk) {
     const int t = blockIdx.x;
-    const int bx = t % nbx, by = (t / nbx) % nby, bc = t / (nbx * nby);
+    const int bx = t % nbx, bc = t / nbx;
     const int m = P.m;
-    const int64_t i = b.lo[0] + (int64_t)bx * 64 + threadIdx.x, hi0 = b.lo[0] + b.len[0];
-    const int64_t j = b.lo[1] + by;   // nby == 1 in 2D and 1D, where j is marched or the only one
+    // z marched: 64 consecutive points of a plane, counted along its rows; y
+    // marched: of the row
+    int64_t i, j;
+    plane_index((int64_t)bx * 64 + threadIdx.x, b.len[0], m == 2 ? b.len[1] : 1, i, j);
+    const bool in = j < (m == 2 ? b.len[1] : 1);
+    i = in ? b.lo[0] + i : b.lo[0];
+    j = in ? b.lo[1] + j : b.lo[1];
     const int64_t m0 = b.lo[m] + (int64_t)bc * chunk;
     const int64_t hm = b.lo[m] + b.len[m], m1 = m0 + chunk < hm ? m0 + chunk : hm;
-    const int64_t I[3] = {i < hi0 ? i : hi0 - 1, j, b.lo[2]};
+    const int64_t I[3] = {i, j, b.lo[2]};
     Slots<S> r[N];
     int64_t Im[N];
 #pragma unroll
@@ -251,7 +260,7 @@ __global__ void __launch_bounds__(64) program_kernel(const PProg P, DF<T> dst, B
 #pragma unroll
         for (int u = 0; u < N; ++u) {
             const double v = P.out >= 0 ? r[u].get(P.out) : P.k[-1 - P.out];
-            if (i < hi0 && p + u < m1) put(m == 2 ? dst(i, j, p + u) : dst(i, p + u, 0), v);
+            if (in && p + u < m1) put(m == 2 ? dst(i, j, p + u) : dst(i, p + u, 0), v);
         }
     }
 }
@@ -415,30 +424,30 @@ static int plan_program(const chmy_pop_t* prog, int n, PProg* P, bool* heavy) {
 template <class T>
 static int program_launch(const PProg& P, const chmy_field_t* dst, const Box3& b, int slots, bool heavy,
                           hipStream_t st) {
-    const int64_t nbx = (b.len[0] + 63) / 64, nby = P.m == 2 ? b.len[1] : 1, nm = b.len[P.m];
+    const int64_t nbx = (b.len[0] * (P.m == 2 ? b.len[1] : 1) + 63) / 64, nm = b.len[P.m];
     // planes per wave: fill whole rounds of the waves the chip holds (12 a CU
     // at these kernels' registers); a wave also spends about two planes' time
     // on the per-chunk operations.  160x144x127: 20 planes, one round
     const int64_t room = 12 * (int64_t)cu_count();
     int64_t chunk = 4, best = INT64_MAX;
     for (int64_t c = 4; c <= 64; c += 4) {
-        const int64_t waves = nbx * nby * ((nm + c - 1) / c), cost = (waves + room - 1) / room * (c + 2);
+        const int64_t waves = nbx * ((nm + c - 1) / c), cost = (waves + room - 1) / room * (c + 2);
         if (cost < best) {
             best = cost;
             chunk = c;
         }
     }
-    const int64_t nb = nbx * nby * ((nm + chunk - 1) / chunk);
+    const int64_t nb = nbx * ((nm + chunk - 1) / chunk);
     if (nb > INT32_MAX) return set_error(CHMY_E_SIZE, "point program: box too large");
     const dim3 grd((unsigned)nb), blk(64);
     const DF<T> d = view<T>(*dst);
-    const int ix = (int)nbx, iy = (int)nby, ic = (int)chunk;
+    const int ix = (int)nbx, ic = (int)chunk;
     if (slots > 16)
         hipLaunchKernelGGL((program_kernel<T, 0, 1, true>), grd, blk, (size_t)slots * 64 * sizeof(double), st, P, d, b, ix,
-                           iy, ic);
-    else if (heavy) hipLaunchKernelGGL((program_kernel<T, 16, 1, true>), grd, blk, 0, st, P, d, b, ix, iy, ic);
-    else if (slots > 8) hipLaunchKernelGGL((program_kernel<T, 16, 2, false>), grd, blk, 0, st, P, d, b, ix, iy, ic);
-    else hipLaunchKernelGGL((program_kernel<T, 8, 4, false>), grd, blk, 0, st, P, d, b, ix, iy, ic);
+                           ic);
+    else if (heavy) hipLaunchKernelGGL((program_kernel<T, 16, 1, true>), grd, blk, 0, st, P, d, b, ix, ic);
+    else if (slots > 8) hipLaunchKernelGGL((program_kernel<T, 16, 2, false>), grd, blk, 0, st, P, d, b, ix, ic);
+    else hipLaunchKernelGGL((program_kernel<T, 8, 4, false>), grd, blk, 0, st, P, d, b, ix, ic);
     CHMY_HIP(hipGetLastError());
     return 0;
 }
