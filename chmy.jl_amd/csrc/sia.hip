@@ -308,6 +308,9 @@ struct SiaStep {   // forward steps H -> Ho, H's Neumann batch included
     int wd;        // also store D(H) of the cells into Dout (for a later adjoint step at H)
     DF<T> Dout;
 };
+struct SiaMid {    // two kept steps: the state between them and its D
+    DF<double> H, D;
+};
 
 // Steps a launch may take: their time steps travel in its argument.
 constexpr int kSiaSteps = 8;
@@ -342,6 +345,10 @@ struct SiaRows {
     using Col = SiaCol<NW, R>;
     double h[R + 2], b[R + 2], a[R];   // [r + 1]: row r
     double gx[R], gy[R + 1], u[R], v[R];
+    __device__ __forceinline__ void load_h(const DF<double>& H, const Col& c) {
+#pragma unroll
+        for (int r = -1; r <= R; ++r) h[r + 1] = c.ld(H, r);
+    }
     __device__ __forceinline__ void load(const SiaF<double>& s, const Col& c) {
 #pragma unroll
         for (int r = -1; r <= R; ++r) {
@@ -419,11 +426,39 @@ __device__ __forceinline__ void sia_face_d(const double* D, double lo, double hi
     }
 }
 
+// A state's owned cells and their Neumann(0) ghosts, dims y then x
+// (batch.jl:20-29): ghosts copy the adjacent cell, corners the diagonal cell.
+template <int NW, int R>
+__device__ __forceinline__ void sia_store(const SiaCol<NW, R>& c, const DF<double>& f, const double* h) {
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+        if (!c.own(r)) continue;
+        double* row = &c.at(f, r);
+        row[0] = h[r];
+        const bool x0 = c.i == 1, x1 = c.i == c.nx;
+        if (x0) row[-1] = h[r];
+        if (x1) row[1] = h[r];
+        if (c.j(r) == 1) {
+            double* g = row - f.sy;
+            g[0] = h[r];
+            if (x0) g[-1] = h[r];
+            if (x1) g[1] = h[r];
+        }
+        if (c.j(r) == c.ny) {
+            double* g = row + f.sy;
+            g[0] = h[r];
+            if (x0) g[-1] = h[r];
+            if (x1) g[1] = h[r];
+        }
+    }
+}
+
 // n forward steps on the region (a ring of 2 n); the owned cells' final H and
-// its ghosts are stored.  With MAXD (a ring of 2 n + 1) the magnitude bits of
+// its ghosts are stored; with KEEP (n at most 2) every state is.  With MAXD (a ring of 2 n + 1) the magnitude bits of
 // the new state's largest owned D come back.
-template <int NW, int R, bool MAXD>
-__device__ __forceinline__ unsigned long long sia_step_cols(const SiaStep<double>& p, const SiaCol<NW, R>& c,
+template <int NW, int R, bool MAXD, bool KEEP = false>
+__device__ __forceinline__ unsigned long long sia_step_cols(const SiaStep<double>& p, const SiaMid& mid,
+                                                            const SiaCol<NW, R>& c,
                                                             const double* dts, int n, double (*ldsH)[NW][64],
                                                             double (*ldsD)[NW][64]) {
     using Col = SiaCol<NW, R>;
@@ -432,15 +467,19 @@ __device__ __forceinline__ unsigned long long sia_step_cols(const SiaStep<double
     typename Col::Edge& eD = *reinterpret_cast<typename Col::Edge*>(ldsD);
     SiaRows<NW, R> k;
     k.load(s, c);
-#pragma unroll 1
-    for (int q = 0; q < n; ++q) {
+    // (two kept steps are written out, so that no view is chosen at run time:
+    // that puts the kernel's arguments in scratch)
+    auto one = [&](int q, auto second) {
         if (q > 0) k.refresh(c, eH);
         k.gradients(s);
         double D[R];
 #pragma unroll
         for (int r = 0; r < R; ++r) {
             D[r] = c.inside(r) ? k.D(s, r) : 0.0;
-            if (p.wd && c.own(r)) c.at(p.Dout, r) = D[r];
+            if (p.wd && c.own(r)) {
+                if constexpr (decltype(second)::value) c.at(mid.D, r) = D[r];
+                else c.at(p.Dout, r) = D[r];
+            }
         }
         c.put(eD, D);
         __syncthreads();
@@ -450,31 +489,20 @@ __device__ __forceinline__ unsigned long long sia_step_cols(const SiaStep<double
         k.update(s, c, fx, fy, dts[q], x);
 #pragma unroll
         for (int r = 0; r < R; ++r) k.h[r + 1] = c.inside(r) ? jmax0(x[r]) : k.h[r + 1];
-    }
-#pragma unroll
-    for (int r = 0; r < R; ++r) {
-        if (!c.own(r)) continue;
-        const double h = k.h[r + 1];
-        double* row = &c.at(p.Ho, r);
-        row[0] = h;
-        // Neumann(0) batch, dims y then x (batch.jl:20-29): ghosts copy the
-        // adjacent cell, corners the diagonal cell
-        const bool x0 = c.i == 1, x1 = c.i == c.nx;
-        if (x0) row[-1] = h;
-        if (x1) row[1] = h;
-        if (c.j(r) == 1) {
-            double* g = row - p.Ho.sy;
-            g[0] = h;
-            if (x0) g[-1] = h;
-            if (x1) g[1] = h;
+    };
+    if constexpr (MAXD) {
+        one(0, std::false_type{});
+    } else if constexpr (KEEP) {
+        one(0, std::false_type{});
+        if (n > 1) {
+            sia_store(c, mid.H, k.h + 1);
+            one(1, std::true_type{});
         }
-        if (c.j(r) == c.ny) {
-            double* g = row + p.Ho.sy;
-            g[0] = h;
-            if (x0) g[-1] = h;
-            if (x1) g[1] = h;
-        }
+    } else {
+#pragma unroll 1
+        for (int q = 0; q < n; ++q) one(q, std::false_type{});
     }
+    sia_store(c, p.Ho, k.h + 1);
     unsigned long long m = 0;
     if constexpr (MAXD) {
         k.refresh(c, eH);
@@ -489,130 +517,149 @@ __device__ __forceinline__ unsigned long long sia_step_cols(const SiaStep<double
 }
 
 template <class T>
-struct SiaAdj {    // one adjoint step at state s.H: lam -> lo, gA += dJ/dlog A
+struct SiaAdj {    // one adjoint step at state s.H, or two (then at H2): lam -> lo, gA += dJ/dlog A
     SiaF<T> s;
     DF<T> lam, lo, gA;
     T dt;
     int rd;        // D(s.H) read from Din (stored by the forward step at s.H) instead of evaluated
     DF<T> Din;
+    int n;         // steps
+    DF<T> H2, D2;  // the second step's state and its D (always stored)
+    T dt2;
 };
 
 // lam' reaches D of the cells 3 away, and an evaluated D the surface of the
 // cell beside that one: the rows -1 and R a wave holds cover it in y, one
 // more lane in x.
 constexpr int kAdjRing = 3;
-__host__ __device__ constexpr int sia_adj_ring(int rd) { return rd ? kAdjRing : kAdjRing + 1; }
+__host__ __device__ constexpr int sia_adj_ring(int rd, int n) { return kAdjRing * n + (rd ? 0 : 1); }
 
-template <int NW, int R>
+// Between two steps lam stays in registers, exact 3 cells further in (a ring
+// of 6 for both); B, A and the gradient's sum are read and written once.
+template <int NW, int R, bool TWO>
 __device__ __forceinline__ void sia_adj_cols(const SiaAdj<double>& p, const SiaCol<NW, R>& c, double (*lds0)[NW][64],
                                              double (*lds1)[NW][64]) {
     using Col = SiaCol<NW, R>;
-    const SiaF<double>& s = p.s;
     typename Col::Edge& e0 = *reinterpret_cast<typename Col::Edge*>(lds0);
     typename Col::Edge& e1 = *reinterpret_cast<typename Col::Edge*>(lds1);
-    const double dt = p.dt;
+    const SiaF<double>& s = p.s;
     const int nx = c.nx, ny = c.ny;
     SiaRows<NW, R> k;
     k.load(s, c);
-    double lam[R], D[R], Dlo, Dhi, fx[R], fy[R + 1];
+    double lam[R], gA[R];
 #pragma unroll
-    for (int r = 0; r < R; ++r) lam[r] = c.ld(p.lam, r);
-    double gA[R];
+    for (int r = 0; r < R; ++r) {
+        lam[r] = c.ld(p.lam, r);
+        gA[r] = s.hasA ? c.ld(p.gA, r) : 0.0;
+    }
+    auto one = [&](const DF<double>& Din, double dt, bool rd) {
+        double D[R], Dlo, Dhi, fx[R], fy[R + 1];
+        if (rd) {   // D of the wave's rows and the two beside them, stored by the forward step at this state
+            const double lo = c.ld(Din, -1), hi = c.ld(Din, R);
 #pragma unroll
-    for (int r = 0; r < R; ++r) gA[r] = s.hasA ? c.ld(p.gA, r) : 0.0;
-    if (p.rd) {   // D of the wave's rows and the two beside them, stored by the forward step at this state
-        const double lo = c.ld(p.Din, -1), hi = c.ld(p.Din, R);
+            for (int r = 0; r < R; ++r) {
+                const double d = c.ld(Din, r);
+                D[r] = c.inside(r) ? d : 0.0;
+            }
+            Dlo = c.inside(-1) ? lo : 0.0;
+            Dhi = c.inside(R) ? hi : 0.0;
+            k.gradients(s);
+        } else {
+            k.gradients(s);
+#pragma unroll
+            for (int r = 0; r < R; ++r) D[r] = c.inside(r) ? k.D(s, r) : 0.0;
+            c.put(e1, D);
+            __syncthreads();
+            c.get(e1, D, Dlo, Dhi);
+        }
+        sia_face_d<NW, R>(D, Dlo, Dhi, fx, fy);
+        // A1: mu
+        double mu[R], mlo, mhi;
+        {
+            double x[R];
+            k.update(s, c, fx, fy, dt, x);
+#pragma unroll
+            for (int r = 0; r < R; ++r) mu[r] = c.inside(r) && x[r] > 0.0 ? lam[r] : 0.0;
+        }
+        c.put(e0, mu);
+        __syncthreads();
+        c.get(e0, mu, mlo, mhi);
+        // A2 + A3: qbar on the faces, Dbar, abar; HD and the log A gradient
+        const bool fxin = c.i >= 2 && c.i <= nx;
+        double qbx[R], qby[R + 1], Dvy[R + 1], abx[R], aby[R], HD[R];
+#pragma unroll
+        for (int r = 0; r <= R; ++r) {
+            qby[r] = dt * s.iy * ((r < R ? mu[r] : mhi) - (r > 0 ? mu[r - 1] : mlo));
+            Dvy[r] = c.j(r) < 2 || c.j(r) > ny ? 0.0 : -k.gy[r] * qby[r];
+        }
+        const int n = s.n;
 #pragma unroll
         for (int r = 0; r < R; ++r) {
-            const double d = c.ld(p.Din, r);
-            D[r] = c.inside(r) ? d : 0.0;
+            qbx[r] = dt * s.ix * (mu[r] - xm1(mu[r]));
+            const double Dvx = fxin ? -k.gx[r] * qbx[r] : 0.0;
+            const double Db = 0.5 * (Dvx + xp1(Dvx)) + 0.5 * (Dvy[r] + Dvy[r + 1]);
+            const double h = k.h[r + 1], av = k.a[r], u = k.u[r], v = k.v[r];
+            const double vm = sqrt(u * u + v * v);
+            const double P = ipow_(vm, n - 1);
+            const double Cc = av * ipow_(h, n + 2) + s.As * ipow_(h, n);
+            if (s.hasA) gA[r] = gA[r] + av * (Db * ipow_(h, n + 2) * P);
+            HD[r] = Db * (double(n + 2) * av * ipow_(h, n + 1) + double(n) * s.As * ipow_(h, n - 1)) * P;
+            double coef = 0.0;
+            if (n >= 3) coef = double(n - 1) * ipow_(vm, n - 3);
+            else if (n == 2 && vm > 0.0) coef = 1.0 / vm;
+            const double Pb = Db * Cc;
+            const bool in = c.inside(r);
+            abx[r] = in ? Pb * coef * u : 0.0;
+            aby[r] = in ? Pb * coef * v : 0.0;
         }
-        Dlo = c.inside(-1) ? lo : 0.0;
-        Dhi = c.inside(R) ? hi : 0.0;
-        k.gradients(s);
-    } else {
-        k.gradients(s);
-#pragma unroll
-        for (int r = 0; r < R; ++r) D[r] = c.inside(r) ? k.D(s, r) : 0.0;
-        c.put(e1, D);
+        double alo, ahi;
+        c.put(e1, aby);
         __syncthreads();
-        c.get(e1, D, Dlo, Dhi);
-    }
-    sia_face_d<NW, R>(D, Dlo, Dhi, fx, fy);
-    // A1: mu
-    double mu[R], mlo, mhi;
-    {
-        double x[R];
-        k.update(s, c, fx, fy, dt, x);
+        c.get(e1, aby, alo, ahi);
+        // A4 + A5: gbar on the faces, then lam'
+        double gby[R + 1];
 #pragma unroll
-        for (int r = 0; r < R; ++r) mu[r] = c.inside(r) && x[r] > 0.0 ? lam[r] : 0.0;
-    }
-    c.put(e0, mu);
-    __syncthreads();
-    c.get(e0, mu, mlo, mhi);
-    // A2 + A3: qbar on the faces, Dbar, abar; HD and the log A gradient
-    const bool fxin = c.i >= 2 && c.i <= nx;
-    double qbx[R], qby[R + 1], Dvy[R + 1], abx[R], aby[R], HD[R];
+        for (int r = 0; r <= R; ++r) {
+            const int f = c.j(r);
+            double g = f >= 2 && f <= ny ? -fy[r] * qby[r] : 0.0;
+            if (f - 1 >= 1) g = g + 0.5 * (r > 0 ? aby[r - 1] : alo);
+            if (f <= ny) g = g + 0.5 * (r < R ? aby[r] : ahi);
+            gby[r] = g;
+        }
 #pragma unroll
-    for (int r = 0; r <= R; ++r) {
-        qby[r] = dt * s.iy * ((r < R ? mu[r] : mhi) - (r > 0 ? mu[r - 1] : mlo));
-        Dvy[r] = c.j(r) < 2 || c.j(r) > ny ? 0.0 : -k.gy[r] * qby[r];
-    }
-    const int n = s.n;
-#pragma unroll
-    for (int r = 0; r < R; ++r) {
-        qbx[r] = dt * s.ix * (mu[r] - xm1(mu[r]));
-        const double Dvx = fxin ? -k.gx[r] * qbx[r] : 0.0;
-        const double Db = 0.5 * (Dvx + xp1(Dvx)) + 0.5 * (Dvy[r] + Dvy[r + 1]);
-        const double h = k.h[r + 1], av = k.a[r], u = k.u[r], v = k.v[r];
-        const double vm = sqrt(u * u + v * v);
-        const double P = ipow_(vm, n - 1);
-        const double Cc = av * ipow_(h, n + 2) + s.As * ipow_(h, n);
-        if (s.hasA && c.own(r)) c.at(p.gA, r) = gA[r] + av * (Db * ipow_(h, n + 2) * P);
-        HD[r] = Db * (double(n + 2) * av * ipow_(h, n + 1) + double(n) * s.As * ipow_(h, n - 1)) * P;
-        double coef = 0.0;
-        if (n >= 3) coef = double(n - 1) * ipow_(vm, n - 3);
-        else if (n == 2 && vm > 0.0) coef = 1.0 / vm;
-        const double Pb = Db * Cc;
-        const bool in = c.inside(r);
-        abx[r] = in ? Pb * coef * u : 0.0;
-        aby[r] = in ? Pb * coef * v : 0.0;
-    }
-    double alo, ahi;
-    c.put(e1, aby);
-    __syncthreads();
-    c.get(e1, aby, alo, ahi);
-    // A4 + A5: gbar on the faces, then lam'
-    double gby[R + 1];
-#pragma unroll
-    for (int r = 0; r <= R; ++r) {
-        const int f = c.j(r);
-        double g = f >= 2 && f <= ny ? -fy[r] * qby[r] : 0.0;
-        if (f - 1 >= 1) g = g + 0.5 * (r > 0 ? aby[r - 1] : alo);
-        if (f <= ny) g = g + 0.5 * (r < R ? aby[r] : ahi);
-        gby[r] = g;
+        for (int r = 0; r < R; ++r) {
+            double gx0 = fxin ? -fx[r] * qbx[r] : 0.0;
+            const double al = xm1(abx[r]);
+            gx0 = c.i - 1 >= 1 ? gx0 + 0.5 * al : gx0;
+            gx0 = c.i <= nx ? gx0 + 0.5 * abx[r] : gx0;
+            const double gx1 = xp1(gx0), gy0 = gby[r], gy1 = gby[r + 1];
+            double t = 0.0;
+            t = t + s.ix * gx0;
+            t = t - s.ix * gx1;
+            t = t + s.iy * gy0;
+            t = t - s.iy * gy1;
+            double l = mu[r] + HD[r] + t;
+            const double m = s.mba * (k.S(r) - s.mbb);
+            if (m < s.mbc) l = l + dt * mu[r] * s.mba;
+            if (c.i == 1) l = l + (-s.ix * gx0);
+            if (c.i == nx) l = l + s.ix * gx1;
+            if (c.j(r) == 1) l = l + (-s.iy * gy0);
+            if (c.j(r) == ny) l = l + s.iy * gy1;
+            lam[r] = l;
+        }
+    };
+    one(p.Din, p.dt, p.rd);
+    if constexpr (TWO) {
+        if (p.n > 1) {
+            k.load_h(p.H2, c);
+            one(p.D2, p.dt2, true);
+        }
     }
 #pragma unroll
     for (int r = 0; r < R; ++r) {
-        double gx0 = fxin ? -fx[r] * qbx[r] : 0.0;
-        const double al = xm1(abx[r]);
-        gx0 = c.i - 1 >= 1 ? gx0 + 0.5 * al : gx0;
-        gx0 = c.i <= nx ? gx0 + 0.5 * abx[r] : gx0;
-        const double gx1 = xp1(gx0), gy0 = gby[r], gy1 = gby[r + 1];
         if (!c.own(r)) continue;
-        double t = 0.0;
-        t = t + s.ix * gx0;
-        t = t - s.ix * gx1;
-        t = t + s.iy * gy0;
-        t = t - s.iy * gy1;
-        double l = mu[r] + HD[r] + t;
-        const double m = s.mba * (k.S(r) - s.mbb);
-        if (m < s.mbc) l = l + dt * mu[r] * s.mba;
-        if (c.i == 1) l = l + (-s.ix * gx0);
-        if (c.i == nx) l = l + s.ix * gx1;
-        if (c.j(r) == 1) l = l + (-s.iy * gy0);
-        if (c.j(r) == ny) l = l + s.iy * gy1;
-        c.at(p.lo, r) = l;
+        c.at(p.lo, r) = lam[r];
+        if (s.hasA) c.at(p.gA, r) = gA[r];
     }
 }
 
@@ -625,7 +672,7 @@ __global__ void __launch_bounds__(NW * 64) sia_steps_kernel(SiaStep<double> f, S
     __shared__ double lds[2][2][NW][64];
     if constexpr (NP > 0) f.s.n = NP;
     const SiaCol<NW, R> c(blockIdx.x % ntx, blockIdx.x / ntx, 2 * d.n, 2 * d.n, nx, ny);
-    sia_step_cols<NW, R, false>(f, c, d.dt, d.n, lds[0], lds[1]);
+    sia_step_cols<NW, R, false>(f, SiaMid{}, c, d.dt, d.n, lds[0], lds[1]);
 }
 
 // The step whose Δt follows from its state's max(D), and the next state's.
@@ -639,7 +686,7 @@ __global__ void __launch_bounds__(NW * 64) sia_rule_kernel(SiaStep<double> f, Si
     if (blockIdx.x == 0 && threadIdx.x == 0 && threadIdx.y == 0) *rule.dt_out = dt;
     constexpr int ring = MAXD ? 3 : 2;
     const SiaCol<NW, R> c(blockIdx.x % ntx, blockIdx.x / ntx, ring, ring, nx, ny);
-    unsigned long long m = sia_step_cols<NW, R, MAXD>(f, c, &dt, 1, lds[0], lds[1]);
+    unsigned long long m = sia_step_cols<NW, R, MAXD>(f, SiaMid{}, c, &dt, 1, lds[0], lds[1]);
     if constexpr (MAXD) {
         for (int o = 32; o > 0; o >>= 1) {
             const unsigned long long q = __shfl_xor(m, o, 64);
@@ -681,10 +728,10 @@ __global__ void __launch_bounds__(256) sia_d_max_kernel(SiaF<T> s, DF<T> D, int6
     }
 }
 
-// Blocks 0 .. na - 1: adjoint regions; the rest: an independent forward step
-// (the recompute of the previous checkpoint segment rides along).
-template <int NP, int NW, int RA, int RF>
-__global__ void __launch_bounds__(NW * 64) sia_adj_kernel(SiaAdj<double> a, SiaStep<double> f, double fdt, int na,
+// Blocks 0 .. na - 1: adjoint regions; the rest: as many independent forward
+// steps (the recompute of the previous checkpoint segment rides along).
+template <int NP, int NW, int RA, int RF, bool TWO>
+__global__ void __launch_bounds__(NW * 64) sia_adj_kernel(SiaAdj<double> a, SiaStep<double> f, SiaMid mid, SiaDts fd, int na,
                                                           int ntxa, int ntxf, int64_t nx, int64_t ny) {
     __shared__ double lds[2][2][NW][64];
     if constexpr (NP > 0) {
@@ -693,11 +740,11 @@ __global__ void __launch_bounds__(NW * 64) sia_adj_kernel(SiaAdj<double> a, SiaS
     }
     const int bid = blockIdx.x;
     if (bid < na) {
-        const SiaCol<NW, RA> c(bid % ntxa, bid / ntxa, sia_adj_ring(a.rd), kAdjRing, nx, ny);
-        sia_adj_cols<NW, RA>(a, c, lds[0], lds[1]);
+        const SiaCol<NW, RA> c(bid % ntxa, bid / ntxa, sia_adj_ring(a.rd, a.n), kAdjRing * a.n, nx, ny);
+        sia_adj_cols<NW, RA, TWO>(a, c, lds[0], lds[1]);
     } else {
-        const SiaCol<NW, RF> c((bid - na) % ntxf, (bid - na) / ntxf, 2, 2, nx, ny);
-        sia_step_cols<NW, RF, false>(f, c, &fdt, 1, lds[0], lds[1]);
+        const SiaCol<NW, RF> c((bid - na) % ntxf, (bid - na) / ntxf, 2 * fd.n, 2 * fd.n, nx, ny);
+        sia_step_cols<NW, RF, false, TWO>(f, mid, c, fd.dt, fd.n, lds[0], lds[1]);
     }
 }
 
@@ -705,11 +752,15 @@ __global__ void __launch_bounds__(NW * 64) sia_adj_kernel(SiaAdj<double> a, SiaS
 // is its serial chain (about 4.5 us a forward step, 5.4 us an adjoint step for
 // one region alone), so forward steps go several to a launch (300 steps of
 // 512^2: 5.1 us each singly, 4.3 in twos, 3.8 in threes, 3.9 in fives on
-// regions of 64 x 64, where the ring's work eats the rest).  Regions of 32 rows while they
-// all fit the CUs at once, else 48 (250x177: 1.14 ms for the gradient of 100
-// steps with 32 rows, 1.20 with 48; 512^2: 4.86 and 4.68 for 300).  The
-// adjoint's regions are 16 rows with 24 for the steps riding along: 3 blocks a
-// CU hold them all at 512^2 (with 16 and 16 rows a second round starts: 5.04).
+// regions of 64 x 64, where the ring's work eats the rest) and adjoint steps
+// two (the gradient with 1 -> 2 a launch, us: 64x51, 100 steps 1067 -> 928 with
+// 8 waves of 2 rows, 1060 with 16; 250x177 1143 -> 1062 with 12 of 2, 1205 with
+// 8; 512^2, 300 steps 4640 -> 4335 with 16 of 3, 4520 with 12 of 4, 6010 with
+// 16 of 4).  Forward regions of 32 rows while they all fit the CUs at once,
+// else 48 (250x177: 1.14 ms for the gradient of 100 steps with 32 rows, 1.20
+// with 48; 512^2: 4.86 and 4.68 for 300).  A single adjoint step's regions are
+// 16 rows with 24 for the step riding along: 3 blocks a CU hold them all at
+// 512^2 (with 16 and 16 rows a second round starts: 5.04).
 constexpr int kSiaMax = 3;                        // forward steps per launch
 constexpr int kNWF = 16, kRF1 = 2, kRF2 = 3;      // forward: waves, rows per wave
 constexpr int kNWA = 8, kRA = 2, kRR = 3;         // adjoint, and the steps riding along
@@ -753,18 +804,31 @@ static void launch_rule(hipStream_t st, const SiaStep<double>& f, const SiaRule&
     else hipLaunchKernelGGL((sia_rule_kernel<0, NW, R, MAXD>), dim3(nb), blk, 0, st, f, r, ntx, nx, ny);
 }
 
-static void launch_adj(hipStream_t st, const SiaAdj<double>& a, const SiaStep<double>* f, double fdt, int64_t nx,
-                       int64_t ny) {
-    constexpr int NW = kNWA, RA = kRA, RF = kRR;
+template <int NW, int RA, int RF, bool TWO>
+static void launch_adj_r(hipStream_t st, const SiaAdj<double>& a, const SiaStep<double>& f, const SiaMid& mid,
+                         const SiaDts& fd, int64_t nx, int64_t ny) {
     int ntxa, ntxf = 1;
-    const int na = sia_regions(nx, ny, sia_adj_ring(a.rd), kAdjRing, NW * RA, &ntxa);
-    const int nf = f ? sia_regions(nx, ny, 2, 2, NW * RF, &ntxf) : 0;
-    const SiaStep<double> g = f ? *f : SiaStep<double>{};
-    const dim3 blk(64, NW);
-    if (a.s.n == 3)
-        hipLaunchKernelGGL((sia_adj_kernel<3, NW, RA, RF>), dim3(na + nf), blk, 0, st, a, g, fdt, na, ntxa, ntxf, nx, ny);
-    else
-        hipLaunchKernelGGL((sia_adj_kernel<0, NW, RA, RF>), dim3(na + nf), blk, 0, st, a, g, fdt, na, ntxa, ntxf, nx, ny);
+    const int na = sia_regions(nx, ny, sia_adj_ring(a.rd, a.n), kAdjRing * a.n, NW * RA, &ntxa);
+    const int nf = fd.n ? sia_regions(nx, ny, 2 * fd.n, 2 * fd.n, NW * RF, &ntxf) : 0;
+    const dim3 blk(64, NW), grd(na + nf);
+    if (a.s.n == 3) hipLaunchKernelGGL((sia_adj_kernel<3, NW, RA, RF, TWO>), grd, blk, 0, st, a, f, mid, fd, na, ntxa, ntxf, nx, ny);
+    else hipLaunchKernelGGL((sia_adj_kernel<0, NW, RA, RF, TWO>), grd, blk, 0, st, a, f, mid, fd, na, ntxa, ntxf, nx, ny);
+}
+
+// fd.n forward steps (0: none) ride along with a.n adjoint steps.  Two steps
+// take the first shape whose blocks all find a CU of their own (the flatter,
+// the shorter a block's chain), the largest regions beyond.
+static void launch_adj(hipStream_t st, const SiaAdj<double>& a, const SiaStep<double>& f, const SiaMid& mid,
+                       const SiaDts& fd, int64_t nx, int64_t ny) {
+    if (a.n == 1 && fd.n <= 1) return launch_adj_r<kNWA, kRA, kRR, false>(st, a, f, mid, fd, nx, ny);
+    auto fits = [&](int nw, int r) {
+        int t;
+        return sia_regions(nx, ny, 2 * kAdjRing, 2 * kAdjRing, nw * r, &t) + sia_regions(nx, ny, 4, 4, nw * (r + 1), &t) <=
+               cu_count();
+    };
+    if (fits(8, 2)) launch_adj_r<8, 2, 3, true>(st, a, f, mid, fd, nx, ny);
+    else if (fits(12, 2)) launch_adj_r<12, 2, 3, true>(st, a, f, mid, fd, nx, ny);
+    else launch_adj_r<16, 3, 4, true>(st, a, f, mid, fd, nx, ny);
 }
 
 template <class T>
@@ -817,7 +881,9 @@ static SiaAdj<double> sia_adjointer(const chmy_grid_t* g, const chmy_field_t* H,
     a.gA = gA ? view<double>(*gA) : a.lo;
     a.dt = dt;
     a.rd = 0;
-    a.Din = a.lo;
+    a.n = 1;
+    a.Din = a.H2 = a.D2 = a.lo;
+    a.dt2 = 0.0;
     return a;
 }
 
@@ -900,22 +966,32 @@ static int sia_reverse_sweep(const chmy_grid_t* g, const chmy_field_t* ckpt, int
     int slot = 0;   // lam_in of the next adjoint step: 0 = lam_a, 1 = lam_b
     for (int sg = nseg - 1; sg >= 0; --sg) {
         const int L = len(sg), Lp = sg > 0 ? len(sg - 1) : 0;
-        for (int r = 0; r < std::max(L, Lp - 1); ++r) {
+        for (int r = 0; r < std::max(L, Lp - 1);) {
             // the recompute of segment sg - 1 (state r -> r + 1) rides along with
-            // adjoint step q = L - 1 - r of segment sg
-            const bool fw = sg > 0 && r + 1 < Lp;
+            // adjoint step q = L - 1 - r of segment sg, two of each to a launch
+            // where the second step's D is stored
+            const int na = r >= L ? 0 : dbuf && r + 2 <= L ? 2 : 1, take = std::max(na, 1);
+            const int nf = std::max(0, std::min(take, Lp - 1 - r));
             SiaStep<double> f{};
-            if (fw) {
-                const chmy_field_t s0 = state(sg - 1, r), s1 = state(sg - 1, r + 1);
+            SiaMid mid{};
+            SiaDts fd{};
+            fd.n = nf;
+            if (nf > 0) {
+                const chmy_field_t s0 = state(sg - 1, r), s1 = state(sg - 1, r + nf);
                 f = sia_stepper(g, &s0, &s1, B, A, p);
+                for (int k = 0; k < nf; ++k) fd.dt[k] = dts[(sg - 1) * stride + r + k];
                 if (dbuf) {
                     f.wd = 1;
                     f.Dout = dfield(sg - 1, r);
                 }
+                if (nf == 2) {
+                    mid.H = view<double>(state(sg - 1, r + 1));
+                    mid.D = dfield(sg - 1, r + 1);
+                }
             }
-            const double* fdt = fw ? &dts[(sg - 1) * stride + r] : nullptr;
-            if (r >= L) {
-                launch_steps(st, f, fdt, 1, nx, ny);
+            if (na == 0) {
+                launch_steps(st, f, fd.dt, 1, nx, ny);
+                r += 1;
                 continue;
             }
             const int q = L - 1 - r;
@@ -928,8 +1004,15 @@ static int sia_reverse_sweep(const chmy_grid_t* g, const chmy_field_t* ckpt, int
                 a.rd = 1;
                 a.Din = dfield(sg, q);
             }
-            launch_adj(st, a, fw ? &f : nullptr, fw ? *fdt : 0.0, nx, ny);
+            a.n = na;
+            if (na == 2) {
+                a.H2 = view<double>(state(sg, q - 1));
+                a.D2 = dfield(sg, q - 1);
+                a.dt2 = dts[sg * stride + q - 1];
+            }
+            launch_adj(st, a, f, mid, fd, nx, ny);
             slot ^= 1;
+            r += na;
         }
     }
     return slot;
@@ -1070,7 +1153,7 @@ int chmy_sia_step_adjoint(const chmy_grid_t* g, const chmy_field_t* H, const chm
     SiaPar p{As, npow, mb_a, mb_b, mb_c, dt};
     if (!work) {   // one tiled pass
         SiaAdj<double> a = sia_adjointer(g, H, lam_in, lam_out, A ? grad_logA : nullptr, B, A, p, dt);
-        launch_adj((hipStream_t)stream, a, nullptr, 0.0, g->n[0], g->n[1]);
+        launch_adj((hipStream_t)stream, a, SiaStep<double>{}, SiaMid{}, SiaDts{}, g->n[0], g->n[1]);
         CHMY_HIP(hipGetLastError());
         return 0;
     }

@@ -378,7 +378,7 @@ def test_adaptive_run_equals_rule_and_step(arch, dims, npow, with_A, dt_max):
 
 
 @pytest.mark.parametrize("npow", [3, 2])
-@pytest.mark.parametrize("n", [(2, 3), (52, 20), (53, 37), (57, 11), (116, 45), (125, 61), (700, 402)])
+@pytest.mark.parametrize("n", [(2, 3), (52, 20), (53, 37), (57, 11), (116, 45), (125, 61), (260, 149), (700, 402)])
 def test_multi_step_regions_equal_single_steps(arch, n, npow):
     """Several steps to a launch, the adaptive step's next max(D) and the
     adjoint's regions at their edges (owned columns 52, 56, 58, 60, rows 10,
