@@ -22,7 +22,7 @@ import torch
 
 from . import _lib
 from .architectures import current_stream
-from .boundary_conditions import Dirichlet, Neumann, batch
+from .boundary_conditions import BatchSet, Dirichlet, FieldBatch, Neumann, batch
 from .fields import Field, TensorField, VectorField, set_storage
 from .function_field import as_field
 from .grids import Center, UniformGrid, spacing
@@ -123,6 +123,18 @@ class PTStokes:
         bs = self._bcs.get(key)
         if bs is None:
             bs = free_slip_batch(self.grid, V, self.normal_values)
+            self._bcs[key] = bs
+        bs.apply()
+
+    def _apply_bc_both(self, Va, Vb):
+        """apply_bc on two vector fields in one launch (the sets share no field)."""
+        key = (id(Va[0]), id(Vb[0]))
+        bs = self._bcs.get(key)
+        if bs is None:
+            a, b = (free_slip_batch(self.grid, v, self.normal_values) for v in (Va, Vb))
+            bs = BatchSet(self.grid, [tuple(FieldBatch(list(p.fields) + list(q.fields),
+                                                       list(p.conditions) + list(q.conditions))
+                                            for p, q in zip(da, db)) for da, db in zip(a.per_dim, b.per_dim)])
             self._bcs[key] = bs
         bs.apply()
 
@@ -231,8 +243,7 @@ class PTStokes:
                   C.byref(self.rhog.desc()) if self.rhog is not None else None,
                   counts, comp, conds, ITER_EXACT if self.exact else 0, self.eta_s, self.eta_ve_s, self.G,
                   self.dt, self.p["dtau_Pr"], self.p["dtau_r"], self.p["nudtau"], current_stream())
-        self.apply_bc(V_first)
-        self.apply_bc(self.V2)
+        self._apply_bc_both(V_first, self.V2)
         self._swap()
         self.iters += 2
 
