@@ -1370,14 +1370,10 @@ __global__ void __launch_bounds__(kFX * kTB3Y<T>) fused3d_tb_kernel(Fused3<T> a,
     }
 }
 
-#ifndef CHMY_FUSED_ZCHUNK64
-#define CHMY_FUSED_ZCHUNK64 16
-#endif
 #ifndef CHMY_FUSED_ZCHUNK32
 #define CHMY_FUSED_ZCHUNK32 12
 #endif
-template <class T>
-constexpr int kZChunk = std::is_same<T, double>::value ? CHMY_FUSED_ZCHUNK64 : CHMY_FUSED_ZCHUNK32;
+constexpr int kZChunk32 = CHMY_FUSED_ZCHUNK32;
 template <class T>
 constexpr int kBY3 = std::is_same<T, double>::value ? CHMY_FUSED_BY64 : CHMY_FUSED_BY32;
 template <class T>
@@ -1543,10 +1539,12 @@ static int fused_launch(const chmy_grid_t* g, const chmy_field_t* V, const chmy_
             CHMY_HIP(hipGetLastError());
             return 0;
         }
-        a.kchunk = kZChunk<T>;
         a.ntx = (int32_t)((g->n[0] + 2 + kTW3<T> - 3) / (kTW3<T> - 2));
         a.nty = (int32_t)((g->n[1] + 2 + kBY3<T> - 2) / (kBY3<T> - 1));
-        a.nchunks = (int32_t)((g->n[2] + 2 + kZChunk<T> - 1) / kZChunk<T>);
+        // FP64: one block a CU, as the pass (175x159x143 265 -> 234 us, 255^3 1137 ->
+        // 1117 against 16 planes); FP32 blocks share a CU and keep a fixed length
+        a.kchunk = sizeof(T) == 8 ? tb3_chunk((int64_t)a.ntx * a.nty, g->n[2] + 2) : kZChunk32;
+        a.nchunks = (int32_t)((g->n[2] + 2 + a.kchunk - 1) / a.kchunk);
         a.has_rg = rg != nullptr;
         a.write_res = wres;
         a.ix = T(g->inv_spacing[0]);
