@@ -750,9 +750,11 @@ __global__ void __launch_bounds__(NW * 64) sia_adj_kernel(SiaAdj<double> a, SiaS
 
 // Shapes, each the best measured of 4..16 waves by 1..6 rows.  A launch's floor
 // is its serial chain (about 4.5 us a forward step, 5.4 us an adjoint step for
-// one region alone), so forward steps go several to a launch (300 steps of
-// 512^2: 5.1 us each singly, 4.3 in twos, 3.8 in threes, 3.9 in fives on
-// regions of 64 x 64, where the ring's work eats the rest) and adjoint steps
+// one region alone), so forward steps go several to a launch: up to five while
+// the regions' own 44 x 28 cells cover the grid in one round of the CUs, else
+// three, where the ring's work counts (300 steps of 512^2 within the gradient,
+// us a step: 5.1 singly, 4.3 in twos, 3.8 in threes, 3.1 in fives; gradient 4319
+// -> 4098 from three to five, 64x51 935 -> 872, 250x177 1072 -> 1006), and adjoint steps
 // two (the gradient with 1 -> 2 a launch, us: 64x51, 100 steps 1067 -> 928 with
 // 8 waves of 2 rows, 1060 with 16; 250x177 1143 -> 1062 with 12 of 2, 1205 with
 // 8; 512^2, 300 steps 4640 -> 4335 with 16 of 3, 4520 with 12 of 4, 6010 with
@@ -761,7 +763,7 @@ __global__ void __launch_bounds__(NW * 64) sia_adj_kernel(SiaAdj<double> a, SiaS
 // with 48; 512^2: 4.86 and 4.68 for 300).  A single adjoint step's regions are
 // 16 rows with 24 for the step riding along: 3 blocks a CU hold them all at
 // 512^2 (with 16 and 16 rows a second round starts: 5.04).
-constexpr int kSiaMax = 3;                        // forward steps per launch
+constexpr int kSiaMax = 5, kSiaMany = 3;          // forward steps per launch: one round, more
 constexpr int kNWF = 16, kRF1 = 2, kRF2 = 3;      // forward: waves, rows per wave
 constexpr int kNWA = 8, kRA = 2, kRR = 3;         // adjoint, and the steps riding along
 constexpr int kNWD = 16, kRD = 1;                 // the adaptive step
@@ -891,7 +893,7 @@ static SiaAdj<double> sia_adjointer(const chmy_grid_t* g, const chmy_field_t* H,
 // its last are not stored, so each must have a later state in the same
 // storage (looked for over the next 8), and the output must not touch the
 // input (a block reads cells that its neighbours own).
-static int sia_run_length(const chmy_field_t* st, int nstates, int q) {
+static int sia_run_length(const chmy_field_t* st, int nstates, int q, int longest) {
     const auto same = [](const chmy_field_t& a, const chmy_field_t& b) {
         return a.data == b.data && a.halo[0] == b.halo[0] && a.halo[1] == b.halo[1];
     };
@@ -905,7 +907,7 @@ static int sia_run_length(const chmy_field_t* st, int nstates, int q) {
         return false;
     };
     int most = 1;
-    while (most < kSiaMax && q + most + 1 < nstates && replaced(q + most)) ++most;
+    while (most < longest && q + most + 1 < nstates && replaced(q + most)) ++most;
     for (int n = most; n > 1; --n)
         if (apart(st[q], st[q + n])) return n;
     return 1;
@@ -1192,8 +1194,11 @@ int chmy_sia_run(const chmy_grid_t* g, const chmy_field_t* states, int nstates, 
             return set_error(CHMY_E_ARG, "states[%d] and states[%d] share storage", q, q + 1);
     const SiaPar p{As, npow, mb_a, mb_b, mb_c, 0.0};
     hipStream_t st = (hipStream_t)stream;
+    int ntx;
+    const int longest = sia_regions(g->n[0], g->n[1], 2 * kSiaMax, 2 * kSiaMax, kNWF * kRF2, &ntx) <= cu_count() ? kSiaMax
+                                                                                                               : kSiaMany;
     for (int q = 0; q + 1 < nstates;) {
-        const int n = sia_run_length(states, nstates, q);
+        const int n = sia_run_length(states, nstates, q, longest);
         const SiaStep<double> f = sia_stepper(g, &states[q], &states[q + n], B, A, p);
         launch_steps(st, f, dts + q, n, g->n[0], g->n[1]);
         q += n;
