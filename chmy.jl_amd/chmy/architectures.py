@@ -65,7 +65,8 @@ def activate(arch, priority="normal"):
 
 
 def heuristic_groupsize(backend, nd):
-    """Work-group shape of the HIP kernels: one wave64 along x, 4 rows in y."""
+    """A work-group of 256 threads, one wave64 along x and 4 rows in y (the
+    per-point kernels lay their 256 points along the rows of a plane)."""
     return {1: (256,), 2: (64, 4), 3: (64, 4, 1)}[nd]
 
 
