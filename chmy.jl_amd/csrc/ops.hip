@@ -166,14 +166,14 @@ __global__ void __launch_bounds__(256) diffusion_step_bc_kernel(Box3 box, Box3 r
 // value is the expression of diffusion_value on the same operands; the
 // neighbour beyond a boundary is the batch's own fma step of the cell (the
 // stored ghost in the first step), so every stored value has the bits of as
-// many launches of the step.  q is not stored and the corner ghosts (which no
-// cell reads) are left alone: the caller runs the last two steps one by one,
-// and they write both buffers' ghosts, corners included, and q.
+// many launches of the step.  q is not stored, so the caller runs the last step
+// by itself; in 3D the last two, since the edge and corner ghosts (which no
+// cell reads, but q on the ghosts does) are left alone there.
 //
 // Why: a step of 256^2 cells is one 5 us launch for 0.5 MB of data, most of it
 // the wait for the launch before it.  Measured, us per step of a 100-step call,
-// one launch each -> now: 2D FP64 64^2 4.7 -> 0.95, 256^2 5.1 -> 0.96, 500x480
-// 5.5 -> 1.5, 1024^2 11.4 -> 3.5 (FP32 10.0 -> 2.8); 3D 20^3 5.6 -> 3.5, 64^3
+// one launch each -> now: 2D FP64 64^2 4.7 -> 0.88, 256^2 5.1 -> 0.87, 500x480
+// 5.5 -> 1.4, 1024^2 11.4 -> 3.5 (FP32 10.0 -> 2.8); 3D 20^3 5.6 -> 3.5, 64^3
 // 12.6 -> 3.7, 160^3 58.6 -> 25.7 (FP32 45 -> 15).  Bound by the chain of LDS
 // reads and barriers (0.1 us a step) and the launches on small grids, by
 // vector issue and LDS on large ones.
@@ -291,6 +291,23 @@ __global__ void __launch_bounds__(NT) diffusion_tile_kernel(const DiffTile<T> p)
             const int64_t st = d == 0 ? 1 : d == 1 ? p.C.sy : p.C.sz;
             if (d == M ? i == 1 : g0[d & 1][0]) p.Co.p[o - st] = ghost_of(p.r, d, 0, c[q]);
             if (d == M ? i == p.n[M] : g0[d & 1][1]) p.Co.p[o + st] = ghost_of(p.r, d, 1, c[q]);
+        }
+        if constexpr (ND == 2) {
+            // what else the batch writes: the corners (y's rule, then x's), and its
+            // tangential range's last index n + 2, from points that no step changes
+            const bool gy[2] = {i == 1, i == p.n[1]};
+            const int64_t sy = p.C.sy;
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
+                const int a_ = k & 1, b_ = k >> 1;
+                const int64_t dx = a_ ? 1 : -1, dy = b_ ? sy : -sy;
+                if (g0[0][a_] && gy[b_]) p.Co.p[o + dx + dy] = ghost_of(p.r, 0, a_, ghost_of(p.r, 1, b_, c[q]));
+            }
+#pragma unroll
+            for (int k = 0; k < 2; ++k) {
+                if (g0[0][k] && gy[1]) p.Co.p[o + 2 * sy + (k ? 1 : -1)] = ghost_of(p.r, 0, k, p.Co.p[o + 2 * sy]);
+                if (gy[k] && g0[0][1]) p.Co.p[o + 2 + (k ? sy : -sy)] = ghost_of(p.r, 1, k, p.Co.p[o + 2]);
+            }
         }
     }
 }
@@ -640,13 +657,13 @@ static int diffusion_tile_any(int nd, int k, int64_t cells, const DiffTile<T>& a
                                  : diffusion_tile_launch<T, 3, 28, 12, 12, kDiffK3, 8>(a, k, C, p, s);
 }
 
-// All but the last two steps in passes of up to 8 (2D) or 2 (3D) steps, as many
+// All but the last step (3D: two) in passes of up to 8 (2D) or 2 (3D) steps, as many
 // passes as leave the buffers where single steps would (a pass flips the
 // parity once); *done steps were taken.
 template <class T>
 static int diffusion_passes(const chmy_grid_t* g, const chmy_field_t* C0, const chmy_field_t* C1, const SideRules& r,
                             double chi, double dt, int niter, int* p, int* done, hipStream_t s) {
-    const int steps = niter - 2, nd = g->nd;
+    const int nd = g->nd, steps = niter - (nd == 2 ? 1 : 2);
     int64_t cells = 1;
     for (int d = 0; d < nd; ++d) cells *= g->n[d];
     if (nd < 2 || steps < 2) return 0;
