@@ -766,7 +766,7 @@ __global__ void __launch_bounds__(NW * 64) sia_adj_kernel(SiaAdj<double> a, SiaS
 constexpr int kSiaMax = 5, kSiaMany = 3;          // forward steps per launch: one round, more
 constexpr int kNWF = 16, kRF1 = 2, kRF2 = 3;      // forward: waves, rows per wave
 constexpr int kNWA = 8, kRA = 2, kRR = 3;         // adjoint, and the steps riding along
-constexpr int kNWD = 16, kRD = 1;                 // the adaptive step
+constexpr int kNWD = 8, kRD = 2;                  // the adaptive step (us for 24: 250x230 203, 400x390 243; 16 x 1: 206, 260)
 static_assert(kSiaMax <= kSiaSteps && kNWF * kRF1 > 4 * kSiaMax && 64 > 4 * kSiaMax && kNWA * kRA > 2 * kAdjRing &&
                   kNWA * kRR > 4 && kNWD * kRD > 6,
               "a region owns at least one row and column");
