@@ -9,6 +9,7 @@ struct Shape2 {
     static constexpr int KM = KM_, W = W_, PT = PT_, TX = kFX - 2 * KM, TY = W * PT - 2 * KM;
 };
 using Small2 = Shape2<7, 16, 1>;
+using Flat2 = Shape2<5, 16, 1>;
 using Mid2 = Shape2<6, 16, 2>;
 using Large2 = Shape2<8, 16, 3>;
 using Dense2 = Shape2<5, 8, 3>;
@@ -22,17 +23,23 @@ using Dense2 = Shape2<5, 8, 3>;
 // 231 / 246 (221 tiles of Large2), 800x640 340 / 313 / 297 (357 tiles),
 // 1400x1200 693 / 633 / 592; 41 at 2047^2 1734 (Large2) / 1584; other waves,
 // rows and lengths for the last one: <4, 8, 3> 1775, <6, 8, 3> 1668, <5, 16, 3>
-// 1982, <6, 12, 4> 1840, <5, 6, 4> 2512.  400x380: Mid2 and Dense2 alike.
+// 1982, <6, 12, 4> 1840, <5, 6, 4> 2512.  400x380: Mid2 and Dense2 alike.  Mid2 /
+// Flat2, 33 iterations: 200x150 188 / 152, 280x240 190 / 156, 160x150 in the
+// exact form 250 / 184 (<5, 14, 1> 153 / 188 / 183, <6, 15, 1> 158 / 191 / 197).
 static int64_t tiles2(int64_t nbx, int64_t nby, int tx, int ty) { return ((nbx + tx - 1) / tx) * ((nby + ty - 1) / ty); }
 template <class Sh>
 static bool one_round(int64_t nbx, int64_t nby) {
     return tiles2(nbx, nby, Sh::TX, Sh::TY) <= cu_count();
 }
 static int shape2(int64_t nbx, int64_t nby) {
-    return one_round<Small2>(nbx, nby) ? 0 : one_round<Mid2>(nbx, nby) ? 1 : one_round<Large2>(nbx, nby) ? 2 : 3;
+    return one_round<Small2>(nbx, nby)  ? 0
+           : one_round<Flat2>(nbx, nby) ? 1
+           : one_round<Mid2>(nbx, nby)  ? 2
+           : one_round<Large2>(nbx, nby) ? 3
+                                         : 4;
 }
 int multi2d_most(const chmy_grid_t* g) {
-    const int k[4] = {Small2::KM, Mid2::KM, Large2::KM, Dense2::KM};
+    const int k[5] = {Small2::KM, Flat2::KM, Mid2::KM, Large2::KM, Dense2::KM};
     return k[shape2(g->n[0] + 2, g->n[1] + 2)];
 }
 
@@ -244,8 +251,9 @@ void multi2d_launch(Fused2<T> a, const FreeSlip2& fs, bool fv, bool exact, bool 
     };
     switch (shape2(nbx, nby)) {
         case 0: go(Small2{}); break;
-        case 1: go(Mid2{}); break;
-        case 2: go(Large2{}); break;
+        case 1: go(Flat2{}); break;
+        case 2: go(Mid2{}); break;
+        case 3: go(Large2{}); break;
         default: go(Dense2{}); break;
     }
 }

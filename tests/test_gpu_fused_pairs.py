@@ -377,10 +377,12 @@ def test_several_iterations_per_pass_2d(arch, T, forcing, exact, visc, rhog, dim
 
 
 @pytest.mark.parametrize("T,forcing", [(np.float64, None), (np.float32, "bf16")])
-@pytest.mark.parametrize("dims,niter", [((860, 559), 11), ((538, 1010), 8), ((1027, 640), 6)])
-def test_many_tiles_per_cu_2d(arch, T, forcing, dims, niter):
-    """Grids of several tiles a CU (8 waves, 54 x 14 points a tile; tiles that
-    end at, past and inside the box) against single iterations, bitwise."""
+@pytest.mark.parametrize("dims,niter", [((860, 559), 11), ((538, 1010), 8), ((1027, 640), 6),   # 54 x 14 points
+                                        ((322, 94), 11), ((161, 150), 8), ((300, 101), 16)])    # 54 x 6
+def test_more_tile_shapes_2d(arch, T, forcing, dims, niter):
+    """Grids of several tiles a CU (8 waves of three rows a tile) and the flat
+    tiles of 16 waves with five iterations a pass; tiles that end at, past and
+    inside the box, against single iterations, bitwise."""
     g = chmy.UniformGrid(arch, origin=(-0.5, -0.5), extent=(1.0, 1.3), dims=dims)
     a = _run(arch, g, T, False, "field", forcing, GENERAL, niter, True, 29)
     b = _run(arch, g, T, False, "field", forcing, GENERAL, niter, False, 29)
