@@ -298,7 +298,9 @@ int chmy_stokes_iter(const chmy_grid_t* grid, const chmy_field_t* V, const chmy_
  * eight in 2D; CHMY_ITER_SINGLE (in `flags`) keeps single iterations, and
  * CHMY_ITER_PAIRS is accepted and ignored.  A pass writes set 1-p like one
  * iteration, so the parity flips once per pass; results are bitwise those of
- * single iterations. */
+ * single iterations.  The V batch has been applied to the set the call ends
+ * on; between 2D passes the next pass applies it to the V it reads, so the
+ * other set's ghosts may be from before it. */
 int chmy_stokes_iterate(const chmy_grid_t* grid, const chmy_field_t* V0, const chmy_field_t* tau0,
                         const chmy_field_t* Pr0, const chmy_field_t* V1, const chmy_field_t* tau1,
                         const chmy_field_t* Pr1, const chmy_field_t* tau_old, const chmy_field_t* eta,
