@@ -165,10 +165,24 @@ inline Box3 box3(const chmy_box_t& b, int nd) {
 // KernelAbstractions launch over an empty worksize does no work).
 inline bool no_work(const Box3& b) { return b.len[0] <= 0 || b.len[1] <= 0 || b.len[2] <= 0; }
 
+// A line of nb blocks as a grid.  HIP launches fewer than 2^32 work-items in a
+// grid dimension, so a line of that many or more is folded into rows of
+// kLineRow blocks (whole rounds of the 8 XCDs); the ids that the last row has
+// too many name no tile, and their blocks do nothing.
+constexpr int64_t kLineRow = int64_t(1) << 21, kLineMost = int64_t(1) << 30;
+inline int line_grid(int64_t nb, int threads, dim3* grd) {
+    if (nb > kLineMost) return set_error(CHMY_E_SIZE, "box too large: %lld blocks", (long long)nb);
+    const bool one = nb * threads <= INT64_C(0xffffffff);
+    *grd = one ? dim3((unsigned)nb, 1, 1) : dim3((unsigned)kLineRow, (unsigned)((nb + kLineRow - 1) / kLineRow), 1);
+    return 0;
+}
+__device__ __forceinline__ uint32_t line_id() { return blockIdx.y * gridDim.x + blockIdx.x; }
+__device__ __forceinline__ uint32_t line_ids() { return gridDim.y * gridDim.x; }
+
 // The q-th point of a plane of rows of len0 points, counted along the rows:
 // column a, row c (c >= len1 past the plane).  The 32-bit division unless the
 // plane has 2^32 points (uniform).
-__device__ __forceinline__ void plane_index(int64_t q, int64_t len0, int64_t len1, int64_t& a, int64_t& c) {
+__host__ __device__ __forceinline__ void plane_index(int64_t q, int64_t len0, int64_t len1, int64_t& a, int64_t& c) {
     if (len0 * len1 + 0x10000 < 0x100000000ll) {
         const uint32_t r = (uint32_t)q, n = (uint32_t)len0, k = r / n;
         c = k;
@@ -184,20 +198,29 @@ __device__ __forceinline__ void plane_index(int64_t q, int64_t len0, int64_t len
 // plane, each XCD a contiguous run of them: the planes and rows that a
 // neighbour's point shares are found in that XCD's L2.
 constexpr int kFlat = 256;
-inline dim3 flat_grid(const Box3& b) {
-    return dim3((unsigned)((b.len[0] * b.len[1] + kFlat - 1) / kFlat * b.len[2]), 1, 1);
+inline int flat_grid(const Box3& b, dim3* grd) {
+    int64_t plane, nb;
+    if (__builtin_mul_overflow(b.len[0], b.len[1], &plane) ||
+        __builtin_mul_overflow(plane / kFlat + (plane % kFlat != 0), b.len[2], &nb))
+        nb = INT64_MAX;
+    return line_grid(nb, kFlat, grd);
 }
-__device__ __forceinline__ bool flat_point(const Box3& b, int64_t& i, int64_t& j, int64_t& k) {
-    const uint32_t per = (uint32_t)((b.len[0] * b.len[1] + kFlat - 1) / kFlat), nb = gridDim.x;
+// Lane `lane` of block `bid` of nb: its point, or false.
+__host__ __device__ __forceinline__ bool flat_at(const Box3& b, uint32_t bid, uint32_t nb, uint32_t lane, int64_t& i,
+                                                 int64_t& j, int64_t& k) {
+    const uint32_t per = (uint32_t)((b.len[0] * b.len[1] + kFlat - 1) / kFlat);
     // xcd_remap on unsigned ids
-    const uint32_t run = nb / 8, id = blockIdx.x < 8 * run ? (blockIdx.x % 8) * run + blockIdx.x / 8 : blockIdx.x;
+    const uint32_t run = nb / 8, id = bid < 8 * run ? (bid % 8) * run + bid / 8 : bid;
     const uint32_t e = id / per;
     int64_t a, c;
-    plane_index((int64_t)(id - e * per) * kFlat + threadIdx.x, b.len[0], b.len[1], a, c);
+    plane_index((int64_t)(id - e * per) * kFlat + lane, b.len[0], b.len[1], a, c);
     i = b.lo[0] + a;
     j = b.lo[1] + c;
     k = b.lo[2] + e;
-    return c < b.len[1];
+    return c < b.len[1] && e < b.len[2];
+}
+__device__ __forceinline__ bool flat_point(const Box3& b, int64_t& i, int64_t& j, int64_t& k) {
+    return flat_at(b, line_id(), line_ids(), threadIdx.x, i, j, k);
 }
 
 // Compute units of the current device, read once per device (api.hip).

@@ -235,7 +235,7 @@ __device__ __forceinline__ void program_run(const PProg& P, int q0, int q1, Slot
 // 191x187x189 FP64 271 -> 256 (160x144x127 waits for the host: 161 both).
 template <class T, int S, int N, bool HEAVY>
 __global__ void __launch_bounds__(64) program_kernel(const PProg P, DF<T> dst, Box3 b, int nbx, int chunk) {
-    const int t = blockIdx.x;
+    const int t = line_id();
     const int bx = t % nbx, bc = t / nbx;
     const int m = P.m;
     // z marched: 64 consecutive points of a plane, counted along its rows; y
@@ -247,6 +247,7 @@ __global__ void __launch_bounds__(64) program_kernel(const PProg P, DF<T> dst, B
     j = in ? b.lo[1] + j : b.lo[1];
     const int64_t m0 = b.lo[m] + (int64_t)bc * chunk;
     const int64_t hm = b.lo[m] + b.len[m], m1 = m0 + chunk < hm ? m0 + chunk : hm;
+    if (m0 >= hm) return;   // no chunk
     const int64_t I[3] = {i, j, b.lo[2]};
     Slots<S> r[N];
     int64_t Im[N];
@@ -437,9 +438,9 @@ static int program_launch(const PProg& P, const chmy_field_t* dst, const Box3& b
             chunk = c;
         }
     }
-    const int64_t nb = nbx * ((nm + chunk - 1) / chunk);
-    if (nb > INT32_MAX) return set_error(CHMY_E_SIZE, "point program: box too large");
-    const dim3 grd((unsigned)nb), blk(64);
+    dim3 grd;
+    CHMY_TRY(line_grid(nbx * ((nm + chunk - 1) / chunk), 64, &grd));
+    const dim3 blk(64);
     const DF<T> d = view<T>(*dst);
     const int ix = (int)nbx, ic = (int)chunk;
     if (slots > 16)

@@ -287,7 +287,7 @@ constexpr int kOpB = 256, kOpZ = 4;
 
 template <class T, class Op>
 __global__ void __launch_bounds__(kOpB) op_kernel(Box3 b, DF<T> dst, Op op, int nbx, int kchunk) {
-    const int t = xcd_remap(blockIdx.x, gridDim.x);
+    const int t = xcd_remap(line_id(), line_ids());   // past the last tile: bz past the last chunk
     const int bx = t % nbx, bz = t / nbx;
     int64_t a, c;
     plane_index((int64_t)bx * kOpB + threadIdx.x, b.len[0], b.len[1], a, c);
@@ -382,10 +382,9 @@ static int op_launch(const OpCall& c, const Op& op) {
     const int64_t nbx = (c.b.len[0] * c.b.len[1] + kOpB - 1) / kOpB;
     int kz = kOpZ;
     while (kz > 1 && nbx * ((c.b.len[2] + kz - 1) / kz) < 4096) kz /= 2;
-    const int64_t nb = nbx * ((c.b.len[2] + kz - 1) / kz);
-    if (nb > INT32_MAX) return set_error(CHMY_E_SIZE, "operator: box too large");
-    hipLaunchKernelGGL((op_kernel<T, Op>), dim3((unsigned)nb), dim3(kOpB, 1, 1), 0, c.s, c.b, view<T>(*c.dst), op, (int)nbx,
-                       kz);
+    dim3 grd;
+    CHMY_TRY(line_grid(nbx * ((c.b.len[2] + kz - 1) / kz), kOpB, &grd));
+    hipLaunchKernelGGL((op_kernel<T, Op>), grd, dim3(kOpB, 1, 1), 0, c.s, c.b, view<T>(*c.dst), op, (int)nbx, kz);
     CHMY_HIP(hipGetLastError());
     return 0;
 }

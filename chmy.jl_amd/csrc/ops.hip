@@ -206,8 +206,9 @@ __global__ void __launch_bounds__(NT) diffusion_tile_kernel(const DiffTile<T> p)
     using Sh = DiffShape<T, ND, TX, TY, TZ, KS, PT>;
     constexpr int RX = Sh::RX, RY = Sh::RY, M = Sh::M, SM = Sh::SM;
     __shared__ T buf[2][Sh::COLS * Sh::RM];
-    const int t = xcd_remap(blockIdx.x, gridDim.x);
-    const int bx = t % p.nb[0], by = (t / p.nb[0]) % p.nb[1], bz = ND == 3 ? t / (p.nb[0] * p.nb[1]) : 0;
+    const int t = xcd_remap(line_id(), line_ids());
+    const int row = t / p.nb[0], bx = t - row * p.nb[0], by = ND == 3 ? row % p.nb[1] : row, bz = ND == 3 ? row / p.nb[1] : 0;
+    if (ND == 3 ? bz >= p.nb[2] : by >= p.nb[1]) return;   // no tile (whole block: no barrier passed)
     const int col = threadIdx.x % Sh::COLS, strip = threadIdx.x / Sh::COLS;
     const int a[3] = {col % RX, ND == 3 ? col / RX : strip * PT, strip * PT};
     const int org[3] = {1 + bx * TX - KS, 1 + by * TY - KS, ND == 3 ? 1 + bz * TZ - KS : 0};
@@ -420,8 +421,8 @@ __global__ void __launch_bounds__(64 * kThY) thermal_step3_kernel(Box3 b, DF<T> 
                                                                   T nlam, T dt, T i0, T i1, T i2, int nbx, int nby,
                                                                   int kchunk) {
     const int lane = threadIdx.x, r = threadIdx.y;
-    const int lt = xcd_remap(blockIdx.x, gridDim.x);
-    const int bx = lt % nbx, by = (lt / nbx) % nby, bz = lt / (nbx * nby);
+    const int lt = xcd_remap(line_id(), line_ids());
+    const int bx = lt % nbx, by = (lt / nbx) % nby, bz = lt / nbx / nby;
     const int64_t hi0 = b.lo[0] + b.len[0], hi1 = b.lo[1] + b.len[1], hi2 = b.lo[2] + b.len[2];
     const int64_t i = b.lo[0] + (int64_t)bx * 64 + lane, j = b.lo[1] + (int64_t)by * kThY + r;
     const int64_t kb = b.lo[2] + (int64_t)bz * kchunk;
@@ -493,11 +494,12 @@ template <class T>
 __global__ void __launch_bounds__(64 * kTh2Y) thermal_step2_kernel(Thermal2<T> a) {
     __shared__ T s1[2][kTh2Y][64];
     const int lane = threadIdx.x, ty = __builtin_amdgcn_readfirstlane(threadIdx.y);
-    const int lt = xcd_remap(blockIdx.x, gridDim.x);
-    const int bx = lt % a.nbx, by = (lt / a.nbx) % a.nby, bz = lt / (a.nbx * a.nby);
+    const int lt = xcd_remap(line_id(), line_ids());
+    const int bx = lt % a.nbx, by = (lt / a.nbx) % a.nby, bz = lt / a.nbx / a.nby;
     const int n0 = a.n[0], n1 = a.n[1], n2 = a.n[2];
     const int i = bx * 60 - 1 + lane, j = by * (kTh2Y - 2) + ty;   // lane 2 and row 1 of the first tile: cell 1
     const int kb = 1 + bz * a.kchunk, ke = min(kb + a.kchunk, n2 + 1);
+    if (kb > n2) return;   // no tile (whole block: no barrier passed)
     const uint32_t ic = (uint32_t)min(max(i, 0), n0 + 1);
     const int jc = min(max(j, 0), n1 + 1);
     const bool own = lane >= 2 && lane <= 61 && i <= n0 && ty >= 1 && ty <= kTh2Y - 2 && j <= n1;
@@ -610,7 +612,8 @@ static int diffusion_launch(const chmy_grid_t* g, const chmy_box_t* box, const c
     DFL<T> c = lview<T>(*Cf);
     DFL<T> q0 = lview<T>(q[0]);
     DFL<T> q1 = g->nd > 1 ? lview<T>(q[1]) : q0, q2 = g->nd > 2 ? lview<T>(q[2]) : q0;
-    dim3 grd = flat_grid(b);
+    dim3 grd;
+    CHMY_TRY(flat_grid(b, &grd));
     if (flux)
         hipLaunchKernelGGL(diffusion_flux_kernel<T>, grd, blk2(), 0, s, b, c, q0, q1, q2, g->nd, -T(scalar),
                            T(g->inv_spacing[0]), T(g->inv_spacing[1]), T(g->inv_spacing[2]));
@@ -634,8 +637,10 @@ static int diffusion_tile_launch(const DiffTile<T>& base, int steps, const DF<T>
         a.nb[d] = (int32_t)q;
         nb *= q;
     }
-    hipLaunchKernelGGL((diffusion_tile_kernel<T, ND, TX, TY, TZ, KS, PT>), dim3((unsigned)nb),
-                       dim3(DiffShape<T, ND, TX, TY, TZ, KS, PT>::NT), 0, s, a);
+    constexpr int NT = DiffShape<T, ND, TX, TY, TZ, KS, PT>::NT;
+    dim3 grd;
+    CHMY_TRY(line_grid(nb, NT, &grd));
+    hipLaunchKernelGGL((diffusion_tile_kernel<T, ND, TX, TY, TZ, KS, PT>), grd, dim3(NT), 0, s, a);
     CHMY_HIP(hipGetLastError());
     return 0;
 }
@@ -702,7 +707,9 @@ static int copy_launch(const chmy_grid_t* g, const chmy_box_t& bx, const chmy_fi
     for (int q = 0; q < nt; ++q) { c.src[c.n] = lview<T>(tau[q]); c.dst[c.n] = lview<T>(tauo[q]); ++c.n; }
     Box3 b = box3(bx, g->nd);
     if (no_work(b)) return 0;
-    hipLaunchKernelGGL(copy_kernel<T>, flat_grid(b), blk2(), 0, s, b, c);
+    dim3 grd;
+    CHMY_TRY(flat_grid(b, &grd));
+    hipLaunchKernelGGL(copy_kernel<T>, grd, blk2(), 0, s, b, c);
     CHMY_HIP(hipGetLastError());
     return 0;
 }
@@ -715,7 +722,8 @@ static int thermal_launch(const chmy_grid_t* g, const chmy_box_t& bx, const chmy
     DFL<T> t = lview<T>(*Tf), o = lview<T>(other[0]);
     DFL<T> q0 = lview<T>(q[0]);
     DFL<T> q1 = g->nd > 1 ? lview<T>(q[1]) : q0, q2 = g->nd > 2 ? lview<T>(q[2]) : q0;
-    dim3 grd = flat_grid(b);
+    dim3 grd;
+    CHMY_TRY(flat_grid(b, &grd));
     if (flux) {
         DFL<T> v1 = g->nd > 1 ? lview<T>(other[1]) : o, v2 = g->nd > 2 ? lview<T>(other[2]) : o;
         hipLaunchKernelGGL(thermal_flux_kernel<T>, grd, blk2(), 0, s, b, t, o, v1, v2, q0, q1, q2, g->nd, -T(scalar),
@@ -768,7 +776,8 @@ int chmy_diffusion_step(const chmy_grid_t* g, const chmy_box_t* box, const chmy_
         DFL<T> c = lview<T>(*C), co = lview<T>(*C_out);
         DFL<T> q0 = lview<T>(q[0]);
         DFL<T> q1 = g->nd > 1 ? lview<T>(q[1]) : q0, q2 = g->nd > 2 ? lview<T>(q[2]) : q0;
-        dim3 grd = flat_grid(b);
+        dim3 grd;
+        CHMY_TRY(flat_grid(b, &grd));
         hipLaunchKernelGGL(diffusion_step_kernel<T>, grd, blk2(), 0, (hipStream_t)stream, b, c, co, q0, q1, q2,
                            g->nd, -T(chi), T(dt), T(g->inv_spacing[0]), T(g->inv_spacing[1]),
                            T(g->inv_spacing[2]));
@@ -827,9 +836,10 @@ int chmy_diffusion_iterate(const chmy_grid_t* g, const chmy_field_t* C0, const c
             DFL<T> c[2] = {lview<T>(*C0), lview<T>(*C1)};
             DFL<T> q0 = lview<T>(q[0]);
             DFL<T> q1 = g->nd > 1 ? lview<T>(q[1]) : q0, q2 = g->nd > 2 ? lview<T>(q[2]) : q0;
+            dim3 grd;
+            CHMY_TRY(flat_grid(reg, &grd));
             int it = 0;
             CHMY_TRY(diffusion_passes<T>(g, C0, C1, rules, chi, dt, niter, &p, &it, (hipStream_t)stream));
-            const dim3 grd = flat_grid(reg);
             for (; it < niter; ++it) {
                 hipLaunchKernelGGL(diffusion_step_bc_kernel<T>, grd, blk2(), 0, (hipStream_t)stream, b, reg, c[p],
                                    c[1 - p], q0, q1, q2, g->nd, -T(chi), T(dt), T(g->inv_spacing[0]),
@@ -927,16 +937,17 @@ int chmy_thermal_step(const chmy_grid_t* g, const chmy_box_t* box, const chmy_fi
             const int nbx = (int)((b.len[0] + 63) / 64), nby = (int)((b.len[1] + kThY - 1) / kThY);
             const int64_t nch = (b.len[2] + 15) / 16;
             const int kchunk = (int)((b.len[2] + nch - 1) / nch);
-            const int64_t nb = (int64_t)nbx * nby * nch;
-            if (nb > INT32_MAX) return set_error(CHMY_E_SIZE, "thermal step: box too large");
-            hipLaunchKernelGGL(thermal_step3_kernel<T>, dim3((unsigned)nb), dim3(64, kThY, 1), 0, (hipStream_t)stream,
+            dim3 grd;
+            CHMY_TRY(line_grid((int64_t)nbx * nby * nch, 64 * kThY, &grd));
+            hipLaunchKernelGGL(thermal_step3_kernel<T>, grd, dim3(64, kThY, 1), 0, (hipStream_t)stream,
                                b, view<T>(*Tf), view<T>(*T_out), view<T>(*To), view<T>(V[0]), view<T>(V[1]),
                                view<T>(V[2]), view<T>(qT[0]), view<T>(qT[1]), view<T>(qT[2]), -T(lam), T(dt),
                                T(g->inv_spacing[0]), T(g->inv_spacing[1]), T(g->inv_spacing[2]), nbx, nby, kchunk);
             CHMY_HIP(hipGetLastError());
             return 0;
         }
-        dim3 grd = flat_grid(b);
+        dim3 grd;
+        CHMY_TRY(flat_grid(b, &grd));
         hipLaunchKernelGGL(thermal_step_kernel<T>, grd, blk2(), 0, (hipStream_t)stream, b, t, to, o, v0, v1, v2, q0,
                            q1, q2, g->nd, -T(lam), T(dt), T(g->inv_spacing[0]), T(g->inv_spacing[1]),
                            T(g->inv_spacing[2]));
@@ -986,9 +997,9 @@ int chmy_thermal_step2(const chmy_grid_t* g, const chmy_field_t* Tf, const chmy_
                 a.kchunk = k;
             }
         }
-        const int64_t nb = tiles * ((a.n[2] + a.kchunk - 1) / a.kchunk);
-        if (nb > INT32_MAX) return set_error(CHMY_E_SIZE, "thermal step: box too large");
-        hipLaunchKernelGGL(thermal_step2_kernel<T>, dim3((unsigned)nb), dim3(64, kTh2Y, 1), 0, (hipStream_t)stream, a);
+        dim3 grd;
+        CHMY_TRY(line_grid(tiles * ((a.n[2] + a.kchunk - 1) / a.kchunk), 64 * kTh2Y, &grd));
+        hipLaunchKernelGGL(thermal_step2_kernel<T>, grd, dim3(64, kTh2Y, 1), 0, (hipStream_t)stream, a);
         CHMY_HIP(hipGetLastError());
         return 0;
     };
@@ -1005,12 +1016,13 @@ int chmy_maxloc(const chmy_grid_t* g, const chmy_box_t* box, const chmy_field_t*
     Box3 b = box3(bx, g->nd);
     if (no_work(b)) return 0;
     hipStream_t s = (hipStream_t)stream;
+    dim3 grd;
+    CHMY_TRY(flat_grid(b, &grd));
     if (src->dtype == CHMY_F64)
-        hipLaunchKernelGGL(maxloc_kernel<double>, flat_grid(b), blk2(), 0, s, b, lview<double>(*dst),
-                           lview<double>(*src), g->nd);
+        hipLaunchKernelGGL(maxloc_kernel<double>, grd, blk2(), 0, s, b, lview<double>(*dst), lview<double>(*src),
+                           g->nd);
     else
-        hipLaunchKernelGGL(maxloc_kernel<float>, flat_grid(b), blk2(), 0, s, b, lview<float>(*dst),
-                           lview<float>(*src), g->nd);
+        hipLaunchKernelGGL(maxloc_kernel<float>, grd, blk2(), 0, s, b, lview<float>(*dst), lview<float>(*src), g->nd);
     CHMY_HIP(hipGetLastError());
     return 0;
 }

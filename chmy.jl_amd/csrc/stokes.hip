@@ -205,7 +205,9 @@ static int stress_launch(const chmy_grid_t* g, const chmy_box_t& bx, const chmy_
     a.dr = T(dr);
     Box3 b = box3(bx, nd);
     if (no_work(b)) return 0;
-    const dim3 blk(kFlat, 1, 1), grd = flat_grid(b);
+    const dim3 blk(kFlat, 1, 1);
+    dim3 grd;
+    CHMY_TRY(flat_grid(b, &grd));
     if (nd == 2) {
         if (eta) hipLaunchKernelGGL((stress_kernel<T, 2, true>), grd, blk, 0, s, b, a);
         else hipLaunchKernelGGL((stress_kernel<T, 2, false>), grd, blk, 0, s, b, a);
@@ -239,7 +241,9 @@ static int velocity_launch(const chmy_grid_t* g, const chmy_box_t& bx, const chm
     a.nu = T(nu);
     Box3 b = box3(bx, nd);
     if (no_work(b)) return 0;
-    const dim3 blk(kFlat, 1, 1), grd = flat_grid(b);
+    const dim3 blk(kFlat, 1, 1);
+    dim3 grd;
+    CHMY_TRY(flat_grid(b, &grd));
     if (nd == 2) {
         if (eml) hipLaunchKernelGGL((velocity_kernel<T, 2, true>), grd, blk, 0, s, b, a);
         else hipLaunchKernelGGL((velocity_kernel<T, 2, false>), grd, blk, 0, s, b, a);

@@ -182,7 +182,9 @@ static int residual_launch(const chmy_grid_t* g, const chmy_box_t& bx, const chm
     a.Gdt = T(G) * T(dt);
     Box3 b = box3(bx, nd);
     if (no_work(b)) return 0;
-    const dim3 blk(kFlat, 1, 1), grd = flat_grid(b);
+    const dim3 blk(kFlat, 1, 1);
+    dim3 grd;
+    CHMY_TRY(flat_grid(b, &grd));
     if (nd == 2 && eta) hipLaunchKernelGGL((residual_kernel<T, TO, 2, true>), grd, blk, 0, s, b, a);
     else if (nd == 2) hipLaunchKernelGGL((residual_kernel<T, TO, 2, false>), grd, blk, 0, s, b, a);
     else if (eta) hipLaunchKernelGGL((residual_kernel<T, TO, 3, true>), grd, blk, 0, s, b, a);
@@ -197,6 +199,8 @@ static int accumulate_launch(const chmy_grid_t* g, const chmy_box_t& bx, const c
                              const chmy_field_t* tauc, const chmy_field_t* Prc, hipStream_t s) {
     const Box3 b = box3(bx, g->nd);
     if (no_work(b)) return 0;
+    dim3 grd;
+    CHMY_TRY(flat_grid(b, &grd));
     auto go = [&](auto nd) {
         constexpr int ND = decltype(nd)::value, NT = ND == 2 ? 3 : 6;
         AccArgs<T, TO, ND + NT + 1> a;
@@ -204,7 +208,7 @@ static int accumulate_launch(const chmy_grid_t* g, const chmy_box_t& bx, const c
         for (int c = 0; c < NT; ++c) { a.x[ND + c] = view<T>(tau[c]); a.d[ND + c] = view<TO>(tauc[c]); }
         a.x[ND + NT] = view<T>(*Pr);
         a.d[ND + NT] = view<TO>(*Prc);
-        hipLaunchKernelGGL((accumulate_kernel<T, TO, ND + NT + 1>), flat_grid(b), dim3(kFlat, 1, 1), 0, s, b, a);
+        hipLaunchKernelGGL((accumulate_kernel<T, TO, ND + NT + 1>), grd, dim3(kFlat, 1, 1), 0, s, b, a);
     };
     if (g->nd == 2) go(std::integral_constant<int, 2>{});
     else go(std::integral_constant<int, 3>{});
