@@ -5,7 +5,7 @@ fails here."""
 import os
 import re
 
-from test_gpu_dispatch_shapes import PASS_SIZES
+from test_gpu_dispatch_shapes import ADJOINT_SIZES, FORWARD_SIZES, PASS_SIZES
 
 CSRC = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "chmy.jl_amd", "csrc")
 CUS, LANES = 256, 64
@@ -33,6 +33,36 @@ def pass_shape(dims):
     return "Dense2"
 
 
+def regions(n, rx, ry, rows):
+    return up(n[0], LANES - 2 * rx) * up(n[1], rows - 2 * ry)
+
+
+def constants(src):
+    return {k: int(v) for line in re.findall(r"^constexpr int (k\w+ = \d+(?:, k\w+ = \d+)*);", src, re.M)
+            for k, v in re.findall(r"(k\w+) = (\d+)", line)}
+
+
 def test_pass_sizes():
     for name, sizes in PASS_SIZES.items():
         assert [pass_shape(d) for d in sizes] == [name] * len(sizes)
+
+
+def test_adjoint_sizes():
+    src = source("sia.hip")
+    ring = constants(src)["kAdjRing"]
+    order = [tuple(map(int, m)) for m in re.findall(r"if \(fits\((\d+), (\d+)\)\) launch_adj_r<\1, \2, ", src)]
+    assert order + [(16, 3)] == list(ADJOINT_SIZES)
+    for want, sizes in ADJOINT_SIZES.items():
+        for n in sizes:
+            fit = [s for s in order if regions(n, 2 * ring, 2 * ring, s[0] * s[1]) +
+                   regions(n, 4, 4, s[0] * (s[1] + 1)) <= CUS]
+            assert (fit + [(16, 3)])[0] == want, n
+
+
+def test_forward_sizes():
+    c = constants(source("sia.hip"))
+    assert {c["kSiaMax"], c["kSiaMany"]} == set(FORWARD_SIZES)
+    for want, sizes in FORWARD_SIZES.items():
+        for n in sizes:
+            one = regions(n, 2 * c["kSiaMax"], 2 * c["kSiaMax"], c["kNWF"] * c["kRF2"]) <= CUS
+            assert (c["kSiaMax"] if one else c["kSiaMany"]) == want, n

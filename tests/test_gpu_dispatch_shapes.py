@@ -1,11 +1,16 @@
-"""Every shape that the 2D multi-iteration passes choose from by grid size,
-bitwise against single iterations.  The sizes are listed under the shape they reach; tests/test_dispatch_sizes.py
+"""Every shape that the 2D multi-iteration passes and the SIA launches choose
+from by grid size, bitwise against single iterations and single steps.  The
+sizes are listed under the shape they reach; tests/test_dispatch_sizes.py
 holds the lists to the shapes' constants in the sources."""
 import numpy as np
 import pytest
+import torch
 
 import chmy
+from chmy.sia import SIA
+from _helpers import dev
 from test_gpu_fused_pairs import GENERAL, _compare, _run
+from test_gpu_sia import _setup
 
 pytestmark = pytest.mark.gpu
 
@@ -15,6 +20,11 @@ PASS_SIZES = {"Small2": [(49, 3), (101, 66)],
               "Mid2": [(414, 378), (415, 379), (400, 380)],
               "Large2": [(478, 638), (481, 639)],
               "Dense2": [(862, 558), (863, 559)]}
+# adjoint pairs: waves and rows of a region
+ADJOINT_SIZES = {(8, 2): [(57, 11), (104, 52)], (12, 2): [(260, 180), (261, 181), (300, 200)], (16, 3): [(512, 437)]}
+# forward steps a launch may take
+FORWARD_SIZES = {5: [(250, 177)], 3: [(800, 520), (833, 541)]}
+
 
 @pytest.fixture(scope="module")
 def arch():
@@ -41,3 +51,36 @@ def test_passes_of_the_other_shapes_2d(arch, shape, dims, niter):
     a = _run(arch, g, np.float64, False, "field", None, GENERAL, niter, True, 41)
     b = _run(arch, g, np.float64, False, "field", None, GENERAL, niter, False, 41)
     _compare(a, b, f"{shape} dims {dims} niter {niter}")
+
+
+@pytest.mark.parametrize("npow", [3, 2])
+@pytest.mark.parametrize("n", sum(ADJOINT_SIZES.values(), []) + sum(FORWARD_SIZES.values(), []))
+def test_sia_gradient_over_shapes(arch, n, npow):
+    """Seven steps and two checkpoints: segments of four states and of three,
+    so that paired and single adjoint steps and riding steps mix.  The run
+    against the per-point step, the reverse sweep against the five gather
+    passes, bitwise."""
+    g, og, H, hH, B, hB, A, hA = _setup(arch, n=n, seed=23)
+    S = SIA(arch, g, hB.arr, logA=np.log(hA.arr), As=0.5, npow=npow, mb=(0.5, 0.3, 0.25))
+    dt = 1e-2 * min(e / m for e, m in zip(g.extent, n)) ** 2
+    dts = [dt * (1 + 0.1 * k) for k in range(7)]
+    want = [hH.arr.copy()]
+    S.reset(hH.arr)
+    for d in dts:
+        S.step(d)
+        S.H.swap(S.H2)
+        want.append(dev(S.H).copy())
+    S.reset(hH.arr)
+    S.forward(7, dts)
+    assert np.array_equal(dev(S.H), want[7]) and np.array_equal(dev(S.H2), want[6])
+    last = torch.from_numpy(want[7][2:-2, 2:-2].T.copy()).to(S.lam.data.device)
+    obs = last * 0.97
+    _, grad = S.gradient(hH.arr, obs, 7, dts, ncheck=2)
+    lam = S.lam.interior().clone()
+    for a in (S.grad, S.lam, S.lam2):
+        a.data.zero_()
+    S.lam.interior().copy_(last - obs)
+    for k in reversed(range(7)):
+        S.reset(want[k])
+        S._adjoint_step(S.H, dts[k], passes=5)
+    assert torch.equal(S.lam.interior(), lam) and torch.equal(S.grad.interior(), grad)
