@@ -151,6 +151,7 @@ int sia_scratch_ptr(void** p);
 struct Box3 {
     int64_t lo[3];
     int64_t len[3];
+    int32_t spread = 0;   // flat_at's order of blocks
 };
 inline Box3 box3(const chmy_box_t& b, int nd) {
     Box3 r;
@@ -195,22 +196,44 @@ __host__ __device__ __forceinline__ void plane_index(int64_t q, int64_t len0, in
 
 // Per-point kernels: blocks of 256 consecutive points of a plane (counted along
 // x and on into the next row, so no lane idles at a row's end), plane after
-// plane, each XCD a contiguous run of them: the planes and rows that a
-// neighbour's point shares are found in that XCD's L2.
+// plane.  Which XCD takes which blocks (ids congruent mod 8 go to one XCD)
+// depends on what the launch's arrays hold together:
+//  - up to the 256 MB cache behind the L2s, each XCD one contiguous run: the
+//    planes and rows that a neighbour's point shares are found in its L2;
+//  - beyond, runs of 32 blocks, so that the XCDs work side by side.  Eight runs
+//    far apart are eight places of HBM read and written at once, and a plane of
+//    every array is more than an L2 holds anyway.
+// Measured, FP64, us, 64 x 4 grid -> one run an XCD -> runs of 32: diffusion
+// step (5 arrays) 159x143x127 33 -> 23 -> 28, 207x191x175 (277 MB) 81 -> 93 -> 67,
+// 250^3 216 -> 237 -> 186, 400^3 842 -> 980 -> 750; compute_q (4 arrays)
+// 207x191x175 (221 MB) 59 -> 38 -> 42, 400^3 605 -> 690 -> 628; update_C
+// 1000x1000x60 497 -> 548 -> 487.  Runs of 16, 64 and 128: within 3% of 32,
+// 128 up to 9% slower (one step of chmy_diffusion_iterate, 250^3).
 constexpr int kFlat = 256;
-inline int flat_grid(const Box3& b, dim3* grd) {
+constexpr uint32_t kFlatRun = 32;
+constexpr int64_t kFlatCache = int64_t(256) << 20;
+// point_bytes: what a point of the box keeps in the caches, over all arrays
+// that the launch reads or writes (not those stored past them).
+inline int flat_grid(Box3& b, int64_t point_bytes, dim3* grd) {
     int64_t plane, nb;
     if (__builtin_mul_overflow(b.len[0], b.len[1], &plane) ||
         __builtin_mul_overflow(plane / kFlat + (plane % kFlat != 0), b.len[2], &nb))
         nb = INT64_MAX;
-    return line_grid(nb, kFlat, grd);
+    CHMY_TRY(line_grid(nb, kFlat, grd));
+    b.spread = nb * kFlat > kFlatCache / point_bytes;
+    return 0;
 }
 // Lane `lane` of block `bid` of nb: its point, or false.
 __host__ __device__ __forceinline__ bool flat_at(const Box3& b, uint32_t bid, uint32_t nb, uint32_t lane, int64_t& i,
                                                  int64_t& j, int64_t& k) {
     const uint32_t per = (uint32_t)((b.len[0] * b.len[1] + kFlat - 1) / kFlat);
-    // xcd_remap on unsigned ids
-    const uint32_t run = nb / 8, id = bid < 8 * run ? (bid % 8) * run + bid / 8 : bid;
+    uint32_t id = bid;   // the blocks past the last whole round of the XCDs keep theirs
+    if (b.spread) {
+        constexpr uint32_t G = 8 * kFlatRun;
+        if ((bid | (G - 1)) < nb) id = bid / G * G + bid % 8 * kFlatRun + bid % G / 8;
+    } else if (bid < nb / 8 * 8) {
+        id = bid % 8 * (nb / 8) + bid / 8;
+    }
     const uint32_t e = id / per;
     int64_t a, c;
     plane_index((int64_t)(id - e * per) * kFlat + lane, b.len[0], b.len[1], a, c);

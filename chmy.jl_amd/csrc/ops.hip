@@ -613,7 +613,7 @@ static int diffusion_launch(const chmy_grid_t* g, const chmy_box_t* box, const c
     DFL<T> q0 = lview<T>(q[0]);
     DFL<T> q1 = g->nd > 1 ? lview<T>(q[1]) : q0, q2 = g->nd > 2 ? lview<T>(q[2]) : q0;
     dim3 grd;
-    CHMY_TRY(flat_grid(b, &grd));
+    CHMY_TRY(flat_grid(b, (1 + g->nd) * sizeof(T), &grd));
     if (flux)
         hipLaunchKernelGGL(diffusion_flux_kernel<T>, grd, blk2(), 0, s, b, c, q0, q1, q2, g->nd, -T(scalar),
                            T(g->inv_spacing[0]), T(g->inv_spacing[1]), T(g->inv_spacing[2]));
@@ -708,7 +708,7 @@ static int copy_launch(const chmy_grid_t* g, const chmy_box_t& bx, const chmy_fi
     Box3 b = box3(bx, g->nd);
     if (no_work(b)) return 0;
     dim3 grd;
-    CHMY_TRY(flat_grid(b, &grd));
+    CHMY_TRY(flat_grid(b, 2 * c.n * sizeof(T), &grd));
     hipLaunchKernelGGL(copy_kernel<T>, grd, blk2(), 0, s, b, c);
     CHMY_HIP(hipGetLastError());
     return 0;
@@ -723,7 +723,7 @@ static int thermal_launch(const chmy_grid_t* g, const chmy_box_t& bx, const chmy
     DFL<T> q0 = lview<T>(q[0]);
     DFL<T> q1 = g->nd > 1 ? lview<T>(q[1]) : q0, q2 = g->nd > 2 ? lview<T>(q[2]) : q0;
     dim3 grd;
-    CHMY_TRY(flat_grid(b, &grd));
+    CHMY_TRY(flat_grid(b, (flux ? 1 + 2 * g->nd : 2 + g->nd) * sizeof(T), &grd));
     if (flux) {
         DFL<T> v1 = g->nd > 1 ? lview<T>(other[1]) : o, v2 = g->nd > 2 ? lview<T>(other[2]) : o;
         hipLaunchKernelGGL(thermal_flux_kernel<T>, grd, blk2(), 0, s, b, t, o, v1, v2, q0, q1, q2, g->nd, -T(scalar),
@@ -777,7 +777,7 @@ int chmy_diffusion_step(const chmy_grid_t* g, const chmy_box_t* box, const chmy_
         DFL<T> q0 = lview<T>(q[0]);
         DFL<T> q1 = g->nd > 1 ? lview<T>(q[1]) : q0, q2 = g->nd > 2 ? lview<T>(q[2]) : q0;
         dim3 grd;
-        CHMY_TRY(flat_grid(b, &grd));
+        CHMY_TRY(flat_grid(b, (2 + g->nd) * sizeof(T), &grd));
         hipLaunchKernelGGL(diffusion_step_kernel<T>, grd, blk2(), 0, (hipStream_t)stream, b, c, co, q0, q1, q2,
                            g->nd, -T(chi), T(dt), T(g->inv_spacing[0]), T(g->inv_spacing[1]),
                            T(g->inv_spacing[2]));
@@ -837,7 +837,7 @@ int chmy_diffusion_iterate(const chmy_grid_t* g, const chmy_field_t* C0, const c
             DFL<T> q0 = lview<T>(q[0]);
             DFL<T> q1 = g->nd > 1 ? lview<T>(q[1]) : q0, q2 = g->nd > 2 ? lview<T>(q[2]) : q0;
             dim3 grd;
-            CHMY_TRY(flat_grid(reg, &grd));
+            CHMY_TRY(flat_grid(reg, (2 + g->nd) * sizeof(T), &grd));
             int it = 0;
             CHMY_TRY(diffusion_passes<T>(g, C0, C1, rules, chi, dt, niter, &p, &it, (hipStream_t)stream));
             for (; it < niter; ++it) {
@@ -947,7 +947,7 @@ int chmy_thermal_step(const chmy_grid_t* g, const chmy_box_t* box, const chmy_fi
             return 0;
         }
         dim3 grd;
-        CHMY_TRY(flat_grid(b, &grd));
+        CHMY_TRY(flat_grid(b, (3 + 2 * g->nd) * sizeof(T), &grd));
         hipLaunchKernelGGL(thermal_step_kernel<T>, grd, blk2(), 0, (hipStream_t)stream, b, t, to, o, v0, v1, v2, q0,
                            q1, q2, g->nd, -T(lam), T(dt), T(g->inv_spacing[0]), T(g->inv_spacing[1]),
                            T(g->inv_spacing[2]));
@@ -1017,7 +1017,7 @@ int chmy_maxloc(const chmy_grid_t* g, const chmy_box_t* box, const chmy_field_t*
     if (no_work(b)) return 0;
     hipStream_t s = (hipStream_t)stream;
     dim3 grd;
-    CHMY_TRY(flat_grid(b, &grd));
+    CHMY_TRY(flat_grid(b, 2 * (src->dtype == CHMY_F64 ? 8 : 4), &grd));
     if (src->dtype == CHMY_F64)
         hipLaunchKernelGGL(maxloc_kernel<double>, grd, blk2(), 0, s, b, lview<double>(*dst), lview<double>(*src),
                            g->nd);

@@ -207,7 +207,7 @@ static int stress_launch(const chmy_grid_t* g, const chmy_box_t& bx, const chmy_
     if (no_work(b)) return 0;
     const dim3 blk(kFlat, 1, 1);
     dim3 grd;
-    CHMY_TRY(flat_grid(b, &grd));
+    CHMY_TRY(flat_grid(b, (1 + nd + 2 * (nd == 2 ? 3 : 6) + (eta ? 1 : 0)) * sizeof(T), &grd));
     if (nd == 2) {
         if (eta) hipLaunchKernelGGL((stress_kernel<T, 2, true>), grd, blk, 0, s, b, a);
         else hipLaunchKernelGGL((stress_kernel<T, 2, false>), grd, blk, 0, s, b, a);
@@ -243,7 +243,7 @@ static int velocity_launch(const chmy_grid_t* g, const chmy_box_t& bx, const chm
     if (no_work(b)) return 0;
     const dim3 blk(kFlat, 1, 1);
     dim3 grd;
-    CHMY_TRY(flat_grid(b, &grd));
+    CHMY_TRY(flat_grid(b, (1 + nd + (nd == 2 ? 3 : 6) + (eml ? 1 : 0) + (rg ? 1 : 0)) * sizeof(T), &grd));
     if (nd == 2) {
         if (eml) hipLaunchKernelGGL((velocity_kernel<T, 2, true>), grd, blk, 0, s, b, a);
         else hipLaunchKernelGGL((velocity_kernel<T, 2, false>), grd, blk, 0, s, b, a);

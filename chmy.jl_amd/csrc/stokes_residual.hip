@@ -184,7 +184,8 @@ static int residual_launch(const chmy_grid_t* g, const chmy_box_t& bx, const chm
     if (no_work(b)) return 0;
     const dim3 blk(kFlat, 1, 1);
     dim3 grd;
-    CHMY_TRY(flat_grid(b, &grd));
+    const int64_t point = (1 + nd + 2 * nt + (eta ? 1 : 0) + (dV ? 1 + nd : 0)) * sizeof(T) + (1 + nd + nt) * sizeof(TO);
+    CHMY_TRY(flat_grid(b, point, &grd));
     if (nd == 2 && eta) hipLaunchKernelGGL((residual_kernel<T, TO, 2, true>), grd, blk, 0, s, b, a);
     else if (nd == 2) hipLaunchKernelGGL((residual_kernel<T, TO, 2, false>), grd, blk, 0, s, b, a);
     else if (eta) hipLaunchKernelGGL((residual_kernel<T, TO, 3, true>), grd, blk, 0, s, b, a);
@@ -197,10 +198,10 @@ template <class T, class TO>
 static int accumulate_launch(const chmy_grid_t* g, const chmy_box_t& bx, const chmy_field_t* V,
                              const chmy_field_t* tau, const chmy_field_t* Pr, const chmy_field_t* Vc,
                              const chmy_field_t* tauc, const chmy_field_t* Prc, hipStream_t s) {
-    const Box3 b = box3(bx, g->nd);
+    Box3 b = box3(bx, g->nd);
     if (no_work(b)) return 0;
     dim3 grd;
-    CHMY_TRY(flat_grid(b, &grd));
+    CHMY_TRY(flat_grid(b, (1 + g->nd + (g->nd == 2 ? 3 : 6)) * (sizeof(T) + sizeof(TO)), &grd));
     auto go = [&](auto nd) {
         constexpr int ND = decltype(nd)::value, NT = ND == 2 ? 3 : 6;
         AccArgs<T, TO, ND + NT + 1> a;

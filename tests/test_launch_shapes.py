@@ -1,7 +1,7 @@
 """Grids of the per-point kernels, on the host: HIP launches fewer than 2^32
 work-items in one grid dimension, so longer lines of blocks are folded; every
-tile of a box must still belong to exactly one block, and blocks without one
-must see no point.  A host program includes the library's own launch header
+tile of a box must still belong to exactly one block, in either order of the
+blocks over the XCDs, and blocks without one must see no point.  A host program includes the library's own launch header
 and walks all block ids."""
 import os
 import shutil
@@ -24,11 +24,13 @@ using namespace chmy;
     (long long)b.len[0], (long long)b.len[1], (long long)b.len[2]); std::exit(1); } } while (0)
 static Box3 box(int64_t x, int64_t y, int64_t z) { return Box3{{0, 3, 1}, {x, y, z}}; }
 
-// every block id of the box's grid: the tile that its lane 0 names (all lanes when `lanes`)
-static void walk(int64_t x, int64_t y, int64_t z, bool lanes) {
+// every block id of the box's grid: the tile that its lane 0 names (all lanes
+// when `lanes`), in either order of the blocks
+static void walk(int64_t x, int64_t y, int64_t z, bool lanes, bool spread) {
     Box3 b = box(x, y, z);
     dim3 g;
-    CHECK(flat_grid(b, &g) == 0);
+    CHECK(flat_grid(b, 8, &g) == 0);
+    b.spread = spread;
     CHECK((uint64_t)g.x * kFlat < (1ull << 32) && g.y < 65536 && g.z == 1);
     const uint64_t n = (uint64_t)g.x * g.y, per = (uint64_t)((x * y + kFlat - 1) / kFlat);
     CHECK(n >= per * z && (g.y == 1 || g.x % 8 == 0));
@@ -64,13 +66,16 @@ static void walk(int64_t x, int64_t y, int64_t z, bool lanes) {
 int main() {
     for (int64_t x : {1, 3, 255, 256, 257, 700})
         for (int64_t y : {1, 2, 9})
-            for (int64_t z : {1, 4, 33}) walk(x, y, z, true);
-    walk(65535, 65536, 1, false);        // 2^32 - 2^16 points
-    walk(65536, 65536, 1, false);        // 2^32, the 64-bit division
-    walk(1626, 1626, 1626, false);
-    walk(1626, 1627, 1626, false);
-    walk(3, 2, 16777217, false);         // a block a plane
-    walk((int64_t(1) << 32) + 5, 1, 1, false);
+            for (int64_t z : {1, 4, 33, 600})
+                for (bool spread : {false, true}) walk(x, y, z, z < 600, spread);
+    for (bool spread : {false, true}) {
+        walk(65535, 65536, 1, false, spread);        // 2^32 - 2^16 points
+        walk(65536, 65536, 1, false, spread);        // 2^32, the 64-bit division
+        walk(1626, 1626, 1626, false, spread);
+        walk(1626, 1627, 1626, false, spread);
+        walk(3, 2, 16777217, false, spread);         // a block a plane
+        walk((int64_t(1) << 32) + 5, 1, 1, false, spread);
+    }
     for (int threads : {64, 256, 768, 1024})
         for (int64_t nb : {int64_t(1), int64_t(1) << 22, (int64_t(1) << 24) - 1, int64_t(1) << 24, (int64_t(1) << 26) + 1, kLineMost}) {
             Box3 b = box(nb, threads, 0);
@@ -81,12 +86,14 @@ int main() {
             CHECK((uint64_t)g.x * g.y < (1ull << 31));
         }
     dim3 g;
-    Box3 b = box(0, 0, 0);
+    Box3 b = box(256, 4, 1024);   // 2^20 points: 256 bytes each are the cache's size
+    CHECK(flat_grid(b, 256, &g) == 0 && !b.spread && flat_grid(b, 257, &g) == 0 && b.spread);
+    b = box(0, 0, 0);
     CHECK(line_grid(kLineMost + 1, 64, &g) == CHMY_E_SIZE);
     b = box(int64_t(1) << 30, int64_t(1) << 30, 1);
-    CHECK(flat_grid(b, &g) == CHMY_E_SIZE);
+    CHECK(flat_grid(b, 8, &g) == CHMY_E_SIZE);
     b = box(int64_t(1) << 40, int64_t(1) << 40, 3);
-    CHECK(flat_grid(b, &g) == CHMY_E_SIZE);
+    CHECK(flat_grid(b, 8, &g) == CHMY_E_SIZE);
     std::printf("ok\n");
     return 0;
 }
