@@ -62,18 +62,6 @@ struct DF {
     __device__ __forceinline__ T& at(int64_t o) const { return p[o]; }
 };
 
-// Same, carrying locations and dimensionality for the generic operators.
-template <class T>
-struct DFL {
-    T* p;
-    int64_t st[3];
-    int32_t loc[3];
-    int32_t nd;
-    __device__ __forceinline__ T& operator()(int64_t i, int64_t j, int64_t k) const {
-        return p[i * st[0] + j * st[1] + k * st[2]];
-    }
-};
-
 inline int64_t pad_of(const chmy_field_t& f, int d) { return f.n[d] + 4 * (int64_t)f.halo[d]; }
 
 template <class T>
@@ -87,19 +75,6 @@ DF<T> view(const chmy_field_t& f) {
     if (f.nd >= 2) off += (2 * (int64_t)f.halo[1] - 1) * v.sy;
     if (f.nd >= 3) off += (2 * (int64_t)f.halo[2] - 1) * v.sz;
     v.p = static_cast<T*>(f.data) + off;
-    return v;
-}
-
-template <class T>
-DFL<T> lview(const chmy_field_t& f) {
-    DFL<T> v;
-    DF<T> b = view<T>(f);
-    v.p = b.p;
-    v.st[0] = 1;
-    v.st[1] = b.sy;
-    v.st[2] = b.sz;
-    for (int d = 0; d < 3; ++d) v.loc[d] = d < f.nd ? f.loc[d] : 0;
-    v.nd = f.nd;
     return v;
 }
 

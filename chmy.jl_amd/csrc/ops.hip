@@ -2,9 +2,13 @@
 // the viscosity max-neighbourhood.  Each thread owns one logical index I of the
 // box, 256 consecutive points of a plane a block (flat_point).  These are
 // bandwidth-bound streaming kernels; the fused Stokes iteration lives in
-// stokes_fused.hip.  159x143x127 FP64, us, 64 x 4 blocks -> flat ones: thermal
-// flux 37.5 -> 31, update 34 -> 28.6, update_old! (loads before stores) 69 -> 60;
-// a diffusion step through the Launcher at 160x150x140 111 -> 94.
+// stokes_fused.hip.  In FP32 on large boxes the address arithmetic bounds them
+// too, so the views carry a unit x stride (a 64-bit product a point and array
+// less): us, 64 x 4 blocks -> flat ones -> with unit strides, a step of
+// chmy_diffusion_iterate FP32 3000^2 44.2 -> 48.2 -> 43.4, 400^3 728 -> 777 ->
+// 710; compute_q FP64 400^3 606 -> 630 -> 597.  159x143x127 FP64: thermal flux
+// 36.2 -> 25.8 -> 25.9, update 26.8 -> 19.8 -> 19.3, update_old! (loads before
+// stores) 69 -> 62, a step of the loop 44.4 -> 35 -> 33.7.
 #include <cstring>
 
 #include "stokes_pt.hpp"
@@ -22,14 +26,14 @@ __device__ __forceinline__ Ix3 box_index(const Box3& b, bool& ok) {
 }
 
 template <class T>
-__device__ __forceinline__ T& g_at(const DFL<T>& f, Ix3 I) { return f(I.i, I.j, I.k); }
+__device__ __forceinline__ T& g_at(const DF<T>& f, Ix3 I) { return f(I.i, I.j, I.k); }
 __device__ __forceinline__ Ix3 sh(Ix3 I, int d, int64_t s) {
     if (d == 0) I.i += s; else if (d == 1) I.j += s; else I.k += s;
     return I;
 }
 // ------------------------------------------------------------------ diffusion
 template <class T>
-__global__ void __launch_bounds__(256) diffusion_flux_kernel(Box3 b, DFL<T> C, DFL<T> q0, DFL<T> q1, DFL<T> q2,
+__global__ void __launch_bounds__(256) diffusion_flux_kernel(Box3 b, DF<T> C, DF<T> q0, DF<T> q1, DF<T> q2,
                                                              int nd, T nchi, T i0, T i1, T i2) {
     bool ok;
     Ix3 I = box_index(b, ok);
@@ -41,7 +45,7 @@ __global__ void __launch_bounds__(256) diffusion_flux_kernel(Box3 b, DFL<T> C, D
 }
 
 template <class T>
-__global__ void __launch_bounds__(256) diffusion_update_kernel(Box3 b, DFL<T> C, DFL<T> q0, DFL<T> q1, DFL<T> q2,
+__global__ void __launch_bounds__(256) diffusion_update_kernel(Box3 b, DF<T> C, DF<T> q0, DF<T> q1, DF<T> q2,
                                                                int nd, T dt, T i0, T i1, T i2) {
     bool ok;
     Ix3 I = box_index(b, ok);
@@ -62,8 +66,8 @@ __global__ void __launch_bounds__(256) diffusion_update_kernel(Box3 b, DFL<T> C,
 // compute_q! stores it), q_D at I+e recomputed when I+e is in the box, else
 // read from q's storage; C[I] - Δt divg(q)[I].
 template <class T>
-__device__ __forceinline__ T diffusion_value(const Box3& b, const DFL<T>& C, const DFL<T>& q0, const DFL<T>& q1,
-                                             const DFL<T>& q2, int nd, T nchi, T dt, const T* isp, Ix3 I,
+__device__ __forceinline__ T diffusion_value(const Box3& b, const DF<T>& C, const DF<T>& q0, const DF<T>& q1,
+                                             const DF<T>& q2, int nd, T nchi, T dt, const T* isp, Ix3 I,
                                              bool store_q) {
     const T c = g_at(C, I);
     const int64_t hi[3] = {b.lo[0] + b.len[0], b.lo[1] + b.len[1], b.lo[2] + b.len[2]};
@@ -72,7 +76,7 @@ __device__ __forceinline__ T diffusion_value(const Box3& b, const DFL<T>& C, con
 #pragma unroll
     for (int d = 0; d < 3; ++d) {
         if (d >= nd) break;
-        const DFL<T>& qd = d == 0 ? q0 : (d == 1 ? q1 : q2);
+        const DF<T>& qd = d == 0 ? q0 : (d == 1 ? q1 : q2);
         const T ql = nchi * ((c - g_at(C, sh(I, d, -1))) * isp[d]);
         if (store_q) g_at(qd, I) = ql;
         const Ix3 J = sh(I, d, 1);
@@ -84,8 +88,8 @@ __device__ __forceinline__ T diffusion_value(const Box3& b, const DFL<T>& C, con
 }
 
 template <class T>
-__global__ void __launch_bounds__(256) diffusion_step_kernel(Box3 b, DFL<T> C, DFL<T> Co, DFL<T> q0, DFL<T> q1,
-                                                             DFL<T> q2, int nd, T nchi, T dt, T i0, T i1, T i2) {
+__global__ void __launch_bounds__(256) diffusion_step_kernel(Box3 b, DF<T> C, DF<T> Co, DF<T> q0, DF<T> q1,
+                                                             DF<T> q2, int nd, T nchi, T dt, T i0, T i1, T i2) {
     bool ok;
     Ix3 I = box_index(b, ok);
     if (!ok) return;
@@ -111,8 +115,8 @@ struct SideRules {
 // each writing dim's rule from the highest to the lowest, the batch's own fma
 // steps.  q is stored on the box as the step stores it.
 template <class T>
-__global__ void __launch_bounds__(256) diffusion_step_bc_kernel(Box3 box, Box3 reg, DFL<T> C, DFL<T> Co, DFL<T> q0,
-                                                                DFL<T> q1, DFL<T> q2, int nd, T nchi, T dt, T i0,
+__global__ void __launch_bounds__(256) diffusion_step_bc_kernel(Box3 box, Box3 reg, DF<T> C, DF<T> Co, DF<T> q0,
+                                                                DF<T> q1, DF<T> q2, int nd, T nchi, T dt, T i0,
                                                                 T i1, T i2, SideRules r) {
     bool ok;
     const Ix3 P = box_index(reg, ok);
@@ -316,7 +320,7 @@ __global__ void __launch_bounds__(NT) diffusion_tile_kernel(const DiffTile<T> p)
 // ------------------------------------------------------------------ update_old!
 template <class T>
 struct Copy7 {
-    DFL<T> src[7], dst[7];
+    DF<T> src[7], dst[7];
     int n;
 };
 
@@ -336,8 +340,8 @@ __global__ void __launch_bounds__(256) copy_kernel(Box3 b, Copy7<T> c) {
 
 // ------------------------------------------------------------------ thermal
 template <class T>
-__global__ void __launch_bounds__(256) thermal_flux_kernel(Box3 b, DFL<T> Tf, DFL<T> V0, DFL<T> V1, DFL<T> V2,
-                                                           DFL<T> q0, DFL<T> q1, DFL<T> q2, int nd, T nlam, T i0,
+__global__ void __launch_bounds__(256) thermal_flux_kernel(Box3 b, DF<T> Tf, DF<T> V0, DF<T> V1, DF<T> V2,
+                                                           DF<T> q0, DF<T> q1, DF<T> q2, int nd, T nlam, T i0,
                                                            T i1, T i2) {
     bool ok;
     Ix3 I = box_index(b, ok);
@@ -347,8 +351,8 @@ __global__ void __launch_bounds__(256) thermal_flux_kernel(Box3 b, DFL<T> Tf, DF
 #pragma unroll
     for (int d = 0; d < 3; ++d) {   // constant indices once unrolled: no stack arrays
         if (d >= nd) break;
-        const DFL<T>& Vd = d == 0 ? V0 : (d == 1 ? V1 : V2);
-        const DFL<T>& qd = d == 0 ? q0 : (d == 1 ? q1 : q2);
+        const DF<T>& Vd = d == 0 ? V0 : (d == 1 ? V1 : V2);
+        const DF<T>& qd = d == 0 ? q0 : (d == 1 ? q1 : q2);
         // qT_D = ((-λ ∂_D T) + max(V_D,0) left_D T) + min(V_D,0) right_D T
         // (stokes_3d_inc_ve_T.jl:59-71); T Center: left = T[I-e], right = T[I]
         const T tl = g_at(Tf, sh(I, d, -1));
@@ -363,8 +367,8 @@ __global__ void __launch_bounds__(256) thermal_flux_kernel(Box3 b, DFL<T> Tf, DF
 // read from qT's storage; T_out[I] = T_old[I] - Δt divg(qT)[I].  T and T_out
 // are distinct buffers.
 template <class T>
-__global__ void __launch_bounds__(256) thermal_step_kernel(Box3 b, DFL<T> Tf, DFL<T> Tout, DFL<T> To, DFL<T> V0,
-                                                           DFL<T> V1, DFL<T> V2, DFL<T> q0, DFL<T> q1, DFL<T> q2,
+__global__ void __launch_bounds__(256) thermal_step_kernel(Box3 b, DF<T> Tf, DF<T> Tout, DF<T> To, DF<T> V0,
+                                                           DF<T> V1, DF<T> V2, DF<T> q0, DF<T> q1, DF<T> q2,
                                                            int nd, T nlam, T dt, T i0, T i1, T i2) {
     bool ok;
     Ix3 I = box_index(b, ok);
@@ -377,8 +381,8 @@ __global__ void __launch_bounds__(256) thermal_step_kernel(Box3 b, DFL<T> Tf, DF
 #pragma unroll
     for (int d = 0; d < 3; ++d) {
         if (d >= nd) break;
-        const DFL<T>& Vd = d == 0 ? V0 : (d == 1 ? V1 : V2);
-        const DFL<T>& qd = d == 0 ? q0 : (d == 1 ? q1 : q2);
+        const DF<T>& Vd = d == 0 ? V0 : (d == 1 ? V1 : V2);
+        const DF<T>& qd = d == 0 ? q0 : (d == 1 ? q1 : q2);
         const T tl = g_at(Tf, sh(I, d, -1));
         const T v = g_at(Vd, I);
         const T ql = (nlam * ((tc - tl) * isp[d]) + jmax0(v) * tl) + jmin0(v) * tc;
@@ -574,8 +578,8 @@ __global__ void __launch_bounds__(64 * kTh2Y) thermal_step2_kernel(Thermal2<T> a
 }
 
 template <class T>
-__global__ void __launch_bounds__(256) thermal_update_kernel(Box3 b, DFL<T> Tf, DFL<T> To, DFL<T> q0, DFL<T> q1,
-                                                             DFL<T> q2, int nd, T dt, T i0, T i1, T i2) {
+__global__ void __launch_bounds__(256) thermal_update_kernel(Box3 b, DF<T> Tf, DF<T> To, DF<T> q0, DF<T> q1,
+                                                             DF<T> q2, int nd, T dt, T i0, T i1, T i2) {
     bool ok;
     Ix3 I = box_index(b, ok);
     if (!ok) return;
@@ -587,7 +591,7 @@ __global__ void __launch_bounds__(256) thermal_update_kernel(Box3 b, DFL<T> Tf, 
 
 // ------------------------------------------------------------------ maxloc
 template <class T>
-__global__ void __launch_bounds__(256) maxloc_kernel(Box3 b, DFL<T> dst, DFL<T> src, int nd) {
+__global__ void __launch_bounds__(256) maxloc_kernel(Box3 b, DF<T> dst, DF<T> src, int nd) {
     bool ok;
     Ix3 I = box_index(b, ok);
     if (!ok) return;
@@ -609,9 +613,9 @@ static int diffusion_launch(const chmy_grid_t* g, const chmy_box_t* box, const c
     CHMY_TRY(check_box(g, box, &bx));
     Box3 b = box3(bx, g->nd);
     if (no_work(b)) return 0;
-    DFL<T> c = lview<T>(*Cf);
-    DFL<T> q0 = lview<T>(q[0]);
-    DFL<T> q1 = g->nd > 1 ? lview<T>(q[1]) : q0, q2 = g->nd > 2 ? lview<T>(q[2]) : q0;
+    DF<T> c = view<T>(*Cf);
+    DF<T> q0 = view<T>(q[0]);
+    DF<T> q1 = g->nd > 1 ? view<T>(q[1]) : q0, q2 = g->nd > 2 ? view<T>(q[2]) : q0;
     dim3 grd;
     CHMY_TRY(flat_grid(b, (1 + g->nd) * sizeof(T), &grd));
     if (flux)
@@ -703,8 +707,8 @@ static int copy_launch(const chmy_grid_t* g, const chmy_box_t& bx, const chmy_fi
     Copy7<T> c;
     int nt = g->nd == 2 ? 3 : 6;
     c.n = 0;
-    if (Tf) { c.src[c.n] = lview<T>(*Tf); c.dst[c.n] = lview<T>(*To); ++c.n; }
-    for (int q = 0; q < nt; ++q) { c.src[c.n] = lview<T>(tau[q]); c.dst[c.n] = lview<T>(tauo[q]); ++c.n; }
+    if (Tf) { c.src[c.n] = view<T>(*Tf); c.dst[c.n] = view<T>(*To); ++c.n; }
+    for (int q = 0; q < nt; ++q) { c.src[c.n] = view<T>(tau[q]); c.dst[c.n] = view<T>(tauo[q]); ++c.n; }
     Box3 b = box3(bx, g->nd);
     if (no_work(b)) return 0;
     dim3 grd;
@@ -719,13 +723,13 @@ static int thermal_launch(const chmy_grid_t* g, const chmy_box_t& bx, const chmy
                           const chmy_field_t* other, double scalar, bool flux, hipStream_t s) {
     Box3 b = box3(bx, g->nd);
     if (no_work(b)) return 0;
-    DFL<T> t = lview<T>(*Tf), o = lview<T>(other[0]);
-    DFL<T> q0 = lview<T>(q[0]);
-    DFL<T> q1 = g->nd > 1 ? lview<T>(q[1]) : q0, q2 = g->nd > 2 ? lview<T>(q[2]) : q0;
+    DF<T> t = view<T>(*Tf), o = view<T>(other[0]);
+    DF<T> q0 = view<T>(q[0]);
+    DF<T> q1 = g->nd > 1 ? view<T>(q[1]) : q0, q2 = g->nd > 2 ? view<T>(q[2]) : q0;
     dim3 grd;
     CHMY_TRY(flat_grid(b, (flux ? 1 + 2 * g->nd : 2 + g->nd) * sizeof(T), &grd));
     if (flux) {
-        DFL<T> v1 = g->nd > 1 ? lview<T>(other[1]) : o, v2 = g->nd > 2 ? lview<T>(other[2]) : o;
+        DF<T> v1 = g->nd > 1 ? view<T>(other[1]) : o, v2 = g->nd > 2 ? view<T>(other[2]) : o;
         hipLaunchKernelGGL(thermal_flux_kernel<T>, grd, blk2(), 0, s, b, t, o, v1, v2, q0, q1, q2, g->nd, -T(scalar),
                            T(g->inv_spacing[0]), T(g->inv_spacing[1]), T(g->inv_spacing[2]));
     } else {
@@ -773,9 +777,9 @@ int chmy_diffusion_step(const chmy_grid_t* g, const chmy_box_t* box, const chmy_
     if (no_work(b)) return 0;
     auto launch = [&](auto zero) -> int {
         using T = decltype(zero);
-        DFL<T> c = lview<T>(*C), co = lview<T>(*C_out);
-        DFL<T> q0 = lview<T>(q[0]);
-        DFL<T> q1 = g->nd > 1 ? lview<T>(q[1]) : q0, q2 = g->nd > 2 ? lview<T>(q[2]) : q0;
+        DF<T> c = view<T>(*C), co = view<T>(*C_out);
+        DF<T> q0 = view<T>(q[0]);
+        DF<T> q1 = g->nd > 1 ? view<T>(q[1]) : q0, q2 = g->nd > 2 ? view<T>(q[2]) : q0;
         dim3 grd;
         CHMY_TRY(flat_grid(b, (2 + g->nd) * sizeof(T), &grd));
         hipLaunchKernelGGL(diffusion_step_kernel<T>, grd, blk2(), 0, (hipStream_t)stream, b, c, co, q0, q1, q2,
@@ -833,9 +837,9 @@ int chmy_diffusion_iterate(const chmy_grid_t* g, const chmy_field_t* C0, const c
         for (int d = 0; d < g->nd; ++d) reg.len[d] = b.len[d] + 1;   // [0, n+2]
         auto run = [&](auto zero) -> int {
             using T = decltype(zero);
-            DFL<T> c[2] = {lview<T>(*C0), lview<T>(*C1)};
-            DFL<T> q0 = lview<T>(q[0]);
-            DFL<T> q1 = g->nd > 1 ? lview<T>(q[1]) : q0, q2 = g->nd > 2 ? lview<T>(q[2]) : q0;
+            DF<T> c[2] = {view<T>(*C0), view<T>(*C1)};
+            DF<T> q0 = view<T>(q[0]);
+            DF<T> q1 = g->nd > 1 ? view<T>(q[1]) : q0, q2 = g->nd > 2 ? view<T>(q[2]) : q0;
             dim3 grd;
             CHMY_TRY(flat_grid(reg, (2 + g->nd) * sizeof(T), &grd));
             int it = 0;
@@ -919,10 +923,10 @@ int chmy_thermal_step(const chmy_grid_t* g, const chmy_box_t* box, const chmy_fi
     if (no_work(b)) return 0;
     auto launch = [&](auto zero) -> int {
         using T = decltype(zero);
-        DFL<T> t = lview<T>(*Tf), to = lview<T>(*T_out), o = lview<T>(*To);
-        DFL<T> v0 = lview<T>(V[0]), q0 = lview<T>(qT[0]);
-        DFL<T> v1 = g->nd > 1 ? lview<T>(V[1]) : v0, v2 = g->nd > 2 ? lview<T>(V[2]) : v0;
-        DFL<T> q1 = g->nd > 1 ? lview<T>(qT[1]) : q0, q2 = g->nd > 2 ? lview<T>(qT[2]) : q0;
+        DF<T> t = view<T>(*Tf), to = view<T>(*T_out), o = view<T>(*To);
+        DF<T> v0 = view<T>(V[0]), q0 = view<T>(qT[0]);
+        DF<T> v1 = g->nd > 1 ? view<T>(V[1]) : v0, v2 = g->nd > 2 ? view<T>(V[2]) : v0;
+        DF<T> q1 = g->nd > 1 ? view<T>(qT[1]) : q0, q2 = g->nd > 2 ? view<T>(qT[2]) : q0;
         // 3D with one stride set per location (Center; each V_D with qT_D): the z-march
         bool march = g->nd == 3;
         if (march) {
@@ -1019,10 +1023,10 @@ int chmy_maxloc(const chmy_grid_t* g, const chmy_box_t* box, const chmy_field_t*
     dim3 grd;
     CHMY_TRY(flat_grid(b, 2 * (src->dtype == CHMY_F64 ? 8 : 4), &grd));
     if (src->dtype == CHMY_F64)
-        hipLaunchKernelGGL(maxloc_kernel<double>, grd, blk2(), 0, s, b, lview<double>(*dst), lview<double>(*src),
+        hipLaunchKernelGGL(maxloc_kernel<double>, grd, blk2(), 0, s, b, view<double>(*dst), view<double>(*src),
                            g->nd);
     else
-        hipLaunchKernelGGL(maxloc_kernel<float>, grd, blk2(), 0, s, b, lview<float>(*dst), lview<float>(*src), g->nd);
+        hipLaunchKernelGGL(maxloc_kernel<float>, grd, blk2(), 0, s, b, view<float>(*dst), view<float>(*src), g->nd);
     CHMY_HIP(hipGetLastError());
     return 0;
 }
