@@ -152,7 +152,8 @@ inline int line_grid(int64_t nb, int threads, dim3* grd) {
     *grd = one ? dim3((unsigned)nb, 1, 1) : dim3((unsigned)kLineRow, (unsigned)((nb + kLineRow - 1) / kLineRow), 1);
     return 0;
 }
-__device__ __forceinline__ uint32_t line_id() { return blockIdx.y * gridDim.x + blockIdx.x; }
+// (rows have kLineRow blocks whenever there are several: no read of the grid's size)
+__device__ __forceinline__ uint32_t line_id() { return blockIdx.y * (uint32_t)kLineRow + blockIdx.x; }
 __device__ __forceinline__ uint32_t line_ids() { return gridDim.y * gridDim.x; }
 
 // The q-th point of a plane of rows of len0 points, counted along the rows:
