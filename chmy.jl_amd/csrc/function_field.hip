@@ -22,7 +22,8 @@
 //  - each operation runs on 4 (8 slots) or 2 (16 slots) planes at once, which
 //    shares its decoding and gives independent work to overlap.
 // Programs that need more slots keep the file in LDS; those, and the ones that
-// call sin, cos, tanh or pow, whose code is large, run one plane at a time.
+// call sin, cos, tanh or pow, whose code is large, run one plane at a time (two
+// runs of a line: 141 VGPRs).
 //  - sums, products, negations and squares become FMA with constant operands
 //    that give the same bits, so most operations take the first branch.
 // Bound by instruction issue: per operation and 4 planes about 65 vector and 83
@@ -43,6 +44,7 @@
 // pow are the device math library's and may differ from the host's by an ulp.
 #include <algorithm>
 #include <cmath>
+#include <type_traits>
 
 #include "common.hpp"
 
@@ -69,7 +71,7 @@ struct PIns {
 struct PProg {
     int32_t npro, n;     // operations [0, npro) once per chunk, [npro, n) per plane
     int32_t out;         // the stored value's operand
-    int32_t m;           // the marched dim (nd - 1; 2 in 1D, of length 1)
+    int32_t m;           // the marched dim (nd - 1; in 1D x, 64 points at a time)
     double o[3], h[3], ih[3];
     Axes3 ax;            // FunctionAxis tables (p == nullptr: uniform dim)
     PIns op[kPMaxOps + 1];   // (one past the end is read ahead)
@@ -226,42 +228,56 @@ __device__ __forceinline__ void program_run(const PProg& P, int q0, int q1, Slot
     }
 }
 
-// One wave: 64 consecutive points of a plane (of a row where y is marched), a
-// chunk of planes of the marched dim, N planes at a time.  Lanes and planes
-// past the box evaluate its first or last indices and store nothing.  With 64
-// columns of one row a wave instead, 160 points took three waves: us at
-// 160x144x127 FP64 66 -> 53 (42 operations), 46 -> 42 (27), 36 -> 29 (11 with
-// loads); all three and their host side at 140x187x170 FP32 238 -> 187,
-// 191x187x189 FP64 271 -> 256 (160x144x127 waits for the host: 161 both).
-template <class T, int S, int N, bool HEAVY>
+// One wave: 64 consecutive points of a plane (of a row where y is marched; in
+// 1D, ROW, of the line), a chunk of planes of the marched dim (ROW: of runs of
+// 64 points), N at a time.  Lanes and planes past the box evaluate its first or
+// last indices and store nothing.  With 64 columns of one row a wave instead,
+// 160 points took three waves: us at 160x144x127 FP64 66 -> 53 (42 operations),
+// 46 -> 42 (27), 36 -> 29 (11 with loads); all three and their host side at
+// 140x187x170 FP32 238 -> 187, 191x187x189 FP64 271 -> 256 (160x144x127 waits
+// for the host: 161 both).
+template <class T, int S, int N, bool HEAVY, bool ROW>
 __global__ void __launch_bounds__(64) program_kernel(const PProg P, DF<T> dst, Box3 b, int nbx, int chunk) {
     const int t = line_id();
-    const int bx = t % nbx, bc = t / nbx;
+    const int bx = ROW ? 0 : t % nbx, bc = ROW ? t : t / nbx;
     const int m = P.m;
     // z marched: 64 consecutive points of a plane, counted along its rows; y
     // marched: of the row
-    int64_t i, j;
-    plane_index((int64_t)bx * 64 + threadIdx.x, b.len[0], m == 2 ? b.len[1] : 1, i, j);
-    const bool in = j < (m == 2 ? b.len[1] : 1);
-    i = in ? b.lo[0] + i : b.lo[0];
-    j = in ? b.lo[1] + j : b.lo[1];
-    const int64_t m0 = b.lo[m] + (int64_t)bc * chunk;
-    const int64_t hm = b.lo[m] + b.len[m], m1 = m0 + chunk < hm ? m0 + chunk : hm;
-    if (m0 >= hm) return;   // no chunk
-    const int64_t I[3] = {i, j, b.lo[2]};
+    int64_t i = b.lo[0] + threadIdx.x, j = b.lo[1];
+    bool in = true;
+    if constexpr (!ROW) {
+        plane_index((int64_t)bx * 64 + threadIdx.x, b.len[0], m == 2 ? b.len[1] : 1, i, j);
+        in = j < (m == 2 ? b.len[1] : 1);
+        i = in ? b.lo[0] + i : b.lo[0];
+        j = in ? b.lo[1] + j : b.lo[1];
+    }
+    const int64_t m0 = (ROW ? 0 : b.lo[m]) + (int64_t)bc * chunk;
+    const int64_t hm = ROW ? (b.len[0] + 63) / 64 : b.lo[m] + b.len[m], m1 = m0 + chunk < hm ? m0 + chunk : hm;
+    // (a block past the last chunk, m0 >= hm, marches no plane; its part per chunk loads no field)
+    const int64_t I[3] = {i, j, b.lo[2]}, last = b.lo[0] + b.len[0] - 1;   // (the line's last point)
     Slots<S> r[N];
     int64_t Im[N];
+    // the index along the marched dim at step p of the march
+    auto along = [&](int64_t p) -> int64_t {
+        if (!ROW) return p < m1 ? p : m1 - 1;
+        const int64_t x = i + 64 * p;
+        return x < last ? x : last;
+    };
 #pragma unroll
-    for (int u = 0; u < N; ++u) Im[u] = m0;
+    for (int u = 0; u < N; ++u) Im[u] = along(m0);
     program_run<S, N, HEAVY>(P, 0, P.npro, r, I, Im);
     for (int64_t p = m0; p < m1; p += N) {
 #pragma unroll
-        for (int u = 0; u < N; ++u) Im[u] = p + u < m1 ? p + u : m1 - 1;
+        for (int u = 0; u < N; ++u) Im[u] = along(p + u);
         program_run<S, N, HEAVY>(P, P.npro, P.n, r, I, Im);
 #pragma unroll
         for (int u = 0; u < N; ++u) {
             const double v = P.out >= 0 ? r[u].get(P.out) : P.k[-1 - P.out];
-            if (in && p + u < m1) put(m == 2 ? dst(i, j, p + u) : dst(i, p + u, 0), v);
+            if constexpr (ROW) {
+                if (p + u < m1 && i + 64 * (p + u) <= last) put(dst(Im[u], 0, 0), v);
+            } else {
+                if (in && p + u < m1) put(m == 2 ? dst(i, j, p + u) : dst(i, p + u, 0), v);
+            }
         }
     }
 }
@@ -425,32 +441,48 @@ static int plan_program(const chmy_pop_t* prog, int n, PProg* P, bool* heavy) {
 template <class T>
 static int program_launch(const PProg& P, const chmy_field_t* dst, const Box3& b, int slots, bool heavy,
                           hipStream_t st) {
-    const int64_t nbx = (b.len[0] * (P.m == 2 ? b.len[1] : 1) + 63) / 64, nm = b.len[P.m];
-    // planes per wave: fill whole rounds of the waves the chip holds (12 a CU
-    // at these kernels' registers); a wave also spends about two planes' time
-    // on the per-chunk operations.  160x144x127: 20 planes, one round
-    const int64_t room = 12 * (int64_t)cu_count();
-    int64_t chunk = 4, best = INT64_MAX;
-    for (int64_t c = 4; c <= 64; c += 4) {
-        const int64_t waves = nbx * ((nm + c - 1) / c), cost = (waves + room - 1) / room * (c + 2);
-        if (cost < best) {
-            best = cost;
-            chunk = c;
-        }
-    }
-    dim3 grd;
-    CHMY_TRY(line_grid(nbx * ((nm + chunk - 1) / chunk), 64, &grd));
-    const dim3 blk(64);
+    const bool row = P.m == 0;
+    const int64_t nbx = row ? 1 : (b.len[0] * (P.m == 2 ? b.len[1] : 1) + 63) / 64;
+    const int64_t nm = row ? (b.len[0] + 63) / 64 : b.len[P.m];
     const DF<T> d = view<T>(*dst);
-    const int ix = (int)nbx, ic = (int)chunk;
-    if (slots > 16)
-        hipLaunchKernelGGL((program_kernel<T, 0, 1, true>), grd, blk, (size_t)slots * 64 * sizeof(double), st, P, d, b, ix,
-                           ic);
-    else if (heavy) hipLaunchKernelGGL((program_kernel<T, 16, 1, true>), grd, blk, 0, st, P, d, b, ix, ic);
-    else if (slots > 8) hipLaunchKernelGGL((program_kernel<T, 16, 2, false>), grd, blk, 0, st, P, d, b, ix, ic);
-    else hipLaunchKernelGGL((program_kernel<T, 8, 4, false>), grd, blk, 0, st, P, d, b, ix, ic);
-    CHMY_HIP(hipGetLastError());
-    return 0;
+    auto go = [&](auto s, auto n, auto h, auto line) -> int {
+        constexpr int S = decltype(s)::value, N = decltype(n)::value;
+        constexpr bool HEAVY = decltype(h)::value, ROW = decltype(line)::value;
+        // planes per wave: fill whole rounds of the waves the chip holds (12 a CU
+        // at these kernels' registers); a wave also spends about two planes' time
+        // on the per-chunk operations.  160x144x127: 20 planes, one round.  On a
+        // line no operation is per chunk, so short chunks that balance: twice the
+        // runs that share the decoding (four times: 3-5% more below 10^6 points,
+        // whole rounds: 10-60% more at 2 10^6), one run with the file in LDS
+        int64_t chunk = S ? 2 * N : 1, best = INT64_MAX;
+        const int64_t room = 12 * (int64_t)cu_count();
+        for (int64_t c = 4; !ROW && c <= 64; c += 4) {
+            const int64_t waves = nbx * ((nm + c - 1) / c), cost = (waves + room - 1) / room * (c + 2);
+            if (cost < best) {
+                best = cost;
+                chunk = c;
+            }
+        }
+        dim3 grd;
+        CHMY_TRY(line_grid(nbx * ((nm + chunk - 1) / chunk), 64, &grd));
+        const size_t lds = S ? 0 : (size_t)slots * 64 * sizeof(double);
+        hipLaunchKernelGGL((program_kernel<T, S, N, HEAVY, ROW>), grd, dim3(64), lds, st, P, d, b, (int)nbx, (int)chunk);
+        CHMY_HIP(hipGetLastError());
+        return 0;
+    };
+    auto by_slots = [&](auto line) -> int {
+        using I0 = std::integral_constant<int, 0>;
+        using I1 = std::integral_constant<int, 1>;
+        using I2 = std::integral_constant<int, 2>;
+        using I4 = std::integral_constant<int, 4>;
+        using I8 = std::integral_constant<int, 8>;
+        using I16 = std::integral_constant<int, 16>;
+        if (slots > 16) return go(I0{}, I1{}, std::true_type{}, line);
+        if (heavy) return go(I16{}, std::conditional_t<decltype(line)::value, I2, I1>{}, std::true_type{}, line);
+        if (slots > 8) return go(I16{}, I2{}, std::false_type{}, line);
+        return go(I8{}, I4{}, std::false_type{}, line);
+    };
+    return row ? by_slots(std::true_type{}) : by_slots(std::false_type{});
 }
 
 }  // namespace chmy
@@ -482,7 +514,7 @@ int chmy_set_program(const chmy_grid_t* g, const chmy_field_t* dst, const chmy_b
     if (b.len[0] == 0 || b.len[1] == 0 || b.len[2] == 0) return 0;
     PProg P;
     std::memset(&P, 0, sizeof P);
-    P.m = g->nd == 1 ? 2 : g->nd - 1;
+    P.m = g->nd - 1;
     for (int d = 0; d < 3; ++d) {
         P.o[d] = d < g->nd ? g->origin[d] : 0.0;
         P.h[d] = d < g->nd ? g->spacing[d] : 0.0;

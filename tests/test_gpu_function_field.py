@@ -283,3 +283,38 @@ def test_program_register_files_and_plane_chunks(arch, dims, wide, sine):
     chmy.set_(f, func, g)
     want = host_values(ogrid(g), f, func, ())
     assert np.array_equal(f.interior().cpu().numpy(), want)
+
+
+@pytest.mark.parametrize("n", [1, 63, 64, 65, 255, 256, 257, 1000003])
+@pytest.mark.parametrize("dtype", [torch.float64, torch.float32, torch.bfloat16])
+def test_programs_on_lines(arch, n, dtype):
+    """1D, where a wave marches along the line 64 points at a time: lines that
+    end inside, at and past a run and a chunk of runs (several at 1000003),
+    each register file, with indices, coordinates and loads at offsets; in f64
+    on the host, then rounded once, so bitwise."""
+    g = chmy.UniformGrid(arch, origin=(-0.4,), extent=(1.7,), dims=(n,))
+    H = chmy.Field(arch, g, (Cc(),))
+    h = np.random.default_rng(n).uniform(-1.0, 1.0, H.data.shape)
+    chmy.set_storage(H, h)
+    ix = np.arange(1, n + 1)
+    for wide, sine in ((3, False), (12, False), (20, False), (3, True)):
+        def func(g_, l, i, H):
+            v = [H[i + k % 3 - 1] * (0.3 + k) + i for k in range(wide)]
+            s = v[0] * v[-1]
+            for k in range(1, wide):
+                s = s - v[k] * v[wide - 1 - k]
+            return 0.0 * np.sin(s) + s if sine else s
+        v = [h[ix + 1 + k % 3 - 1] * (0.3 + k) + ix for k in range(wide)]   # H[i] is storage i + 1
+        want = v[0] * v[-1]
+        for k in range(1, wide):
+            want = want - v[k] * v[wide - 1 - k]
+        f = chmy.Field(arch, g, (Cc(),), dtype)
+        f.data.fill_(7.0)
+        chmy.set_(f, func, g, discrete=True, parameters=(H,))
+        got = f.data.cpu()
+        assert torch.equal(got[2:-2], torch.from_numpy(want).float().to(dtype) if dtype == torch.bfloat16
+                           else torch.from_numpy(want).to(dtype)), (wide, sine)
+        assert bool((got[:2] == 7.0).all()) and bool((got[-2:] == 7.0).all())
+    f = chmy.Field(arch, g, (Vv(),))
+    chmy.set_(f, lambda x: x * x - 0.5, g)
+    assert np.array_equal(f.interior().cpu().numpy(), host_values(ogrid(g), f, lambda x: x * x - 0.5, ()))
