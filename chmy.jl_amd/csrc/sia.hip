@@ -763,12 +763,21 @@ __global__ void __launch_bounds__(NW * 64) sia_adj_kernel(SiaAdj<double> a, SiaS
 // with 48; 512^2: 4.86 and 4.68 for 300).  A single adjoint step's regions are
 // 16 rows with 24 for the step riding along: 3 blocks a CU hold them all at
 // 512^2 (with 16 and 16 rows a second round starts: 5.04).
+// A single forward step (every state kept, or recomputed for the adjoint) has a
+// ring of 2, so smaller regions waste little and a block's waves wait for
+// fewer others: 4 waves of 2 rows up to two blocks a CU, 8 of 2 up to one, then
+// the shapes of several steps.  40 steps with every state kept, n = 3 / 8, us,
+// a 256-thread tile a block -> 16 waves -> now: 64x64 162 / 193 -> 197 / 254 ->
+// 155 / 190, 250x230 162 / 198 -> 203 / 254 -> 157 / 189, 400x390 185 / 222 -> 203 /
+// 251 -> 167 / 197; 512x512 (unchanged) 211 / 249 -> 203 / 250.  (4 x 3 and 6 x 2:
+// 4-15% more up to 250x230, 8 x 1: 5% more at n = 3.)
 constexpr int kSiaMax = 5, kSiaMany = 3;          // forward steps per launch: one round, more
 constexpr int kNWF = 16, kRF1 = 2, kRF2 = 3;      // forward: waves, rows per wave
+constexpr int kNWS = 4, kNWT = 8, kRS = 2;        // a single forward step: waves up to two blocks a CU, up to one, rows
 constexpr int kNWA = 8, kRA = 2, kRR = 3;         // adjoint, and the steps riding along
 constexpr int kNWD = 8, kRD = 2;                  // the adaptive step (us for 24: 250x230 203, 400x390 243; 16 x 1: 206, 260)
 static_assert(kSiaMax <= kSiaSteps && kNWF * kRF1 > 4 * kSiaMax && 64 > 4 * kSiaMax && kNWA * kRA > 2 * kAdjRing &&
-                  kNWA * kRR > 4 && kNWD * kRD > 6,
+                  kNWA * kRR > 4 && kNWD * kRD > 6 && kNWS * kRS > 4,
               "a region owns at least one row and column");
 
 static int sia_regions(int64_t nx, int64_t ny, int rx, int ry, int rows, int* ntx) {
@@ -778,22 +787,27 @@ static int sia_regions(int64_t nx, int64_t ny, int rx, int ry, int rows, int* nt
 }
 
 // n = 3 (Glen's law as sia.jl uses it) takes the unrolled kernels
-template <int R>
+template <int NW, int R>
 static void launch_steps_r(hipStream_t st, const SiaStep<double>& f, const SiaDts& d, int64_t nx, int64_t ny) {
     int ntx;
-    const int nb = sia_regions(nx, ny, 2 * d.n, 2 * d.n, kNWF * R, &ntx);
-    const dim3 blk(64, kNWF);
-    if (f.s.n == 3) hipLaunchKernelGGL((sia_steps_kernel<3, kNWF, R>), dim3(nb), blk, 0, st, f, d, ntx, nx, ny);
-    else hipLaunchKernelGGL((sia_steps_kernel<0, kNWF, R>), dim3(nb), blk, 0, st, f, d, ntx, nx, ny);
+    const int nb = sia_regions(nx, ny, 2 * d.n, 2 * d.n, NW * R, &ntx);
+    const dim3 blk(64, NW);
+    if (f.s.n == 3) hipLaunchKernelGGL((sia_steps_kernel<3, NW, R>), dim3(nb), blk, 0, st, f, d, ntx, nx, ny);
+    else hipLaunchKernelGGL((sia_steps_kernel<0, NW, R>), dim3(nb), blk, 0, st, f, d, ntx, nx, ny);
 }
 
 static void launch_steps(hipStream_t st, const SiaStep<double>& f, const double* dts, int n, int64_t nx, int64_t ny) {
     SiaDts d{};
     d.n = n;
     for (int q = 0; q < n; ++q) d.dt[q] = dts[q];
-    int ntx;
-    if (sia_regions(nx, ny, 2 * n, 2 * n, kNWF * kRF1, &ntx) <= cu_count()) launch_steps_r<kRF1>(st, f, d, nx, ny);
-    else launch_steps_r<kRF2>(st, f, d, nx, ny);
+    auto fits = [&](int rows, int blocks) {
+        int ntx;
+        return sia_regions(nx, ny, 2 * n, 2 * n, rows, &ntx) <= blocks * cu_count();
+    };
+    if (n == 1 && fits(kNWS * kRS, 2)) launch_steps_r<kNWS, kRS>(st, f, d, nx, ny);
+    else if (n == 1 && fits(kNWT * kRS, 1)) launch_steps_r<kNWT, kRS>(st, f, d, nx, ny);
+    else if (fits(kNWF * kRF1, 1)) launch_steps_r<kNWF, kRF1>(st, f, d, nx, ny);
+    else launch_steps_r<kNWF, kRF2>(st, f, d, nx, ny);
 }
 
 template <bool MAXD>

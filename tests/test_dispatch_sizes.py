@@ -5,7 +5,7 @@ fails here."""
 import os
 import re
 
-from test_gpu_dispatch_shapes import ADJOINT_SIZES, FORWARD_SIZES, PASS_SIZES
+from test_gpu_dispatch_shapes import ADJOINT_SIZES, FORWARD_SIZES, PASS_SIZES, SINGLE_SIZES
 
 CSRC = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "chmy.jl_amd", "csrc")
 CUS, LANES = 256, 64
@@ -66,3 +66,17 @@ def test_forward_sizes():
         for n in sizes:
             one = regions(n, 2 * c["kSiaMax"], 2 * c["kSiaMax"], c["kNWF"] * c["kRF2"]) <= CUS
             assert (c["kSiaMax"] if one else c["kSiaMany"]) == want, n
+
+
+def test_single_step_sizes():
+    src = source("sia.hip")
+    c = constants(src)
+    body = src[src.index("static void launch_steps("):]
+    order = [(c[w], c[r], int(k)) for w, r, k in re.findall(r"if \((?:n == 1 && )?fits\((k\w+) \* (k\w+), (\d+)\)\)",
+                                                            body[:body.index("\n}")])]
+    last = (c["kNWF"], c["kRF2"])
+    assert [o[:2] for o in order] + [last] == list(SINGLE_SIZES)
+    for want, sizes in SINGLE_SIZES.items():
+        for n in sizes:
+            fit = [(w, r) for w, r, k in order if regions(n, 2, 2, w * r) <= k * CUS]
+            assert (fit + [last])[0] == want, n

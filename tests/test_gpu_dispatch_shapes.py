@@ -24,6 +24,9 @@ PASS_SIZES = {"Small2": [(49, 3), (101, 66)],
 ADJOINT_SIZES = {(8, 2): [(57, 11), (104, 52)], (12, 2): [(260, 180), (261, 181), (300, 200)], (16, 3): [(512, 437)]}
 # forward steps a launch may take
 FORWARD_SIZES = {5: [(250, 177)], 3: [(800, 520), (833, 541)]}
+# single forward steps: waves and rows of a region
+SINGLE_SIZES = {(4, 2): [(60, 4), (61, 5), (300, 196)], (8, 2): [(360, 372), (361, 373)], (16, 2): [(480, 476), (481, 477)],
+                (16, 3): [(840, 616), (841, 617)]}
 
 
 @pytest.fixture(scope="module")
@@ -84,3 +87,22 @@ def test_sia_gradient_over_shapes(arch, n, npow):
         S.reset(want[k])
         S._adjoint_step(S.H, dts[k], passes=5)
     assert torch.equal(S.lam.interior(), lam) and torch.equal(S.grad.interior(), grad)
+
+
+@pytest.mark.parametrize("npow", [3, 2])
+@pytest.mark.parametrize("n", sum(SINGLE_SIZES.values(), []))
+def test_sia_single_steps_over_shapes(arch, n, npow):
+    """A run that keeps every state, one step a launch, against the per-point
+    step and its Neumann batch, bitwise over the storage."""
+    g, og, H, hH, B, hB, A, hA = _setup(arch, n=n, seed=29)
+    S = SIA(arch, g, hB.arr, logA=np.log(hA.arr), As=0.5, npow=npow, mb=(0.5, 0.3, 0.25))
+    dt = 1e-2 * min(e / m for e, m in zip(g.extent, n)) ** 2
+    dts = [dt * (1 + 0.1 * k) for k in range(3)]
+    S.reset(hH.arr)
+    states = [S._field() for _ in range(4)]
+    states[0].data.copy_(S.H.data)
+    S.run(states, dts)
+    for k, d in enumerate(dts):
+        S.step(d)
+        S.H.swap(S.H2)
+        assert torch.equal(states[k + 1].data, S.H.data), k
