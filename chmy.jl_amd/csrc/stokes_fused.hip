@@ -1902,7 +1902,7 @@ int chmy_stokes_iterate(const chmy_grid_t* g, const chmy_field_t* V0, const chmy
     const chmy_field_t* T[2] = {tau0, tau1};
     const chmy_field_t* P[2] = {Pr0, Pr1};
     // free-slip batches run iterations in passes (the batch in-kernel between
-    // them), two in 3D and up to `most` in 2D; a pass writes the other set, as
+    // them), two in 3D and up to eight in 2D; a pass writes the other set, as
     // one iteration does, so the parity flips once per pass.  CHMY_ITER_SINGLE
     // keeps single iterations (CHMY_ITER_PAIRS, once the 3D opt-in, is accepted and ignored)
     const bool single = ((flags | flags_last) & CHMY_ITER_SINGLE) != 0;
@@ -1913,23 +1913,21 @@ int chmy_stokes_iterate(const chmy_grid_t* g, const chmy_field_t* V0, const chmy
     const bool tb2 = CHMY_FUSED_TB && !single && nd == 2 && free_slip_2d(g, bc_counts, bc_comp, bcs, &fs);
     const bool tb3 = !single && !(rhog && f_V) && nd == 3 && free_slip_3d(g, bc_counts, bc_comp, bcs, &fs3);
     const bool tb = tb2 || tb3;
-    const int most = tb2 ? multi2d_most(g) : 1;
     int p = *parity_inout;
     for (int it = 0; it < niter;) {
         const int fl = it == niter - 1 ? flags_last : flags;
         const int fl2 = it + 1 == niter - 1 ? flags_last : flags;
-        // 2D: a run of iterations of the same flags in passes of up to `most`, three
-        // or more each, evenly long (a remainder of one or two would take a launch
-        // that moves the state for itself)
+        // 2D: a run of iterations of the same flags
         const int run = flags == flags_last ? niter - it : it < niter - 1 ? niter - 1 - it : 1;
-        if (tb2 && run > 2 && !(fl & CHMY_ITER_RESIDUAL)) {
-            const int passes = (run + most - 1) / most, m = (run + passes - 1) / passes;
+        const bool fx = Pr0 && Pr0->dtype == CHMY_F32 && (fl & CHMY_ITER_EXACT);
+        const int m = tb2 && !(fl & CHMY_ITER_RESIDUAL) ? multi2d_next(g, fx, f_V != nullptr, run) : 0;
+        if (m > 0) {
             fs.iters = m;
             CHMY_TRY(stokes_iter_impl(g, Vs[p], T[p], P[p], Vs[1 - p], T[1 - p], P[1 - p], tau_old, eta, eta_ml, rhog,
                                       f_V, f_P, divV, r_V, fl, eta_s, eta_ve_s, G, dt, dtau_Pr, dtau_r, nudtau,
                                       stream, &fs, nullptr));
             it += m;
-            fs.pre = m < run;   // the rest of the run is passes: the next applies the batch
+            fs.pre = multi2d_next(g, fx, f_V != nullptr, run - m) > 0;   // another such pass follows: it applies the batch
             if (fs.pre) {
                 p = 1 - p;
                 continue;

@@ -38,9 +38,27 @@ static int shape2(int64_t nbx, int64_t nby) {
            : one_round<Large2>(nbx, nby) ? 3
                                          : 4;
 }
-int multi2d_most(const chmy_grid_t* g) {
-    const int k[5] = {Small2::KM, Flat2::KM, Mid2::KM, Large2::KM, Dense2::KM};
-    return k[shape2(g->n[0] + 2, g->n[1] + 2)];
+
+// A run of iterations is cut into evenly long passes of at most the shape's
+// iterations, three or more each (a remainder of one or two would take a launch
+// that moves the state for itself).  FP32 in the exact form on large grids takes
+// passes of five and two instead: there the two-iteration pass streams at its
+// best while the divisions and the ring, five deep however short the pass,
+// bound this one.  2047^2, variable eta, us per iteration: passes of 3 / 4 / 5 52 /
+// 49 / 46, of 2 48, single 69; 4000^2 (6 iterations in 3 + 3 against 2 + 2 + 2) 199
+// against 166.  The line: at 1400^2 two passes of 3 and three of 2 take the same;
+// with forcing, which a pass reads once for all its iterations, two of 4 and
+// four of 2 do at 2500^2 (three of 2 10% less than two of 3).
+int multi2d_next(const chmy_grid_t* g, bool f32_exact, bool forced, int run) {
+    const int64_t nbx = g->n[0] + 2, nby = g->n[1] + 2;
+    const int km[5] = {Small2::KM, Flat2::KM, Mid2::KM, Large2::KM, Dense2::KM};
+    const int shape = shape2(nbx, nby), most = km[shape];
+    if (run < 3) return 0;
+    const int64_t line = (forced ? 10 : 5) * (int64_t(1) << 19);
+    if (f32_exact && shape == 4 && nbx * nby >= line && run != 3)
+        return run >= 2 * most || (run >= most && run % 2) ? most : 0;
+    const int passes = (run + most - 1) / most;
+    return (run + passes - 1) / passes;
 }
 
 // Up to KM PT iterations of a tile on chip (build extension): the state is

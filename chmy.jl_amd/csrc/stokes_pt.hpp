@@ -175,10 +175,11 @@ struct FreeSlip2 {
     int32_t pre;     // the batch is still to be applied to the V the pass reads
 };
 
-// The most iterations of a 2D pass over this grid (stokes_multi2d.hip).
-int multi2d_most(const chmy_grid_t* g);
+// Iterations of the next 2D pass of a run (stokes_multi2d.hip); 0: none, the
+// run goes on in passes of two and single iterations.
+int multi2d_next(const chmy_grid_t* g, bool f32_exact, bool forced, int run);
 
-// fs.iters (at most multi2d_most) iterations in one launch; `a` holds everything but the tiling.
+// fs.iters (as multi2d_next gives them) iterations in one launch; `a` holds everything but the tiling.
 template <class T>
 void multi2d_launch(Fused2<T> a, const FreeSlip2& fs, bool fv, bool exact, bool bf, bool rg, hipStream_t s);
 

@@ -56,6 +56,22 @@ def test_passes_of_the_other_shapes_2d(arch, shape, dims, niter):
     _compare(a, b, f"{shape} dims {dims} niter {niter}")
 
 
+@pytest.mark.parametrize("dims,niter,forcing", [((1699, 1541), 4, None), ((1699, 1541), 6, None), ((1699, 1541), 7, None),
+                                                ((1699, 1541), 13, None), ((1699, 1541), 22, None), ((1690, 1540), 6, None),
+                                                ((1699, 1541), 6, "bf16"), ((2290, 2290), 8, "bf16"),
+                                                ((2290, 2290), 17, "bf16")])
+def test_fp32_exact_passes_of_five_and_two(arch, dims, niter, forcing):
+    """FP32, exact form, at and below the size from which runs are cut into
+    passes of five and two iterations: pairs only, a five and pairs, fives and
+    pairs (the batch is the next pass's before a five, a launch before a pair).
+    Bitwise; the random state overflows after 17 iterations, and a NaN counts as
+    a NaN (IEEE 754 leaves its sign open: Inf - Inf by the order of operands)."""
+    g = chmy.UniformGrid(arch, origin=(-0.5, -0.5), extent=(1.0, 1.3), dims=dims)
+    a, b = ([np.where(np.isnan(x), np.float32("nan"), x) for x in
+             _run(arch, g, np.float32, True, "field", forcing, GENERAL, niter, pairs, 43)] for pairs in (True, False))
+    _compare(a, b, f"dims {dims} niter {niter}")
+
+
 @pytest.mark.parametrize("npow", [3, 2])
 @pytest.mark.parametrize("n", sum(ADJOINT_SIZES.values(), []) + sum(FORWARD_SIZES.values(), []))
 def test_sia_gradient_over_shapes(arch, n, npow):
