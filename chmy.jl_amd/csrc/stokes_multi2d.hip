@@ -44,9 +44,9 @@ static int shape2(int64_t nbx, int64_t nby) {
 // that moves the state for itself).  FP32 in the exact form on large grids takes
 // passes of five and two instead: there the two-iteration pass streams at its
 // best while the divisions and the ring, five deep however short the pass,
-// bound this one.  2047^2, variable eta, us per iteration: passes of 3 / 4 / 5 52 /
-// 49 / 46, of 2 48, single 69; 4000^2 (6 iterations in 3 + 3 against 2 + 2 + 2) 199
-// against 166.  The line: at 1400^2 two passes of 3 and three of 2 take the same;
+// bound this one.  2047^2, variable eta, us per iteration: passes of 3 / 4 / 5 54 /
+// 49 / 47, of 2 48, single 71; 4000^2 (6 iterations in 3 + 3 against 2 + 2 + 2) 198
+// against 171 (and fives 174).  The line: at 1400^2 two passes of 3 and three of 2 take the same;
 // with forcing, which a pass reads once for all its iterations, two of 4 and
 // four of 2 do at 2500^2 (three of 2 10% less than two of 3).
 int multi2d_next(const chmy_grid_t* g, bool f32_exact, bool forced, int run) {
