@@ -103,8 +103,10 @@ class SIA:
         self._neumann(H_out)
 
     def run(self, states, dts):
-        """states[q] -> states[q+1] for the given Δt (one tiled launch per step,
-        Neumann batch included)."""
+        """states[q] -> states[q+1] for the given Δt, Neumann batch included, up
+        to five steps to a launch.  Afterwards each field holds the last of the
+        states that name it; a state whose field a later one reuses may not have
+        been written in between."""
         if len(states) < 2:
             return
         d = (C.c_double * (len(states) - 1))(*[float(x) for x in dts])

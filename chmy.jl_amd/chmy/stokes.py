@@ -184,8 +184,9 @@ class PTStokes:
     def iterate(self, niter, residual_last=False, pairs=True):
         """niter PT iterations in one native call (fused kernel + V batch,
         buffers alternating); (V, tau, Pr) hold the result afterwards.  With
-        the free-slip batch they run in pairs (one pass per two iterations,
-        bitwise the same results); pairs=False keeps single iterations."""
+        the free-slip batch they run in passes (two iterations each in 3D, up
+        to eight in 2D, bitwise the same results; in 2D the other set's V may
+        lack the batch); pairs=False keeps single iterations."""
         if niter <= 0:
             return
         g = self.grid

@@ -88,8 +88,8 @@ class StokesThermal:
         err = None
         if it == 1:
             # no thermal update: the iterations between checks run in one
-            # native call (in 2D two per pass), with the residual fields
-            # written by the last one
+            # native call (passes of two in 3D, of up to eight in 2D), with the
+            # residual fields written by the last one
             q = 0
             while q < niter:
                 k = min(ncheck - q % ncheck, niter - q)

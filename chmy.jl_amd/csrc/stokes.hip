@@ -5,9 +5,9 @@
 // with -ffp-contract=off so f64 results equal the CPU semantics bit for bit.
 // Both are bound by HBM (24 and 17 arrays a launch in 3D).  159x143x127 FP64,
 // 64 x 4 blocks with loads between stores -> flat blocks, each XCD a contiguous
-// run, every load before the first store, and divV and r_V (never read again
-// by the iteration) past the caches: stress 124 -> 109 us (5.1 TB/s), velocity
-// 100 -> 84 us (4.7 TB/s).
+// run (or runs of 32 blocks, flat_at), every load before the first store, and
+// divV and r_V (never read again by the iteration) past the caches: stress 124
+// -> 106 us (5.2 TB/s), velocity 100 -> 87 us (4.5 TB/s).
 #include "common.hpp"
 
 namespace chmy {

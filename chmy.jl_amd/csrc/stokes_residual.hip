@@ -13,10 +13,11 @@
 // attainable accuracy.
 // 207x191x175, bf16 forcing, us: residual 478 -> 374 with flat blocks, every
 // load before the first store and eta's form a template parameter (its
-// run-time test cut the loads into groups waited for one by one); 1.08 GB, 219
-// at the copy rate; the rest is about 60 loads a point at 4 waves a SIMD (106
-// VGPRs; held to 5 or 6 waves it takes 392 and 557).  Accumulate 316 -> 294
-// (1.38 GB, 4.7 TB/s).
+// run-time test cut the loads into groups waited for one by one), -> 344 with
+// the blocks in runs of 32 (flat_at); 1.08 GB, 219 at the copy rate; the rest
+// is about 60 loads a point at 4 waves a SIMD (106 VGPRs; held to 5 or 6 waves
+// it took 392 and 557 against 374).  Accumulate 316 -> 294 -> 275 (1.38 GB, 5.0
+// TB/s).
 #include <type_traits>
 
 #include "common.hpp"

@@ -202,8 +202,8 @@ int chmy_diffusion_step(const chmy_grid_t* grid, const chmy_box_t* box, const ch
  * *parity_inout into 1-p, then the C batch (bc_counts[2*dim+side-1] <= 1
  * entries, the conditions in bcs, as chmy_bc_batchset) on 1-p.  When every
  * (dim, side) has one rule with a scalar (or no) value, the batch runs inside
- * the step's launch, and in 2D and 3D all but the last two steps run several
- * to a launch (same bits in both buffers and q).  On return *parity_inout
+ * the step's launch, and all but the last step (2D) or the last two (3D) run
+ * several to a launch (same bits in both buffers and q).  On return *parity_inout
  * names the buffer holding C (build extension). */
 int chmy_diffusion_iterate(const chmy_grid_t* grid, const chmy_field_t* C0, const chmy_field_t* C1,
                            const chmy_field_t* q, const int32_t* bc_counts, const chmy_bc_t* bcs, double chi,
@@ -402,7 +402,7 @@ int chmy_sia_step(const chmy_grid_t* grid, const chmy_field_t* H, const chmy_fie
 /* Adjoint of chmy_sia_step + Neumann batch (build extension): given the step's
  * input state H (with halos) and lam_in = dJ/dH_out (cells), writes
  * lam_out = dJ/dH (cells) and adds dJ/dlog(A) into grad_logA (if A != NULL).
- * work == NULL: one tiled pass (LDS-staged D, mu, abar).  Otherwise five
+ * work == NULL: one launch over register columns.  Otherwise five
  * gather passes through 8 scratch fields {mu: Center, Dvx, gdx: (Vertex,Center),
  * Dvy, gdy: (Center,Vertex), ax, ay, HD: Center}; both give the same bits. */
 int chmy_sia_step_adjoint(const chmy_grid_t* grid, const chmy_field_t* H, const chmy_field_t* lam_in,
@@ -411,10 +411,12 @@ int chmy_sia_step_adjoint(const chmy_grid_t* grid, const chmy_field_t* H, const 
                           double dt, const chmy_field_t* work, void* stream);
 /* The time loop of sia.jl:71-96 with a given Δt sequence (the reference's
  * adaptive rule evaluated beforehand, or fixed): states[q] -> states[q+1]
- * by one step followed by the H Neumann batch (sia.jl:81), both in one tiled
- * launch, for q = 0..nstates-2.  Consecutive states must not share storage;
- * a plain run alternates two fields, a checkpointed run passes its
- * checkpoint fields at the stored steps (build extension: no copies). */
+ * by one step followed by the H Neumann batch (sia.jl:81), for q =
+ * 0..nstates-2, up to five steps to a launch.  Consecutive states must not
+ * share storage; a plain run alternates two fields, a checkpointed run passes
+ * its checkpoint fields at the stored steps (build extension: no copies).
+ * On return every field holds the last of the states that name it; a state
+ * whose storage a later one takes over may not have been written in between. */
 int chmy_sia_run(const chmy_grid_t* grid, const chmy_field_t* states, int nstates, const chmy_field_t* B,
                  const chmy_field_t* A, double As, int npow, double mb_a, double mb_b, double mb_c,
                  const double* dts, void* stream);
